@@ -383,7 +383,7 @@ int run_front(Pipeline& pl, const sr_surfels* g, int* radii, uint32_t capacity, 
 
 // Scatter into tile buckets, sort every tile, split into quadrant sub-lists,
 // then the acceptance pass over all (quadrant, chunk) work items.
-int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st, bool pairs = true) {
+int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st) {
   uint32_t* counters = pl.counters();
   char* bin = pl.bin;
   const BinLayout& bl = pl.bl;
@@ -425,7 +425,6 @@ int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st, bool p
   sa.work_count = counters + 2;
   sa.q_flag = (uint32_t*)(pl.img + pl.il.q_flag);
   SR_STAGE(3, dbg, st, "sort", launch_sort_tiles(sa, st));
-  if (!pairs) return SR_OK;  // the _part variant's blend walks the sub-lists itself
   AcceptArgs aa{};
   aa.vs = pl.vs;
   aa.ranges = sa.ranges;
@@ -445,6 +444,7 @@ int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st, bool p
   aa.q_flag = sa.q_flag;
   aa.frag_fill = (unsigned long long*)(counters + 4);
   aa.frag_cap = (uint32_t)bl.frag_cap;
+  aa.part = pl.part ? 1 : 0;
   const size_t items = work_capacity(pl.capacity, pl.vs.B, pl.il.T);
   SR_STAGE(8, dbg, st, "accept", launch_accept(aa, items, st));
   SR_STAGE(10, dbg, st, "pair_offsets", launch_pair_offsets(aa, st));
@@ -454,7 +454,8 @@ int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st, bool p
   return SR_OK;
 }
 
-int run_blend_fwd(Pipeline& pl, float* out_color, float* out_others, bool dbg, hipStream_t st) {
+int run_blend_fwd(Pipeline& pl, float* out_color, float* out_others, bool dbg, hipStream_t st,
+                  const float* sem = nullptr, float* out_sem = nullptr) {
   BlendArgs ba{};
   ba.vs = pl.vs;
   ba.ranges = (const uint32_t*)(pl.img + pl.il.ranges);
@@ -473,13 +474,29 @@ int run_blend_fwd(Pipeline& pl, float* out_color, float* out_others, bool dbg, h
   ba.n_contrib = (uint32_t*)(pl.img + pl.il.n_contrib);
   ba.out_color = out_color;
   ba.out_others = out_others;
+  ba.part = pl.part ? 1 : 0;
+  ba.S = pl.S;
+  ba.sem = sem;
+  ba.out_sem = out_sem;
   SR_STAGE(4, dbg, st, "blend_fwd", launch_blend_fwd(ba, st));
+  if (pl.S > 0) SR_STAGE(4, dbg, st, "blend_semantics", launch_blend_semantics(ba, st));
+  return SR_OK;
+}
+
+// The image state an empty binning leaves for the blend: no sub-list entry,
+// no pair, any order.
+int clear_lists(Pipeline& pl, bool dbg, hipStream_t st) {
+  const size_t nq = (size_t)pl.il.T * quads_per_tile(pl.vs.B);
+  SR_STAGE(3, dbg, st, "clear", launch_fill_u32((uint32_t*)(pl.img + pl.il.sub_count), 0u, nq, st));
+  SR_STAGE(3, dbg, st, "clear", launch_fill_u32((uint32_t*)(pl.img + pl.il.q_flag), 0u, nq, st));
+  SR_STAGE(3, dbg, st, "clear", launch_fill_u32((uint32_t*)(pl.img + pl.il.lane_range), 0u, nq * 128, st));
+  SR_STAGE(3, dbg, st, "clear", launch_iota_u32((uint32_t*)(pl.img + pl.il.q_order), nq, st));
   return SR_OK;
 }
 
 int run_backward(Pipeline& pl, const sr_surfels* g, const int* radii, const float* dL_dcolor,
                  const float* dL_dothers, const RecordGrads& rg, sr_grads* gr, bool blend, bool dbg,
-                 hipStream_t st) {
+                 hipStream_t st, const float* dL_dsem = nullptr, float* dL_dsemantics = nullptr) {
   if (blend) {
     BlendBwdArgs ba{};
     ba.vs = pl.vs;
@@ -505,6 +522,10 @@ int run_backward(Pipeline& pl, const sr_surfels* g, const int* radii, const floa
     ba.pos_quads = (const uint16_t*)(pl.bin + pl.bl.pos_quads);
     ba.part = (float*)(pl.bin + pl.bl.part);
     ba.part_nz = (uint8_t*)(pl.bin + pl.bl.part_nz);
+    ba.is_part = pl.part ? 1 : 0;
+    ba.S = pl.S;
+    ba.dL_dsem = dL_dsem;
+    ba.sem_part = (float*)(pl.bin + pl.bl.sem_part);
     SR_STAGE(6, dbg, st, "blend_bwd", launch_blend_bwd(ba, st));
     SR_STAGE(9, dbg, st, "blend_bwd_grad",
              launch_blend_bwd_grad(ba, work_capacity(pl.capacity, pl.vs.B, pl.il.T), st));
@@ -541,7 +562,10 @@ int run_backward(Pipeline& pl, const sr_surfels* g, const int* radii, const floa
   pb.dL_dmean3D = gr->dL_dmeans3D;
   pb.dL_dscales = gr->dL_dscales;
   pb.dL_drots = gr->dL_drotations;
-  SR_STAGE(7, dbg, st, "preprocess_bwd", launch_preprocess_bwd(pb, st));
+  pb.S = pl.S;
+  pb.sem_part = blend ? (const float*)(pl.bin + pl.bl.sem_part) : nullptr;
+  pb.dL_dsem = dL_dsemantics;
+  SR_STAGE(7, dbg, st, "preprocess_bwd", pl.part ? launch_part_preprocess_bwd(pb, st) : launch_preprocess_bwd(pb, st));
   return SR_OK;
 }
 
@@ -627,13 +651,13 @@ size_t sr_state_offset(const char* name, int P, int W, int H, int tile, int L) {
   return (size_t)-1;
 }
 
-int sr_forward(const sr_settings* s, const sr_surfels* g, sr_alloc_fn alloc, void* ctx, float* out_color,
-               float* out_others, int* radii, int* num_rendered, sr_stream_t stream_) {
-  hipStream_t st = (hipStream_t)stream_;
-  int rc = validate(s, g);
-  if (rc != SR_OK) return rc;
-  if (!alloc || !out_color || !out_others || !num_rendered) return fail(SR_ERR_INVALID, "NULL output");
-  if (g->P > 0 && (!radii || !g->opacities)) return fail(SR_ERR_INVALID, "radii and opacities must not be NULL");
+namespace {
+// Forward of one view, either variant (part: S semantic channels, 8 aux
+// channels); the entry points have checked their arguments.
+int forward_view(const sr_settings* s, const sr_surfels* g, bool part, int S, const float* semantics,
+                 sr_alloc_fn alloc, void* ctx, float* out_color, float* out_semantic, float* out_others, int* radii,
+                 int* num_rendered, hipStream_t st) {
+  int rc;
   const int P = g->P, W = s->image_width, H = s->image_height, B = s->tile;
   const bool dbg = s->debug != 0;
   const int cap = s->capacity;
@@ -643,7 +667,8 @@ int sr_forward(const sr_settings* s, const sr_surfels* g, sr_alloc_fn alloc, voi
     // The reference glue skips the rasteriser for P == 0 and returns its
     // zero-filled outputs (rasterize_points.cu:85-87, 99).
     SR_STAGE(4, dbg, st, "clear", launch_fill_f32(out_color, 0.0f, 3 * (size_t)W * H, st));
-    SR_STAGE(4, dbg, st, "clear", launch_fill_f32(out_others, 0.0f, 7 * (size_t)W * H, st));
+    SR_STAGE(4, dbg, st, "clear", launch_fill_f32(out_others, 0.0f, (part ? 8 : 7) * (size_t)W * H, st));
+    if (S > 0) SR_STAGE(4, dbg, st, "clear", launch_fill_f32(out_semantic, 0.0f, (size_t)S * W * H, st));
     return SR_OK;
   }
   const ViewSet vs = single_view(W, H, B, s->tanfovx, s->tanfovy);
@@ -657,6 +682,8 @@ int sr_forward(const sr_settings* s, const sr_surfels* g, sr_alloc_fn alloc, voi
   pl.P = P;
   pl.s_D = s->sh_degree;
   pl.prefiltered = s->prefiltered;
+  pl.part = part;
+  pl.S = S;
   pl.mod = s->scale_modifier;
   pl.pair_store = s->pair_store;
   pl.pair_capacity = s->pair_capacity;
@@ -676,7 +703,7 @@ int sr_forward(const sr_settings* s, const sr_surfels* g, sr_alloc_fn alloc, voi
     // exceed it.  The instance count is copied back right after the scan
     // and waited for only once the rest is enqueued, by when it has long
     // arrived, so the stream never drains mid-forward.
-    pl.bl = bin_layout(cap, B, il.T, s->pair_store, s->pair_capacity, 0, s->slot_capacity);
+    pl.bl = bin_layout(cap, B, il.T, s->pair_store, s->pair_capacity, S, s->slot_capacity);
     pl.bin = (char*)alloc(ctx, pl.bl.total, 1);
     if (!pl.bin) return fail(SR_ERR_ALLOC, "allocation callback failed");
     pl.capacity = cap;
@@ -687,7 +714,7 @@ int sr_forward(const sr_settings* s, const sr_surfels* g, sr_alloc_fn alloc, voi
     if (!counted) return fail(SR_ERR_HIP, "hipEventCreate failed");
     SR_HIP(hipEventRecord(counted, st));
     rc = run_binning(pl, radii, dbg, st);
-    if (rc == SR_OK) rc = run_blend_fwd(pl, out_color, out_others, dbg, st);
+    if (rc == SR_OK) rc = run_blend_fwd(pl, out_color, out_others, dbg, st, semantics, out_semantic);
     if (rc == SR_OK) rc = post_pair_count(pl, st);
     SR_HIP(hipEventSynchronize(counted));
     if (rc != SR_OK) return rc;
@@ -710,36 +737,40 @@ int sr_forward(const sr_settings* s, const sr_surfels* g, sr_alloc_fn alloc, voi
   *num_rendered = L;
   // the slots the forward needs, exactly (the slot region is the layout's
   // last, so the backward locates everything without this count)
-  const int S = (int)(host[8] > 0u ? host[8] : 1u);
-  pl.bl = bin_layout(L, B, il.T, s->pair_store, s->pair_capacity, 0, S);
+  const int slots = (int)(host[8] > 0u ? host[8] : 1u);
+  pl.bl = bin_layout(L, B, il.T, s->pair_store, s->pair_capacity, S, slots);
   pl.bin = (char*)alloc(ctx, pl.bl.total, 1);
   if (!pl.bin) return fail(SR_ERR_ALLOC, "allocation callback failed");
   pl.capacity = L;
   if (L > 0) {
     rc = run_binning(pl, radii, dbg, st);
     if (rc != SR_OK) return rc;
-    rc = run_blend_fwd(pl, out_color, out_others, dbg, st);
+    rc = run_blend_fwd(pl, out_color, out_others, dbg, st, semantics, out_semantic);
     if (rc != SR_OK) return rc;
     return post_pair_count(pl, st);
-  } else {
-    SR_STAGE(3, dbg, st, "clear",
-             launch_fill_u32((uint32_t*)(img + il.sub_count), 0u, (size_t)il.T * quads_per_tile(B), st));
-    SR_STAGE(3, dbg, st, "clear",
-             launch_fill_u32((uint32_t*)(img + il.q_flag), 0u, (size_t)il.T * quads_per_tile(B), st));
-    SR_STAGE(3, dbg, st, "clear",
-             launch_fill_u32((uint32_t*)(img + il.lane_range), 0u, (size_t)il.T * quads_per_tile(B) * 128, st));
-    SR_STAGE(3, dbg, st, "clear", launch_iota_u32((uint32_t*)(img + il.q_order), (size_t)il.T * quads_per_tile(B), st));
   }
-  return run_blend_fwd(pl, out_color, out_others, dbg, st);
+  rc = clear_lists(pl, dbg, st);
+  if (rc != SR_OK) return rc;
+  return run_blend_fwd(pl, out_color, out_others, dbg, st, semantics, out_semantic);
 }
+}  // namespace
 
-int sr_backward(const sr_settings* s, const sr_surfels* g, int R, const int* radii, void* geom_buf,
-                const void* bin_buf, const void* img_buf, const float* dL_dcolor, const float* dL_dothers,
-                sr_grads* gr, sr_stream_t stream_) {
-  hipStream_t st = (hipStream_t)stream_;
+int sr_forward(const sr_settings* s, const sr_surfels* g, sr_alloc_fn alloc, void* ctx, float* out_color,
+               float* out_others, int* radii, int* num_rendered, sr_stream_t stream_) {
   int rc = validate(s, g);
   if (rc != SR_OK) return rc;
-  if (!gr || !dL_dcolor || !dL_dothers) return fail(SR_ERR_INVALID, "NULL gradient argument");
+  if (!alloc || !out_color || !out_others || !num_rendered) return fail(SR_ERR_INVALID, "NULL output");
+  if (g->P > 0 && (!radii || !g->opacities)) return fail(SR_ERR_INVALID, "radii and opacities must not be NULL");
+  return forward_view(s, g, false, 0, nullptr, alloc, ctx, out_color, nullptr, out_others, radii, num_rendered,
+                      (hipStream_t)stream_);
+}
+
+namespace {
+// Backward of one view, either variant.
+int backward_view(const sr_settings* s, const sr_surfels* g, bool part, int S, int R, const int* radii,
+                  void* geom_buf, const void* bin_buf, const void* img_buf, const float* dL_dcolor,
+                  const float* dL_dsemantic, const float* dL_dothers, sr_grads* gr, float* dL_dsemantics,
+                  hipStream_t st) {
   const int P = g->P, W = s->image_width, H = s->image_height, B = s->tile;
   if (P == 0) return SR_OK;
   if (!geom_buf || !img_buf || !radii) return fail(SR_ERR_INVALID, "forward state missing");
@@ -751,6 +782,8 @@ int sr_backward(const sr_settings* s, const sr_surfels* g, int R, const int* rad
   Pipeline pl{};
   pl.vs = single_view(W, H, B, s->tanfovx, s->tanfovy);
   pl.P = P;
+  pl.part = part;
+  pl.S = S;
   pl.s_D = s->sh_degree;
   pl.vm = s->viewmatrix;
   pl.pm = s->projmatrix;
@@ -761,7 +794,7 @@ int sr_backward(const sr_settings* s, const sr_surfels* g, int R, const int* rad
   // the binning arrays are laid out for the forward's capacity (R when 0)
   const int cap = s->capacity > 0 ? s->capacity : R;
   if (cap < R) return fail(SR_ERR_INVALID, "capacity %d below num_rendered %d", s->capacity, R);
-  pl.bl = bin_layout(cap, B, pl.il.T, s->pair_store, s->pair_capacity);
+  pl.bl = bin_layout(cap, B, pl.il.T, s->pair_store, s->pair_capacity, S);
   pl.geom = (char*)geom_buf;
   pl.img = (char*)img_buf;
   pl.bin = (char*)bin_buf;
@@ -769,28 +802,27 @@ int sr_backward(const sr_settings* s, const sr_surfels* g, int R, const int* rad
   // With one view the per-record gradient arrays are the outputs themselves;
   // the backward writes every output once, so nothing is cleared first.
   RecordGrads rg{gr->dL_dtransMat, gr->dL_dmeans2D, gr->dL_dopacity, gr->dL_dcolors};
-  return run_backward(pl, g, radii, dL_dcolor, dL_dothers, rg, gr, R > 0 && bin_buf != nullptr, dbg, st);
+  return run_backward(pl, g, radii, dL_dcolor, dL_dothers, rg, gr, R > 0 && bin_buf != nullptr, dbg, st,
+                      dL_dsemantic, dL_dsemantics);
+}
+}  // namespace
+
+int sr_backward(const sr_settings* s, const sr_surfels* g, int R, const int* radii, void* geom_buf,
+                const void* bin_buf, const void* img_buf, const float* dL_dcolor, const float* dL_dothers,
+                sr_grads* gr, sr_stream_t stream_) {
+  int rc = validate(s, g);
+  if (rc != SR_OK) return rc;
+  if (!gr || !dL_dcolor || !dL_dothers) return fail(SR_ERR_INVALID, "NULL gradient argument");
+  return backward_view(s, g, false, 0, R, radii, geom_buf, bin_buf, img_buf, dL_dcolor, nullptr, dL_dothers, gr,
+                       nullptr, (hipStream_t)stream_);
 }
 
 // ---- the _part variant -----------------------------------------------------
 namespace {
-PartArgs part_args(const Pipeline& pl, const float* sem) {
-  PartArgs pa{};
-  pa.vs = pl.vs;
-  pa.S = pl.S;
-  pa.ranges = (const uint32_t*)(pl.img + pl.il.ranges);
-  pa.sub = (const uint2*)(pl.bin + pl.bl.sub);
-  pa.sub_count = (const uint32_t*)(pl.img + pl.il.sub_count);
-  pa.rec = (const float4*)(pl.geom + pl.gl.rec);
-  pa.sem = sem;
-  pa.bg = pl.bg;
-  return pa;
-}
-
 int validate_part(const sr_settings* s, const sr_surfels* g, int S, const float* semantics) {
   int rc = validate(s, g);
   if (rc != SR_OK) return rc;
-  if (S < 0 || S > 16) return fail(SR_ERR_INVALID, "semantic channels must be in [0, 16] (got %d)", S);
+  if (S < 0 || S > kMaxSem) return fail(SR_ERR_INVALID, "semantic channels must be in [0, 16] (got %d)", S);
   if (g->P > 0 && S > 0 && !semantics) return fail(SR_ERR_INVALID, "semantics must not be NULL");
   return SR_OK;
 }
@@ -799,153 +831,25 @@ int validate_part(const sr_settings* s, const sr_surfels* g, int S, const float*
 int sr_forward_part(const sr_settings* s, const sr_surfels* g, int S, const float* semantics, sr_alloc_fn alloc,
                     void* ctx, float* out_color, float* out_semantic, float* out_others, int* radii,
                     int* num_rendered, sr_stream_t stream_) {
-  hipStream_t st = (hipStream_t)stream_;
   int rc = validate_part(s, g, S, semantics);
   if (rc != SR_OK) return rc;
   if (!alloc || !out_color || !out_others || !num_rendered || (S > 0 && !out_semantic))
     return fail(SR_ERR_INVALID, "NULL output");
   if (g->P > 0 && (!radii || !g->opacities)) return fail(SR_ERR_INVALID, "radii and opacities must not be NULL");
-  const int P = g->P, W = s->image_width, H = s->image_height, B = s->tile;
-  const bool dbg = s->debug != 0;
-  *num_rendered = 0;
-  if (P == 0) {
-    SR_STAGE(4, dbg, st, "clear", launch_fill_f32(out_color, 0.0f, 3 * (size_t)W * H, st));
-    SR_STAGE(4, dbg, st, "clear", launch_fill_f32(out_others, 0.0f, 8 * (size_t)W * H, st));
-    if (S > 0) SR_STAGE(4, dbg, st, "clear", launch_fill_f32(out_semantic, 0.0f, (size_t)S * W * H, st));
-    return SR_OK;
-  }
-  Pipeline pl{};
-  pl.vs = single_view(W, H, B, s->tanfovx, s->tanfovy);
-  pl.P = P;
-  pl.s_D = s->sh_degree;
-  pl.prefiltered = s->prefiltered;
-  pl.mod = s->scale_modifier;
-  pl.part = true;
-  pl.S = S;
-  pl.vm = s->viewmatrix;
-  pl.pm = s->projmatrix;
-  pl.campos = s->campos;
-  pl.bg = s->bg;
-  pl.gl = geom_layout((size_t)P);
-  pl.il = image_layout(pl.vs);
-  pl.geom = (char*)alloc(ctx, pl.gl.total, 0);
-  pl.img = (char*)alloc(ctx, pl.il.total, 2);
-  if (!pl.geom || !pl.img) return fail(SR_ERR_ALLOC, "allocation callback failed");
-  uint32_t* host = pinned_counters();
-  if (!host) return fail(SR_ERR_HIP, "hipHostMalloc failed");
-  rc = run_front(pl, g, radii, 0xFFFFFFFFu, 0xFFFFFFFFu, dbg, st);
-  if (rc != SR_OK) return rc;
-  SR_HIP(hipMemcpyAsync(host, pl.counters(), 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  SR_HIP(hipStreamSynchronize(st));
-  if (host[1] & kErrPrefiltered)
-    return fail(SR_ERR_PREFILTERED, "Point is filtered although prefiltered is set. This shouldn't happen!");
-  const int L = (int)host[0];
-  *num_rendered = L;
-  pl.bl = bin_layout(L, B, pl.il.T, 0, 1, S);
-  pl.bin = (char*)alloc(ctx, pl.bl.total, 1);
-  if (!pl.bin) return fail(SR_ERR_ALLOC, "allocation callback failed");
-  pl.capacity = L;
-  if (L > 0) {
-    rc = run_binning(pl, radii, dbg, st, false);
-    if (rc != SR_OK) return rc;
-  } else {
-    SR_STAGE(3, dbg, st, "clear",
-             launch_fill_u32((uint32_t*)(pl.img + pl.il.sub_count), 0u, (size_t)pl.il.T * quads_per_tile(B), st));
-  }
-  PartArgs pa = part_args(pl, semantics);
-  pa.final_T = (float*)(pl.img + pl.il.final_T);
-  pa.n_contrib = (uint32_t*)(pl.img + pl.il.n_contrib);
-  pa.out_color = out_color;
-  pa.out_sem = out_semantic;
-  pa.out_others = out_others;
-  SR_STAGE(4, dbg, st, "blend_fwd", launch_part_blend_fwd(pa, st));
-  return SR_OK;
+  return forward_view(s, g, true, S, semantics, alloc, ctx, out_color, out_semantic, out_others, radii, num_rendered,
+                      (hipStream_t)stream_);
 }
 
 int sr_backward_part(const sr_settings* s, const sr_surfels* g, int S, const float* semantics, int R,
                      const int* radii, void* geom_buf, const void* bin_buf, const void* img_buf,
                      const float* dL_dcolor, const float* dL_dsemantic, const float* dL_dothers, sr_grads* gr,
                      float* dL_dsemantics, sr_stream_t stream_) {
-  hipStream_t st = (hipStream_t)stream_;
   int rc = validate_part(s, g, S, semantics);
   if (rc != SR_OK) return rc;
   if (!gr || !dL_dcolor || !dL_dothers || (S > 0 && (!dL_dsemantic || !dL_dsemantics)))
     return fail(SR_ERR_INVALID, "NULL gradient argument");
-  const int P = g->P, W = s->image_width, H = s->image_height, B = s->tile;
-  if (P == 0) return SR_OK;
-  if (!geom_buf || !img_buf || !radii) return fail(SR_ERR_INVALID, "forward state missing");
-  if (R < 0) return fail(SR_ERR_INVALID, "num_rendered must be >= 0");
-  if (!gr->dL_dmeans2D || !gr->dL_dcolors || !gr->dL_dopacity || !gr->dL_dmeans3D || !gr->dL_dtransMat ||
-      !gr->dL_dscales || !gr->dL_drotations || (g->shs && !gr->dL_dsh))
-    return fail(SR_ERR_INVALID, "gradient output missing");
-  const bool dbg = s->debug != 0;
-  Pipeline pl{};
-  pl.vs = single_view(W, H, B, s->tanfovx, s->tanfovy);
-  pl.P = P;
-  pl.s_D = s->sh_degree;
-  pl.part = true;
-  pl.S = S;
-  pl.vm = s->viewmatrix;
-  pl.pm = s->projmatrix;
-  pl.campos = s->campos;
-  pl.bg = s->bg;
-  pl.gl = geom_layout((size_t)P);
-  pl.il = image_layout(pl.vs);
-  pl.bl = bin_layout(R, B, pl.il.T, 0, 1, S);
-  pl.geom = (char*)geom_buf;
-  pl.img = (char*)img_buf;
-  pl.bin = (char*)bin_buf;
-  pl.capacity = R;
-  const bool blend = R > 0 && bin_buf != nullptr;
-  if (blend) {
-    PartArgs pa = part_args(pl, semantics);
-    pa.final_T_in = (const float*)(pl.img + pl.il.final_T);
-    pa.n_contrib_in = (const uint32_t*)(pl.img + pl.il.n_contrib);
-    pa.dL_dpix = dL_dcolor;
-    pa.dL_dsem = dL_dsemantic;
-    pa.dL_dothers = dL_dothers;
-    pa.pos_slot = (const uint32_t*)(pl.bin + pl.bl.pos_slot);
-    pa.pos_quads = (const uint16_t*)(pl.bin + pl.bl.pos_quads);
-    pa.part = (float*)(pl.bin + pl.bl.part);
-    pa.sem_part = (float*)(pl.bin + pl.bl.sem_part);
-    pa.part_nz = (uint8_t*)(pl.bin + pl.bl.part_nz);
-    SR_STAGE(6, dbg, st, "blend_bwd", launch_part_blend_bwd(pa, st));
-  }
-  PreprocessBwdArgs pb{};
-  pb.vs = pl.vs;
-  pb.P = P;
-  pb.D = pl.s_D;
-  pb.M = g->M;
-  pb.counters = pl.counters();
-  pb.tiles = (const uint32_t*)(pl.geom + pl.gl.tiles);
-  pb.roff = (const uint32_t*)(pl.geom + pl.gl.roff);
-  pb.rslot = (const uint2*)(pl.geom + pl.gl.rslot);
-  pb.part = blend ? (const float*)(pl.bin + pl.bl.part) : nullptr;
-  pb.part_nz = blend ? (const uint8_t*)(pl.bin + pl.bl.part_nz) : nullptr;
-  pb.sem_part = blend ? (const float*)(pl.bin + pl.bl.sem_part) : nullptr;
-  pb.S = S;
-  pb.means3D = g->means3D;
-  pb.scales = g->scales;
-  pb.rots = g->rotations;
-  pb.shs = g->shs;
-  pb.tprec = g->transMat_precomp;
-  pb.rec = (const float4*)(pl.geom + pl.gl.rec);
-  pb.radii = radii;
-  pb.clamped = (const uint8_t*)(pl.geom + pl.gl.clamped);
-  pb.vm = pl.vm;
-  pb.pm = pl.pm;
-  pb.campos = pl.campos;
-  pb.dL_dtransMat = gr->dL_dtransMat;
-  pb.dL_dcolors = gr->dL_dcolors;
-  pb.dL_dopacity = gr->dL_dopacity;
-  pb.dL_dsh = gr->dL_dsh;
-  pb.dL_dmean2D = gr->dL_dmeans2D;
-  pb.dL_dmean3D = gr->dL_dmeans3D;
-  pb.dL_dscales = gr->dL_dscales;
-  pb.dL_drots = gr->dL_drotations;
-  pb.dL_dsem = dL_dsemantics;
-  SR_STAGE(7, dbg, st, "preprocess_bwd", launch_part_preprocess_bwd(pb, st));
-  return SR_OK;
+  return backward_view(s, g, true, S, R, radii, geom_buf, bin_buf, img_buf, dL_dcolor, dL_dsemantic, dL_dothers, gr,
+                       dL_dsemantics, (hipStream_t)stream_);
 }
 
 size_t sr_batch_workspace_bytes(const sr_views* v, int P, int capacity) {

@@ -47,10 +47,11 @@ static_assert(kGradGroup >= 1 && 64 % kGradGroup == 0, "groups tile the 64 pixel
 // tile-list position pos of quadrant q as five float4 in its slot.  Every
 // entry of every sub-list sets its flag exactly once per backward and
 // stores its sums when any is non-zero, so neither buffer needs clearing.
+// (also: some pixel has a semantic gradient for the slot, _part variant).
 template <class G>
-SR_DEV void store_part(const BlendBwdArgs& a, uint32_t pos, int q, G g) {
+SR_DEV void store_part(const BlendBwdArgs& a, uint32_t pos, int q, G g, bool also = false) {
   const size_t slot = slot_of(a.pos_slot, a.pos_quads, pos, q);
-  bool nz = false;
+  bool nz = also;
 #pragma unroll
   for (int k = 0; k < 18; ++k) nz |= g(k) != 0.0f;
   a.part_nz[slot] = nz ? 1 : 0;  // most entries blend no pixel of the quadrant: only a flag
@@ -70,8 +71,10 @@ struct PixelBwd {
   int median_contributor;
   float dLp0, dLp1, dLp2, dLn0, dLn1, dLn2;
   float dL_ddepth, dL_daccum, dL_dreg, dL_dmedian;
+  float dL_dmaxw;  // _part: median weight's
 };
 
+template <bool kPart>
 SR_DEV PixelBwd pixel_bwd(const BlendBwdArgs& a, const ViewInfo& vi, bool inside, uint32_t pxi, uint32_t pyi) {
   PixelBwd p{};
   const size_t HW = (size_t)vi.H * vi.W, pid = (size_t)vi.W * pyi + pxi, pb = vi.pix_base;
@@ -79,7 +82,7 @@ SR_DEV PixelBwd pixel_bwd(const BlendBwdArgs& a, const ViewInfo& vi, bool inside
     const float* final_T = a.final_T + 3 * pb;
     const uint32_t* n_contrib = a.n_contrib + 2 * pb;
     const float* dL_dpix = a.dL_dpix + 3 * pb;
-    const float* dL_dothers = a.dL_dothers + 7 * pb;
+    const float* dL_dothers = a.dL_dothers + (kPart ? 8 : 7) * pb;
     p.T_final = final_T[pid];
     p.final_D = final_T[pid + HW];
     p.final_D2 = final_T[pid + 2 * HW];
@@ -95,6 +98,7 @@ SR_DEV PixelBwd pixel_bwd(const BlendBwdArgs& a, const ViewInfo& vi, bool inside
     p.dLn2 = dL_dothers[4 * HW + pid];
     p.dL_dmedian = dL_dothers[5 * HW + pid];
     p.dL_dreg = dL_dothers[6 * HW + pid];
+    if (kPart) p.dL_dmaxw = dL_dothers[7 * HW + pid];
   }
   p.final_A = 1.0f - p.T_final;
   float bg_dot = 0.0f;
@@ -119,6 +123,7 @@ struct ChainBwd {
   float last_dL_dT = 0.0f, last_alpha = 0.0f;
   // nc = (normal.xyz, r); m_d, m2 = m_d * m_d, dmd_dd = distortion weight,
   // its square and its derivative
+  template <bool kPart>
   SR_DEV float4 step(const PixelBwd& p, float alpha, float c_d, float m_d, float m2, float dmd_dd,
                      uint32_t contributor, const float4& nc, float g, float bl) {
     T = T / (1.0f - alpha);
@@ -134,7 +139,10 @@ struct ChainBwd {
     last_c2 = bl;
     dL_dalpha += (bl - acc_r2) * p.dLp2;
     float dL_dz = 0.0f, dL_dweight = 0.0f;
-    if ((int)contributor == p.median_contributor - 1) dL_dz += p.dL_dmedian;
+    if ((int)contributor == p.median_contributor - 1) {
+      dL_dz += p.dL_dmedian;
+      if (kPart) dL_dweight += p.dL_dmaxw;
+    }
     dL_dweight += ((p.final_D2 + m2 * p.final_A) - (2.0f * m_d) * p.final_D) * p.dL_dreg;
     dL_dalpha += dL_dweight - last_dL_dT;
     last_dL_dT = dL_dweight * alpha + (1.0f - alpha) * last_dL_dT;
@@ -160,31 +168,6 @@ struct ChainBwd {
     dL_dz += (alpha * T) * p.dL_ddepth;
     return make_float4(w, dL_dalpha, dL_dz, 0.0f);
   }
-  // The state updates of step() alone, with the same operations in the same
-  // order (so a chain resumed from a saved state continues bit for bit).
-  SR_DEV void advance(const PixelBwd& p, float alpha, float c_d, float m_d, float m2, const float4& nc, float g,
-                      float bl) {
-    T = T / (1.0f - alpha);
-    acc_r0 = last_alpha * last_c0 + (1.0f - last_alpha) * acc_r0;
-    last_c0 = nc.w;
-    acc_r1 = last_alpha * last_c1 + (1.0f - last_alpha) * acc_r1;
-    last_c1 = g;
-    acc_r2 = last_alpha * last_c2 + (1.0f - last_alpha) * acc_r2;
-    last_c2 = bl;
-    float dL_dweight = 0.0f;
-    dL_dweight += ((p.final_D2 + m2 * p.final_A) - (2.0f * m_d) * p.final_D) * p.dL_dreg;
-    last_dL_dT = dL_dweight * alpha + (1.0f - alpha) * last_dL_dT;
-    accum_depth_rec = last_alpha * last_depth + (1.0f - last_alpha) * accum_depth_rec;
-    last_depth = c_d;
-    accum_alpha_rec = last_alpha + (1.0f - last_alpha) * accum_alpha_rec;
-    acc_n0 = last_alpha * last_n0 + (1.0f - last_alpha) * acc_n0;
-    last_n0 = nc.x;
-    acc_n1 = last_alpha * last_n1 + (1.0f - last_alpha) * acc_n1;
-    last_n1 = nc.y;
-    acc_n2 = last_alpha * last_n2 + (1.0f - last_alpha) * acc_n2;
-    last_n2 = nc.z;
-    last_alpha = alpha;
-  }
 };
 static_assert(sizeof(ChainBwd) == 18 * sizeof(float), "chain state is 18 floats");
 
@@ -205,13 +188,16 @@ struct SegMap {
   float b[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};  // r, g, b, depth, n0, n1, n2, alpha
   // one pair (alpha, distortion weight m_d) after the pair behind it (la,
   // values l: r, g, b, depth, n0, n1, n2)
-  SR_DEV void add(const PixelBwd& p, float la, const float* l, float alpha, float m_d, float m2) {
+  template <bool kPart>
+  SR_DEV void add(const PixelBwd& p, float la, const float* l, float alpha, float m_d, float m2,
+                  uint32_t contributor) {
     const float om = 1.0f - la;
 #pragma unroll
     for (int x = 0; x < 7; ++x) b[x] = la * l[x] + om * b[x];
     b[7] = la + om * b[7];
     A = om * A;
-    const float dw = ((p.final_D2 + m2 * p.final_A) - (2.0f * m_d) * p.final_D) * p.dL_dreg;
+    float dw = ((p.final_D2 + m2 * p.final_A) - (2.0f * m_d) * p.final_D) * p.dL_dreg;
+    if (kPart && (int)contributor == p.median_contributor - 1) dw = p.dL_dmaxw + dw;
     const float oa = 1.0f - alpha;
     b2 = dw * alpha + oa * b2;
     A2 = oa * A2;
@@ -314,11 +300,13 @@ SR_DEV void pair_grads(float dLp0, float dLp1, float dLp2, float dLn0, float dLn
 // per-pixel chain carries only the recurrences.  A quadrant some of whose
 // pairs missed the store (q_flag) instead runs the whole backward here over
 // staged records, recomputing those pairs.
+template <bool kPart>
 __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
   __shared__ float4 s_q0[64], s_q1[64], s_q2[64], s_q3[64], s_q4[64];
   __shared__ uint2 s_e[64];
   __shared__ float s_acc[kNumG][64];
   __shared__ float s_tmp[kNumG][65];
+  __shared__ uint32_t s_took[kPart ? 64 : 1];   // _part: the entry has a pixel with a semantic gradient
   __shared__ float s_map[8][8][kSegMapFloats];  // per pixel of the wave, each segment's SegMap
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   if (a.counters[1] & kErrCapacity) return;
@@ -338,7 +326,7 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
   const uint32_t pxi = (uint32_t)(tx * B + (q % QX) * kQuad + (pix & 7));
   const uint32_t pyi = (uint32_t)(ty * B + (q / QX) * kQuad + (pix >> 3));
   const bool inside = lane_ok && pxi < (uint32_t)vi.W && pyi < (uint32_t)vi.H;
-  const float pixx = (float)pxi, pixy = (float)pyi;
+  const float pixx = pixel_centre<kPart>((int)pxi), pixy = pixel_centre<kPart>((int)pyi);
   ChainBwd ch;
 
   if (!staged) {
@@ -361,7 +349,7 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
     const int n = (int)rg.y, f0 = (int)rg.x;
     const int seg_len = max(kChainSegMin, (n + 7) / 8);
     const int nseg = (n + seg_len - 1) / seg_len;
-    const PixelBwd px = pixel_bwd(a, vi, n > 0, qxi, qyi);
+    const PixelBwd px = pixel_bwd<kPart>(a, vi, n > 0, qxi, qyi);
     // walk pairs f0 + hi down to f0 + lo, calling fn(index, p0, p1, p2)
     auto walk = [&](int lo, int hi, auto&& fn) {
       float4 g0[kChainPre], g1[kChainPre], g2[kChainPre];
@@ -416,7 +404,7 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
 #pragma unroll
       for (int x = 0; x < 7; ++x) pl[x] = l[x];
       walk(lo, hi, [&](int, const float4& c0, const float4& c1, const float4& c2) {
-        m.add(px, pa, pl, c0.w, c0.y, c0.z);
+        m.add<kPart>(px, pa, pl, c0.w, c0.y, kPart ? c0.y * c0.y : c0.z, __float_as_uint(c2.z));
         pa = c0.w;
         pl[0] = c1.w;
         pl[1] = c2.x;
@@ -445,7 +433,8 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
       ch.last_n1 = l[5];
       ch.last_n2 = l[6];
       walk(lo, hi, [&](int k, const float4& c0, const float4& c1, const float4& c2) {
-        a.ps.fW[f0 + k] = ch.step(px, c0.w, c0.x, c0.y, c0.z, c2.w, __float_as_uint(c2.z), c1, c2.x, c2.y);
+        a.ps.fW[f0 + k] = ch.step<kPart>(px, c0.w, c0.x, c0.y, kPart ? c0.y * c0.y : c0.z, c2.w,
+                                         __float_as_uint(c2.z), c1, c2.x, c2.y);
       });
     }
     return;
@@ -457,7 +446,7 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
   const uint2* list = a.sub + (size_t)Q * rbeg + (size_t)q * ntile;
   const uint64_t* masks = a.masks + mask_base(Q, rbeg, ntile, tile, q);
   const uint32_t* frag_off = a.frag_off + mask_base(Q, rbeg, ntile, tile, q);
-  const PixelBwd px = pixel_bwd(a, vi, inside, pxi, pyi);
+  const PixelBwd px = pixel_bwd<kPart>(a, vi, inside, pxi, pyi);
   ch.T = px.T_final;
   // The pixel's run is cut into the stored path's segments (the forward
   // recorded how many pairs the pixel blended): while a segment's pairs go
@@ -472,8 +461,14 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
   int seg = (n_run + seg_len - 1) / seg_len - 1, seg_start = seg * seg_len, idx = n_run;
   const int nch = (cnt + 63) / 64;
   const bool active = inside && px.last_contributor > 0;
-  const float mcoef = kFar / (kFar - kNear);
-  const float dmd_num = kFar * kNear, dmd_den0 = kFar - kNear;
+  // the pixel's semantic gradients (_part)
+  float dLs[kPart ? kMaxSem : 1];
+#pragma unroll
+  for (int x = 0; x < (kPart ? kMaxSem : 1); ++x) {
+    const size_t HW = (size_t)vi.H * vi.W;
+    dLs[x] = kPart && inside && x < a.S
+                 ? a.dL_dsem[(size_t)a.S * vi.pix_base + x * HW + (size_t)vi.W * pyi + pxi] : 0.0f;
+  }
   ChunkRegs nx{};
   uint2 v2 = make_uint2(0u, 0u);
   if (nch > 0) {
@@ -494,6 +489,7 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
     }
 #pragma unroll
     for (int k = 0; k < kNumG; ++k) s_acc[k][lane] = 0.0f;
+    if (kPart) s_took[lane] = 0u;
     __syncthreads();
     if (c > 0) {  // in flight while this chunk runs
       const uint2 ve = v2;
@@ -515,22 +511,22 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
 #pragma unroll
         for (int k = 0; k < kNumG; ++k) gk[k] = 0.0f;
         bool took = false;
+        float took_w = 0.0f;
         const uint32_t contributor = s_e[j].y;  // 0-based position in the tile list
         if (hit && contributor < px.last_contributor) {
           const float4 q2 = s_q2[j];
           Pair e;  // a flagged quadrant has no stored pairs: recompute
           if (eval_pair<false>(pixx, pixy, s_q0[j], s_q1[j], q2, 0.0f, e)) {
             const float c_d = e.depth;
-            const float m_d = mcoef * (1.0f - kNear / c_d);
-            const float dmd_dd = dmd_num / ((dmd_den0 * c_d) * c_d);
+            const float m_d = dist_weight<kPart>(c_d), dmd_dd = dist_weight_grad<kPart>(c_d);
             const float4 q3 = s_q3[j], q4 = s_q4[j];
             --idx;  // this pair's place in the run
             if (seg >= 1) {
               float l[7];
               chain_last(ch, l);
-              seg_map.add(px, ch.last_alpha, l, e.alpha, m_d, m_d * m_d);
+              seg_map.add<kPart>(px, ch.last_alpha, l, e.alpha, m_d, m_d * m_d, contributor);
             }
-            const float4 g = ch.step(px, e.alpha, c_d, m_d, m_d * m_d, dmd_dd, contributor, q3, q4.x, q4.y);
+            const float4 g = ch.step<kPart>(px, e.alpha, c_d, m_d, m_d * m_d, dmd_dd, contributor, q3, q4.x, q4.y);
             if (idx == seg_start && seg >= 1) {  // the next pair starts segment seg - 1
               seg_map.apply(fold);
               ch.T = fold.T;
@@ -550,13 +546,13 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
             pair_grads(px.dLp0, px.dLp1, px.dLp2, px.dLn0, px.dLn1, px.dLn2, e, s_q1[j], q2.w, g.x, g.y, g.z,
                        pixx, pixy, [&](int k, float v) { gk[k] += v; });
             took = true;
+            took_w = g.x;
           }
         }
         const uint64_t tookm = __ballot(took);
-#pragma unroll
-        for (int k = 0; k < kNumG; ++k) s_tmp[k][lane] = gk[k];
-        __syncthreads();
-        if (lane < kNumG) {  // grouped exactly as the per-pair gradient pass sums
+        // row `lane` of s_tmp summed over the pixels of tookm, grouped
+        // exactly as the per-pair gradient pass sums
+        auto grouped = [&]() {
           float acc = 0.0f, grp = 0.0f;
           int in_grp = 0;
           for (uint64_t mm = tookm; mm != 0ull; mm &= mm - 1ull) {
@@ -568,13 +564,27 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
             }
           }
           if (in_grp > 0) acc += grp;
-          s_acc[lane][j] = acc;
-        }
+          return acc;
+        };
+#pragma unroll
+        for (int k = 0; k < kNumG; ++k) s_tmp[k][lane] = gk[k];
         __syncthreads();
+        if (lane < kNumG) s_acc[lane][j] = grouped();
+        __syncthreads();
+        if (kPart && a.S > 0 && tookm != 0ull) {  // semantics get their own gradient only
+#pragma unroll
+          for (int x = 0; x < kMaxSem; ++x) s_tmp[x][lane] = took_w * dLs[x];
+          __syncthreads();
+          if (lane < a.S)
+            a.sem_part[slot_of(a.pos_slot, a.pos_quads, rbeg + s_e[j].y, q) * (size_t)a.S + lane] = grouped();
+          if (lane == 0) s_took[j] = 1u;
+          __syncthreads();
+        }
       }
     }
     __syncthreads();
-    if (lane < m) store_part(a, rbeg + s_e[lane].y, q, [&](int k) { return s_acc[k][lane]; });
+    if (lane < m)
+      store_part(a, rbeg + s_e[lane].y, q, [&](int k) { return s_acc[k][lane]; }, kPart && s_took[lane] != 0u);
   }
 }
 
@@ -582,7 +592,8 @@ hipError_t launch_blend_bwd(const BlendBwdArgs& a, hipStream_t s) {
   if (a.vs.T == 0) return hipSuccess;
   if (a.vs.B != 8 && a.vs.B != 16 && a.vs.B != 32) return hipErrorInvalidValue;
   const unsigned nblk = (unsigned)(a.vs.T * quads_per_tile(a.vs.B));
-  hipLaunchKernelGGL(k_blend_bwd, dim3(nblk * kSplitBwd), dim3(64), 0, s, a);
+  if (a.is_part) hipLaunchKernelGGL(k_blend_bwd<true>, dim3(nblk * kSplitBwd), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL(k_blend_bwd<false>, dim3(nblk * kSplitBwd), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 
@@ -630,6 +641,9 @@ SR_DEV uint64_t wave_transpose64(uint64_t x, int lane) {
 // entry's sums go to its (position, quadrant) slot of the partial-gradient
 // buffer.  The recompute path of pass 1 groups its sums the same way, so
 // the partials have the same bits whichever quadrants missed the pair store.
+// kSem: the _part variant's semantic channels, rounded up (0: none), whose
+// gradients w dL/dsem are summed the same way into sem_part.
+template <bool kPart, int kSem>
 __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
   __shared__ uint4 s_pm[64];    // per pixel: trimmed mask (lo, hi), first stored pair of the chunk
   __shared__ float4 s_pg[64];   // per pixel: dL/dpixel (rgb), dL/dnormal.x
@@ -639,7 +653,8 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
   __shared__ unsigned long long s_col[64];         // per entry: the pixels that blended it
   __shared__ uint32_t s_tbase[64];                 // per entry: its first group
   __shared__ uint8_t s_towner[64 * (64 / kGradGroup)];  // entry of every group
-  __shared__ float s_grp[kNumG][64];               // group sums of the round
+  __shared__ float s_grp[kNumG + kSem][64];        // group sums of the round
+  __shared__ float s_dls[kSem > 0 ? kSem : 1][64]; // per pixel: dL/dsem
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   const int lane = threadIdx.x;
   if (a.counters[1] & kErrCapacity) return;
@@ -671,7 +686,7 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
       const size_t HW = (size_t)vi.H * vi.W, pid = (size_t)vi.W * pyi + pxi, pb = vi.pix_base;
       lc = a.n_contrib[2 * pb + pid];
       const float* dL_dpix = a.dL_dpix + 3 * pb;
-      const float* dL_dothers = a.dL_dothers + 7 * pb;
+      const float* dL_dothers = a.dL_dothers + (kPart ? 8 : 7) * pb;
       pg = make_float4(dL_dpix[pid], dL_dpix[HW + pid], dL_dpix[2 * HW + pid], dL_dothers[2 * HW + pid]);
       pn = make_float2(dL_dothers[3 * HW + pid], dL_dothers[4 * HW + pid]);
     }
@@ -690,6 +705,12 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
     s_e0[lane] = q0;
     s_e1[lane] = q1;
     s_e2[lane] = q2;
+#pragma unroll
+    for (int x = 0; x < kSem; ++x) {
+      const size_t HW = (size_t)vi.H * vi.W;
+      s_dls[x][lane] = mask && x < a.S
+                           ? a.dL_dsem[(size_t)a.S * vi.pix_base + x * HW + (size_t)vi.W * pyi + pxi] : 0.0f;
+    }
     __syncthreads();
     if (mask) {
       // entries in front of the last contributor: positions rise along the
@@ -716,14 +737,14 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
     s_tbase[lane] = tbase;
     for (uint32_t i = 0; i < ng; ++i) s_towner[tbase + i] = (uint8_t)lane;
     __syncthreads();
-    float acc[kNumG];
+    float acc[kNumG + kSem];
 #pragma unroll
-    for (int k = 0; k < kNumG; ++k) acc[k] = 0.0f;
+    for (int k = 0; k < kNumG + kSem; ++k) acc[k] = 0.0f;
     for (uint32_t base = 0; base < ntask; base += 64) {  // uniform
       const uint32_t t = base + (uint32_t)lane;
-      float g[kNumG];
+      float g[kNumG + kSem];
 #pragma unroll
-      for (int k = 0; k < kNumG; ++k) g[k] = 0.0f;
+      for (int k = 0; k < kNumG + kSem; ++k) g[k] = 0.0f;
       if (t < ntask) {
         const int j = s_towner[t];
         const uint32_t gi = t - s_tbase[j];
@@ -753,34 +774,48 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
           if (p < 0) continue;
           const float4 g4 = s_pg[p];
           const float2 n2 = s_pn[p];
-          const float pixx = (float)(bx + (p & 7)), pixy = (float)(by + (p >> 3));
+          const float pixx = pixel_centre<kPart>(bx + (p & 7)), pixy = pixel_centre<kPart>(by + (p >> 3));
           // the pair itself (s, G, planes) recomputed exactly as the
           // acceptance pass evaluated it: cheaper than fetching it
           Pair e;
           (void)eval_pair<false>(pixx, pixy, r0, r1, r2, 0.0f, e);
           pair_grads(g4.x, g4.y, g4.z, g4.w, n2.x, n2.y, e, r1, r2.w, fw[k].x, fw[k].y, fw[k].z, pixx, pixy,
                      [&](int s, float val) { g[s] += val; });
+#pragma unroll
+          for (int x = 0; x < kSem; ++x) g[kNumG + x] += fw[k].x * s_dls[x][p];
         }
       }
 #pragma unroll
-      for (int k = 0; k < kNumG; ++k) s_grp[k][lane] = g[k];
+      for (int k = 0; k < kNumG + kSem; ++k) s_grp[k][lane] = g[k];
       __syncthreads();
       // the entry's lane adds its groups of this round, in order
       const uint32_t lo = max(tbase, base), hi = min(tbase + ng, base + 64u);
       for (uint32_t u = lo; u < hi; ++u) {
 #pragma unroll
-        for (int k = 0; k < kNumG; ++k) acc[k] += s_grp[k][u - base];
+        for (int k = 0; k < kNumG + kSem; ++k) acc[k] += s_grp[k][u - base];
       }
       __syncthreads();
     }
-    if (has) store_part(a, rbeg + v.y, q, [&](int k) { return acc[k]; });
+    if (has) {
+      store_part(a, rbeg + v.y, q, [&](int k) { return acc[k]; }, kSem > 0 && ng > 0u);
+      if (kSem > 0 && ng > 0u) {
+        float* d = a.sem_part + slot_of(a.pos_slot, a.pos_quads, rbeg + v.y, q) * (size_t)a.S;
+#pragma unroll
+        for (int x = 0; x < kSem; ++x)
+          if (x < a.S) d[x] = acc[kNumG + x];
+      }
+    }
   }
 }
 
 hipError_t launch_blend_bwd_grad(const BlendBwdArgs& a, size_t max_items, hipStream_t s) {
   if (max_items == 0) return hipSuccess;
   const unsigned grid = (unsigned)(max_items < 65536 ? max_items : 65536);
-  hipLaunchKernelGGL(k_blend_bwd_grad, dim3(grid), dim3(64), 0, s, a);
+  if (!a.is_part) hipLaunchKernelGGL((k_blend_bwd_grad<false, 0>), dim3(grid), dim3(64), 0, s, a);
+  else if (a.S == 0) hipLaunchKernelGGL((k_blend_bwd_grad<true, 0>), dim3(grid), dim3(64), 0, s, a);
+  else if (a.S <= 4) hipLaunchKernelGGL((k_blend_bwd_grad<true, 4>), dim3(grid), dim3(64), 0, s, a);
+  else if (a.S <= 8) hipLaunchKernelGGL((k_blend_bwd_grad<true, 8>), dim3(grid), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL((k_blend_bwd_grad<true, 16>), dim3(grid), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 

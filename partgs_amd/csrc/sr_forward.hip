@@ -1484,6 +1484,7 @@ hipError_t launch_sort_tiles(const SortArgs& a, hipStream_t s) {
 // bulk of the pair evaluations, runs balanced over the whole GPU; the blend
 // kernels then visit only accepted pairs.
 // ---------------------------------------------------------------------------
+template <bool kPart>
 __global__ __launch_bounds__(64) void k_accept(AcceptArgs a) {
   __shared__ float4 s_q0[64], s_q1[64], s_q2[64];
   __shared__ float s_rej[64];
@@ -1553,7 +1554,8 @@ __global__ __launch_bounds__(64) void k_accept(AcceptArgs a) {
         const uint32_t dy = (r * kDiv[bw]) >> 9, dx = r - dy * bw;
         const int lx = (int)(g & 15u) + (int)dx, ly = (int)((g >> 4) & 15u) + (int)dy;
         Pair e;
-        if (eval_pair<true>((float)(qx0 + lx), (float)(qy0 + ly), s_q0[j], s_q1[j], s_q2[j], s_rej[j], e)) {
+        if (eval_pair<true>(pixel_centre<kPart>(qx0 + lx), pixel_centre<kPart>(qy0 + ly), s_q0[j], s_q1[j], s_q2[j],
+                            s_rej[j], e)) {
           const int p = ly * kQuad + lx;
           atomicOr(&s_mask[p], 1ull << j);
           atomicAdd(&s_logT[p], __log2f(1.0f - e.alpha));
@@ -1570,7 +1572,8 @@ __global__ __launch_bounds__(64) void k_accept(AcceptArgs a) {
 hipError_t launch_accept(const AcceptArgs& a, size_t max_items, hipStream_t s) {
   if (max_items == 0) return hipSuccess;
   const unsigned grid = (unsigned)(max_items < 65536 ? max_items : 65536);
-  hipLaunchKernelGGL(k_accept, dim3(grid), dim3(64), 0, s, a);
+  if (a.part) hipLaunchKernelGGL(k_accept<true>, dim3(grid), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL(k_accept<false>, dim3(grid), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 
@@ -1755,17 +1758,17 @@ hipError_t launch_pair_offsets(const AcceptArgs& a, hipStream_t s) {
 // bits), so consecutive lanes write consecutive records of a pixel's run.
 // Each lane recomputes its pair and stores the entry data the blend chains
 // need.
+template <bool kPart>
 __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
   __shared__ float4 s_q0[64], s_q1[64], s_q2[64], s_q3[64], s_q4[64];
   __shared__ uint32_t s_pos[64];
   __shared__ unsigned long long s_mask[64];
   __shared__ uint32_t s_start[64], s_foff[64];
   __shared__ uint8_t s_owner[64 * 64];  // pixel of every pair slot
+  __shared__ uint32_t s_rid[kPart ? 64 : 1];
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   const int lane = threadIdx.x;
   if (a.counters[1] & kErrCapacity) return;
-  const float mcoef = kFar / (kFar - kNear);
-  const float dmd_num = kFar * kNear, dmd_den0 = kFar - kNear;
   const uint32_t nwork = *a.work_count;
   for (uint32_t w = blockIdx.x; w < nwork; w += gridDim.x) {
     const uint2 item = a.work[nwork - 1u - w];  // from the end: see work_capacity
@@ -1809,6 +1812,7 @@ __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
       s_q3[lane] = rc[3];
       s_q4[lane] = rc[4];
       s_pos[lane] = v.y;
+      if (kPart) s_rid[lane] = v.x;
     }
     __syncthreads();
     for (uint32_t base = 0; base < total; base += 64) {
@@ -1818,13 +1822,13 @@ __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
       const uint32_t k = t - s_start[p];
       const int j = select_bit(s_mask[p], k);
       Pair e;
-      eval_pair<false>((float)(qx0 + (p & 7)), (float)(qy0 + (p >> 3)), s_q0[j], s_q1[j], s_q2[j], 0.0f, e);
+      eval_pair<false>(pixel_centre<kPart>(qx0 + (p & 7)), pixel_centre<kPart>(qy0 + (p >> 3)), s_q0[j], s_q1[j],
+                       s_q2[j], 0.0f, e);
       const float4 q3 = s_q3[j], q4 = s_q4[j];
       // the distortion weight m(depth) and its derivative, as the blends form them
-      const float m_d = mcoef * (1.0f - kNear / e.depth);
-      const float dmd_dd = dmd_num / ((dmd_den0 * e.depth) * e.depth);
+      const float m_d = dist_weight<kPart>(e.depth), dmd_dd = dist_weight_grad<kPart>(e.depth);
       float4* pr = a.ps.rec + kPairQuads * (size_t)(s_foff[p] + k);
-      pr[0] = make_float4(e.depth, m_d, m_d * m_d, e.alpha);
+      pr[0] = make_float4(e.depth, m_d, kPart ? __uint_as_float(s_rid[j]) : m_d * m_d, e.alpha);
       pr[1] = q3;
       pr[2] = make_float4(q4.x, q4.y, __uint_as_float(s_pos[j]), dmd_dd);
     }
@@ -1834,7 +1838,8 @@ __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
 hipError_t launch_pair_write(const AcceptArgs& a, size_t max_items, hipStream_t s) {
   if (max_items == 0) return hipSuccess;
   const unsigned grid = (unsigned)(max_items < 65536 ? max_items : 65536);
-  hipLaunchKernelGGL(k_pair_write, dim3(grid), dim3(64), 0, s, a);
+  if (a.part) hipLaunchKernelGGL(k_pair_write<true>, dim3(grid), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL(k_pair_write<false>, dim3(grid), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 
@@ -1861,6 +1866,10 @@ constexpr int kPre = SR_FWD_PREFETCH;  // stored pairs a lane fetches ahead in t
 // instructions (role values are picked by select), so the serial chain of a
 // long pixel costs a quarter of the full update per pair; each accumulator
 // sees exactly the reference's operations in order.
+// The _part variant sums (x alpha) T where the plain one sums x (alpha T),
+// tracks the median pair's weight, and leaves each blended pair's T in the
+// fW region for the semantic channels' pass.
+template <bool kPart>
 SR_DEV void blend_fwd_stored(const BlendArgs& a, const ViewInfo& vi, int qi, int tx, int ty, int q, int part) {
   static_assert(kSplit == 4, "4 waves of 16 pixels x 4 roles per quadrant");
   const int B = a.vs.B, QX = B / kQuad;
@@ -1880,8 +1889,9 @@ SR_DEV void blend_fwd_stored(const BlendArgs& a, const ViewInfo& vi, int qi, int
   // quad in a0..a2 and w in a3, except that role 0's a3 is the distortion.
   const int qsel = role < 2 ? role : 2;
   float T = 1.0f;
-  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f, median_depth = 0.0f;
+  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f, median_depth = 0.0f, median_weight = 0.0f;
   float median_contributor = -1.0f;
+  float* pair_T = kPart && a.S > 0 ? reinterpret_cast<float*>(a.ps.fW) : nullptr;
   uint32_t last_contributor = 0;
   int blended = 0;
   bool done = !inside;
@@ -1902,6 +1912,7 @@ SR_DEV void blend_fwd_stored(const BlendArgs& a, const ViewInfo& vi, int qi, int
 #pragma unroll
     for (int k = 0; k < kPre; ++k) cq[k] = fq[k];
     const int n = left;
+    const uint32_t f0 = f;
     f += kPre;
     left -= kPre;
     if (left > 0) fetch(f, left);  // next batch in flight
@@ -1922,8 +1933,10 @@ SR_DEV void blend_fwd_stored(const BlendArgs& a, const ViewInfo& vi, int qi, int
       const float w = alpha * T;
       const float A = 1.0f - T;
       // role 0: the distortion term (mm^2 A + M2 - 2 mm M1), a1 = M1, a2 = M2
-      const float x3 = role == 0 ? (v.z * A + a2) - (2.0f * v.y) * a1 : v.w;
-      const float n0 = a0 + v.x * w, n1 = a1 + v.y * w, n2 = a2 + v.z * w, n3 = a3 + x3 * w;
+      const float vz = kPart && role == 0 ? v.y * v.y : v.z;
+      const float x3 = role == 0 ? (vz * A + a2) - (2.0f * v.y) * a1 : v.w;
+      auto weighed = [&](float x) { return kPart ? (x * alpha) * T : x * w; };
+      const float n0 = a0 + weighed(v.x), n1 = a1 + weighed(v.y), n2 = a2 + weighed(vz), n3 = a3 + weighed(x3);
       a0 = ok ? n0 : a0;
       a1 = ok ? n1 : a1;
       a2 = ok ? n2 : a2;
@@ -1931,6 +1944,10 @@ SR_DEV void blend_fwd_stored(const BlendArgs& a, const ViewInfo& vi, int qi, int
       const bool med = ok && T > 0.5f;
       median_depth = med ? depth : median_depth;
       median_contributor = med ? (float)contributor : median_contributor;
+      if (kPart) {
+        median_weight = med ? w : median_weight;
+        if (pair_T != nullptr && ok && role == 0) pair_T[f0 + k] = T;
+      }
       T = ok ? test_T : T;
       last_contributor = ok ? contributor : last_contributor;
       blended += ok ? 1 : 0;
@@ -1940,7 +1957,7 @@ SR_DEV void blend_fwd_stored(const BlendArgs& a, const ViewInfo& vi, int qi, int
   const size_t HW = (size_t)vi.H * vi.W, pid = (size_t)vi.W * pyi + pxi, pb = vi.pix_base;
   float* final_T = a.final_T + 3 * pb;
   float* out_color = a.out_color + 3 * pb;
-  float* out_others = a.out_others + 7 * pb;
+  float* out_others = a.out_others + (kPart ? 8 : 7) * pb;
   if (role == 0) {
     out_others[pid] = a0;
     final_T[pid + HW] = a1;
@@ -1961,14 +1978,17 @@ SR_DEV void blend_fwd_stored(const BlendArgs& a, const ViewInfo& vi, int qi, int
     n_contrib[pid + HW] = f2u(median_contributor);
     out_others[pid + HW] = 1.0f - T;
     out_others[pid + 5 * HW] = median_depth;
+    if (kPart) out_others[pid + 7 * HW] = median_weight;
     // the backward passes walk only the blended prefix of the run
     if (cnt > 0) a.lane_range[(size_t)qi * 64 + pix].y = (uint32_t)blended;
   }
 }
 
+template <bool kPart>
 __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
   __shared__ float4 s_q0[64], s_q1[64], s_q2[64], s_q3[64], s_q4[64];
   __shared__ uint32_t s_pos[64];
+  __shared__ uint32_t s_rid[kPart ? 64 : 1];
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   if (a.counters[1] & kErrCapacity) return;
   const int qi = (int)a.q_order[blockIdx.x / kSplit], part = blockIdx.x % kSplit;
@@ -1980,7 +2000,7 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
   const bool staged = a.q_flag[qi] != 0u;
   if (staged && part != 0) return;  // the staged path uses all 64 lanes of part 0
   if (!staged) {
-    blend_fwd_stored(a, vi, qi, tx, ty, q, part);
+    blend_fwd_stored<kPart>(a, vi, qi, tx, ty, q, part);
     return;
   }
   // staged path: lane = pixel of the quadrant
@@ -1995,37 +2015,49 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
   const uint2* list = a.sub + (size_t)Q * rbeg + (size_t)q * ntile;
   const uint64_t* masks = a.masks + mask_base(Q, rbeg, ntile, tile, q);
   const uint32_t* frag_off = a.frag_off + mask_base(Q, rbeg, ntile, tile, q);
-  const float pixx = (float)pxi, pixy = (float)pyi;
+  const float pixx = pixel_centre<kPart>((int)pxi), pixy = pixel_centre<kPart>((int)pyi);
   float T = 1.0f;
   uint32_t last_contributor = 0;
+  float Sem[kPart ? kMaxSem : 1];
+#pragma unroll
+  for (int ch = 0; ch < (kPart ? kMaxSem : 1); ++ch) Sem[ch] = 0.0f;
+  float median_weight = 0.0f;
   float C0 = 0.0f, C1 = 0.0f, C2 = 0.0f, N0 = 0.0f, N1 = 0.0f, N2 = 0.0f;
   float D = 0.0f, M1 = 0.0f, M2 = 0.0f, distortion = 0.0f, median_depth = 0.0f, median_contributor = -1.0f;
   int blended = 0;
-  const float mcoef = kFar / (kFar - kNear);
   const int nch = (cnt + 63) / 64;
   // One front-to-back step of the reference's update (forward.cu:383-415);
   // false once T would drop below 1e-4 (the pixel is done).  mm is the
   // distortion weight mcoef (1 - near / depth).
-  auto step = [&](float alpha, float depth, float mm, uint32_t pos, const float4& nc, float g, float bl) -> bool {
+  auto step = [&](float alpha, float depth, float mm, uint32_t pos, const float4& nc, float g, float bl,
+                  uint32_t rid) -> bool {
     const float test_T = T * (1.0f - alpha);
     if (test_T < 0.0001f) return false;
     const uint32_t contributor = pos + 1u;
     const float w = alpha * T;
     const float A = 1.0f - T;
-    distortion += (((mm * mm) * A + M2) - (2.0f * mm) * M1) * w;
-    D += depth * w;
-    M1 += mm * w;
-    M2 += (mm * mm) * w;
+    auto weighed = [&](float x) { return kPart ? (x * alpha) * T : x * w; };
+    distortion += weighed(((mm * mm) * A + M2) - (2.0f * mm) * M1);
+    D += weighed(depth);
+    M1 += weighed(mm);
+    M2 += weighed(mm * mm);
     if (T > 0.5f) {
       median_depth = depth;
+      median_weight = w;
       median_contributor = (float)contributor;
     }
-    N0 += nc.x * w;
-    N1 += nc.y * w;
-    N2 += nc.z * w;
-    C0 += nc.w * w;
-    C1 += g * w;
-    C2 += bl * w;
+    N0 += weighed(nc.x);
+    N1 += weighed(nc.y);
+    N2 += weighed(nc.z);
+    C0 += weighed(nc.w);
+    C1 += weighed(g);
+    C2 += weighed(bl);
+    if (kPart) {
+      const float* sr = a.sem + (size_t)rid * a.S;
+#pragma unroll
+      for (int ch = 0; ch < kMaxSem; ++ch)
+        if (ch < a.S) Sem[ch] += weighed(sr[ch]);
+    }
     T = test_T;
     last_contributor = contributor;
     ++blended;
@@ -2047,6 +2079,7 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
       __syncthreads();
       if (lane < m) {
         s_pos[lane] = nx.v.y;
+        if (kPart) s_rid[lane] = nx.v.x;
         s_q0[lane] = nx.q0;
         s_q1[lane] = nx.q1;
         s_q2[lane] = nx.q2;
@@ -2076,7 +2109,7 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
           depth = e.depth;
         }
         const float4 q3 = s_q3[j], q4 = s_q4[j];
-        if (!step(alpha, depth, mcoef * (1.0f - kNear / depth), s_pos[j], q3, q4.x, q4.y)) {
+        if (!step(alpha, depth, dist_weight<kPart>(depth), s_pos[j], q3, q4.x, q4.y, kPart ? s_rid[j] : 0u)) {
           done = true;
           break;
         }
@@ -2089,7 +2122,14 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
     float* final_T = a.final_T + 3 * pb;
     uint32_t* n_contrib = a.n_contrib + 2 * pb;
     float* out_color = a.out_color + 3 * pb;
-    float* out_others = a.out_others + 7 * pb;
+    float* out_others = a.out_others + (kPart ? 8 : 7) * pb;
+    if (kPart) {
+      out_others[pid + 7 * HW] = median_weight;
+      float* out_sem = a.out_sem + (size_t)a.S * pb;
+#pragma unroll
+      for (int ch = 0; ch < kMaxSem; ++ch)
+        if (ch < a.S) out_sem[ch * HW + pid] = Sem[ch];
+    }
     final_T[pid] = T;
     n_contrib[pid] = last_contributor;
     out_color[pid] = C0 + T * a.bg[0];
@@ -2114,7 +2154,63 @@ hipError_t launch_blend_fwd(const BlendArgs& a, hipStream_t s) {
   if (a.vs.T == 0) return hipSuccess;
   if (a.vs.B != 8 && a.vs.B != 16 && a.vs.B != 32) return hipErrorInvalidValue;
   const unsigned nblk = (unsigned)(a.vs.T * quads_per_tile(a.vs.B));
-  hipLaunchKernelGGL(k_blend_fwd, dim3(nblk * kSplit), dim3(64), 0, s, a);
+  if (a.part) hipLaunchKernelGGL(k_blend_fwd<true>, dim3(nblk * kSplit), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL(k_blend_fwd<false>, dim3(nblk * kSplit), dim3(64), 0, s, a);
+  return hipGetLastError();
+}
+
+// Semantic channels of the _part variant (dsp/cuda_rasterizer/forward.cu:417):
+// Sem[ch] += (s[ch] alpha) T over the pixel's blended pairs in order, with
+// the T the blend left per pair.  kLanes lanes per pixel, one channel each:
+// a pair's alpha and T are one broadcast load and its semantics one row
+// gather, and only the sum itself is serial, so kSemPre pairs' loads are in
+// flight.  One wave per 64 / kLanes pixels, quadrants longest chain first.
+// Memory-bound: 20 + 4 S bytes a pair.
+constexpr int kSemPre = 8;
+template <int kLanes>
+__global__ __launch_bounds__(64) void k_blend_semantics(BlendArgs a) {
+  constexpr int kWaves = kLanes, kPix = 64 / kLanes;  // waves per quadrant, pixels per wave
+  const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
+  if (a.counters[1] & kErrCapacity) return;
+  const int qi = (int)a.q_order[blockIdx.x / kWaves], wv = blockIdx.x % kWaves;
+  if (a.q_flag[qi] != 0u) return;  // blended with the quadrant's recomputed pairs
+  const int tile = qi / Q, q = qi % Q;
+  const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
+  const int lt = tile - (int)vi.tile_base;
+  const int lane = threadIdx.x, ch = lane % kLanes, pix = wv * kPix + lane / kLanes;
+  const uint32_t pxi = (uint32_t)((lt % vi.gx) * B + (q % QX) * kQuad + (pix & 7));
+  const uint32_t pyi = (uint32_t)((lt / vi.gx) * B + (q / QX) * kQuad + (pix >> 3));
+  if (pxi >= (uint32_t)vi.W || pyi >= (uint32_t)vi.H || ch >= a.S) return;
+  float sum = 0.0f;
+  if (a.sub_count[qi] > 0u) {
+    const uint2 rg = a.lane_range[(size_t)qi * 64 + pix];
+    const float* pair_T = reinterpret_cast<const float*>(a.ps.fW);
+    for (uint32_t i = 0; i < rg.y; i += kSemPre) {
+      float4 p0[kSemPre];
+      float T[kSemPre], sv[kSemPre];
+#pragma unroll
+      for (int k = 0; k < kSemPre; ++k) {  // past the run's end: its last pair again, not summed
+        const size_t f = rg.x + min(i + (uint32_t)k, rg.y - 1u);
+        p0[k] = a.ps.rec[kPairQuads * f];
+        T[k] = pair_T[f];
+      }
+#pragma unroll
+      for (int k = 0; k < kSemPre; ++k) sv[k] = a.sem[(size_t)__float_as_uint(p0[k].z) * a.S + ch];
+#pragma unroll
+      for (int k = 0; k < kSemPre; ++k)
+        if (i + (uint32_t)k < rg.y) sum += (sv[k] * p0[k].w) * T[k];
+    }
+  }
+  const size_t HW = (size_t)vi.H * vi.W;
+  a.out_sem[(size_t)a.S * vi.pix_base + ch * HW + (size_t)vi.W * pyi + pxi] = sum;
+}
+
+hipError_t launch_blend_semantics(const BlendArgs& a, hipStream_t s) {
+  if (a.vs.T == 0 || a.S <= 0) return hipSuccess;
+  const unsigned nq = (unsigned)(a.vs.T * quads_per_tile(a.vs.B));
+  if (a.S <= 4) hipLaunchKernelGGL(k_blend_semantics<4>, dim3(nq * 4), dim3(64), 0, s, a);
+  else if (a.S <= 8) hipLaunchKernelGGL(k_blend_semantics<8>, dim3(nq * 8), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL(k_blend_semantics<16>, dim3(nq * 16), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 

@@ -183,7 +183,8 @@ constexpr int kPartStride = 20;  // 18 partial gradients, padded to five float4
 //   p1 = (normal.xyz, r)
 //   p2 = (g, b, position of the entry in the tile list (bits), dm/ddepth)
 // (p0, p1 and p2 are what the forward blend's lanes of roles 0, 1 and 2
-// accumulate, in their accumulators' order)
+// accumulate, in their accumulators' order; the _part variant keeps the
+// record number in p0.z instead of m^2, for its semantic channels)
 // A lane's consecutive pairs are consecutive records, so the fill writes
 // whole lines.  (The per-pair gradient pass recomputes s and G.)  fW = (w, dL/dalpha, dL/ddepth, 0) is written by the backward chain
 // pass for the per-pair gradient pass, which recomputes the rest of the pair.  All pairs of one pixel of a quadrant are
@@ -355,6 +356,7 @@ struct AcceptArgs {
   uint32_t* q_flag;
   unsigned long long* frag_fill;
   uint32_t frag_cap;
+  int part;  // the _part variant's pixel centres and records
 };
 
 struct BlendArgs {
@@ -375,6 +377,11 @@ struct BlendArgs {
   uint32_t* n_contrib;
   float* out_color;
   float* out_others;
+  // the _part variant: 8 aux channels and S <= 16 semantic ones
+  int part;
+  int S;
+  const float* sem;  // P x S
+  float* out_sem;    // S planes per view
 };
 
 // Backward blend.  Each (instance, quadrant) entry receives its 18
@@ -405,6 +412,11 @@ struct BlendBwdArgs {
   const uint16_t* pos_quads;
   float* part;        // partial gradients per slot (slot_of)
   uint8_t* part_nz;   // 1 where that slot was stored (any non-zero sum)
+  // the _part variant: 8 aux channels and S <= 16 semantic ones
+  int is_part;
+  int S;
+  const float* dL_dsem;
+  float* sem_part;    // S sums per slot
 };
 
 // Backward preprocess over all views of each surfel.  It first reduces each
@@ -448,37 +460,8 @@ struct PreprocessBwdArgs {
   float* dL_dsem;
 };
 
-// The _part variant's blend passes (one view): the plain pipeline's
-// records, ranges and quadrant sub-lists, plus semantics.
-struct PartArgs {
-  ViewSet vs;
-  int S;                     // semantic channels, <= 16
-  const uint32_t* ranges;
-  const uint2* sub;
-  const uint32_t* sub_count;
-  const float4* rec;
-  const float* sem;          // P x S
-  const float* bg;
-  // forward outputs
-  float* final_T;
-  uint32_t* n_contrib;
-  float* out_color;
-  float* out_sem;            // S x H x W
-  float* out_others;         // 8 x H x W
-  // backward
-  const float* final_T_in;
-  const uint32_t* n_contrib_in;
-  const float* dL_dpix;
-  const float* dL_dsem;
-  const float* dL_dothers;
-  const uint32_t* pos_slot;    // slot_of
-  const uint16_t* pos_quads;
-  float* part;
-  float* sem_part;           // S per slot
-  uint8_t* part_nz;
-};
-
 constexpr int kMaxQuads = 16;
+constexpr int kMaxSem = 16;  // semantic channels of the _part variant
 
 // Bit q set when cull box bx meets quadrant q (of QX x QX) of tile (tx, ty)
 // inside the image; the empty box (32767, 32767, -32768, -32768) meets none.
@@ -520,9 +503,6 @@ __device__ inline size_t slot_of(const uint32_t* pos_slot, const uint16_t* pos_q
 }
 
 // Launchers (return hipGetLastError()).
-hipError_t launch_part_blend_fwd(const PartArgs& a, hipStream_t s);
-hipError_t launch_part_blend_bwd(const PartArgs& a, hipStream_t s);
-
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 hipError_t launch_fill_f32(float* p, float v, size_t n, hipStream_t s);
 // Sets the message sr_last_error() returns on the calling thread; returns code.
@@ -540,6 +520,7 @@ hipError_t launch_pair_write(const AcceptArgs& a, size_t max_items, hipStream_t 
 hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, hipStream_t s);
 hipError_t launch_iota_u32(uint32_t* p, size_t n, hipStream_t s);
 hipError_t launch_blend_fwd(const BlendArgs& a, hipStream_t s);
+hipError_t launch_blend_semantics(const BlendArgs& a, hipStream_t s);
 hipError_t launch_blend_bwd(const BlendBwdArgs& a, hipStream_t s);
 hipError_t launch_blend_bwd_grad(const BlendBwdArgs& a, size_t max_items, hipStream_t s);
 hipError_t launch_preprocess_bwd(const PreprocessBwdArgs& a, hipStream_t s);

@@ -47,11 +47,13 @@ def _semantics(semantics, P, dev):
 
 def rasterize_gaussians_fwd(bg, means3D, colors, opacity, semantics, scales, rotations, scale_modifier,
                             transMat_precomp, viewmatrix, projmatrix, tan_fovx, tan_fovy, image_height, image_width,
-                            sh, degree, campos, prefiltered, debug, tile: int = 16):
+                            sh, degree, campos, prefiltered, debug, tile: int = 16, capacity: int = 0,
+                            pair_capacity: int = 0, slot_capacity: int = 0):
     """RasterizeGaussiansCUDA of the _part variant (dsp/rasterize_points.cu:40-146).
 
     Returns (num_rendered, color (3,H,W), semantic (S,H,W), others (8,H,W),
-    radii (P,) int32, geomBuffer, binningBuffer, imgBuffer)."""
+    radii (P,) int32, geomBuffer, binningBuffer, imgBuffer).  The three
+    capacities are those of the plain rasterize_gaussians_fwd."""
     if means3D.ndimension() != 2 or means3D.size(1) != 3:
         raise RuntimeError("means3D must have dimensions (num_points, 3)")
     lib = _lib.load()
@@ -73,7 +75,7 @@ def rasterize_gaussians_fwd(bg, means3D, colors, opacity, semantics, scales, rot
     others = torch.empty((8, H, W), dtype=torch.float32, device=dev)
     radii = torch.empty((P,), dtype=torch.int32, device=dev)
     s = _settings(a["bg"], scale_modifier, a["viewmatrix"], a["projmatrix"], tan_fovx, tan_fovy, H, W, degree,
-                  a["campos"], prefiltered, debug, tile)
+                  a["campos"], prefiltered, debug, tile, 0, capacity, pair_capacity, slot_capacity)
     g = _surfels(P, means3D, a["sh"], a["colors"], a["opacity"], a["scales"], a["rotations"], a["transMat_precomp"])
     arena = _Arena(dev)
     nr = C.c_int(0)
@@ -83,6 +85,8 @@ def rasterize_gaussians_fwd(bg, means3D, colors, opacity, semantics, scales, rot
                                  _lib.stream_handle(dev))
     if rc == _lib.SR_ERR_ALLOC and arena.error is not None:
         raise arena.error
+    if rc == _lib.SR_ERR_CAPACITY:
+        raise _lib.CapacityError(nr.value, capacity, slots=nr.value <= capacity)
     _lib.check(rc)
     return nr.value, color, semantic, others, radii, arena.get(0), arena.get(1), arena.get(2)
 
@@ -90,8 +94,10 @@ def rasterize_gaussians_fwd(bg, means3D, colors, opacity, semantics, scales, rot
 def rasterize_gaussians_bwd(bg, means3D, radii, colors, semantics, scales, rotations, scale_modifier,
                             transMat_precomp, viewmatrix, projmatrix, tan_fovx, tan_fovy, dL_dout_color,
                             dL_dout_semantic, dL_dout_others, sh, degree, campos, geomBuffer, R, binningBuffer,
-                            imageBuffer, debug, tile: int = 16):
+                            imageBuffer, debug, tile: int = 16, capacity: int = 0, pair_capacity: int = 0,
+                            slot_capacity: int = 0):
     """RasterizeGaussiansBackwardCUDA of the _part variant (dsp/rasterize_points.cu:149-252).
+    The capacities are the forward's.
 
     Returns (dL_dmeans2D, dL_dcolors, dL_dsemantics, dL_dopacity,
     dL_dmeans3D, dL_dtransMat, dL_dsh, dL_dscales, dL_drotations)."""
@@ -115,7 +121,7 @@ def rasterize_gaussians_bwd(bg, means3D, radii, colors, semantics, scales, rotat
     if P != 0:
         dsem = _f32(dL_dout_semantic, "dL_dout_semantic") if S > 0 else None
         s = _settings(a["bg"], scale_modifier, a["viewmatrix"], a["projmatrix"], tan_fovx, tan_fovy, H, W, degree,
-                      a["campos"], False, debug, tile)
+                      a["campos"], False, debug, tile, 0, capacity, pair_capacity, slot_capacity)
         g = _surfels(P, means3D, a["sh"], a["colors"], torch.empty(0, **opts), a["scales"], a["rotations"],
                      a["transMat_precomp"])
         gr = _lib.SrGrads()
