@@ -24,6 +24,7 @@
 // faces at the poles) are generated and differentiated in FP64.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "../../include/surfel_rast.h"
@@ -421,37 +422,83 @@ SR_DEV void to_block(const SdfBlock& k, float ratio, const float* pt, float* d, 
     pinv[r] = ((d[0] * k.R[3 * r] + d[1] * k.R[3 * r + 1]) + d[2] * k.R[3 * r + 2]) / (k.S[r] * ratio);
 }
 
-// The signed distance, and with grad != nullptr its derivatives: grad[0..2]
-// along pinv, grad[3] along e1, grad[4] along e2 (the clamps pass gradient
-// where their input is inside the range, as torch.clamp does).
+// log2 of a positive normal float in double, |error| < 2e-11: x = 2^e m with
+// m in [sqrt(1/2), sqrt(2)), log m = 2 atanh(s) = 2 s (1 + s^2/3 + s^4/5 + ...)
+// for s = (m - 1) / (m + 1), |s| < 0.1716 (the terms from s^4 on need no more
+// than FP32; the quotient is one Newton step in double from the FP32
+// reciprocal).
+SR_DEV double log2_pos(float x) {
+  const uint32_t u = __float_as_uint(x);
+  int e = (int)(u >> 23) - 127;
+  float m = __uint_as_float((u & 0x7fffffu) | 0x3f800000u);
+  if (m > 1.41421356f) {
+    m *= 0.5f;
+    ++e;
+  }
+  const double den = (double)m + 1.0;
+  const double r0 = (double)__builtin_amdgcn_rcpf(m + 1.0f);
+  const double s = (double)(m - 1.0f) * fma(r0, fma(-den, r0, 1.0), r0);
+  const double z = s * s;
+  const float zf = (float)z;
+  const float t = fmaf(fmaf(fmaf(fmaf(1.0f / 13.0f, zf, 1.0f / 11.0f), zf, 1.0f / 9.0f), zf, 1.0f / 7.0f), zf, 0.2f);
+  const double p = fma(z, fma(z, (double)t, 1.0 / 3.0), 1.0);
+  return fma(2.8853900817779268, s * p, (double)e);  // 2 / ln 2
+}
+
+// 2^t rounded to float (0.56 ulp): the Taylor series of 2^f, f in [-1/2, 1/2],
+// its first two terms in double and the rest in FP32.
+SR_DEV float exp2_pos(double t) {
+  const double n = rint(t);
+  const double f = t - n;
+  const float ff = (float)f;
+  float q = 1.52527338e-05f;                 // ln2^7 / 7!
+  q = fmaf(q, ff, 1.54035304e-04f);          // ln2^6 / 6!
+  q = fmaf(q, ff, 1.33335581e-03f);
+  q = fmaf(q, ff, 9.61812911e-03f);
+  q = fmaf(q, ff, 5.55041087e-02f);
+  q = fmaf(q, ff, 2.40226507e-01f);          // ln2^2 / 2
+  const double r = fma(f, fma(f, (double)q, 0.69314718055994531), 1.0);
+  return ldexpf((float)r, (int)n);
+}
+
+// The signed distance, and with kGrad its derivatives: grad[0..2] along
+// pinv, grad[3] along e1, grad[4] along e2 (the clamps pass gradient where
+// their input is inside the range, as torch.clamp does).  Every power is
+// 2^(y log2 x) on one logarithm per base, which the derivatives share: 5
+// logarithms and 10 exponentials with them, against 9 powf and 5 logf.
+template <bool kGrad>
 SR_DEV float implicit_sdf(const float* pinv, float e1, float e2, float* grad) {
-  float q[3], sq[3], base[3], pw[3];
+  constexpr float kLn2 = 0.693147182f;
+  float q[3], sq[3], pw[3];
+  double lb[3];
   const float ie1 = 1.0f / e1, ie2 = 1.0f / e2;
   const float ex[3] = {ie2, ie1, ie2};
+#pragma unroll
   for (int k = 0; k < 3; ++k) {
     q[k] = fminf(fmaxf(pinv[k], -5.0f), 5.0f);
     sq[k] = q[k] * q[k];
-    base[k] = fmaxf(sq[k], kSdfEps);
-    pw[k] = powf(base[k], ex[k]);
+    lb[k] = log2_pos(fmaxf(sq[k], kSdfEps));
+    pw[k] = exp2_pos((double)ex[k] * lb[k]);
   }
   const float xz = pw[0] + pw[2];
-  const float B = fmaxf(xz, kSdfEps);
+  const double lB = log2_pos(fmaxf(xz, kSdfEps));
   const float r21 = e2 / e1;
-  const float Bp = powf(B, r21);
+  const float Bp = exp2_pos((double)r21 * lB);
   const float res = Bp + pw[1];
-  const float A = fmaxf(res, kSdfEps);
+  const double lA = log2_pos(fmaxf(res, kSdfEps));
   const float h = e1 / 2.0f;
-  const float Ap = powf(A, h);
-  if (grad) {
-    const float d_res = res >= kSdfEps ? h * powf(A, h - 1.0f) : 0.0f;
-    const float d_B = xz >= kSdfEps ? d_res * (r21 * powf(B, r21 - 1.0f)) : 0.0f;
-    const float d_r21 = d_res * (Bp * logf(B));
-    float d_e1 = 0.5f * (Ap * logf(A)) + d_r21 * (-e2 / (e1 * e1));
+  const float Ap = exp2_pos((double)h * lA);
+  if constexpr (kGrad) {
+    const float d_res = res >= kSdfEps ? h * exp2_pos((double)(h - 1.0f) * lA) : 0.0f;
+    const float d_B = xz >= kSdfEps ? d_res * (r21 * exp2_pos((double)(r21 - 1.0f) * lB)) : 0.0f;
+    const float d_r21 = d_res * (Bp * (kLn2 * (float)lB));
+    float d_e1 = 0.5f * (Ap * (kLn2 * (float)lA)) + d_r21 * (-e2 / (e1 * e1));
     float d_e2 = d_r21 * ie1;
     const float d_pw[3] = {d_B, d_res, d_B};
+#pragma unroll
     for (int k = 0; k < 3; ++k) {
-      const float d_base = sq[k] >= kSdfEps ? d_pw[k] * (ex[k] * powf(base[k], ex[k] - 1.0f)) : 0.0f;
-      const float d_ex = d_pw[k] * (pw[k] * logf(base[k]));
+      const float d_base = sq[k] >= kSdfEps ? d_pw[k] * (ex[k] * exp2_pos((double)(ex[k] - 1.0f) * lb[k])) : 0.0f;
+      const float d_ex = d_pw[k] * (pw[k] * (kLn2 * (float)lb[k]));
       if (k == 1) d_e1 += d_ex * (-ie1 * ie1);
       else d_e2 += d_ex * (-ie2 * ie2);
       const bool inside = pinv[k] >= -5.0f && pinv[k] <= 5.0f;
@@ -463,41 +510,68 @@ SR_DEV float implicit_sdf(const float* pinv, float e1, float e2, float* grad) {
   return Ap - 1.0f;
 }
 
-__global__ __launch_bounds__(kSdfThreads) void k_sdf_fwd(const float* prm, float ratio, float scale_min,
-                                                         const float* pts, int N, float* sdf) {
-  const int b = blockIdx.y, n = blockIdx.x * kSdfThreads + threadIdx.x;
-  if (n >= N) return;
-  const SdfBlock k = sdf_block(prm, b, scale_min);
-  float d[3], pinv[3];
-  to_block(k, ratio, pts + 3 * (size_t)n, d, pinv);
-  sdf[(size_t)b * N + n] = implicit_sdf(pinv, k.e1, k.e2, nullptr);
+// Points a lane takes: the block's frame (five exponentials, a square root
+// and the rotation) is formed once per lane, so up to eight points share it
+// where that still leaves eight workgroups per CU.
+constexpr int kSdfMaxPts = 8;
+int sdf_pts_per_lane(int B, int N) {
+  const long long groups = (long long)B * ((N + kSdfThreads - 1) / kSdfThreads);
+  return (int)std::min<long long>(kSdfMaxPts, std::max<long long>(1, groups / 2048));
+}
+int sdf_chunks(int B, int N) {
+  const int pts = kSdfThreads * sdf_pts_per_lane(B, N);
+  return (N + pts - 1) / pts;
 }
 
-// Per (block, chunk of 256 points): the 17 sums, each over the chunk's
-// points in a fixed tree order.
+// 16 x 262,144 points: 109 us with powf and the frame formed for every
+// point, 40 us now.
+__global__ __launch_bounds__(kSdfThreads) void k_sdf_fwd(const float* prm, float ratio, float scale_min,
+                                                         const float* __restrict__ pts, int N, int per, float* sdf) {
+  const int b = blockIdx.y;
+  const SdfBlock k = sdf_block(prm, b, scale_min);
+  for (int i = 0; i < per; ++i) {
+    const long long n = ((long long)blockIdx.x * per + i) * kSdfThreads + threadIdx.x;
+    if (n >= N) return;
+    float d[3], pinv[3];
+    to_block(k, ratio, pts + 3 * (size_t)n, d, pinv);
+    sdf[(size_t)b * N + n] = implicit_sdf<false>(pinv, k.e1, k.e2, nullptr);
+  }
+}
+
+// Per (block, chunk of 256 per points): the 17 sums, each lane's points in
+// order, then over the lanes in a fixed tree order.  200 us with powf,
+// 59 us now (16 x 262,144 points).
 __global__ __launch_bounds__(kSdfThreads) void k_sdf_bwd(const float* prm, float ratio, float scale_min,
-                                                         const float* pts, int N, const float* dsdf, float* part) {
+                                                         const float* __restrict__ pts, int N, int per,
+                                                         const float* __restrict__ dsdf, float* part) {
   __shared__ float s_w[kSdfSums][kSdfThreads / 64];
-  const int b = blockIdx.y, n = blockIdx.x * kSdfThreads + threadIdx.x;
+  const int b = blockIdx.y;
+  const SdfBlock k = sdf_block(prm, b, scale_min);
   float c[kSdfSums];
+#pragma unroll
   for (int i = 0; i < kSdfSums; ++i) c[i] = 0.0f;
-  if (n < N) {
-    const SdfBlock k = sdf_block(prm, b, scale_min);
+  for (int i = 0; i < per; ++i) {
+    const long long n = ((long long)blockIdx.x * per + i) * kSdfThreads + threadIdx.x;
+    if (n >= N) break;
     float d[3], pinv[3], gr[5];
     to_block(k, ratio, pts + 3 * (size_t)n, d, pinv);
-    implicit_sdf(pinv, k.e1, k.e2, gr);
+    implicit_sdf<true>(pinv, k.e1, k.e2, gr);
     const float g = dsdf[(size_t)b * N + n];
+#pragma unroll
     for (int r = 0; r < 3; ++r) {
       const float gk = g * gr[r];
-      for (int j = 0; j < 3; ++j) c[3 * r + j] = gk * d[j];
-      c[9 + r] = gk;
-      c[12 + r] = gk * pinv[r];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) c[3 * r + j] += gk * d[j];
+      c[9 + r] += gk;
+      c[12 + r] += gk * pinv[r];
     }
-    c[15] = g * gr[3];
-    c[16] = g * gr[4];
+    c[15] += g * gr[3];
+    c[16] += g * gr[4];
   }
+#pragma unroll
   for (int i = 0; i < kSdfSums; ++i) {
     float v = c[i];
+#pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     if ((threadIdx.x & 63) == 0) s_w[i][threadIdx.x >> 6] = v;
   }
@@ -508,16 +582,28 @@ __global__ __launch_bounds__(kSdfThreads) void k_sdf_bwd(const float* prm, float
   }
 }
 
-// Per block: the chunk sums in a fixed order, then the chain to the 12 block
-// parameters through S = exp(s) + scale_min, R(normalised quaternion) and
-// e = 1.8 sigmoid(.) + 0.1 (dual numbers through make_block).
-__global__ __launch_bounds__(64) void k_sdf_reduce(const float* prm, float ratio, float scale_min, int nchunk,
-                                                   const float* part, float* dprm) {
+// Per block: the chunk sums in a fixed order (kSdfStreams interleaved streams
+// of chunks, then the streams in order: one stream was a chain of a thousand
+// dependent loads, 155 us for 16 x 262,144 points against 5 us), then the
+// chain to the 12 block parameters through S = exp(s) + scale_min,
+// R(normalised quaternion) and e = 1.8 sigmoid(.) + 0.1 (dual numbers through
+// make_block).
+constexpr int kSdfStreams = 15;
+__global__ __launch_bounds__(256) void k_sdf_reduce(const float* prm, float ratio, float scale_min, int nchunk,
+                                                    const float* part, float* dprm) {
+  __shared__ float s_part[kSdfStreams][kSdfSums];
   __shared__ float s_tot[kSdfSums];
   const int b = blockIdx.x;
+  if (threadIdx.x < kSdfStreams * kSdfSums) {
+    const int st = threadIdx.x / kSdfSums, i = threadIdx.x % kSdfSums;
+    float acc = 0.0f;
+    for (int c = st; c < nchunk; c += kSdfStreams) acc += part[((size_t)b * nchunk + c) * kSdfSums + i];
+    s_part[st][i] = acc;
+  }
+  __syncthreads();
   if (threadIdx.x < kSdfSums) {
     float acc = 0.0f;
-    for (int c = 0; c < nchunk; ++c) acc += part[((size_t)b * nchunk + c) * kSdfSums + threadIdx.x];
+    for (int st = 0; st < kSdfStreams; ++st) acc += s_part[st][threadIdx.x];
     s_tot[threadIdx.x] = acc;
   }
   __syncthreads();
@@ -651,8 +737,8 @@ int sb_sdf_fwd(const float* params, int B, float ratio, float scale_min, const f
   if ((long long)B * N == 0) return SR_OK;
   if (!params || !points || !sdf) return sr::set_error(SR_ERR_INVALID, "sb_sdf_fwd: NULL argument");
   if (B > 65535) return sr::set_error(SR_ERR_INVALID, "sb_sdf_fwd: more than 65535 blocks");
-  hipLaunchKernelGGL(sb::k_sdf_fwd, dim3((unsigned)((N + sb::kSdfThreads - 1) / sb::kSdfThreads), (unsigned)B),
-                     dim3(sb::kSdfThreads), 0, (hipStream_t)stream, params, ratio, scale_min, points, N, sdf);
+  hipLaunchKernelGGL(sb::k_sdf_fwd, dim3((unsigned)sb::sdf_chunks(B, N), (unsigned)B), dim3(sb::kSdfThreads), 0,
+                     (hipStream_t)stream, params, ratio, scale_min, points, N, sb::sdf_pts_per_lane(B, N), sdf);
   return hipGetLastError() == hipSuccess ? SR_OK : sr::set_error(SR_ERR_HIP, "sb_sdf_fwd: launch failed");
 }
 
@@ -677,10 +763,10 @@ int sb_sdf_bwd(const float* params, int B, float ratio, float scale_min, const f
   }
   if (!workspace || workspace_bytes < sb_sdf_bwd_workspace_bytes(B, N))
     return sr::set_error(SR_ERR_INVALID, "sb_sdf_bwd: workspace smaller than sb_sdf_bwd_workspace_bytes");
-  const int nchunk = (N + sb::kSdfThreads - 1) / sb::kSdfThreads;
+  const int nchunk = sb::sdf_chunks(B, N);  // at most one per 256 points, which the workspace is sized for
   hipLaunchKernelGGL(sb::k_sdf_bwd, dim3((unsigned)nchunk, (unsigned)B), dim3(sb::kSdfThreads), 0, st, params, ratio,
-                     scale_min, points, N, dL_dsdf, (float*)workspace);
-  hipLaunchKernelGGL(sb::k_sdf_reduce, dim3((unsigned)B), dim3(64), 0, st, params, ratio, scale_min, nchunk,
+                     scale_min, points, N, sb::sdf_pts_per_lane(B, N), dL_dsdf, (float*)workspace);
+  hipLaunchKernelGGL(sb::k_sdf_reduce, dim3((unsigned)B), dim3(256), 0, st, params, ratio, scale_min, nchunk,
                      (const float*)workspace, dL_dparams);
   return hipGetLastError() == hipSuccess ? SR_OK : sr::set_error(SR_ERR_HIP, "sb_sdf_bwd: launch failed");
 }
