@@ -13,10 +13,9 @@
 //   rotations = normalize(rot_to_quat([v1 v2 v0]))                 (get_rotation)
 //   opacities = sigmoid(sq_occ[b])                                  (get_opacity)
 //
-// The backward evaluates the same code on dual numbers, once per block
-// parameter (3 log-scales, 4 quaternion, 3 translation, 2 epsilon logits), so
-// the 12 directional derivatives of every output are exact; they are
-// contracted with the upstream gradients; the per-block sums are formed in
+// The backward takes every surfel's upstream gradient back to the 12 block
+// parameters (3 log-scales, 4 quaternion, 3 translation, 2 epsilon logits)
+// in one reverse sweep; the per-block sums are formed in
 // a fixed order (per-surfel contributions, then one workgroup per block
 // and parameter), so the gradients are deterministic.  Surfels whose
 // triangle is nearly degenerate (|n| < 1e-3 |e1| |e2|, or |n| or |V1 - c|
@@ -73,7 +72,6 @@ template <typename T> SR_DEV Dual<T> fexp(Dual<T> a) {
   const T e = fexp(a.v);
   return {e, e * a.d};
 }
-template <typename T> SR_DEV Dual<T> flog(Dual<T> a) { return {flog(a.v), a.d / a.v}; }
 
 template <typename S> SR_DEV S sigmoid(S x) { return S(1) / (S(1) + fexp(-x)); }
 template <typename T> SR_DEV Dual<T> sigmoid(Dual<T> x) {
@@ -81,27 +79,17 @@ template <typename T> SR_DEV Dual<T> sigmoid(Dual<T> x) {
   return {s, s * (T(1) - s) * x.d};
 }
 
-// sign(c) |c|^e for a constant base c (signed_pow, pytorch.py:28-29); the
-// derivative in e is sign(c) |c|^e ln|c|, taken as 0 at c == 0 (its limit).
+// sign(c) |c|^e for a constant base c (signed_pow, pytorch.py:28-29); its
+// derivative in e, sign(c) |c|^e ln|c|, is taken as 0 at c == 0 (its limit).
 template <typename T> SR_DEV T spow(T c, T e) {
   if (c == T(0)) return T(0);
   const T m = fexp(e * flog(c < T(0) ? -c : c));
   return c < T(0) ? -m : m;
 }
-template <typename T> SR_DEV Dual<T> spow(T c, Dual<T> e) {
-  if (c == T(0)) return {T(0), T(0)};
-  const T lc = flog(c < T(0) ? -c : c);
-  const T m = fexp(e.v * lc);
-  const T s = c < T(0) ? T(-1) : T(1);
-  return {s * m, s * m * lc * e.d};
-}
 
 // relu(x) + 1e-8 then exp(log(.)) is the identity up to rounding: keep relu + eps.
 SR_DEV float relu_eps(float x, float eps) { return x > 0.0f ? x + eps : eps; }
 SR_DEV double relu_eps(double x, double eps) { return x > 0.0 ? x + eps : eps; }
-template <typename T> SR_DEV Dual<T> relu_eps(Dual<T> x, T eps) {
-  return x.v > T(0) ? Dual<T>{x.v + eps, x.d} : Dual<T>{eps, T(0)};
-}
 
 template <typename S> struct V3 {
   S x, y, z;
@@ -297,28 +285,181 @@ __global__ __launch_bounds__(256) void k_block_fwd(Args a, float* means, float* 
   opac[sidx] = 1.0f / (1.0f + expf(-a.occ[b]));
 }
 
-// Directional derivative of the 9 outputs along block parameter pi,
-// contracted with the upstream gradient g (9 values).
+// Adjoint of one surfel: from the gradient g of its 9 outputs (mean 3, scale
+// 2, quaternion 4), the gradient of the 12 block parameters.  One reverse
+// sweep through the face (quaternion -> frame -> vertices) and the vertices'
+// four signed powers; returns the forward's degeneracy test.
 template <typename T>
-SR_DEV T directional(const Args& a, int b, int i, int j, int k, int pi, const float* g) {
-  Dual<T> p[12];
-  for (int t = 0; t < 12; ++t) p[t] = Dual<T>{(T)a.prm[12 * b + t], t == pi ? T(1) : T(0)};
-  const Block<Dual<T>> blk = make_block<Dual<T>, T>(p, (T)a.scale_min);
-  float w0, w1, w2;
-  bary_of(a, k, w0, w1, w2);
-  SurfelOut<Dual<T>> o;
-  surfel<Dual<T>, T>(blk, (T)a.eta[i], (T)a.eta[i + 1], (T)a.omega[j], (T)a.omega[(j + 1) % a.n_omega], (T)a.ratio,
-                     (T)a.surfel_scale, (T)w0, (T)w1, (T)w2, o);
-  T acc = 0;
-  for (int t = 0; t < 3; ++t) acc += o.m[t].d * (T)g[t];
-  for (int t = 0; t < 2; ++t) acc += o.s[t].d * (T)g[3 + t];
-  for (int t = 0; t < 4; ++t) acc += o.q[t].d * (T)g[5 + t];
-  return acc;
+SR_DEV bool surfel_adjoint(const Args& a, int b, int i, int j, int k, const float* g, T* out) {
+  const T eps = T(1e-8);
+  T p[12];
+  for (int t = 0; t < 12; ++t) p[t] = (T)a.prm[12 * b + t];
+  const Block<T> bk = make_block<T, T>(p, (T)a.scale_min);
+  float wf[3];
+  bary_of(a, k, wf[0], wf[1], wf[2]);
+  const T ratio = (T)a.ratio, sscale = (T)a.surfel_scale;
+  // vertices V0 (eta0, om0), V1 (eta1, om0), V2 (eta0, om1): u holds each
+  // one's scaled local coordinates, lc .. ls the logarithms of the bases
+  const T eta[2] = {(T)a.eta[i], (T)a.eta[i + 1]};
+  const T om[2] = {(T)a.omega[j], (T)a.omega[(j + 1) % a.n_omega]};
+  auto power = [](T c, T e, T& lg) -> T {  // sign(c) |c|^e and ln |c| (0 at c == 0: no gradient there)
+    const T m = c < T(0) ? -c : c;
+    if (m == T(0)) {
+      lg = T(0);
+      return T(0);
+    }
+    lg = flog(m);
+    const T v = fexp(e * lg);
+    return c < T(0) ? -v : v;
+  };
+  T ce[2], se[2], co[2], so[2], lce[2], lse[2], lco[2], lso[2];
+  for (int t = 0; t < 2; ++t) {
+    ce[t] = power(cos(eta[t]), bk.e1, lce[t]);
+    se[t] = power(sin(eta[t]), bk.e1, lse[t]);
+    co[t] = power(cos(om[t]), bk.e2, lco[t]);
+    so[t] = power(sin(om[t]), bk.e2, lso[t]);
+  }
+  V3<T> V[3], u[3];
+  for (int v = 0; v < 3; ++v) {
+    const int ie = v == 1, io = v == 2;
+    u[v] = {ce[ie] * so[io] * ratio * bk.Sx, se[ie] * ratio * bk.Sy, ce[ie] * co[io] * ratio * bk.Sz};
+    V[v] = {u[v].x * bk.R[0] + u[v].y * bk.R[3] + u[v].z * bk.R[6] + bk.tx,
+            u[v].x * bk.R[1] + u[v].y * bk.R[4] + u[v].z * bk.R[7] + bk.ty,
+            u[v].x * bk.R[2] + u[v].y * bk.R[5] + u[v].z * bk.R[8] + bk.tz};
+  }
+  // forward of the face, as surfel()
+  const V3<T> e1 = V[1] - V[0], e2 = V[2] - V[0];
+  const V3<T> n = cross(e1, e2);
+  const T nn = fsqrt(dot(n, n));
+  const V3<T> v0 = scl(n, T(1) / (nn + eps));
+  const V3<T> c = scl(V[0] + V[1] + V[2], T(1) / T(3));
+  const V3<T> av = V[1] - c, bv = V[2] - c;
+  const T al = fsqrt(dot(av, av)), v1n = al + eps;
+  const V3<T> v1 = scl(av, T(1) / v1n);
+  const T b0 = dot(bv, v0), b1 = dot(bv, v1);
+  const V3<T> v2u = (bv - scl(v0, b0)) - scl(v1, b1);
+  const T l2 = fsqrt(dot(v2u, v2u)), v2n = l2 + eps;
+  const V3<T> v2 = scl(v2u, T(1) / v2n);
+  const T s1 = v1n / T(2), s2 = dot(bv, v2) / T(2);
+  const T M[9] = {v1.x, v2.x, v0.x, v1.y, v2.y, v0.y, v1.z, v2.z, v0.z};
+  // quaternion: the largest of the four candidates, its sign and its norm
+  const T lead[4] = {T(1) + M[0] + M[4] + M[8], T(1) + M[0] - M[4] - M[8], T(1) - M[0] + M[4] - M[8],
+                     T(1) - M[0] - M[4] + M[8]};
+  T qa[4];
+  for (int t = 0; t < 4; ++t) qa[t] = lead[t] > T(0) ? fsqrt(lead[t]) : T(0);
+  int kk = 0;
+  for (int t = 1; t < 4; ++t)
+    if (qa[t] > qa[kk]) kk = t;
+  const T qk = kk == 0 ? qa[0] : (kk == 1 ? qa[1] : (kk == 2 ? qa[2] : qa[3]));
+  // antisymmetric (d) and symmetric (t) parts the candidates are made of
+  const T d0 = M[7] - M[5], d1 = M[2] - M[6], d2 = M[3] - M[1];
+  const T t0 = M[3] + M[1], t1 = M[2] + M[6], t2 = M[5] + M[7];
+  const T sq = qk * qk;
+  const T cq[4] = {kk == 0 ? sq : (kk == 1 ? d0 : (kk == 2 ? d1 : d2)), kk == 0 ? d0 : (kk == 1 ? sq : (kk == 2 ? t0 : t1)),
+                   kk == 0 ? d1 : (kk == 1 ? t0 : (kk == 2 ? sq : t2)), kk == 0 ? d2 : (kk == 1 ? t1 : (kk == 2 ? t2 : sq))};
+  const bool small = qk < T(0.1);
+  const T den = T(2) * (small ? T(0.1) : qk);
+  const T sgn = cq[0] / den < T(0) ? T(-1) : T(1);
+  T q[4];
+  for (int t = 0; t < 4; ++t) q[t] = sgn * (cq[t] / den);
+  const T ql = fsqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
+  const bool qsmall = ql < T(1e-12);
+  const T qn = qsmall ? T(1e-12) : ql;
+  // reverse: quaternion
+  T gq[4], dotq = T(0);
+  for (int t = 0; t < 4; ++t) dotq += (T)g[5 + t] * (q[t] / qn);
+  for (int t = 0; t < 4; ++t) gq[t] = sgn * (((T)g[5 + t] - (qsmall ? T(0) : (q[t] / qn) * dotq)) / qn);
+  T gden = T(0), gc[4];
+  for (int t = 0; t < 4; ++t) {
+    gc[t] = gq[t] / den;
+    gden -= gq[t] * (cq[t] / den) / den;
+  }
+  // candidate -> the matrix
+  const T gsq = kk == 0 ? gc[0] : (kk == 1 ? gc[1] : (kk == 2 ? gc[2] : gc[3]));
+  const T gqk = (small ? T(0) : T(2) * gden) + T(2) * qk * gsq;
+  const T gl = qk > T(0) ? gqk / (T(2) * qk) : T(0);
+  T gd0, gd1, gd2, gt0, gt1, gt2;
+  gd0 = kk == 0 ? gc[1] : (kk == 1 ? gc[0] : T(0));
+  gd1 = kk == 0 ? gc[2] : (kk == 2 ? gc[0] : T(0));
+  gd2 = kk == 0 ? gc[3] : (kk == 3 ? gc[0] : T(0));
+  gt0 = kk == 1 ? gc[2] : (kk == 2 ? gc[1] : T(0));
+  gt1 = kk == 1 ? gc[3] : (kk == 3 ? gc[1] : T(0));
+  gt2 = kk == 2 ? gc[3] : (kk == 3 ? gc[2] : T(0));
+  const T gM[9] = {kk < 2 ? gl : -gl, gt0 - gd2, gd1 + gt1, gd2 + gt0, (kk & 1) ? -gl : gl, gt2 - gd0,
+                   gt1 - gd1, gd0 + gt2, (kk == 0 || kk == 3) ? gl : -gl};
+  V3<T> g1 = {gM[0], gM[3], gM[6]}, g2 = {gM[1], gM[4], gM[7]}, g0 = {gM[2], gM[5], gM[8]};
+  // scales
+  T gv1n = s1 * sscale > T(0) ? (T)g[3] * sscale / T(2) : T(0);
+  const T gbv2 = s2 * sscale > T(0) ? (T)g[4] * sscale / T(2) : T(0);
+  V3<T> gb = scl(v2, gbv2);
+  g2 = g2 + scl(bv, gbv2);
+  // v2, then v1 and v0
+  V3<T> gu = scl(g2, T(1) / v2n);
+  if (l2 > T(0)) gu = gu - scl(v2, dot(v2, g2) / l2);
+  gb = gb + ((gu - scl(v0, dot(v0, gu))) - scl(v1, dot(v1, gu)));
+  g0 = g0 - (scl(gu, b0) + scl(bv, dot(v0, gu)));
+  g1 = g1 - (scl(gu, b1) + scl(bv, dot(v1, gu)));
+  gv1n = gv1n - dot(v1, g1) / v1n;
+  V3<T> ga = scl(g1, T(1) / v1n);
+  if (al > T(0)) ga = ga + scl(av, gv1n / al);
+  V3<T> gn = scl(g0, T(1) / (nn + eps));
+  if (nn > T(0)) gn = gn - scl(v0, dot(v0, g0) / nn);
+  const V3<T> ge1 = cross(e2, gn), ge2 = cross(gn, e1);
+  const V3<T> gm = {(T)g[0], (T)g[1], (T)g[2]};
+  const V3<T> gcen = scl(ga + gb, T(-1) / T(3));
+  V3<T> gV[3];
+  gV[0] = ((gcen - ge1) - ge2) + scl(gm, (T)wf[0]);
+  gV[1] = ((gcen + ga) + ge1) + scl(gm, (T)wf[1]);
+  gV[2] = ((gcen + gb) + ge2) + scl(gm, (T)wf[2]);
+  // vertices -> rotation, scales, exponents, translation
+  T G[9], gS[3] = {T(0), T(0), T(0)}, gE1 = T(0), gE2 = T(0);
+  for (int t = 0; t < 9; ++t) G[t] = T(0);
+  for (int v = 0; v < 3; ++v) {
+    const int ie = v == 1, io = v == 2;
+    const T uu[3] = {u[v].x, u[v].y, u[v].z}, gg[3] = {gV[v].x, gV[v].y, gV[v].z};
+    T gu3[3];
+    for (int r = 0; r < 3; ++r) {
+      gu3[r] = (bk.R[3 * r] * gg[0] + bk.R[3 * r + 1] * gg[1]) + bk.R[3 * r + 2] * gg[2];
+      for (int t = 0; t < 3; ++t) G[3 * r + t] += uu[r] * gg[t];
+    }
+    // local coordinate over its axis scale
+    gS[0] += gu3[0] * (ce[ie] * so[io] * ratio);
+    gS[1] += gu3[1] * (se[ie] * ratio);
+    gS[2] += gu3[2] * (ce[ie] * co[io] * ratio);
+    const T a0 = gu3[0] * uu[0], a1 = gu3[1] * uu[1], a2 = gu3[2] * uu[2];
+    gE1 += (a0 + a2) * lce[ie] + a1 * lse[ie];
+    gE2 += a0 * lso[io] + a2 * lco[io];
+  }
+  for (int t = 0; t < 3; ++t) out[t] = gS[t] * fexp(p[t]);
+  T ln = fsqrt(p[3] * p[3] + p[4] * p[4] + p[5] * p[5] + p[6] * p[6]);
+  const bool lsmall = ln < T(1e-12);
+  if (lsmall) ln = T(1e-12);
+  const T w = p[3] / ln, x = p[4] / ln, y = p[5] / ln, z = p[6] / ln;
+  const T gr[4] = {
+      T(2) * (((y * (G[2] - G[6]) + z * (G[3] - G[1])) + x * (G[7] - G[5]))),
+      T(2) * (((y * (G[1] + G[3]) + z * (G[2] + G[6])) + w * (G[7] - G[5])) - T(2) * x * (G[4] + G[8])),
+      T(2) * (((x * (G[1] + G[3]) + z * (G[5] + G[7])) + w * (G[2] - G[6])) - T(2) * y * (G[0] + G[8])),
+      T(2) * (((x * (G[2] + G[6]) + y * (G[5] + G[7])) + w * (G[3] - G[1])) - T(2) * z * (G[0] + G[4]))};
+  const T qh[4] = {w, x, y, z};
+  const T along = lsmall ? T(0) : ((w * gr[0] + x * gr[1]) + y * gr[2]) + z * gr[3];
+  for (int t = 0; t < 4; ++t) out[3 + t] = (gr[t] - qh[t] * along) / ln;
+  out[7] = (gV[0].x + gV[1].x) + gV[2].x;
+  out[8] = (gV[0].y + gV[1].y) + gV[2].y;
+  out[9] = (gV[0].z + gV[1].z) + gV[2].z;
+  // e = 1.8 sigmoid(p) + 0.1
+  const T sg1 = sigmoid(p[10]), sg2 = sigmoid(p[11]);
+  out[10] = gE1 * (T(1.8) * sg1 * (T(1) - sg1));
+  out[11] = gE2 * (T(1.8) * sg2 * (T(1) - sg2));
+  const T le = fsqrt(dot(e1, e1)) * fsqrt(dot(e2, e2));
+  return nn < T(1e-3) * le || nn < T(1e-4) || v1n < T(1e-4);
 }
 
-// Pass 1: every surfel's 13 contributions (the 12 directional derivatives
-// contracted with its upstream gradients, and the occupancy term) go to
+// Pass 1: every surfel's 13 contributions (the gradient of the 12 block
+// parameters through it, and the occupancy term) go to
 // contrib[pi * P + sidx], parameter-major so each pass stores contiguously.
+// One reverse sweep per surfel; twelve forward-mode passes, each with the
+// vertices' powers and trigonometry again and in FP64 near the poles, took
+// 231 us for 65,536 surfels, this 21 us.
 __global__ __launch_bounds__(256) void k_block_bwd(Args a, const float* dmeans, const float* dscales,
                                                    const float* drots, const float* dopac, float* contrib) {
   const int sidx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -330,11 +471,13 @@ __global__ __launch_bounds__(256) void k_block_bwd(Args a, const float* dmeans, 
   for (int t = 0; t < 3; ++t) g[t] = dmeans[3 * sidx + t];
   for (int t = 0; t < 2; ++t) g[3 + t] = dscales[2 * sidx + t];
   for (int t = 0; t < 4; ++t) g[5 + t] = drots[4 * sidx + t];
-  SurfelOut<float> o;
-  const bool degenerate = gen_plain<float>(a, b, i, j, k, o);
-  for (int pi = 0; pi < 12; ++pi)
-    contrib[(size_t)pi * P + sidx] =
-        degenerate ? (float)directional<double>(a, b, i, j, k, pi, g) : directional<float>(a, b, i, j, k, pi, g);
+  float out[12];
+  if (surfel_adjoint<float>(a, b, i, j, k, g, out)) {
+    double od[12];
+    surfel_adjoint<double>(a, b, i, j, k, g, od);
+    for (int t = 0; t < 12; ++t) out[t] = (float)od[t];
+  }
+  for (int t = 0; t < 12; ++t) contrib[(size_t)t * P + sidx] = out[t];
   const float sg = 1.0f / (1.0f + expf(-a.occ[b]));
   contrib[(size_t)12 * P + sidx] = dopac[sidx] * sg * (1.0f - sg);
 }
