@@ -186,7 +186,6 @@ struct Pipeline {
   ImageLayout il{};
   BinLayout bl{};
   int capacity = 0;
-  bool side_huge = false;  // huge-tile sort on a second stream (graph-captured batches)
   bool part = false;       // the _part variant
   int S = 0;               // its semantic channels
   uint32_t* counters() const { return (uint32_t*)(img + il.counters); }
@@ -376,8 +375,8 @@ int run_front(Pipeline& pl, const sr_surfels* g, int* radii, uint32_t capacity, 
            launch_scan_tiles(pl.il.T, tile_count, (uint32_t*)(pl.img + pl.il.tile_start),
                              (uint32_t*)(pl.img + pl.il.tile_fill), (uint32_t*)(pl.img + pl.il.ranges), counters,
                              capacity, pl.vs.V * ((pl.P + 255) / 256), (uint32_t*)(pl.geom + pl.gl.bsum),
-                             (uint32_t*)(pl.geom + pl.gl.ssum), slot_capacity, (uint32_t*)(pl.img + pl.il.large), (uint32_t*)(pl.img + pl.il.lchunk_off),
-                             pl.side_huge ? kSmallMax : kLargeMax, st));
+                             (uint32_t*)(pl.geom + pl.gl.ssum), slot_capacity, (uint32_t*)(pl.img + pl.il.large),
+                             (uint32_t*)(pl.img + pl.il.seg_off), st));
   return SR_OK;
 }
 
@@ -409,22 +408,21 @@ int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st) {
   sa.counters = counters;
   sa.large = (const uint32_t*)(pl.img + pl.il.large);
   sa.keys = (uint64_t*)(bin + bl.keys);
-  sa.lmeta = (uint2*)(bin + bl.lmeta);
-  sa.lpre = (uint16_t*)(bin + bl.lpre);
-  sa.lchunk_off = (const uint32_t*)(pl.img + pl.il.lchunk_off);
-  sa.side_huge = pl.side_huge ? 1 : 0;
+  sa.key2 = (uint64_t*)(bin + bl.key2);
+  sa.seg_off = (const uint32_t*)(pl.img + pl.il.seg_off);
+  sa.seg_start = (uint32_t*)(bin + bl.seg_start);
+  sa.seg_hits = (uint32_t*)(bin + bl.seg_hits);
   sa.point_list = (uint32_t*)(bin + bl.point_list);
   sa.cullbox = (const short4*)(pl.geom + pl.gl.cullbox);
   sa.inst_rs = (const uint2*)(bin + bl.inst_rs);
   sa.pos_slot = (uint32_t*)(bin + bl.pos_slot);
   sa.pos_quads = (uint16_t*)(bin + bl.pos_quads);
-  sa.lslot = (uint32_t*)(bin + bl.lslot);
   sa.sub = (uint2*)(bin + bl.sub);
   sa.sub_count = (uint32_t*)(pl.img + pl.il.sub_count);
   sa.work = (uint2*)(bin + bl.work);
   sa.work_count = counters + 2;
   sa.q_flag = (uint32_t*)(pl.img + pl.il.q_flag);
-  SR_STAGE(3, dbg, st, "sort", launch_sort_tiles(sa, st));
+  SR_STAGE(3, dbg, st, "sort", launch_sort_tiles(sa, segment_capacity((size_t)pl.capacity), st));
   AcceptArgs aa{};
   aa.vs = pl.vs;
   aa.ranges = sa.ranges;
@@ -871,13 +869,6 @@ int sr_forward_batched(const sr_views* v, const sr_surfels* g, void* ws, size_t 
   if (ws_bytes < bl.total)
     return fail(SR_ERR_INVALID, "workspace holds %zu bytes, needs %zu", ws_bytes, bl.total);
   Pipeline pl = batch_pipeline(v, g, vs, bl, (char*)ws, capacity);
-  // Many views hold thousands of tiles above kSmallMax instances: sorting
-  // them in chunks and merging by rank does more work in all than one
-  // workgroup per tile, and throughput is what counts here (latency of the
-  // few largest tiles is what counts for one view).  So every tile above
-  // kSmallMax takes the one-workgroup sort, beside the small-tile sort on a
-  // second stream (a captured graph makes the fork cheap).
-  pl.side_huge = true;
   rc = run_front(pl, g, radii, (uint32_t)capacity, (uint32_t)bl.bl.nslot, false, st);
   if (rc == SR_OK) rc = run_binning(pl, radii, false, st);
   if (rc == SR_OK) rc = run_blend_fwd(pl, out_color, out_others, false, st);

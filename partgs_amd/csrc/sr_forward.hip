@@ -8,13 +8,11 @@
 //   k_scatter      per surfel: writes a 64-bit key (depth bits << 32 | surfel
 //                  id) for every covered tile into that tile's bucket.
 //   k_sort_tiles   one workgroup per tile of up to 2048 instances: sorts its
-//                  bucket in LDS (bitonic runs, merge-path levels), emits
+//                  bucket in LDS (depth bins, ranks within a bin), emits
 //                  point_list, then splits the sorted list into
-//                  per-8x8-quadrant sub-lists; larger tiles: one workgroup
-//                  per 2048-key chunk, sorted the same way.
-//   k_merge_chunks the large tiles' chunks merged: every entry placed in the
-//                  tile list and the sub-lists by its ranks in the other
-//                  chunks (binary search in LDS).
+//                  per-8x8-quadrant sub-lists.
+//   k_split_large  larger tiles cut by depth into segments, which k_sort_tiles
+//                  sorts too; k_segment_lists joins their sub-lists.
 //   k_blend_fwd    one wave64 per 8 x 8 quadrant, one lane per pixel: front-
 //                  to-back alpha blending of colour, depth, alpha, normal,
 //                  median depth and depth distortion over the sub-list.
@@ -22,6 +20,8 @@
 // Sorting each tile bucket by (depth bits, surfel id) gives exactly the order
 // of the reference's stable radix sort over (tile, depth) keys emitted in
 // surfel order (dsr/cuda_rasterizer/rasterizer_impl.cu:70-111, 301-309).
+#include <algorithm>
+
 #include "sr_device.h"
 #include "sr_internal.h"
 #include "sr_pair.h"
@@ -613,10 +613,9 @@ SR_DEV void scan1024_excl(uint32_t* s, uint32_t (&x)[N], uint32_t (&total)[N]) {
 }
 
 // Exclusive scan of the tile histogram by one 1024-lane workgroup, with the
-// list of tiles of kSmallMax < n <= large_max (count in counters[3]) and the
-// number of each one's first kSmallMax-key chunk (lchunk_off, followed by
-// the total, which also goes to counters[6]), and the tiles above large_max
-// from the end of the same list (count in counters[7]);
+// list of tiles above kSmallMax instances (count in counters[3]) and the
+// number of each one's first kSegKeys-key segment (seg_off, followed by the
+// total, which also goes to counters[6]);
 // then the same scan for the per-workgroup instance totals of the
 // preprocess (in place), which numbers every record's instances in record
 // order.
@@ -626,30 +625,24 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32
                                                               uint32_t* ranges, uint32_t* counters,
                                                               uint32_t capacity, int nb, uint32_t* bsum,
                                                               uint32_t* ssum, uint32_t slot_capacity,
-                                                              uint32_t* large, uint32_t* lchunk_off,
-                                                              int large_max) {
+                                                              uint32_t* large, uint32_t* seg_off) {
   __shared__ uint32_t s_part[3 * 32];
   const int tid = threadIdx.x;
   const int per = (T + kScanThreads - 1) / kScanThreads;
   const int b = tid * per;
   const int e = min(T, b + per);
-  auto chunks = [](uint32_t c) { return (c + (uint32_t)kSmallMax - 1u) / (uint32_t)kSmallMax; };
-  auto is_large = [&](uint32_t c) { return c > (uint32_t)kSmallMax && c <= (uint32_t)large_max; };
-  // this lane's tiles: instances, large tiles, their chunks, huge tiles
-  uint32_t v1[1] = {0u}, v3[3] = {0u, 0u, 0u};
+  // this lane's tiles: instances, large tiles, their segments
+  uint32_t v3[3] = {0u, 0u, 0u}, tot3[3];
   for (int i = b; i < e; ++i) {
     const uint32_t c = count[i];
-    v1[0] += c;
-    if (is_large(c)) {
-      v3[0] += 1u;
-      v3[1] += chunks(c);
+    v3[0] += c;
+    if (c > (uint32_t)kSmallMax) {
+      v3[1] += 1u;
+      v3[2] += segments_of(c);
     }
-    v3[2] += c > (uint32_t)large_max ? 1u : 0u;
   }
-  uint32_t tot1[1], tot3[3];
-  scan1024_excl(s_part, v1, tot1);
   scan1024_excl(s_part, v3, tot3);
-  uint32_t run = v1[0], at = v3[0], cat = v3[1], hat = v3[2];
+  uint32_t run = v3[0], at = v3[1], sat = v3[2];
   for (int i = b; i < e; ++i) {
     const uint32_t c = count[i];
     start[i] = run;
@@ -657,22 +650,19 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32
     ranges[2 * i] = c ? run : 0u;
     ranges[2 * i + 1] = c ? run + c : 0u;
     run += c;
-    if (is_large(c)) {
+    if (c > (uint32_t)kSmallMax) {
       large[at] = (uint32_t)i;
-      lchunk_off[at] = cat;
-      ++at;
-      cat += chunks(c);
+      seg_off[at++] = sat;
+      sat += segments_of(c);
     }
-    if (c > (uint32_t)large_max) large[T - 1 - (int)hat++] = (uint32_t)i;
   }
   if (tid == kScanThreads - 1) {
-    start[T] = tot1[0];
-    counters[0] = tot1[0];
-    if (tot1[0] > capacity) atomicOr(&counters[1], kErrCapacity);
-    counters[3] = tot3[0];
-    counters[6] = tot3[1];
-    counters[7] = tot3[2];
-    lchunk_off[tot3[0]] = tot3[1];
+    start[T] = tot3[0];
+    counters[0] = tot3[0];
+    if (tot3[0] > capacity) atomicOr(&counters[1], kErrCapacity);
+    counters[3] = tot3[1];
+    counters[6] = tot3[2];
+    seg_off[tot3[1]] = tot3[2];
   }
   // the per-workgroup instance and slot totals of the preprocess, in place
   const int pb = (nb + kScanThreads - 1) / kScanThreads;
@@ -699,10 +689,10 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32
 
 hipError_t launch_scan_tiles(int T, const uint32_t* count, uint32_t* start, uint32_t* fill,
                              uint32_t* ranges, uint32_t* counters, uint32_t capacity, int nb, uint32_t* bsum,
-                             uint32_t* ssum, uint32_t slot_capacity, uint32_t* large, uint32_t* lchunk_off,
-                             int large_max, hipStream_t s) {
+                             uint32_t* ssum, uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off,
+                             hipStream_t s) {
   hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanThreads), 0, s, T, count, start, fill, ranges,
-                     counters, capacity, nb, bsum, ssum, slot_capacity, large, lchunk_off, large_max);
+                     counters, capacity, nb, bsum, ssum, slot_capacity, large, seg_off);
   return hipGetLastError();
 }
 
@@ -797,10 +787,9 @@ hipError_t launch_scatter(const ScatterArgs& a, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-// Per-tile sort.  Tiles with at most kSmallMax instances are sorted by a
-// 256-lane workgroup entirely in LDS (8 keys per lane); larger tiles are cut
-// into kSmallMax-key chunks, each sorted the same way by its own workgroup,
-// and merged by rank (k_sort_tiles, k_merge_chunks).
+// Per-tile sort.  A tile of up to kSmallMax instances is sorted in LDS by one
+// 512-lane workgroup.  A larger one is first split by depth into segments of
+// about kSegKeys keys (k_split_large), which are then sorted like small tiles.
 // ---------------------------------------------------------------------------
 
 // LDS slot of key i in the merge sort: one pad slot after every K keys, so
@@ -899,50 +888,6 @@ SR_DEV int next_pow2(int n) {
 // and holds (surfel id, position in the tile list) pairs.  Each non-empty
 // sub-list appends its 64-entry chunks to the acceptance work list.
 
-// The hit bits of quadrants 4g..4g+3 in the four 16-bit fields of a packed
-// counter (at most kSmallMax < 2^16 entries are counted in one scan, so
-// sums of these never carry from one field into the next).
-SR_DEV uint64_t spread4(uint32_t h, int g) {
-  const uint32_t b = h >> (4 * g);
-  return (uint64_t)(b & 1u) | ((uint64_t)((b >> 1) & 1u) << 16) | ((uint64_t)((b >> 2) & 1u) << 32) |
-         ((uint64_t)((b >> 3) & 1u) << 48);
-}
-SR_DEV uint32_t field16(uint64_t v, int f) { return (uint32_t)(v >> (16 * f)) & 0xffffu; }
-
-// Exclusive scan of one 64-bit value per lane over a 256-lane workgroup;
-// total receives the sum over all lanes.
-SR_DEV uint64_t scan256_excl_u64(uint64_t v, uint64_t* s_w, uint64_t& total) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  uint64_t incl = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t lo = (uint32_t)__shfl_up((int)(uint32_t)incl, d);
-    const uint32_t hi = (uint32_t)__shfl_up((int)(uint32_t)(incl >> 32), d);
-    if (lane >= d) incl += ((uint64_t)hi << 32) | lo;
-  }
-  if (lane == 63) s_w[wave] = incl;
-  __syncthreads();
-  const uint64_t w0 = s_w[0], w1 = s_w[1], w2 = s_w[2], w3 = s_w[3];
-  __syncthreads();
-  total = w0 + w1 + w2 + w3;
-  const uint64_t off = (wave > 0 ? w0 : 0ull) + (wave > 1 ? w1 : 0ull) + (wave > 2 ? w2 : 0ull);
-  return off + incl - v;
-}
-
-// After an LDS sort of cn keys (bucket entries c0 .. c0 + cn - 1 of tile
-// `tile`, whose bucket starts at beg and holds n), by a 256-lane workgroup:
-// lane tid takes the K consecutive sorted entries tid K .. tid K + K - 1,
-// looks up their records and cull boxes (all in flight at once), and one
-// packed scan per four quadrants numbers every entry's hits.
-// kWhole (c0 == beg, cn == n): writes point_list, each position's first
-// slot and quadrant mask (pos_slot, pos_quads) and the quadrant sub-lists,
-// their lengths and the acceptance work items.  Otherwise (one chunk of a
-// larger tile): writes the sorted keys back in place, and per entry
-// (record, quadrant mask) to lmeta, its first slot to lslot and, per
-// quadrant, the number of the chunk's earlier entries that hit it to lpre,
-// for k_merge_chunks.
-constexpr int kSortThreads = 256;
-
 // Called by one whole wave; lane q < Q holds the length of the tile's
 // sub-list q.  Writes the lengths and clears the overflow flags, and appends
 // the sub-lists' 64-entry chunks to the acceptance work list with one atomic
@@ -969,252 +914,219 @@ SR_DEV void append_work(const SortArgs& a, int tile, int Q, uint32_t cnt) {
   }
 }
 
-template <bool kWhole>
-SR_DEV void place_sorted(const SortArgs& a, int tile, uint32_t beg, int n, uint32_t c0, int cn,
-                         const uint64_t* s_keys) {
-  constexpr int K = kSmallMax / kSortThreads;
-  __shared__ uint64_t s_w[kSortThreads / 64];
+// LDS of a tile sort: K keys per lane of NT, and NB bins.
+template <int NT, int K, int NB> struct TileLds {
+  static constexpr int kKeys = NT * K;
+  // the keys (the merge sort pads them by one slot per K), then the bins
+  static constexpr int kBytes = (kKeys + NT) * 8 > kKeys * 8 + (NB + 1) * 4 ? (kKeys + NT) * 8 : kKeys * 8 + (NB + 1) * 4;
+};
+
+// Keys whose depths share one bin are ranked against each other, so a tile
+// with a fuller bin than this (equal or nearly equal depths) goes through the
+// merge sort instead.
+constexpr uint32_t kBinMax = 128;
+
+// Sorts the n <= NT K keys of a bucket at `src` and returns in inst[r] the
+// instance number (the key's low word) of sorted entry r NT + tid.
+//
+// The depths are cut into NB equal bins between the tile's smallest and
+// largest (depth bits, a monotone map), the keys counted into the bins, the
+// bins scanned, and the keys placed by bin; a key's rank is then its bin's
+// start plus the number of smaller keys in the bin.  Keys are unique, so this
+// is the sorted order whatever order the lanes arrive in.  About 6 + n / NB
+// dependent LDS accesses a key, where the merge sort it falls back to makes 50
+// to 300.
+template <int NT, int K, int NB>
+SR_DEV void sort_bucket(const uint64_t* src, int n, char* lds, uint32_t (&inst)[K]) {
+  constexpr int NW = NT / 64, per = NB / NT;
+  static_assert(NB % NT == 0, "whole bins per lane");
+  __shared__ uint32_t s_w[NW];
+  __shared__ uint32_t s_red[2][NW];
+  __shared__ uint32_t s_full;
+  uint64_t* keys = reinterpret_cast<uint64_t*>(lds);
+  uint32_t* bins = reinterpret_cast<uint32_t*>(lds + (size_t)NT * K * 8);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // all K loads in flight: unconditional, the index clamped into the bucket
+  uint64_t kv[K];
+#pragma unroll
+  for (int r = 0; r < K; ++r) kv[r] = src[min(r * NT + tid, n - 1)];
+  uint32_t lo = 0xFFFFFFFFu, hi = 0u;
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    const uint32_t d = (uint32_t)(kv[r] >> 32);
+    lo = min(lo, d);
+    hi = max(hi, d);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
+    hi = max(hi, (uint32_t)__shfl_xor((int)hi, off, 64));
+  }
+  if (lane == 0) {
+    s_red[0][wave] = lo;
+    s_red[1][wave] = hi;
+  }
+  if (tid == 0) s_full = 0u;
+#pragma unroll
+  for (int t = 0; t < per; ++t) bins[t * NT + tid] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    lo = min(lo, s_red[0][w]);
+    hi = max(hi, s_red[1][w]);
+  }
+  const float scale = (float)NB / ((float)(hi - lo) + 1.0f);
+  auto bin_of = [&](uint64_t k) {
+    return min(NB - 1, (int)((float)((uint32_t)(k >> 32) - lo) * scale));
+  };
+  uint32_t at[K];
+#pragma unroll
+  for (int r = 0; r < K; ++r)
+    if (r * NT + tid < n) at[r] = atomicAdd(&bins[bin_of(kv[r])], 1u);
+  __syncthreads();
+  uint32_t c[per], sum = 0u, top = 0u;
+#pragma unroll
+  for (int t = 0; t < per; ++t) {
+    c[t] = bins[tid * per + t];
+    sum += c[t];
+    top = max(top, c[t]);
+  }
+  uint32_t incl = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)incl, off, 64);
+    if (lane >= off) incl += y;
+  }
+  if (lane == 63) s_w[wave] = incl;
+  if (top > kBinMax) s_full = 1u;
+  __syncthreads();
+  if (s_full != 0u) {  // uniform
+#pragma unroll
+    for (int r = 0; r < K; ++r) keys[lds_slot<K>(r * NT + tid)] = r * NT + tid < n ? kv[r] : ~0ull;
+    __syncthreads();
+    merge_sort_lds<NT, K>(keys, max(next_pow2(n), K));
+#pragma unroll
+    for (int r = 0; r < K; ++r) inst[r] = (uint32_t)keys[lds_slot<K>(min(r * NT + tid, n - 1))];
+    __syncthreads();
+    return;
+  }
+  uint32_t run = incl - sum;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) run += w < wave ? s_w[w] : 0u;
+#pragma unroll
+  for (int t = 0; t < per; ++t) {
+    bins[tid * per + t] = run;
+    run += c[t];
+  }
+  if (tid == NT - 1) bins[NB] = run;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < K; ++r)
+    if (r * NT + tid < n) keys[bins[bin_of(kv[r])] + at[r]] = kv[r];
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    at[r] = 0u;
+    if (r * NT + tid < n) {
+      const int b = bin_of(kv[r]);
+      const uint32_t b0 = bins[b], b1 = bins[b + 1];
+      uint32_t below = b0;
+      for (uint32_t m = b0; m < b1; ++m) below += keys[m] < kv[r] ? 1u : 0u;
+      at[r] = below;
+    }
+  }
+  __syncthreads();
+  uint32_t* order = reinterpret_cast<uint32_t*>(lds);
+#pragma unroll
+  for (int r = 0; r < K; ++r)
+    if (r * NT + tid < n) order[at[r]] = (uint32_t)kv[r];
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < K; ++r) inst[r] = order[min(r * NT + tid, n - 1)];
+  __syncthreads();
+}
+
+// Looks up sorted entries' records (inst[r]: the instance of entry
+// r NT + tid of the cnt entries from tile-list position pos on), writes
+// point_list, each position's first slot and quadrant mask, and returns the
+// records and masks (no quadrant past the end).  Consecutive lanes write
+// consecutive positions; the gathers are unconditional (entries past the end
+// repeat the last one), so each round has all K loads in flight.
+template <int NT, int K>
+SR_DEV void place_entries(const SortArgs& a, int tile, uint32_t pos, int cnt, const uint32_t (&inst)[K],
+                          uint32_t (&rid)[K], uint32_t (&hm)[K]) {
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
   const int ltile = tile - (int)vi.tile_base;
   const int tx = ltile % vi.gx, ty = ltile / vi.gx;
   const int tid = threadIdx.x;
-  uint32_t inst[K], rid[K], sl[K], hm[K];  // instance number: the key's low half
-  // the gathers are unconditional (entries past the run read the run's
-  // first entry) so each round has all K loads in flight
+  uint32_t sl[K];
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int i = tid * K + k;
-    inst[k] = (uint32_t)s_keys[lds_slot<K>(i < cn ? i : 0)];
-  }
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const uint2 rs = a.inst_rs[inst[k]];
-    rid[k] = rs.x;
-    sl[k] = rs.y;
+  for (int r = 0; r < K; ++r) {
+    const uint2 rs = a.inst_rs[inst[r]];
+    rid[r] = rs.x;
+    sl[r] = rs.y;
   }
   short4 bx[K];
 #pragma unroll
-  for (int k = 0; k < K; ++k) bx[k] = a.cullbox[rid[k]];
+  for (int r = 0; r < K; ++r) bx[r] = a.cullbox[rid[r]];
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    if (tid * K + k >= cn) {
-      inst[k] = 0u;
-      rid[k] = 0u;
-      bx[k] = make_short4(32767, 32767, -32768, -32768);
+  for (int r = 0; r < K; ++r) {
+    const int i = r * NT + tid;
+    hm[r] = i < cnt ? quad_hits(bx[r], tx, ty, B, QX, Q, vi) : 0u;
+    if (i < cnt) {
+      a.point_list[pos + i] = rid[r];
+      a.pos_slot[pos + i] = sl[r];
+      a.pos_quads[pos + i] = (uint16_t)hm[r];
     }
-  }
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int i = tid * K + k;
-    if (i < cn) {
-      if constexpr (kWhole) {
-        a.point_list[c0 + i] = rid[k];
-        a.pos_slot[c0 + i] = sl[k];
-      } else {
-        a.keys[c0 + i] = s_keys[lds_slot<K>(i)];
-        a.lslot[c0 + i] = sl[k];
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int i = tid * K + k;
-    hm[k] = quad_hits(bx[k], tx, ty, B, QX, Q, vi);
-    if (i < cn) {
-      // for the gradient slots: the instance's quadrants (a chunk's go to
-      // their final positions with the merge)
-      if constexpr (kWhole) a.pos_quads[c0 + i] = (uint16_t)hm[k];
-      else a.lmeta[c0 + i] = make_uint2(rid[k], hm[k]);
-    }
-  }
-  uint2* base = a.sub + (size_t)Q * beg;
-  uint32_t my_cnt = 0;  // kWhole: lane q < Q gets sub-list q's length
-  for (int g = 0; g * 4 < Q; ++g) {  // quadrants 4g .. 4g + 3 (uniform loop)
-    uint64_t cnt = 0;
-#pragma unroll
-    for (int k = 0; k < K; ++k) cnt += spread4(hm[k], g);
-    uint64_t total;
-    uint64_t run = scan256_excl_u64(cnt, s_w, total);
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int i = tid * K + k;
-      if (i < cn) {
-        if constexpr (kWhole) {
-#pragma unroll
-          for (int f = 0; f < 4; ++f) {
-            const int q = 4 * g + f;
-            if (q < Q && ((hm[k] >> q) & 1u))
-              base[(size_t)q * n + field16(run, f)] = make_uint2(rid[k], (uint32_t)i);
-          }
-        } else {
-          uint16_t* d = a.lpre + (size_t)(c0 + i) * Q + 4 * g;
-          if (Q >= 4) *reinterpret_cast<uint64_t*>(d) = run;
-          else *d = (uint16_t)run;
-        }
-      }
-      run += spread4(hm[k], g);
-    }
-    if constexpr (kWhole)
-      if (tid >= 4 * g && tid < min(Q, 4 * g + 4)) my_cnt = field16(total, tid - 4 * g);
-  }
-  if constexpr (kWhole) {
-    if (tid < 64) append_work(a, tile, Q, my_cnt);
   }
 }
 
-// Loads bucket entries c0 .. c0 + cn - 1 (cn <= kSmallMax) into LDS, padded
-// to a power of two, and sorts them.
-SR_DEV void sort_run(const SortArgs& a, uint32_t c0, int cn, uint64_t* s_keys) {
-  constexpr int K = kSmallMax / kSortThreads;
-  const int tid = threadIdx.x;
-  const int S = max(next_pow2(cn), K);
-  // all K loads in flight at once: unconditional (index clamped into the
-  // run), the padding applied afterwards
-  uint64_t kv[K];
+// Appends entries r NT + tid (record rid[r], quadrants hm[r], position
+// first + r NT + tid in the tile's list) to the tile's quadrant sub-lists in
+// order.  Per quadrant, the hits of every (round, wave) are counted by ballot
+// and scanned by one wave.  s_base[q]: entries the sub-list holds already;
+// advanced by the new ones.
+template <int NT, int K>
+SR_DEV void append_sublists(const SortArgs& a, uint32_t beg, int n, int first, int Q, const uint32_t (&rid)[K],
+                            const uint32_t (&hm)[K], uint32_t* s_cnt, uint32_t* s_base) {
+  constexpr int NW = NT / 64, E = K * NW;  // counts per quadrant, in entry order
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 #pragma unroll
-  for (int k = 0; k < K; ++k) kv[k] = a.keys[c0 + (uint32_t)min(tid + k * kSortThreads, cn - 1)];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int i = tid + k * kSortThreads;
-    if (i < S) s_keys[lds_slot<K>(i)] = i < cn ? kv[k] : ~0ull;
+  for (int r = 0; r < K; ++r) {
+    for (int q = 0; q < Q; ++q) {  // uniform
+      const uint64_t m = __ballot((hm[r] >> q) & 1u);
+      if (lane == 0) s_cnt[q * E + r * NW + wave] = (uint32_t)__popcll(m);
+    }
   }
   __syncthreads();
-  merge_sort_lds<kSortThreads, K>(s_keys, S);
-}
-
-// Tiles with more than kSmallMax instances, in two passes over the chunks
-// of the scan's list of them: chunk item i (of counters[6]) is chunk
-// i - lchunk_off[l] of large tile l, the last with lchunk_off[l] <= i; a
-// fixed number of workgroups stride over the items.  The bucket is cut into
-// chunks of kSmallMax keys.  k_sort_tiles sorts each chunk in LDS (in place in
-// `keys`), looks up its records and their quadrants, and stores per entry
-// (record, quadrant mask) in lmeta and, per quadrant, the number of the
-// chunk's earlier entries that hit it (lpre).  k_merge_chunks then places
-// every entry: its position in the tile list is its rank in its own chunk
-// plus, for every other chunk, the number of that chunk's keys below it
-// (binary search in LDS); its position
-// in sub-list q is likewise its own lpre plus the other chunks' hits of q
-// below it.  Keys are unique, so this is the merge of the sorted chunks,
-// and the lists equal those of sorting the whole bucket at once.
-#ifndef SR_CHUNK_BLOCKS
-#define SR_CHUNK_BLOCKS 256
-#endif
-constexpr uint32_t kChunkBlocks = SR_CHUNK_BLOCKS;  // workgroups striding over the chunk items, per pass
-
-// Large tile and chunk of chunk item `it` (< counters[6]).
-SR_DEV void chunk_item(const SortArgs& a, uint32_t it, uint32_t& li, int& c) {
-  uint32_t lo = 0, hi = a.counters[3];  // lchunk_off[lo] <= it < lchunk_off[hi]
-  while (hi - lo > 1u) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (a.lchunk_off[mid] <= it) lo = mid;
-    else hi = mid;
-  }
-  li = lo;
-  c = (int)(it - a.lchunk_off[lo]);
-}
-
-// Hits of quadrants 4g..4g+3 among the first j entries of a sorted chunk of
-// len entries starting at bucket entry c0 (j <= len), packed as by spread4.
-SR_DEV uint64_t chunk_hits_below(const SortArgs& a, uint32_t c0, int len, int j, int Q, int g) {
-  const int at = min(j, len - 1);
-  const uint16_t* p = a.lpre + (size_t)(c0 + (uint32_t)at) * Q + 4 * g;
-  uint64_t v = Q >= 4 ? *reinterpret_cast<const uint64_t*>(p) : (uint64_t)*p;
-  if (j == len) v += spread4(a.lmeta[c0 + (uint32_t)at].y, g);
-  return v;
-}
-
-// Places the entries of chunk c of a large tile (bucket at beg, n entries),
-// whose chunk-sorted keys are in s_tile.
-constexpr int kMergeThreads = 1024;
-SR_DEV void merge_chunk(const SortArgs& a, uint32_t beg, int n, int c, const uint64_t* s_tile) {
-  constexpr int E = kSmallMax / kMergeThreads;  // entries per lane
-  constexpr int kG = 8;                         // chunks searched together
-  const int P = (n + kSmallMax - 1) / kSmallMax;
-  const int Q = quads_per_tile(a.vs.B);
-  const int tid = threadIdx.x;
-  auto chunk_len = [&](int cc) { return min(kSmallMax, n - cc * kSmallMax); };
-  auto key_at = [&](int idx) -> uint64_t { return s_tile[idx]; };
-  const uint32_t c0 = beg + (uint32_t)c * kSmallMax;
-  const int cn = chunk_len(c);
-  uint64_t x[E];
-  uint32_t e[E], rq[E][kMaxQuads];
-  bool ok[E];
+  for (int q = wave; q < Q; q += NW) {
+    static_assert(E <= 64, "one count a lane");
+    const uint32_t c = lane < E ? s_cnt[q * E + lane] : 0u;
+    uint32_t incl = c;
 #pragma unroll
-  for (int r = 0; r < E; ++r) {
-    const int i = tid + r * kMergeThreads;
-    ok[r] = i < cn;
-    x[r] = key_at(c * kSmallMax + (ok[r] ? i : 0));
-    e[r] = (uint32_t)i;
-#pragma unroll
-    for (int g = 0; g < kMaxQuads / 4; ++g) {
-      if (g * 4 < Q) {
-        const uint64_t v = chunk_hits_below(a, c0, cn, ok[r] ? i : 0, Q, g);
-#pragma unroll
-        for (int f = 0; f < 4; ++f) rq[r][4 * g + f] = field16(v, f);
-      }
+    for (int off = 1; off < E; off <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)incl, off, 64);
+      if (lane >= off) incl += y;
     }
+    const uint32_t b0 = s_base[q];
+    if (lane < E) s_cnt[q * E + lane] = b0 + incl - c;
+    if (lane == E - 1) s_base[q] = b0 + incl;
   }
-  for (int cg = 0; cg < P; cg += kG) {
-    // lower bounds of x in chunks cg .. cg + kG - 1, searched together;
-    // every probe stays inside the tile's bucket
-    int pos[E][kG];
-#pragma unroll
-    for (int r = 0; r < E; ++r)
-#pragma unroll
-      for (int j = 0; j < kG; ++j) pos[r][j] = 0;
-    for (int step = kSmallMax; step > 0; step >>= 1) {
-      uint64_t probe[E][kG];
-#pragma unroll
-      for (int r = 0; r < E; ++r)
-#pragma unroll
-        for (int j = 0; j < kG; ++j) {
-          const int cc = cg + j;
-          probe[r][j] = 0;
-          if (cc < P && cc != c) {  // uniform
-            const int p = min(pos[r][j] + step, chunk_len(cc));
-            probe[r][j] = key_at(cc * kSmallMax + p - 1);
-          }
-        }
-#pragma unroll
-      for (int r = 0; r < E; ++r)
-#pragma unroll
-        for (int j = 0; j < kG; ++j) {
-          const int cc = cg + j;
-          if (cc < P && cc != c && pos[r][j] + step <= chunk_len(cc) && probe[r][j] < x[r]) pos[r][j] += step;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kG; ++j) {
-      const int cc = cg + j;
-      if (cc >= P || cc == c) continue;
-      const uint32_t cc0 = beg + (uint32_t)cc * kSmallMax;
-#pragma unroll
-      for (int r = 0; r < E; ++r) {
-        e[r] += (uint32_t)pos[r][j];
-#pragma unroll
-        for (int g = 0; g < kMaxQuads / 4; ++g) {
-          if (g * 4 < Q) {
-            const uint64_t v = chunk_hits_below(a, cc0, chunk_len(cc), pos[r][j], Q, g);
-#pragma unroll
-            for (int f = 0; f < 4; ++f) rq[r][4 * g + f] += field16(v, f);
-          }
-        }
-      }
-    }
-  }
+  __syncthreads();
   uint2* base = a.sub + (size_t)Q * beg;
+  const uint64_t lt = (1ull << lane) - 1ull;
 #pragma unroll
-  for (int r = 0; r < E; ++r) {
-    if (!ok[r]) continue;
-    const uint2 m = a.lmeta[c0 + tid + r * kMergeThreads];
-    a.point_list[beg + e[r]] = m.x;
-    a.pos_slot[beg + e[r]] = a.lslot[c0 + tid + r * kMergeThreads];
-    a.pos_quads[beg + e[r]] = (uint16_t)m.y;
-#pragma unroll
-    for (int q = 0; q < kMaxQuads; ++q)
-      if (q < Q && ((m.y >> q) & 1u)) base[(size_t)q * n + rq[r][q]] = make_uint2(m.x, e[r]);
+  for (int r = 0; r < K; ++r) {
+    for (int q = 0; q < Q; ++q) {
+      const bool hit = (hm[r] >> q) & 1u;
+      const uint64_t m = __ballot(hit);
+      if (hit)
+        base[(size_t)q * n + s_cnt[q * E + r * NW + wave] + (uint32_t)__popcll(m & lt)] =
+            make_uint2(rid[r], (uint32_t)(first + r * NT + tid));
+    }
   }
+  __syncthreads();  // the counts are rewritten by the next call
 }
 
 // Number of elements of A among the first k of merge(A, B) (keys unique).
@@ -1228,50 +1140,41 @@ SR_DEV int co_rank(const uint64_t* A, int na, const uint64_t* Bv, int nb, int k)
   return lo;
 }
 
-// A tile above the chunk path's limit (kLargeMax instances: far denser than
-// a 16 x 16 tile of a typical view; in batches every tile above kSmallMax),
-// by one 1024-lane workgroup: kLargeMax-key chunks sorted in
-// LDS (16 keys per lane), merged pairwise in global memory (merge path; the tile's own lmeta
-// entries, unused for such a tile, are the second buffer), then split into
-// the quadrant sub-lists in rounds of 1024 entries (per-wave ballots and a
-// scan over the waves).  O(n log n), where ranking against every chunk
-// would be O(n^2 / kSmallMax).
-SR_DEV void sort_huge_tile(const SortArgs& a, int tile, uint64_t* s_keys) {
-  constexpr int NT = kMergeThreads, K = kLargeMax / NT, kChunk = kLargeMax, kWaves = NT / 64;
-  __shared__ uint32_t s_wcnt[kMaxQuads][kWaves];
-  __shared__ uint32_t s_woff[kMaxQuads][kWaves];
-  __shared__ uint32_t s_total[kMaxQuads];
-  const uint32_t beg = a.ranges[2 * tile];
-  const int n = (int)(a.ranges[2 * tile + 1] - beg);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  uint64_t* src = a.keys + beg;
-  uint64_t* dst = reinterpret_cast<uint64_t*>(a.lmeta + beg);
-  for (int c0 = 0; c0 < n; c0 += kChunk) {
-    const int cn = min(kChunk, n - c0);
-    const int S = max(next_pow2(cn), K);
-    uint64_t kv[K];  // all loads in flight together (index clamped into the chunk)
-#pragma unroll
-    for (int k = 0; k < K; ++k) kv[k] = src[c0 + min(tid + k * NT, cn - 1)];
+// The large tiles' split, one 1024-lane workgroup per tile of the scan's list
+// (striding): the depths are cut into kSplitBins equal bins between the tile's
+// smallest and largest, and the keys moved bin by bin into key2.  Segment s of
+// the tile starts at the first bin boundary at or after kSegKeys s keys, so
+// segments hold kSegKeys keys give or take a bin, and their sorts, one
+// workgroup each, put the tile in order.  A segment above kSmallMax keys (more
+// than kSegKeys nearly equal depths in one bin) is sorted here: chunks in LDS,
+// then pairwise merges between the tile's two key buffers.
+constexpr int kSplitThreads = 1024, kSplitBins = 4096, kSplitRun = 4;
+constexpr int kSplitChunk = kSplitThreads * kSplitRun;  // keys of one LDS merge sort
+
+// Sorts n keys at v by chunks and merges; other: a buffer as large.
+SR_DEV void sort_range(uint64_t* v, uint64_t* other, int n, uint64_t* lds) {
+  constexpr int NT = kSplitThreads, K = kSplitRun;
+  const int tid = threadIdx.x;
+  for (int c0 = 0; c0 < n; c0 += kSplitChunk) {
+    const int cn = min(kSplitChunk, n - c0);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int i = tid + k * NT;
-      if (i < S) s_keys[lds_slot<K>(i)] = i < cn ? kv[k] : ~0ull;
+      lds[lds_slot<K>(i)] = i < cn ? v[c0 + i] : ~0ull;
     }
     __syncthreads();
-    merge_sort_lds<NT, K>(s_keys, S);
-    for (int i = tid; i < cn; i += NT) src[c0 + i] = s_keys[lds_slot<K>(i)];
+    merge_sort_lds<NT, K>(lds, max(next_pow2(cn), K));
+    for (int i = tid; i < cn; i += NT) v[c0 + i] = lds[lds_slot<K>(i)];
   }
   __syncthreads();
-  for (int w = kChunk; w < n; w <<= 1) {
+  uint64_t *src = v, *dst = other;
+  for (int w = kSplitChunk; w < n; w <<= 1) {
     for (int a0 = 0; a0 < n; a0 += 2 * w) {
-      const int na = min(w, n - a0);
-      const int nb = max(0, min(w, n - a0 - w));
-      const uint64_t* A = src + a0;
-      const uint64_t* Bv = src + a0 + na;
+      const int na = min(w, n - a0), nb = max(0, min(w, n - a0 - w));
+      const uint64_t *A = src + a0, *Bv = src + a0 + na;
       uint64_t* out = dst + a0;
-      const int total = na + nb;
-      const int per = (total + NT - 1) / NT;
+      const int total = na + nb, per = (total + NT - 1) / NT;
       const int k0 = min(total, tid * per), k1 = min(total, k0 + per);
       if (k0 < k1) {
         int i = co_rank(A, na, Bv, nb, k0);
@@ -1287,209 +1190,261 @@ SR_DEV void sort_huge_tile(const SortArgs& a, int tile, uint64_t* s_keys) {
     src = dst;
     dst = t;
   }
-  for (int i = tid; i < n; i += NT) {
-    const uint2 rs = a.inst_rs[(uint32_t)src[i]];
-    a.point_list[beg + i] = rs.x;
-    a.pos_slot[beg + i] = rs.y;
-  }
-  const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
-  const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
-  const int ltile = tile - (int)vi.tile_base;
-  const int tx = ltile % vi.gx, ty = ltile / vi.gx;
-  uint2* base = a.sub + (size_t)Q * beg;
-  if (tid < kMaxQuads) s_total[tid] = 0;
+  if (src != v)
+    for (int i = tid; i < n; i += NT) v[i] = src[i];
   __syncthreads();
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  // the next round's record and cull box are fetched a round ahead
-  const short4 kNone = make_short4(32767, 32767, -32768, -32768);
-  uint32_t id_next = tid < n ? a.point_list[beg + tid] : 0u;
-  short4 bx_next = tid < n ? a.cullbox[id_next] : kNone;
-  for (int c = 0; c < n; c += NT) {  // uniform
-    const int e = c + tid;
-    const bool valid = e < n;
-    const uint32_t id = id_next;
-    const short4 bx = bx_next;
-    if (e + NT < n) {
-      id_next = a.point_list[beg + e + NT];
-      bx_next = a.cullbox[id_next];
-    }
-    const uint32_t hm = valid ? quad_hits(bx, tx, ty, B, QX, Q, vi) : 0u;
-#pragma unroll
-    for (int q = 0; q < kMaxQuads; ++q) {
-      if (q < Q) {
-        const uint64_t m = __ballot((hm >> q) & 1u);
-        if (lane == 0) s_wcnt[q][wave] = (uint32_t)__popcll(m);
-      }
-    }
-    if (valid) a.pos_quads[beg + e] = (uint16_t)hm;
-    __syncthreads();
-    if (tid < Q * kWaves) {  // per quadrant, the waves' first slots
-      const int q = tid / kWaves, w = tid % kWaves;
-      const uint32_t c0 = s_wcnt[q][w];
-      uint32_t incl = c0;
-#pragma unroll
-      for (int d = 1; d < kWaves; d <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)incl, d, kWaves);
-        if (w >= d) incl += y;
-      }
-      const uint32_t t0 = s_total[q];
-      s_woff[q][w] = t0 + incl - c0;
-      if (w == kWaves - 1) s_total[q] = t0 + incl;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < kMaxQuads; ++q) {  // the ballots again: each lane's rank within its wave
-      if (q < Q) {
-        const uint64_t m = __ballot((hm >> q) & 1u);
-        if ((hm >> q) & 1u) base[(size_t)q * n + s_woff[q][wave] + (uint32_t)__popcll(m & lt)] = make_uint2(id, (uint32_t)e);
-      }
-    }
-  }
-  if (tid < Q) {
-    const uint32_t cnt = s_total[tid];
-    a.sub_count[(size_t)tile * Q + tid] = cnt;
-    a.q_flag[(size_t)tile * Q + tid] = 0u;
-    const uint32_t nch = (cnt + 63u) / 64u;
-    if (nch > 0) {
-      const uint32_t w0 = atomicAdd(a.work_count, nch);
-      for (uint32_t ch = 0; ch < nch; ++ch) a.work[w0 + ch] = make_uint2((uint32_t)(tile * Q + tid), ch);
-    }
-  }
 }
 
-// The counters[7] huge tiles, one workgroup each (striding).
-__global__ __launch_bounds__(kMergeThreads) void k_sort_huge(SortArgs a) {
-  __shared__ uint64_t s_keys[kLargeMax + kLargeMax / (kLargeMax / kMergeThreads)];
+__global__ __launch_bounds__(kSplitThreads) void k_split_large(SortArgs a) {
+  constexpr int NT = kSplitThreads, NB = kSplitBins, per = NB / NT, kU = 8, NW = NT / 64;
+  __shared__ __align__(16) uint64_t lds[kSplitChunk + NT];  // the bins, or a chunk of the fallback
+  __shared__ uint32_t s_lo[NW], s_hi[NW], s_w[NW];
+  static_assert(sizeof(lds) >= (NB + 1) * 4, "the bins fit");
   if (a.counters[1] & kErrCapacity) return;
-  for (uint32_t h = blockIdx.x; h < a.counters[7]; h += gridDim.x) {
-    __syncthreads();  // s_keys may still be read for the previous tile
-    sort_huge_tile(a, (int)a.large[a.vs.T - 1 - h], s_keys);
+  uint32_t* bins = reinterpret_cast<uint32_t*>(lds);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (uint32_t l = blockIdx.x; l < a.counters[3]; l += gridDim.x) {
+    const int tile = (int)a.large[l];
+    const uint32_t beg = a.ranges[2 * tile];
+    const int n = (int)(a.ranges[2 * tile + 1] - beg);
+    const uint64_t* src = a.keys + beg;
+    uint64_t* dst = a.key2 + beg;
+    uint32_t* seg = a.seg_start + a.seg_off[l];
+    const int nseg = (int)segments_of((uint32_t)n);
+    auto each = [&](auto&& fn) {  // every key of the tile, kU loads in flight a lane
+      for (int i0 = 0; i0 < n; i0 += kU * NT) {
+        uint64_t k[kU];
+#pragma unroll
+        for (int t = 0; t < kU; ++t) k[t] = src[min(i0 + t * NT + tid, n - 1)];
+#pragma unroll
+        for (int t = 0; t < kU; ++t)
+          if (i0 + t * NT + tid < n) fn(k[t]);
+      }
+    };
+    uint32_t lo = 0xFFFFFFFFu, hi = 0u;
+    each([&](uint64_t k) {
+      const uint32_t d = (uint32_t)(k >> 32);
+      lo = min(lo, d);
+      hi = max(hi, d);
+    });
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
+      hi = max(hi, (uint32_t)__shfl_xor((int)hi, off, 64));
+    }
+    __syncthreads();  // the previous tile's readers are done
+    if (lane == 0) {
+      s_lo[wave] = lo;
+      s_hi[wave] = hi;
+    }
+#pragma unroll
+    for (int t = 0; t < per; ++t) bins[t * NT + tid] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      lo = min(lo, s_lo[w]);
+      hi = max(hi, s_hi[w]);
+    }
+    const float scale = (float)NB / ((float)(hi - lo) + 1.0f);
+    auto bin_of = [&](uint64_t k) { return min(NB - 1, (int)((float)((uint32_t)(k >> 32) - lo) * scale)); };
+    each([&](uint64_t k) { atomicAdd(&bins[bin_of(k)], 1u); });
+    __syncthreads();
+    uint32_t c[per], sum = 0u;
+#pragma unroll
+    for (int t = 0; t < per; ++t) {
+      c[t] = bins[tid * per + t];
+      sum += c[t];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)incl, off, 64);
+      if (lane >= off) incl += y;
+    }
+    if (lane == 63) s_w[wave] = incl;
+    __syncthreads();
+    uint32_t run = incl - sum;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) run += w < wave ? s_w[w] : 0u;
+    // segment s starts at the first bin boundary that is >= kSegKeys s
+#pragma unroll
+    for (int t = 0; t < per; ++t) {
+      bins[tid * per + t] = run;
+      const uint32_t end = run + c[t];
+      for (uint32_t sg = run / kSegKeys + 1u; sg <= end / kSegKeys && sg < (uint32_t)nseg; ++sg) seg[sg] = beg + end;
+      run = end;
+    }
+    if (tid == 0) seg[0] = beg;
+    __syncthreads();
+    each([&](uint64_t k) { dst[atomicAdd(&bins[bin_of(k)], 1u)] = k; });
+    __syncthreads();
+    for (int sg = 0; sg < nseg; ++sg) {  // uniform
+      const uint32_t s0 = seg[sg], s1 = sg + 1 < nseg ? seg[sg + 1] : beg + (uint32_t)n;
+      if (s1 - s0 > (uint32_t)kSmallMax) {
+        sort_range(a.key2 + s0, a.keys + s0, (int)(s1 - s0), lds);
+        __syncthreads();
+      }
+    }
   }
 }
 
-// The counters[6] chunk items of the large tiles, one workgroup each
-// (striding).
-__global__ __launch_bounds__(kMergeThreads) void k_merge_chunks(SortArgs a) {
-  __shared__ uint64_t s_tile[kLargeMax];
+// Large tile and segment of segment item `it` (< counters[6]).
+struct Segment {
+  int tile, n, nseg, sg;
+  uint32_t beg, s0, item0;  // tile's first key, segment's first, item of segment 0
+  int cnt;
+};
+SR_DEV Segment segment_item(const SortArgs& a, uint32_t it) {
+  uint32_t lo = 0, hi = a.counters[3];  // seg_off[lo] <= it < seg_off[hi]
+  while (hi - lo > 1u) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (a.seg_off[mid] <= it) lo = mid;
+    else hi = mid;
+  }
+  Segment g;
+  g.tile = (int)a.large[lo];
+  g.beg = a.ranges[2 * g.tile];
+  g.n = (int)(a.ranges[2 * g.tile + 1] - g.beg);
+  g.nseg = (int)segments_of((uint32_t)g.n);
+  g.item0 = a.seg_off[lo];
+  g.sg = (int)(it - g.item0);
+  g.s0 = a.seg_start[it];
+  g.cnt = (int)((g.sg + 1 < g.nseg ? a.seg_start[it + 1] : g.beg + (uint32_t)g.n) - g.s0);
+  return g;
+}
+
+// Small tiles and segments, one 512-lane workgroup each: the first seg_blocks
+// workgroups stride over the segments (workgroups b, b + seg_blocks, ...), so
+// these start first; workgroup seg_blocks + t sorts tile t when it holds at
+// most kSmallMax instances.  A segment's quadrant hits are counted here and its
+// sub-list entries placed by k_segment_lists.  Latency-bound: 300k surfels at
+// 800 x 600 put about 1,650 instances in each of 350 tiles, so a CU holds two
+// or three sorts and what counts is each one's chain of LDS and gather
+// latencies.  With the split and the segments' lists 64 us there, and 195 us
+// for 1M surfels at 1237 x 823; 256-lane merge sorts of 8 keys a lane, with
+// larger tiles cut into 2,048-key chunks merged by rank (and above 16,384 by
+// one workgroup), took 92 and 624 us.  One workgroup for each tile of up to
+// 16,384 was no better than those on the tiles it bounds (75 us for 8,192
+// keys, 132 us for 16,384).
+constexpr int kSortThreads = 512, kSortKeys = kSmallMax / 512, kSortBins = 2048;
+__global__ __launch_bounds__(kSortThreads) void k_sort_tiles(SortArgs a, uint32_t seg_blocks) {
+  constexpr int NT = kSortThreads, K = kSortKeys;
+  __shared__ __align__(16) char lds[TileLds<NT, K, kSortBins>::kBytes];
+  __shared__ uint32_t s_base[kMaxQuads];
+  static_assert(kMaxQuads * K * (NT / 64) * 4 <= (int)sizeof(lds), "the quadrant counts fit");
   if (a.counters[1] & kErrCapacity) return;
   const int Q = quads_per_tile(a.vs.B);
   const int tid = threadIdx.x;
-  for (uint32_t it = blockIdx.x; it < a.counters[6]; it += gridDim.x) {
-    __syncthreads();  // s_tile may still be read for the previous item
-    uint32_t li;
-    int c;
-    chunk_item(a, it, li, c);
-    const int tile = (int)a.large[li];
-    const uint32_t beg = a.ranges[2 * tile];
-    const int n = (int)(a.ranges[2 * tile + 1] - beg);
-    const int P = (n + kSmallMax - 1) / kSmallMax;
-    for (int i = tid; i < n; i += kMergeThreads) s_tile[i] = a.keys[beg + i];
-    __syncthreads();
-    merge_chunk(a, beg, n, c, s_tile);
-    // the tile's sub-list lengths and acceptance work items, by its chunk 0
-    if (c == 0 && tid < 64) {
-      uint32_t cnt = 0;
-      if (tid < Q)
-        for (int cc = 0; cc < P; ++cc) {
-          const int len = min(kSmallMax, n - cc * kSmallMax);
-          cnt += field16(chunk_hits_below(a, beg + (uint32_t)cc * kSmallMax, len, len, Q, tid / 4), tid % 4);
+  uint32_t inst[K], rid[K], hm[K];
+  if (blockIdx.x < seg_blocks) {
+    for (uint32_t it = blockIdx.x; it < a.counters[6]; it += seg_blocks) {
+      const Segment g = segment_item(a, it);
+      if (tid < Q) s_base[tid] = 0u;
+      __syncthreads();
+      // one round, unless the segment was too full for one and is sorted already
+      for (int c0 = 0; c0 < g.cnt; c0 += NT * K) {
+        const int cn = min(NT * K, g.cnt - c0);
+        if (g.cnt <= NT * K) {
+          sort_bucket<NT, K, kSortBins>(a.key2 + g.s0, cn, lds, inst);
+        } else {
+#pragma unroll
+          for (int r = 0; r < K; ++r) inst[r] = (uint32_t)a.key2[g.s0 + c0 + min(r * NT + tid, cn - 1)];
         }
-      append_work(a, tile, Q, cnt);
-    }
-  }
-}
-
-// Every tile's sort in one launch of 256-lane workgroups.  The first
-// kChunkBlocks workgroups sort the chunks of the large tiles (workgroup b:
-// chunk items b + k kChunkBlocks), so they are dispatched first; workgroup
-// kChunkBlocks + t sorts tile t when it holds at most kSmallMax instances
-// (and writes empty sub-lists for an empty tile).
-__global__ __launch_bounds__(kSortThreads) void k_sort_tiles(SortArgs a) {
-  __shared__ uint64_t s_keys[kSmallMax + kSmallMax / (kSmallMax / kSortThreads)];
-  if (a.counters[1] & kErrCapacity) return;
-  if (blockIdx.x < kChunkBlocks) {
-    for (uint32_t it = blockIdx.x; it < a.counters[6]; it += kChunkBlocks) {
-      uint32_t li;
-      int c;
-      chunk_item(a, it, li, c);
-      const int tile = (int)a.large[li];
-      const uint32_t beg = a.ranges[2 * tile];
-      const int n = (int)(a.ranges[2 * tile + 1] - beg);
-      const uint32_t c0 = beg + (uint32_t)c * kSmallMax;
-      const int cn = min(kSmallMax, n - c * kSmallMax);
-      sort_run(a, c0, cn, s_keys);
-      place_sorted<false>(a, tile, beg, n, c0, cn, s_keys);
-      __syncthreads();  // s_keys is refilled for the next chunk
+        place_entries<NT, K>(a, g.tile, g.s0 + c0, cn, inst, rid, hm);
+        for (int q = 0; q < Q; ++q) {
+          uint32_t hits = 0;
+#pragma unroll
+          for (int r = 0; r < K; ++r) hits += (uint32_t)__popcll(__ballot((hm[r] >> q) & 1u));
+          if ((tid & 63) == 0 && hits) atomicAdd(&s_base[q], hits);
+        }
+      }
+      __syncthreads();
+      if (tid < Q) a.seg_hits[(size_t)it * Q + tid] = s_base[tid];
+      __syncthreads();
     }
     return;
   }
-  const int tile = (int)(blockIdx.x - kChunkBlocks);
+  const int tile = (int)(blockIdx.x - seg_blocks);
   const uint32_t beg = a.ranges[2 * tile];
   const int n = (int)(a.ranges[2 * tile + 1] - beg);
   if (n > kSmallMax) return;
   if (n <= 0) {
-    const int Q = quads_per_tile(a.vs.B);
-    if ((int)threadIdx.x < Q) {
-      a.sub_count[(size_t)tile * Q + threadIdx.x] = 0;
-      a.q_flag[(size_t)tile * Q + threadIdx.x] = 0u;
+    if (tid < Q) {
+      a.sub_count[(size_t)tile * Q + tid] = 0;
+      a.q_flag[(size_t)tile * Q + tid] = 0u;
     }
     return;
   }
-  sort_run(a, beg, n, s_keys);
-  place_sorted<true>(a, tile, beg, n, beg, n, s_keys);
+  sort_bucket<NT, K, kSortBins>(a.keys + beg, n, lds, inst);
+  place_entries<NT, K>(a, tile, beg, n, inst, rid, hm);
+  if (tid < Q) s_base[tid] = 0u;
+  __syncthreads();
+  append_sublists<NT, K>(a, beg, n, 0, Q, rid, hm, reinterpret_cast<uint32_t*>(lds), s_base);
+  if (tid < 64) append_work(a, tile, Q, tid < Q ? s_base[tid] : 0u);
 }
 
-// A second stream per (host thread, device) with fork/join events, for the
-// huge-tile sort beside the others.  Default priority; created on first use.
-struct SideStream {
-  hipStream_t s = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-};
-static hipError_t side_stream(SideStream*& out) {
-  thread_local SideStream cache[16];
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= 16) return hipErrorInvalidDevice;
-  SideStream& c = cache[dev];
-  if (c.s == nullptr) {
-    e = hipStreamCreateWithFlags(&c.s, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&c.fork, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&c.join, hipEventDisableTiming);
-    if (e != hipSuccess) return e;
+// The segments' sub-list entries, one workgroup each (striding): a segment's
+// entries follow those of the tile's earlier segments.  The first segment's
+// workgroup also writes the sub-list lengths and the acceptance work items.
+__global__ __launch_bounds__(kSortThreads) void k_segment_lists(SortArgs a) {
+  constexpr int NT = kSortThreads, K = kSortKeys;
+  __shared__ uint32_t s_cnt[kMaxQuads * K * (NT / 64)];
+  __shared__ uint32_t s_base[kMaxQuads], s_all[kMaxQuads];
+  if (a.counters[1] & kErrCapacity) return;
+  const int Q = quads_per_tile(a.vs.B);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (uint32_t it = blockIdx.x; it < a.counters[6]; it += gridDim.x) {
+    const Segment g = segment_item(a, it);
+    for (int q = wave; q < Q; q += NT / 64) {
+      uint32_t before = 0u, all = 0u;
+      for (int t = lane; t < g.nseg; t += 64) {
+        const uint32_t h = a.seg_hits[(size_t)(g.item0 + (uint32_t)t) * Q + q];
+        all += h;
+        before += t < g.sg ? h : 0u;
+      }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) {
+        before += (uint32_t)__shfl_xor((int)before, off, 64);
+        all += (uint32_t)__shfl_xor((int)all, off, 64);
+      }
+      if (lane == 0) {
+        s_base[q] = before;
+        s_all[q] = all;
+      }
+    }
+    __syncthreads();
+    if (g.sg == 0 && wave == 0) append_work(a, g.tile, Q, lane < Q ? s_all[lane] : 0u);
+    for (int c0 = 0; c0 < g.cnt; c0 += NT * K) {
+      uint32_t rid[K], hm[K];
+#pragma unroll
+      for (int r = 0; r < K; ++r) {
+        const int i = c0 + r * NT + tid;
+        const uint32_t pos = g.s0 + (uint32_t)min(i, g.cnt - 1);
+        rid[r] = a.point_list[pos];
+        hm[r] = a.pos_quads[pos];
+      }
+#pragma unroll
+      for (int r = 0; r < K; ++r) hm[r] = c0 + r * NT + tid < g.cnt ? hm[r] : 0u;
+      append_sublists<NT, K>(a, g.beg, g.n, (int)(g.s0 - g.beg) + c0, Q, rid, hm, s_cnt, s_base);
+    }
+    __syncthreads();
   }
-  out = &c;
-  return hipSuccess;
 }
 
-hipError_t launch_sort_tiles(const SortArgs& a, hipStream_t s) {
+hipError_t launch_sort_tiles(const SortArgs& a, size_t max_segments, hipStream_t s) {
   if (a.vs.T == 0) return hipSuccess;
-  hipError_t e = hipSuccess;
-  SideStream* side = nullptr;
-  if (a.side_huge) {  // fork before the tile sort, so the huge-tile sort does not wait for it
-    e = side_stream(side);
-    if (e == hipSuccess) e = hipEventRecord(side->fork, s);
-    if (e == hipSuccess) e = hipStreamWaitEvent(side->s, side->fork, 0);
-    if (e != hipSuccess) return e;
-  }
-  // issued first: its many small workgroups are dispatched before the huge
-  // tiles' (each of which takes a whole CU's LDS)
-  hipLaunchKernelGGL(k_sort_tiles, dim3(kChunkBlocks + a.vs.T), dim3(kSortThreads), 0, s, a);
+  const unsigned T = (unsigned)a.vs.T;
+  // as many workgroups as run at once several times over, so the uneven
+  // tiles and segments of a large batch balance
+  const unsigned segs = (unsigned)std::min<size_t>(max_segments, 8192);
+  hipLaunchKernelGGL(k_split_large, dim3(std::min(T, 4096u)), dim3(kSplitThreads), 0, s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_sort_tiles, dim3(segs + T), dim3(kSortThreads), 0, s, a, segs);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const hipStream_t hs = a.side_huge ? side->s : s;  // stream of the huge-tile sort
-  // batches: one workgroup per possible tile, so the dispatcher balances
-  // thousands of uneven sorts; one view: a few striding workgroups
-  const unsigned huge_blocks = a.side_huge ? (unsigned)a.vs.T : kChunkBlocks;
-  hipLaunchKernelGGL(k_sort_huge, dim3(huge_blocks), dim3(kMergeThreads), 0, hs, a);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_merge_chunks, dim3(kChunkBlocks), dim3(kMergeThreads), 0, s, a);
-  e = hipGetLastError();
-  if (e != hipSuccess || !a.side_huge) return e;
-  e = hipEventRecord(side->join, hs);
-  if (e == hipSuccess) e = hipStreamWaitEvent(s, side->join, 0);
-  return e;
+  hipLaunchKernelGGL(k_segment_lists, dim3(segs), dim3(kSortThreads), 0, s, a);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------

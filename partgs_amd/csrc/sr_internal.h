@@ -119,7 +119,7 @@ inline GeomLayout geom_layout(size_t R) {
 // Image state: per-tile binning tables and per-pixel blend state of all views.
 struct ImageLayout {
   int T, N;
-  size_t counters, tile_count, tile_start, tile_fill, ranges, large, lchunk_off, sub_count, q_flag, lane_range, q_cost,
+  size_t counters, tile_count, tile_start, tile_fill, ranges, large, seg_off, sub_count, q_flag, lane_range, q_cost,
       q_order, final_T, n_contrib, total;
 };
 inline ImageLayout image_layout(const ViewSet& vs) {
@@ -129,14 +129,14 @@ inline ImageLayout image_layout(const ViewSet& vs) {
   size_t off = 0;
   l.counters = off; off += kAlign;  // [0] instances, [1] error flags, [2] work items,
                                     // [3] large tiles, [4..5] pair-store fill,
-                                    // [6] chunks of the large tiles, [7] huge tiles,
+                                    // [6] segments of the large tiles,
                                     // [8] partial-gradient slots
   l.tile_count = off; off += align_up((size_t)l.T * 4);
   l.tile_start = off; off += align_up(((size_t)l.T + 1) * 4);
   l.tile_fill = off; off += align_up((size_t)l.T * 4);
   l.ranges = off; off += align_up((size_t)l.T * 8);
   l.large = off; off += align_up((size_t)l.T * 4);  // tiles for the large-tile sort
-  l.lchunk_off = off; off += align_up(((size_t)l.T + 1) * 4);  // their first chunk numbers
+  l.seg_off = off; off += align_up(((size_t)l.T + 1) * 4);  // their first segment numbers
   l.sub_count = off; off += align_up((size_t)l.T * quads_per_tile(vs.B) * 4);
   l.q_flag = off; off += align_up((size_t)l.T * quads_per_tile(vs.B) * 4);  // 1: the quadrant missed the pair store
   l.lane_range = off; off += align_up((size_t)l.T * quads_per_tile(vs.B) * 64 * 8);  // (first pair, pairs) per pixel
@@ -156,8 +156,6 @@ inline ImageLayout image_layout(int W, int H, int B) { return image_layout(singl
 //   pos_slot   position in the concatenated sorted tile lists -> the first
 //              slot of the instance there
 //   pos_quads  position -> the quadrants whose sub-lists hold the instance
-//   lslot      large-tile sort: per entry of a sorted chunk, its first slot
-//              (the merge moves it to pos_slot)
 //   part       one slot per sub-list entry, i.e. per (instance, quadrant
 //              holding it): the 18 per-surfel partial gradients the
 //              backward blend summed over that quadrant's pixels
@@ -168,8 +166,8 @@ inline ImageLayout image_layout(int W, int H, int B) { return image_layout(singl
 //              atomic.  The slot array is the layout's last region, so its
 //              size (slot capacity) does not move any other offset.
 struct BinLayout {
-  size_t keys, lmeta, lpre, point_list, sub, masks, chunk_T, work, frag_off, total;
-  size_t inst_rs, pos_slot, pos_quads, lslot, part, part_nz;
+  size_t keys, key2, seg_start, seg_hits, point_list, sub, masks, chunk_T, work, frag_off, total;
+  size_t inst_rs, pos_slot, pos_quads, part, part_nz;
   size_t nslot;  // slots the part region holds
   size_t prec, fW;
   size_t frag_cap;
@@ -208,13 +206,21 @@ __host__ __device__ inline size_t mask_base(int Q, uint32_t beg, uint32_t n, int
 }
 // (quadrant, chunk) work items, appended by the tile sorts as they finish;
 // the kernels that walk the list take it from the end, so the items of the
-// large tiles (appended last, by the chunk merge and the huge-tile sort)
+// large tiles (appended last, by the sorts of the large tiles)
 // start first (measured: 4 us less per 300k-surfel 800x600 step, in the
 // passes that follow).
 inline size_t work_capacity(int L, int B, int T) {
   const size_t Q = (size_t)quads_per_tile(B);
   return Q * ((size_t)T + ((size_t)(L > 0 ? L : 1) + 63) / 64);
 }
+// Tiles with at most kSmallMax instances are sorted by one workgroup each;
+// larger ones are split by depth into segments of about kSegKeys keys.
+constexpr int kSmallMax = 2048;
+constexpr uint32_t kSegKeys = 1024;
+__host__ __device__ inline uint32_t segments_of(uint32_t n) { return (n + kSegKeys - 1u) / kSegKeys; }
+// Segments of all large tiles of n instances: a tile above kSmallMax has at
+// most n / kSegKeys + 1, that is 1.5 n / kSegKeys.
+inline size_t segment_capacity(size_t n) { return n / kSegKeys + n / kSmallMax + 1; }
 // slot_capacity: slots the part region is sized for; 0 sizes it for every
 // (instance, quadrant), which no batch can exceed.
 inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_capacity = 0, int sem = 0,
@@ -224,10 +230,9 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
   const size_t n = (size_t)(L > 0 ? L : 1);
   const size_t Q = (size_t)quads_per_tile(B);
   b.keys = off; off += align_up(n * 8);
-  // large-tile sort: per entry of a sorted 2048-key chunk, (record, quadrant
-  // mask) and, per quadrant, the chunk's hits before it (16-bit each)
-  b.lmeta = off; off += align_up(n * 8);
-  b.lpre = off; off += align_up(n * Q * 2);
+  b.key2 = off; off += align_up(n * 8);  // large tiles: the keys split by depth
+  b.seg_start = off; off += align_up(segment_capacity(n) * 4);     // per segment of a large tile its first key
+  b.seg_hits = off; off += align_up(segment_capacity(n) * Q * 4);  // and its entries per quadrant
   b.point_list = off; off += align_up(n * 4);
   b.sub = off; off += align_up(n * Q * 8);  // uint2 (surfel id, position in tile)
   b.masks = off; off += align_up((n * Q + (size_t)kQuad * kQuad * Q * (size_t)T) * 8);
@@ -238,7 +243,6 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
   b.inst_rs = off; off += align_up(n * 8);
   b.pos_slot = off; off += align_up(n * 4);
   b.pos_quads = off; off += align_up(n * 2);
-  b.lslot = off; off += align_up(n * 4);
   b.nslot = slot_capacity > 0 ? (size_t)slot_capacity : n * Q;
   b.part_nz = off; off += align_up(n * Q);  // per slot: 1 when the slot holds sums
   b.frag_cap = pair_capacity > 0 ? (size_t)pair_capacity
@@ -306,30 +310,21 @@ struct ScatterArgs {
   uint64_t* keys;
 };
 
-// Tiles with at most kSmallMax instances are sorted by one 256-lane
-// workgroup each; up to kLargeMax in kSmallMax-key chunks that are then
-// merged by rank; larger ("huge") ones by one 1024-lane workgroup each.
-constexpr int kSmallMax = 2048;
-constexpr int kLargeMax = 16384;
-
 struct SortArgs {
   ViewSet vs;
   const uint32_t* ranges;
   const uint32_t* counters;
-  const uint32_t* large;  // counters[3] tiles of kSmallMax < n <= large_max from the start, then
-                          // counters[7] tiles of n > large_max from the end (large[T - 1 - h]);
-                          // large_max is kLargeMax, or kSmallMax for batches (no chunk path)
-  const uint32_t* lchunk_off;  // per large tile its first kSmallMax-key chunk (counters[6] in all)
-  int side_huge;               // host: sort the huge tiles on a second stream beside the rest
+  const uint32_t* large;    // the counters[3] tiles above kSmallMax instances
+  const uint32_t* seg_off;  // per large tile its first segment (counters[6] in all)
+  uint32_t* seg_start;
+  uint32_t* seg_hits;
   uint64_t* keys;
-  uint2* lmeta;
-  uint16_t* lpre;
+  uint64_t* key2;
   uint32_t* point_list;
   const short4* cullbox;
   const uint2* inst_rs;
   uint32_t* pos_slot;
   uint16_t* pos_quads;
-  uint32_t* lslot;
   uint2* sub;
   uint32_t* sub_count;
   uint2* work;          // (quadrant index, chunk) items for the acceptance pass
@@ -510,10 +505,10 @@ int set_error(int code, const char* msg);
 hipError_t launch_preprocess(const PreprocessArgs& a, hipStream_t s);
 hipError_t launch_scan_tiles(int T, const uint32_t* count, uint32_t* start, uint32_t* fill,
                              uint32_t* ranges, uint32_t* counters, uint32_t capacity, int nb, uint32_t* bsum,
-                             uint32_t* ssum, uint32_t slot_capacity, uint32_t* large, uint32_t* lchunk_off,
-                             int large_max, hipStream_t s);
+                             uint32_t* ssum, uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off,
+                             hipStream_t s);
 hipError_t launch_scatter(const ScatterArgs& a, hipStream_t s);
-hipError_t launch_sort_tiles(const SortArgs& a, hipStream_t s);
+hipError_t launch_sort_tiles(const SortArgs& a, size_t max_segments, hipStream_t s);
 hipError_t launch_accept(const AcceptArgs& a, size_t max_items, hipStream_t s);
 hipError_t launch_pair_offsets(const AcceptArgs& a, hipStream_t s);
 hipError_t launch_pair_write(const AcceptArgs& a, size_t max_items, hipStream_t s);
