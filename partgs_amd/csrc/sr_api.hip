@@ -366,7 +366,6 @@ int run_front(Pipeline& pl, const sr_surfels* g, int* radii, uint32_t capacity, 
   pa.tiles = (uint32_t*)(pl.geom + pl.gl.tiles);
   pa.clamped = (uint8_t*)(pl.geom + pl.gl.clamped);
   pa.cullbox = (short4*)(pl.geom + pl.gl.cullbox);
-  pa.bsum = (uint32_t*)(pl.geom + pl.gl.bsum);
   pa.ssum = (uint32_t*)(pl.geom + pl.gl.ssum);
   pa.tile_count = tile_count;
   pa.counters = counters;
@@ -374,7 +373,7 @@ int run_front(Pipeline& pl, const sr_surfels* g, int* radii, uint32_t capacity, 
   SR_STAGE(1, dbg, st, "scan",
            launch_scan_tiles(pl.il.T, tile_count, (uint32_t*)(pl.img + pl.il.tile_start),
                              (uint32_t*)(pl.img + pl.il.tile_fill), (uint32_t*)(pl.img + pl.il.ranges), counters,
-                             capacity, pl.vs.V * ((pl.P + 255) / 256), (uint32_t*)(pl.geom + pl.gl.bsum),
+                             capacity, pl.vs.V * ((pl.P + 255) / 256),
                              (uint32_t*)(pl.geom + pl.gl.ssum), slot_capacity, (uint32_t*)(pl.img + pl.il.large),
                              (uint32_t*)(pl.img + pl.il.seg_off), st));
   return SR_OK;
@@ -393,12 +392,10 @@ int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st) {
   sc.depths = (const float*)(pl.geom + pl.gl.depths);
   sc.radii = radii;
   sc.counters = counters;
-  sc.bsum = (const uint32_t*)(pl.geom + pl.gl.bsum);
   sc.ssum = (const uint32_t*)(pl.geom + pl.gl.ssum);
   sc.cullbox = (const short4*)(pl.geom + pl.gl.cullbox);
-  sc.roff = (uint32_t*)(pl.geom + pl.gl.roff);
   sc.rslot = (uint2*)(pl.geom + pl.gl.rslot);
-  sc.inst_rs = (uint2*)(bin + bl.inst_rs);
+  sc.pay = (uint2*)(bin + bl.pay);
   sc.tile_fill = (uint32_t*)(pl.img + pl.il.tile_fill);
   sc.keys = (uint64_t*)(bin + bl.keys);
   SR_STAGE(2, dbg, st, "scatter", launch_scatter(sc, st));
@@ -413,8 +410,8 @@ int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st) {
   sa.seg_start = (uint32_t*)(bin + bl.seg_start);
   sa.seg_hits = (uint32_t*)(bin + bl.seg_hits);
   sa.point_list = (uint32_t*)(bin + bl.point_list);
-  sa.cullbox = (const short4*)(pl.geom + pl.gl.cullbox);
-  sa.inst_rs = (const uint2*)(bin + bl.inst_rs);
+  sa.pay = (const uint2*)(bin + bl.pay);
+  sa.pay2 = (uint2*)(bin + bl.pay2);
   sa.pos_slot = (uint32_t*)(bin + bl.pos_slot);
   sa.pos_quads = (uint16_t*)(bin + bl.pos_quads);
   sa.sub = (uint2*)(bin + bl.sub);
@@ -535,7 +532,6 @@ int run_backward(Pipeline& pl, const sr_surfels* g, const int* radii, const floa
   pb.M = g->M;
   pb.counters = pl.counters();
   pb.tiles = (const uint32_t*)(pl.geom + pl.gl.tiles);
-  pb.roff = (const uint32_t*)(pl.geom + pl.gl.roff);
   pb.rslot = (const uint2*)(pl.geom + pl.gl.rslot);
   pb.part = blend ? (const float*)(pl.bin + pl.bl.part) : nullptr;
   pb.part_nz = blend ? (const uint8_t*)(pl.bin + pl.bl.part_nz) : nullptr;

@@ -490,11 +490,12 @@ SR_DEV bool preprocess_one(const PreprocessArgs& a, int v, int idx, size_t r, in
 // keeps hot tiles (thousands of instances) off a single global counter.
 constexpr int kHistTiles = 4096;
 
-// Exclusive scan of one value per lane over a 256-lane workgroup (four
-// waves); every lane must call it.  Returns the lane's exclusive prefix and
-// the workgroup total.
-SR_DEV uint32_t block_scan256(uint32_t x, uint32_t* s_w, uint32_t& total) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Exclusive scan of one value per lane over a group of 256 consecutive lanes
+// (four waves; a workgroup holds one or more groups, s_w four words each);
+// every lane must call it.  Returns the lane's exclusive prefix and the
+// group's total.
+SR_DEV uint32_t group_scan256(uint32_t x, uint32_t* s_w, uint32_t& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, first = wave & ~3;
   uint32_t incl = x;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -504,15 +505,15 @@ SR_DEV uint32_t block_scan256(uint32_t x, uint32_t* s_w, uint32_t& total) {
   if (lane == 63) s_w[wave] = incl;
   __syncthreads();
   uint32_t off = 0;
-  for (int w = 0; w < wave; ++w) off += s_w[w];
-  total = (s_w[0] + s_w[1]) + (s_w[2] + s_w[3]);
+  for (int w = first; w < wave; ++w) off += s_w[w];
+  total = (s_w[first] + s_w[first + 1]) + (s_w[first + 2] + s_w[first + 3]);
   return off + incl - x;
 }
 
 // Grid: (surfel blocks, views); a workgroup's surfels all belong to view
 // blockIdx.y, so its tile histogram is that view's.  Each workgroup also
-// stores its records' instance total in bsum (view-major), which the tile
-// scan turns into the first instance index of every workgroup.
+// stores its records' slot total in ssum (view-major), which the tile scan
+// turns into the first slot of every workgroup.
 // Partial-gradient slots of a record: one per (instance, quadrant holding
 // it), the quadrants found as the sort's sub-lists find them.
 SR_DEV uint32_t record_slots(short4 bx, int x0, int y0, int x1, int y1, int B, const ViewInfo& vi) {
@@ -522,7 +523,6 @@ SR_DEV uint32_t record_slots(short4 bx, int x0, int y0, int x1, int y1, int B, c
 
 __global__ __launch_bounds__(256) void k_preprocess(PreprocessArgs a) {
   __shared__ uint32_t s_hist[kHistTiles];
-  __shared__ uint32_t s_wsum[4];
   __shared__ uint32_t s_ssum[4];
   const int v = blockIdx.y;
   const int gx = a.vs.v[v].gx;
@@ -536,11 +536,9 @@ __global__ __launch_bounds__(256) void k_preprocess(PreprocessArgs a) {
   const bool ok = idx < a.P && preprocess_one(a, v, idx, (size_t)v * a.P + idx, x0, y0, x1, y1);
   {
     uint32_t total = 0;
-    (void)block_scan256(ok ? (uint32_t)(x1 - x0) * (uint32_t)(y1 - y0) : 0u, s_wsum, total);
-    if (threadIdx.x == 0) a.bsum[(size_t)v * gridDim.x + blockIdx.x] = total;
     // the cull box was stored by preprocess_one (this thread)
     const uint32_t ns = ok ? record_slots(a.cullbox[(size_t)v * a.P + idx], x0, y0, x1, y1, a.vs.B, a.vs.v[v]) : 0u;
-    (void)block_scan256(ns, s_ssum, total);
+    (void)group_scan256(ns, s_ssum, total);
     if (threadIdx.x == 0) a.ssum[(size_t)v * gridDim.x + blockIdx.x] = total;
   }
   if (ok) {
@@ -616,15 +614,14 @@ SR_DEV void scan1024_excl(uint32_t* s, uint32_t (&x)[N], uint32_t (&total)[N]) {
 // list of tiles above kSmallMax instances (count in counters[3]) and the
 // number of each one's first kSegKeys-key segment (seg_off, followed by the
 // total, which also goes to counters[6]);
-// then the same scan for the per-workgroup instance totals of the
-// preprocess (in place), which numbers every record's instances in record
-// order.
+// then the same scan for the per-workgroup slot totals of the preprocess (in
+// place), which numbers every record's slots in record order.
 constexpr int kScanThreads = 1024;
 __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32_t* count,
                                                               uint32_t* start, uint32_t* fill,
                                                               uint32_t* ranges, uint32_t* counters,
-                                                              uint32_t capacity, int nb, uint32_t* bsum,
-                                                              uint32_t* ssum, uint32_t slot_capacity,
+                                                              uint32_t capacity, int nb, uint32_t* ssum,
+                                                              uint32_t slot_capacity,
                                                               uint32_t* large, uint32_t* seg_off) {
   __shared__ uint32_t s_part[3 * 32];
   const int tid = threadIdx.x;
@@ -664,35 +661,29 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32
     counters[6] = tot3[2];
     seg_off[tot3[1]] = tot3[2];
   }
-  // the per-workgroup instance and slot totals of the preprocess, in place
+  // the per-workgroup slot totals of the preprocess, in place
   const int pb = (nb + kScanThreads - 1) / kScanThreads;
   const int b2 = tid * pb, e2 = min(nb, b2 + pb);
-  uint32_t w2[2] = {0u, 0u}, wt[2];
+  uint32_t w1[1] = {0u}, wt[1];
+  for (int i = b2; i < e2; ++i) w1[0] += ssum[i];
+  scan1024_excl(s_part, w1, wt);
+  uint32_t run3 = w1[0];
   for (int i = b2; i < e2; ++i) {
-    w2[0] += bsum[i];
-    w2[1] += ssum[i];
-  }
-  scan1024_excl(s_part, w2, wt);
-  uint32_t run2 = w2[0], run3 = w2[1];
-  for (int i = b2; i < e2; ++i) {
-    const uint32_t c = bsum[i], d = ssum[i];
-    bsum[i] = run2;
+    const uint32_t d = ssum[i];
     ssum[i] = run3;
-    run2 += c;
     run3 += d;
   }
   if (tid == 0) {
-    counters[8] = wt[1];
-    if (wt[1] > slot_capacity) atomicOr(&counters[1], kErrCapacity | kErrSlots);
+    counters[8] = wt[0];
+    if (wt[0] > slot_capacity) atomicOr(&counters[1], kErrCapacity | kErrSlots);
   }
 }
 
 hipError_t launch_scan_tiles(int T, const uint32_t* count, uint32_t* start, uint32_t* fill,
-                             uint32_t* ranges, uint32_t* counters, uint32_t capacity, int nb, uint32_t* bsum,
-                             uint32_t* ssum, uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off,
-                             hipStream_t s) {
+                             uint32_t* ranges, uint32_t* counters, uint32_t capacity, int nb, uint32_t* ssum,
+                             uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off, hipStream_t s) {
   hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanThreads), 0, s, T, count, start, fill, ranges,
-                     counters, capacity, nb, bsum, ssum, slot_capacity, large, seg_off);
+                     counters, capacity, nb, ssum, slot_capacity, large, seg_off);
   return hipGetLastError();
 }
 
@@ -700,16 +691,20 @@ hipError_t launch_scan_tiles(int T, const uint32_t* count, uint32_t* start, uint
 // buckets.  With few enough tiles, each workgroup first counts its instances
 // per tile in LDS, reserves one contiguous block per tile with a single
 // global atomic, then hands out slots inside the block with LDS atomics.
-// Instances are numbered in record order (record r's k-th tile, row-major
-// in its rectangle, is instance roff[r] + k) and the key's low word is the
-// instance number, which orders equal depths by record exactly as the
-// reference's (tile | depth, record) sort does; inst_rs maps it back to the
-// record (and to the instance's first partial-gradient slot).
-__global__ __launch_bounds__(256) void k_scatter(ScatterArgs a) {
+// The key's low word is the record number, which orders equal depths by
+// record exactly as the reference's (tile | depth, record) sort does.  Beside
+// each key goes what the sort would otherwise gather per entry from all over
+// the records: the instance's first partial-gradient slot and its quadrant
+// mask (pay).  Bound by the global atomics on the hot tiles and the chain
+// behind them: 1,024 surfels a workgroup make a quarter of the atomics 256 do.
+// 300k surfels at 800 x 600: 21 us, where 256 surfels a workgroup and 8-byte
+// (record, slot) pairs stored by instance number took 41; a million surfels
+// and 16 views: 528 us, was 901.
+constexpr int kScatterThreads = 1024;
+__global__ __launch_bounds__(kScatterThreads) void k_scatter(ScatterArgs a) {
   __shared__ uint32_t s_cnt[kHistTiles];
   __shared__ uint32_t s_base[kHistTiles];
-  __shared__ uint32_t s_wsum[4];
-  __shared__ uint32_t s_ssum[4];
+  __shared__ uint32_t s_ssum[kScatterThreads / 64];
   if (a.counters[1] & kErrCapacity) return;
   const int v = blockIdx.y;
   const int B = a.vs.B, gx = a.vs.v[v].gx, gy = a.vs.v[v].gy;
@@ -719,43 +714,46 @@ __global__ __launch_bounds__(256) void k_scatter(ScatterArgs a) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   const size_t r = (size_t)v * a.P + idx;
   int x0 = 0, y0 = 0, x1 = 0, y1 = 0;
-  uint64_t hi = 0;
+  uint64_t key = 0;
   const bool ok = idx < a.P && a.radii[r] > 0;
   if (ok) {
     const float4 q2 = a.rec[(size_t)kRecQuads * r + 2];
     get_rect(q2.y, q2.z, a.radii[r], B, gx, gy, x0, y0, x1, y1);
-    hi = (uint64_t)__float_as_uint(a.depths[r]) << 32;
+    key = (uint64_t)__float_as_uint(a.depths[r]) << 32 | (uint32_t)r;
   }
-  uint32_t total = 0;
-  const uint32_t inst0 =
-      a.bsum[(size_t)v * gridDim.x + blockIdx.x] +
-      block_scan256(ok ? (uint32_t)(x1 - x0) * (uint32_t)(y1 - y0) : 0u, s_wsum, total);
-  if (idx < a.P) a.roff[r] = inst0;
   // partial-gradient slots: the record's run, and each instance's first
   // slot (its quadrants' slots follow in quadrant order)
   const ViewInfo& vi = a.vs.v[v];
   const short4 bx = ok ? a.cullbox[r] : make_short4(32767, 32767, -32768, -32768);
   const uint32_t ns = ok ? record_slots(bx, x0, y0, x1, y1, B, vi) : 0u;
-  const uint32_t slot0 = a.ssum[(size_t)v * gridDim.x + blockIdx.x] + block_scan256(ns, s_ssum, total);
+  const int groups = (a.P + 255) / 256;  // of 256 records, per view, as the preprocess counted them
+  const int group = min(idx / 256, groups - 1);
+  uint32_t total = 0;
+  const uint32_t slot0 = a.ssum[(size_t)v * groups + group] + group_scan256(ns, s_ssum, total);
   if (idx < a.P) a.rslot[r] = make_uint2(slot0, ns);
-  if (ok) {
-    const int QX = B / kQuad;
-    uint32_t i = inst0, sl = slot0;
+  const int QX = B / kQuad;
+  // quadrant columns and rows of the image that the box meets
+  const int qc0 = bx.x > 0 ? bx.x / kQuad : 0, qc1 = min(bx.z >= 0 ? bx.z / kQuad : -1, (vi.W - 1) / kQuad);
+  const int qr0 = bx.y > 0 ? bx.y / kQuad : 0, qr1 = min(bx.w >= 0 ? bx.w / kQuad : -1, (vi.H - 1) / kQuad);
+  // place(t) gives the bucket position of this lane's instance in tile t
+  auto emit = [&](auto&& place) {
+    uint32_t sl = slot0;
     for (int ty = y0; ty < y1; ++ty) {
-      const uint32_t rows = (uint32_t)quad_span(bx.y, bx.w, ty * QX, ty * QX + QX, vi.H);
+      const int ra = max(qr0 - ty * QX, 0), rb = min(qr1 - ty * QX, QX - 1);
       for (int tx = x0; tx < x1; ++tx) {
-        a.inst_rs[i++] = make_uint2((uint32_t)r, sl);
-        sl += rows * (uint32_t)quad_span(bx.x, bx.z, tx * QX, tx * QX + QX, vi.W);
+        const int ca = max(qc0 - tx * QX, 0), cb = min(qc1 - tx * QX, QX - 1);
+        const uint32_t cols = ca <= cb ? (2u << cb) - (1u << ca) : 0u;
+        uint32_t mask = 0u;
+        for (int q = ra; q <= rb; ++q) mask |= cols << (q * QX);
+        const uint32_t at = place(ty * gx + tx);
+        a.keys[at] = key;
+        a.pay[at] = make_uint2(sl, mask);
+        sl += (uint32_t)__popc(mask);
       }
     }
-  }
-  uint64_t* keys = a.keys;
+  };
   if (!lds) {
-    if (ok) {
-      uint32_t i = inst0;
-      for (int ty = y0; ty < y1; ++ty)
-        for (int tx = x0; tx < x1; ++tx) keys[atomicAdd(&tile_fill[ty * gx + tx], 1u)] = hi | i++;
-    }
+    if (ok) emit([&](int t) { return atomicAdd(&tile_fill[t], 1u); });
     return;
   }
   for (int t = threadIdx.x; t < T; t += blockDim.x) s_cnt[t] = 0;
@@ -770,19 +768,13 @@ __global__ __launch_bounds__(256) void k_scatter(ScatterArgs a) {
     s_cnt[t] = 0;
   }
   __syncthreads();
-  if (ok) {
-    uint32_t i = inst0;
-    for (int ty = y0; ty < y1; ++ty)
-      for (int tx = x0; tx < x1; ++tx) {
-        const int t = ty * gx + tx;
-        keys[s_base[t] + atomicAdd(&s_cnt[t], 1u)] = hi | i++;
-      }
-  }
+  if (ok) emit([&](int t) { return s_base[t] + atomicAdd(&s_cnt[t], 1u); });
 }
 
 hipError_t launch_scatter(const ScatterArgs& a, hipStream_t s) {
   if (a.P == 0 || a.vs.V == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_scatter, dim3((a.P + 255) / 256, a.vs.V), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(k_scatter, dim3((a.P + kScatterThreads - 1) / kScatterThreads, a.vs.V), dim3(kScatterThreads), 0,
+                     s, a);
   return hipGetLastError();
 }
 
@@ -926,8 +918,9 @@ template <int NT, int K, int NB> struct TileLds {
 // merge sort instead.
 constexpr uint32_t kBinMax = 128;
 
-// Sorts the n <= NT K keys of a bucket at `src` and returns in inst[r] the
-// instance number (the key's low word) of sorted entry r NT + tid.
+// Sorts the n <= NT K keys of a bucket at `src` and returns in ent[r], for
+// sorted entry r NT + tid, the record (the key's low word) and the entry's
+// place in the unsorted bucket.
 //
 // The depths are cut into NB equal bins between the tile's smallest and
 // largest (depth bits, a monotone map), the keys counted into the bins, the
@@ -937,7 +930,7 @@ constexpr uint32_t kBinMax = 128;
 // dependent LDS accesses a key, where the merge sort it falls back to makes 50
 // to 300.
 template <int NT, int K, int NB>
-SR_DEV void sort_bucket(const uint64_t* src, int n, char* lds, uint32_t (&inst)[K]) {
+SR_DEV void sort_bucket(const uint64_t* src, int n, char* lds, uint2 (&ent)[K]) {
   constexpr int NW = NT / 64, per = NB / NT;
   static_assert(NB % NT == 0, "whole bins per lane");
   __shared__ uint32_t s_w[NW];
@@ -1005,78 +998,70 @@ SR_DEV void sort_bucket(const uint64_t* src, int n, char* lds, uint32_t (&inst)[
     for (int r = 0; r < K; ++r) keys[lds_slot<K>(r * NT + tid)] = r * NT + tid < n ? kv[r] : ~0ull;
     __syncthreads();
     merge_sort_lds<NT, K>(keys, max(next_pow2(n), K));
+    // each lane's own keys' ranks: lower bounds in the sorted keys
 #pragma unroll
-    for (int r = 0; r < K; ++r) inst[r] = (uint32_t)keys[lds_slot<K>(min(r * NT + tid, n - 1))];
-    __syncthreads();
-    return;
-  }
-  uint32_t run = incl - sum;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) run += w < wave ? s_w[w] : 0u;
-#pragma unroll
-  for (int t = 0; t < per; ++t) {
-    bins[tid * per + t] = run;
-    run += c[t];
-  }
-  if (tid == NT - 1) bins[NB] = run;
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < K; ++r)
-    if (r * NT + tid < n) keys[bins[bin_of(kv[r])] + at[r]] = kv[r];
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < K; ++r) {
-    at[r] = 0u;
-    if (r * NT + tid < n) {
-      const int b = bin_of(kv[r]);
-      const uint32_t b0 = bins[b], b1 = bins[b + 1];
-      uint32_t below = b0;
-      for (uint32_t m = b0; m < b1; ++m) below += keys[m] < kv[r] ? 1u : 0u;
+    for (int r = 0; r < K; ++r) {
+      uint32_t below = 0u;
+      for (int w = NT * K / 2; w > 0; w >>= 1)
+        if ((int)below + w <= n && keys[lds_slot<K>((int)below + w - 1)] < kv[r]) below += (uint32_t)w;
       at[r] = below;
+    }
+  } else {
+    uint32_t run = incl - sum;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) run += w < wave ? s_w[w] : 0u;
+#pragma unroll
+    for (int t = 0; t < per; ++t) {
+      bins[tid * per + t] = run;
+      run += c[t];
+    }
+    if (tid == NT - 1) bins[NB] = run;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < K; ++r)
+      if (r * NT + tid < n) keys[bins[bin_of(kv[r])] + at[r]] = kv[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+      at[r] = 0u;
+      if (r * NT + tid < n) {
+        const int b = bin_of(kv[r]);
+        const uint32_t b0 = bins[b], b1 = bins[b + 1];
+        uint32_t below = b0;
+        for (uint32_t m = b0; m < b1; ++m) below += keys[m] < kv[r] ? 1u : 0u;
+        at[r] = below;
+      }
     }
   }
   __syncthreads();
-  uint32_t* order = reinterpret_cast<uint32_t*>(lds);
+  uint2* order = reinterpret_cast<uint2*>(lds);
 #pragma unroll
   for (int r = 0; r < K; ++r)
-    if (r * NT + tid < n) order[at[r]] = (uint32_t)kv[r];
+    if (r * NT + tid < n) order[at[r]] = make_uint2((uint32_t)kv[r], (uint32_t)(r * NT + tid));
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < K; ++r) inst[r] = order[min(r * NT + tid, n - 1)];
+  for (int r = 0; r < K; ++r) ent[r] = order[min(r * NT + tid, n - 1)];
   __syncthreads();
 }
 
-// Looks up sorted entries' records (inst[r]: the instance of entry
-// r NT + tid of the cnt entries from tile-list position pos on), writes
-// point_list, each position's first slot and quadrant mask, and returns the
-// records and masks (no quadrant past the end).  Consecutive lanes write
-// consecutive positions; the gathers are unconditional (entries past the end
-// repeat the last one), so each round has all K loads in flight.
+// Writes point_list, first slot and quadrant mask of the cnt sorted entries
+// from tile-list position pos on (entry r NT + tid: record ent[r].x, payload
+// pay[ent[r].y]), consecutive lanes at consecutive positions, and returns the
+// masks (none past the end).
 template <int NT, int K>
-SR_DEV void place_entries(const SortArgs& a, int tile, uint32_t pos, int cnt, const uint32_t (&inst)[K],
-                          uint32_t (&rid)[K], uint32_t (&hm)[K]) {
-  const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
-  const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
-  const int ltile = tile - (int)vi.tile_base;
-  const int tx = ltile % vi.gx, ty = ltile / vi.gx;
+SR_DEV void place_entries(const SortArgs& a, const uint2* pay, uint32_t pos, int cnt, const uint2 (&ent)[K],
+                          uint32_t (&hm)[K]) {
   const int tid = threadIdx.x;
-  uint32_t sl[K];
+  uint2 p[K];  // all loads in flight
 #pragma unroll
-  for (int r = 0; r < K; ++r) {
-    const uint2 rs = a.inst_rs[inst[r]];
-    rid[r] = rs.x;
-    sl[r] = rs.y;
-  }
-  short4 bx[K];
-#pragma unroll
-  for (int r = 0; r < K; ++r) bx[r] = a.cullbox[rid[r]];
+  for (int r = 0; r < K; ++r) p[r] = pay[ent[r].y];
 #pragma unroll
   for (int r = 0; r < K; ++r) {
     const int i = r * NT + tid;
-    hm[r] = i < cnt ? quad_hits(bx[r], tx, ty, B, QX, Q, vi) : 0u;
+    hm[r] = i < cnt ? p[r].y : 0u;
     if (i < cnt) {
-      a.point_list[pos + i] = rid[r];
-      a.pos_slot[pos + i] = sl[r];
+      a.point_list[pos + i] = ent[r].x;
+      a.pos_slot[pos + i] = p[r].x;
       a.pos_quads[pos + i] = (uint16_t)hm[r];
     }
   }
@@ -1145,7 +1130,8 @@ SR_DEV int co_rank(const uint64_t* A, int na, const uint64_t* Bv, int nb, int k)
 // smallest and largest, and the keys moved bin by bin into key2.  Segment s of
 // the tile starts at the first bin boundary at or after kSegKeys s keys, so
 // segments hold kSegKeys keys give or take a bin, and their sorts, one
-// workgroup each, put the tile in order.  A segment above kSmallMax keys (more
+// workgroup each, put the tile in order; the payloads move along (24 us for
+// 300k surfels at 800 x 600, 14 of them the keys').  A segment above kSmallMax keys (more
 // than kSegKeys nearly equal depths in one bin) is sorted here: chunks in LDS,
 // then pairwise merges between the tile's two key buffers.
 constexpr int kSplitThreads = 1024, kSplitBins = 4096, kSplitRun = 4;
@@ -1211,18 +1197,18 @@ __global__ __launch_bounds__(kSplitThreads) void k_split_large(SortArgs a) {
     uint64_t* dst = a.key2 + beg;
     uint32_t* seg = a.seg_start + a.seg_off[l];
     const int nseg = (int)segments_of((uint32_t)n);
-    auto each = [&](auto&& fn) {  // every key of the tile, kU loads in flight a lane
+    auto each = [&](auto&& fn) {  // every key of the tile with its place, kU loads in flight a lane
       for (int i0 = 0; i0 < n; i0 += kU * NT) {
         uint64_t k[kU];
 #pragma unroll
         for (int t = 0; t < kU; ++t) k[t] = src[min(i0 + t * NT + tid, n - 1)];
 #pragma unroll
         for (int t = 0; t < kU; ++t)
-          if (i0 + t * NT + tid < n) fn(k[t]);
+          if (i0 + t * NT + tid < n) fn(k[t], i0 + t * NT + tid);
       }
     };
     uint32_t lo = 0xFFFFFFFFu, hi = 0u;
-    each([&](uint64_t k) {
+    each([&](uint64_t k, int) {
       const uint32_t d = (uint32_t)(k >> 32);
       lo = min(lo, d);
       hi = max(hi, d);
@@ -1247,7 +1233,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_split_large(SortArgs a) {
     }
     const float scale = (float)NB / ((float)(hi - lo) + 1.0f);
     auto bin_of = [&](uint64_t k) { return min(NB - 1, (int)((float)((uint32_t)(k >> 32) - lo) * scale)); };
-    each([&](uint64_t k) { atomicAdd(&bins[bin_of(k)], 1u); });
+    each([&](uint64_t k, int) { atomicAdd(&bins[bin_of(k)], 1u); });
     __syncthreads();
     uint32_t c[per], sum = 0u;
 #pragma unroll
@@ -1276,12 +1262,34 @@ __global__ __launch_bounds__(kSplitThreads) void k_split_large(SortArgs a) {
     }
     if (tid == 0) seg[0] = beg;
     __syncthreads();
-    each([&](uint64_t k) { dst[atomicAdd(&bins[bin_of(k)], 1u)] = k; });
+    const uint2* pay = a.pay + beg;
+    uint2* pay2 = a.pay2 + beg;
+    each([&](uint64_t k, int i) {
+      const uint32_t at = atomicAdd(&bins[bin_of(k)], 1u);
+      dst[at] = k;
+      pay2[at] = pay[i];
+    });
     __syncthreads();
     for (int sg = 0; sg < nseg; ++sg) {  // uniform
       const uint32_t s0 = seg[sg], s1 = sg + 1 < nseg ? seg[sg + 1] : beg + (uint32_t)n;
       if (s1 - s0 > (uint32_t)kSmallMax) {
-        sort_range(a.key2 + s0, a.keys + s0, (int)(s1 - s0), lds);
+        // merges between key2 and the tile's sub-list space (8 bytes an
+        // instance and quadrant, not written yet); the payloads then follow
+        // their keys by binary search
+        const int Q = quads_per_tile(a.vs.B), m = (int)(s1 - s0);
+        uint64_t* v = a.key2 + s0;
+        sort_range(v, reinterpret_cast<uint64_t*>(a.sub + (size_t)Q * s0), m, lds);
+        const uint64_t first = v[0], last = v[m - 1];
+        each([&](uint64_t k, int i) {
+          if (k < first || k > last) return;
+          int lo2 = 0, hi2 = m - 1;  // v[lo2] <= k
+          while (lo2 < hi2) {
+            const int mid = (lo2 + hi2 + 1) >> 1;
+            if (v[mid] <= k) lo2 = mid;
+            else hi2 = mid - 1;
+          }
+          pay2[(s0 - beg) + (uint32_t)lo2] = pay[i];
+        });
         __syncthreads();
       }
     }
@@ -1320,12 +1328,14 @@ SR_DEV Segment segment_item(const SortArgs& a, uint32_t it) {
 // sub-list entries placed by k_segment_lists.  Latency-bound: 300k surfels at
 // 800 x 600 put about 1,650 instances in each of 350 tiles, so a CU holds two
 // or three sorts and what counts is each one's chain of LDS and gather
-// latencies.  With the split and the segments' lists 64 us there, and 195 us
-// for 1M surfels at 1237 x 823; 256-lane merge sorts of 8 keys a lane, with
-// larger tiles cut into 2,048-key chunks merged by rank (and above 16,384 by
-// one workgroup), took 92 and 624 us.  One workgroup for each tile of up to
-// 16,384 was no better than those on the tiles it bounds (75 us for 8,192
-// keys, 132 us for 16,384).
+// latencies.  25 us there, and 481 for a million surfels and 16 views, where
+// looking each entry's record up by instance number and then its cull box took
+// 38 and 1,031.  256-lane merge sorts of 8 keys a lane, with larger tiles cut
+// into 2,048-key chunks merged by rank (and above 16,384 by one workgroup),
+// took 92 us (with the split and the segments' lists now 60) and 624 us for 1M
+// surfels at 1237 x 823.  One workgroup for each tile of up to 16,384 was no
+// better than those on the tiles it bounds (75 us for 8,192 keys, 132 us for
+// 16,384).
 constexpr int kSortThreads = 512, kSortKeys = kSmallMax / 512, kSortBins = 2048;
 __global__ __launch_bounds__(kSortThreads) void k_sort_tiles(SortArgs a, uint32_t seg_blocks) {
   constexpr int NT = kSortThreads, K = kSortKeys;
@@ -1335,7 +1345,8 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_tiles(SortArgs a, uint32_
   if (a.counters[1] & kErrCapacity) return;
   const int Q = quads_per_tile(a.vs.B);
   const int tid = threadIdx.x;
-  uint32_t inst[K], rid[K], hm[K];
+  uint2 ent[K];
+  uint32_t rid[K], hm[K];
   if (blockIdx.x < seg_blocks) {
     for (uint32_t it = blockIdx.x; it < a.counters[6]; it += seg_blocks) {
       const Segment g = segment_item(a, it);
@@ -1345,12 +1356,15 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_tiles(SortArgs a, uint32_
       for (int c0 = 0; c0 < g.cnt; c0 += NT * K) {
         const int cn = min(NT * K, g.cnt - c0);
         if (g.cnt <= NT * K) {
-          sort_bucket<NT, K, kSortBins>(a.key2 + g.s0, cn, lds, inst);
+          sort_bucket<NT, K, kSortBins>(a.key2 + g.s0, cn, lds, ent);
         } else {
 #pragma unroll
-          for (int r = 0; r < K; ++r) inst[r] = (uint32_t)a.key2[g.s0 + c0 + min(r * NT + tid, cn - 1)];
+          for (int r = 0; r < K; ++r) {
+            const int i = min(r * NT + tid, cn - 1);
+            ent[r] = make_uint2((uint32_t)a.key2[g.s0 + c0 + i], (uint32_t)i);
+          }
         }
-        place_entries<NT, K>(a, g.tile, g.s0 + c0, cn, inst, rid, hm);
+        place_entries<NT, K>(a, a.pay2 + g.s0 + c0, g.s0 + c0, cn, ent, hm);
         for (int q = 0; q < Q; ++q) {
           uint32_t hits = 0;
 #pragma unroll
@@ -1375,8 +1389,10 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_tiles(SortArgs a, uint32_
     }
     return;
   }
-  sort_bucket<NT, K, kSortBins>(a.keys + beg, n, lds, inst);
-  place_entries<NT, K>(a, tile, beg, n, inst, rid, hm);
+  sort_bucket<NT, K, kSortBins>(a.keys + beg, n, lds, ent);
+  place_entries<NT, K>(a, a.pay + beg, beg, n, ent, hm);
+#pragma unroll
+  for (int r = 0; r < K; ++r) rid[r] = ent[r].x;
   if (tid < Q) s_base[tid] = 0u;
   __syncthreads();
   append_sublists<NT, K>(a, beg, n, 0, Q, rid, hm, reinterpret_cast<uint32_t*>(lds), s_base);

@@ -95,7 +95,7 @@ __device__ inline int view_of_tile(const ViewSet& vs, uint32_t t) {
 
 // Geometry state: one entry per record (surfel, view).
 struct GeomLayout {
-  size_t rec, depths, tiles, clamped, roff, cullbox, bsum, ssum, rslot, total;
+  size_t rec, depths, tiles, clamped, cullbox, ssum, rslot, total;
 };
 // Workgroups of 256 records, per view, that preprocess and scatter use:
 // at most R / 256 + one partial workgroup per view.
@@ -107,9 +107,7 @@ inline GeomLayout geom_layout(size_t R) {
   g.depths = off; off += align_up(R * 4);
   g.tiles = off; off += align_up(R * 4);
   g.clamped = off; off += align_up(R * 4);  // 3 flags + pad per record
-  g.roff = off; off += align_up(R * 4);     // first instance number of the record
   g.cullbox = off; off += align_up(R * 8);   // short4 inclusive pixel box
-  g.bsum = off; off += align_up(record_groups(R) * 4);  // instances per workgroup, then their scan
   g.ssum = off; off += align_up(record_groups(R) * 4);  // partial-gradient slots per workgroup, then their scan
   g.rslot = off; off += align_up(R * 8);  // uint2 per record: first slot, slots
   g.total = off;
@@ -149,10 +147,10 @@ inline ImageLayout image_layout(const ViewSet& vs) {
 }
 inline ImageLayout image_layout(int W, int H, int B) { return image_layout(single_view(W, H, B)); }
 
-// Binning state: one entry per (surfel, tile) instance.  Instances are
-// numbered in record order: record r's k-th tile (row-major in its tile
-// rectangle) is instance roff[r] + k.
-//   inst_rs    instance -> (record, its first partial-gradient slot)
+// Binning state: one entry per (surfel, tile) instance.
+//   pay        bucket position -> (first partial-gradient slot, quadrant
+//              mask) of the instance there, written beside its key; pay2
+//              beside key2
 //   pos_slot   position in the concatenated sorted tile lists -> the first
 //              slot of the instance there
 //   pos_quads  position -> the quadrants whose sub-lists hold the instance
@@ -167,7 +165,7 @@ inline ImageLayout image_layout(int W, int H, int B) { return image_layout(singl
 //              size (slot capacity) does not move any other offset.
 struct BinLayout {
   size_t keys, key2, seg_start, seg_hits, point_list, sub, masks, chunk_T, work, frag_off, total;
-  size_t inst_rs, pos_slot, pos_quads, part, part_nz;
+  size_t pay, pay2, pos_slot, pos_quads, part, part_nz;
   size_t nslot;  // slots the part region holds
   size_t prec, fW;
   size_t frag_cap;
@@ -240,7 +238,8 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
   b.chunk_T = off; off += align_up(nslots * 4);  // per mask slot: product of (1 - alpha) over its pairs
   b.work = off; off += align_up(work_capacity(L, B, T) * 8);
   b.frag_off = off; off += align_up(nslots * 4);
-  b.inst_rs = off; off += align_up(n * 8);
+  b.pay = off; off += align_up(n * 8);
+  b.pay2 = off; off += align_up(n * 8);
   b.pos_slot = off; off += align_up(n * 4);
   b.pos_quads = off; off += align_up(n * 2);
   b.nslot = slot_capacity > 0 ? (size_t)slot_capacity : n * Q;
@@ -287,7 +286,6 @@ struct PreprocessArgs {
   uint32_t* tiles;
   uint8_t* clamped;
   short4* cullbox;
-  uint32_t* bsum;
   uint32_t* ssum;  // partial-gradient slots per workgroup
   uint32_t* tile_count;
   uint32_t* counters;
@@ -300,14 +298,12 @@ struct ScatterArgs {
   const float* depths;
   const int* radii;
   const uint32_t* counters;
-  const uint32_t* bsum;
   const uint32_t* ssum;  // first slot of each workgroup
   const short4* cullbox;
-  uint32_t* roff;
   uint2* rslot;    // per record: first slot, slots
-  uint2* inst_rs;  // per instance: record, first slot
   uint32_t* tile_fill;
   uint64_t* keys;
+  uint2* pay;
 };
 
 struct SortArgs {
@@ -321,8 +317,8 @@ struct SortArgs {
   uint64_t* keys;
   uint64_t* key2;
   uint32_t* point_list;
-  const short4* cullbox;
-  const uint2* inst_rs;
+  const uint2* pay;
+  uint2* pay2;
   uint32_t* pos_slot;
   uint16_t* pos_quads;
   uint2* sub;
@@ -424,7 +420,6 @@ struct PreprocessBwdArgs {
   int P, D, M;
   const uint32_t* counters;
   const uint32_t* tiles;
-  const uint32_t* roff;
   const uint2* rslot;  // per record: first slot, slots
   const float* part;
   const uint8_t* part_nz;
@@ -504,9 +499,8 @@ hipError_t launch_fill_f32(float* p, float v, size_t n, hipStream_t s);
 int set_error(int code, const char* msg);
 hipError_t launch_preprocess(const PreprocessArgs& a, hipStream_t s);
 hipError_t launch_scan_tiles(int T, const uint32_t* count, uint32_t* start, uint32_t* fill,
-                             uint32_t* ranges, uint32_t* counters, uint32_t capacity, int nb, uint32_t* bsum,
-                             uint32_t* ssum, uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off,
-                             hipStream_t s);
+                             uint32_t* ranges, uint32_t* counters, uint32_t capacity, int nb, uint32_t* ssum,
+                             uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off, hipStream_t s);
 hipError_t launch_scatter(const ScatterArgs& a, hipStream_t s);
 hipError_t launch_sort_tiles(const SortArgs& a, size_t max_segments, hipStream_t s);
 hipError_t launch_accept(const AcceptArgs& a, size_t max_items, hipStream_t s);
