@@ -18,7 +18,9 @@ Every call runs on the HIP library; there is no CPU path.
 """
 from __future__ import annotations
 
+import collections
 import ctypes as C
+import threading
 from typing import NamedTuple
 
 import torch
@@ -219,23 +221,80 @@ def mark_visible(means3D, viewmatrix, projmatrix):
     return present
 
 
-# Binning capacity per (device, tile, width, height): the last instance
-# count with an eighth of headroom.  The first forward of a key sizes its
-# binning buffer from the exact count (one stream synchronisation
-# mid-forward, as the reference); later ones enqueue the whole forward at
-# once and only fall back to a larger capacity when the count outgrows it.
-# The accepted-pair store follows the pairs per instance of the latest
-# completed forward on the device with the same tile (read back without
-# waiting) times the instance capacity, so it shares the capacity's eighth
-# of headroom; pairs beyond the store are recomputed with the same results.
+# Buffer sizes per (device, tile, width, height[, variant]).  The first forward
+# of a key sizes its binning buffer from the exact instance count (one stream
+# synchronisation mid-forward, as the reference); later ones take the last
+# count with an eighth of headroom, enqueue the whole forward at once and only
+# fall back to a larger capacity when the count outgrows it.
+# The accepted-pair store and the partial-gradient slots take the largest
+# counts that completed forwards of the key needed (read back without waiting),
+# with the same headroom.  Sized from the latest forward alone they run out
+# whenever views or scenes that differ by more than the headroom alternate, and
+# pairs beyond the store are recomputed by each pass that needs them: two
+# scenes of 300k surfels at 800 x 600 in turn took 1,844 us a forward and
+# backward, and take 705 with the larger of their counts.  The largest count
+# fades by a 1,024th a forward, so that a scene which lost surfels gives its
+# memory back.
 _capacity_hint = {}
-_pair_ratio = {}
-_slot_ratio = {}  # partial-gradient slots per instance, likewise
-_PAIRS_PER_INSTANCE = 8.0  # before any count is known
+_pair_hint = {}  # accepted pairs
+_slot_hint = {}  # partial-gradient slots
+_PAIRS_PER_INSTANCE = 8  # before any count is known
+_INT_MAX = 0x7FFFFFFF
+_recent = threading.local()  # (instances, key) of the thread's latest forwards
 
 
 def _grown(n: int) -> int:
     return n + n // 8 + 1024
+
+
+def _note_count(hint, seen):
+    """Enters a completed forward's (count, instances) into the hint of its key."""
+    if seen is None:
+        return
+    for n, key in _recent.forwards:
+        if n == seen[1]:
+            old = hint.get(key, 0)
+            hint[key] = max(seen[0], old - old // 1024)
+            return
+
+
+def _forward_sized(key, debug, forward):
+    """Runs forward(capacity, pair_capacity, slot_capacity), which returns a
+    tuple headed by the instance count, with the key's buffer sizes, and again
+    with larger ones while it raises CapacityError.  Returns the result and the
+    sizes."""
+    if not hasattr(_recent, "forwards"):
+        _recent.forwards = collections.deque(maxlen=8)
+    with torch.cuda.device(key[0]):
+        _note_count(_pair_hint, _lib.pair_count())
+        _note_count(_slot_hint, _lib.slot_count())
+    hint = cap = 0 if debug else _capacity_hint.get(key, 0)
+    while True:
+        pcap = scap = 0
+        if cap > 0:
+            pairs, slots = _pair_hint.get(key, 0), _slot_hint.get(key, 0)
+            pcap = min(_grown(pairs) if pairs else _PAIRS_PER_INSTANCE * cap, _INT_MAX)
+            scap = min(_grown(slots), _INT_MAX) if slots else 0  # 0: every (instance, quadrant)
+        try:
+            out = forward(cap, pcap, scap)
+            break
+        except _lib.CapacityError as e:
+            if e.slots:
+                _slot_hint.pop(key, None)
+            else:
+                cap = _grown(e.needed)
+    n = out[0]
+    # keep the hint tracking the count: set by an exact or a retried forward,
+    # shrunk (with what was measured under it) when the count fell far below it
+    shrunk = _grown(n) * 4 < cap
+    if cap != hint or cap == 0 or shrunk:
+        _capacity_hint[key] = _grown(n)
+    if shrunk:
+        _pair_hint.pop(key, None)
+        _slot_hint.pop(key, None)
+        _recent.forwards = collections.deque((f for f in _recent.forwards if f[1] != key), maxlen=8)
+    _recent.forwards.appendleft((n, key))
+    return out, (cap, pcap, scap)
 
 
 class _RasterizeGaussians(torch.autograd.Function):
@@ -244,50 +303,15 @@ class _RasterizeGaussians(torch.autograd.Function):
     @staticmethod
     def forward(ctx, means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
                 raster_settings):
-        tile = getattr(raster_settings, "tile", 16)
-        key = (means3D.device, tile, int(raster_settings.image_width), int(raster_settings.image_height))
-        hint = 0 if raster_settings.debug else _capacity_hint.get(key, 0)
-        cap = hint
-        rkey = (means3D.device, tile)
-        with torch.cuda.device(means3D.device):
-            seen = _lib.pair_count()
-            seen_slots = _lib.slot_count()
-        if seen is not None and seen[1] > 0 and rkey in _pair_ratio:
-            _pair_ratio[rkey] = seen[0] / seen[1]
-        if seen_slots is not None and seen_slots[1] > 0 and rkey in _slot_ratio:
-            _slot_ratio[rkey] = seen_slots[0] / seen_slots[1]
-        while True:
-            ratio = _pair_ratio.get(rkey) or _PAIRS_PER_INSTANCE
-            # the capacity already holds an eighth more instances than the
-            # last count: pairs and slots per instance scale with it
-            pcap = min(int(ratio * cap) + 4096, 0x7FFFFFFF) if cap > 0 else 0
-            sratio = _slot_ratio.get(rkey)
-            scap = min(int(sratio * cap) + 1024, 0x7FFFFFFF) if cap > 0 and sratio else 0
-            try:
-                num_rendered, color, depth, radii, geomBuffer, binningBuffer, imgBuffer = rasterize_gaussians_fwd(
-                    raster_settings.bg, means3D, colors_precomp, opacities, scales, rotations,
-                    raster_settings.scale_modifier, cov3Ds_precomp, raster_settings.viewmatrix,
-                    raster_settings.projmatrix, raster_settings.tanfovx, raster_settings.tanfovy,
-                    raster_settings.image_height, raster_settings.image_width, sh, raster_settings.sh_degree,
-                    raster_settings.campos, raster_settings.prefiltered, raster_settings.debug, tile,
-                    capacity=cap, pair_capacity=pcap, slot_capacity=scap)
-                break
-            except _lib.CapacityError as e:
-                if e.slots:
-                    _slot_ratio[rkey] = 0.0  # this forward: every (instance, quadrant)
-                else:
-                    cap = _grown(e.needed)
-        # keep the hint tracking the count: set by an exact or a retried
-        # forward, shrunk when the count fell far below it
-        if cap != hint or cap == 0 or _grown(num_rendered) * 4 < cap:
-            _capacity_hint[key] = _grown(num_rendered)
-        # from now on the pair store and the slots follow the measured counts
-        _pair_ratio.setdefault(rkey, 0.0)
-        _slot_ratio.setdefault(rkey, 0.0)
-        ctx.pair_capacity = pcap
-        ctx.slot_capacity = scap
-        ctx.raster_settings = raster_settings
-        ctx.capacity = cap
+        rs = raster_settings
+        tile = getattr(rs, "tile", 16)
+        key = (means3D.device, tile, int(rs.image_width), int(rs.image_height))
+        out, ctx.sizes = _forward_sized(key, rs.debug, lambda cap, pcap, scap: rasterize_gaussians_fwd(
+            rs.bg, means3D, colors_precomp, opacities, scales, rotations, rs.scale_modifier, cov3Ds_precomp,
+            rs.viewmatrix, rs.projmatrix, rs.tanfovx, rs.tanfovy, rs.image_height, rs.image_width, sh, rs.sh_degree,
+            rs.campos, rs.prefiltered, rs.debug, tile, capacity=cap, pair_capacity=pcap, slot_capacity=scap))
+        num_rendered, color, depth, radii, geomBuffer, binningBuffer, imgBuffer = out
+        ctx.raster_settings = rs
         ctx.num_rendered = num_rendered
         ctx.save_for_backward(colors_precomp, means3D, scales, rotations, cov3Ds_precomp, radii, sh, geomBuffer,
                               binningBuffer, imgBuffer)
@@ -301,6 +325,7 @@ class _RasterizeGaussians(torch.autograd.Function):
     def backward(ctx, grad_out_color, grad_radii, grad_depth):
         num_rendered = ctx.num_rendered
         rs = ctx.raster_settings
+        cap, pcap, scap = ctx.sizes
         colors_precomp, means3D, scales, rotations, cov3Ds_precomp, radii, sh, geomBuffer, binningBuffer, imgBuffer = (
             ctx.saved_tensors)
         if grad_out_color is None:
@@ -312,7 +337,7 @@ class _RasterizeGaussians(torch.autograd.Function):
             rs.bg, means3D, radii, colors_precomp, scales, rotations, rs.scale_modifier, cov3Ds_precomp,
             rs.viewmatrix, rs.projmatrix, rs.tanfovx, rs.tanfovy, grad_out_color, grad_depth, sh, rs.sh_degree,
             rs.campos, geomBuffer, num_rendered, binningBuffer, imgBuffer, rs.debug, getattr(rs, "tile", 16),
-            capacity=ctx.capacity, pair_capacity=ctx.pair_capacity, slot_capacity=ctx.slot_capacity)
+            capacity=cap, pair_capacity=pcap, slot_capacity=scap)
         return (grad_means3D, grad_means2D, grad_sh, grad_colors_precomp, grad_opacities, grad_scales,
                 grad_rotations, grad_cov3Ds_precomp, None)
 

@@ -27,7 +27,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .rasterizer import _Arena, _f32, _settings, _surfels, mark_visible
+from .rasterizer import _Arena, _f32, _forward_sized, _settings, _surfels, mark_visible
 
 MAX_SEMANTIC_TYPES = 16
 
@@ -146,14 +146,16 @@ class _RasterizeGaussians(torch.autograd.Function):
     @staticmethod
     def forward(ctx, means3D, means2D, sh, colors_precomp, opacities, semantics, scales, rotations, cov3Ds_precomp,
                 raster_settings):
-        tile = getattr(raster_settings, "tile", 16)
-        num_rendered, color, semantic, depth, radii, geomBuffer, binningBuffer, imgBuffer = rasterize_gaussians_fwd(
-            raster_settings.bg, means3D, colors_precomp, opacities, semantics, scales, rotations,
-            raster_settings.scale_modifier, cov3Ds_precomp, raster_settings.viewmatrix, raster_settings.projmatrix,
-            raster_settings.tanfovx, raster_settings.tanfovy, raster_settings.image_height,
-            raster_settings.image_width, sh, raster_settings.sh_degree, raster_settings.campos,
-            raster_settings.prefiltered, raster_settings.debug, tile)
-        ctx.raster_settings = raster_settings
+        rs = raster_settings
+        tile = getattr(rs, "tile", 16)
+        key = (means3D.device, tile, int(rs.image_width), int(rs.image_height), "part")
+        out, ctx.sizes = _forward_sized(key, rs.debug, lambda cap, pcap, scap: rasterize_gaussians_fwd(
+            rs.bg, means3D, colors_precomp, opacities, semantics, scales, rotations, rs.scale_modifier,
+            cov3Ds_precomp, rs.viewmatrix, rs.projmatrix, rs.tanfovx, rs.tanfovy, rs.image_height, rs.image_width, sh,
+            rs.sh_degree, rs.campos, rs.prefiltered, rs.debug, tile, capacity=cap, pair_capacity=pcap,
+            slot_capacity=scap))
+        num_rendered, color, semantic, depth, radii, geomBuffer, binningBuffer, imgBuffer = out
+        ctx.raster_settings = rs
         ctx.num_rendered = num_rendered
         ctx.save_for_backward(colors_precomp, semantics, means3D, scales, rotations, cov3Ds_precomp, radii, sh,
                               geomBuffer, binningBuffer, imgBuffer)
@@ -180,7 +182,7 @@ class _RasterizeGaussians(torch.autograd.Function):
             rs.bg, means3D, radii, colors_precomp, semantics, scales, rotations, rs.scale_modifier, cov3Ds_precomp,
             rs.viewmatrix, rs.projmatrix, rs.tanfovx, rs.tanfovy, grad_out_color, grad_out_semantic, grad_depth, sh,
             rs.sh_degree, rs.campos, geomBuffer, ctx.num_rendered, binningBuffer, imgBuffer, rs.debug,
-            getattr(rs, "tile", 16))
+            getattr(rs, "tile", 16), *ctx.sizes)
         if semantics.ndimension() != 2:
             grad_semantics = None
         return (grad_means3D, grad_means2D, grad_sh, grad_colors_precomp, grad_opacities, grad_semantics, grad_scales,
