@@ -130,13 +130,18 @@ hipEvent_t counts_event() {
   if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) e = nullptr;
   return e;
 }
-// Pinned 64-byte landing zone for the forward counters (instances, error flags, slots).
-// Pinned 8-byte landing zone for the instance count and error flags.
+// Pinned memory the kernels write: portable, since a thread may use several
+// devices, and coherent, since the host reads it after an event.
+uint32_t* pinned_words(size_t n) {
+  void* p = nullptr;
+  const unsigned flags = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
+  return hipHostMalloc(&p, n * sizeof(uint32_t), flags) == hipSuccess ? (uint32_t*)p : nullptr;
+}
+// The calling thread's landing zone for the tile scan's counts (instances,
+// error flags, slots).
 uint32_t* pinned_counters() {
   thread_local uint32_t* p = nullptr;
-  if (!p) {
-    if (hipHostMalloc((void**)&p, 16 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) p = nullptr;
-  }
+  if (!p) p = pinned_words(16);
   return p;
 }
 
@@ -188,6 +193,8 @@ struct Pipeline {
   int capacity = 0;
   bool part = false;       // the _part variant
   int S = 0;               // its semantic channels
+  uint32_t* host_front = nullptr;   // pinned words for the tile scan's counts, or null
+  uint32_t* host_counts = nullptr;  // pinned words for the forward's final counts, or null
   uint32_t* counters() const { return (uint32_t*)(img + il.counters); }
 };
 
@@ -200,8 +207,8 @@ PairStore pair_store(char* bin, const BinLayout& bl) {
 
 // Pinned landing zones and events for the accepted-pair count of recent
 // forwards, per (host thread, device): a ring of kPairSlots, so enqueuing a
-// forward only ever waits for the copy of the forward kPairSlots before it
-// (long finished), never for the one still running.
+// forward only ever waits for the one kPairSlots before it (long finished),
+// never for the one still running.
 constexpr int kPairSlots = 4;
 constexpr int kCountWords = 16;
 struct PairCount {
@@ -218,26 +225,34 @@ PairCount& pair_count_slot() {
   return slots[dev];
 }
 
-// Enqueues the copy of the instance, pair and slot counts (counters[0..8])
-// of the forward just enqueued into the next slot of the ring.
-int post_pair_count(Pipeline& pl, hipStream_t st) {
+// The ring's next slot, for the forward being enqueued to write its counts
+// (counters[0..8]) into; NULL on failure.
+uint32_t* next_count_slot(int& rc) {
   PairCount& pc = pair_count_slot();
+  rc = SR_OK;
   if (!pc.host) {
-    if (hipHostMalloc((void**)&pc.host, kPairSlots * kCountWords * sizeof(uint32_t), hipHostMallocDefault) !=
-        hipSuccess) {
-      pc.host = nullptr;
-      return fail(SR_ERR_HIP, "hipHostMalloc failed");
+    uint32_t* host = pinned_words(kPairSlots * kCountWords);
+    for (int k = 0; host && k < kPairSlots; ++k)
+      if (!pc.ev[k] && hipEventCreateWithFlags(&pc.ev[k], hipEventDisableTiming) != hipSuccess) pc.ev[k] = nullptr;
+    if (!host || !pc.ev[kPairSlots - 1]) {
+      rc = fail(SR_ERR_HIP, "no pinned memory or event for the counts");
+      return nullptr;
     }
-    for (int k = 0; k < kPairSlots; ++k)
-      if (hipEventCreateWithFlags(&pc.ev[k], hipEventDisableTiming) != hipSuccess)
-        return fail(SR_ERR_HIP, "hipEventCreate failed");
+    pc.host = host;
   }
-  const int k = pc.next;
-  if (pc.seq[k] != 0) SR_HIP(hipEventSynchronize(pc.ev[k]));  // the copy of kPairSlots forwards ago
-  SR_HIP(hipMemcpyAsync(pc.host + kCountWords * k, pl.counters(), 9 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  SR_HIP(hipEventRecord(pc.ev[k], st));
-  pc.seq[k] = pc.next_seq++;
-  pc.next = (k + 1) % kPairSlots;
+  // written kPairSlots forwards ago
+  if (pc.seq[pc.next] != 0 && hipEventSynchronize(pc.ev[pc.next]) != hipSuccess) {
+    rc = fail(SR_ERR_HIP, "hipEventSynchronize failed");
+    return nullptr;
+  }
+  return pc.host + kCountWords * pc.next;
+}
+// Marks the slot as in use by the forward just enqueued.
+int post_counts(hipStream_t st) {
+  PairCount& pc = pair_count_slot();
+  SR_HIP(hipEventRecord(pc.ev[pc.next], st));
+  pc.seq[pc.next] = pc.next_seq++;
+  pc.next = (pc.next + 1) % kPairSlots;
   return SR_OK;
 }
 
@@ -375,7 +390,7 @@ int run_front(Pipeline& pl, const sr_surfels* g, int* radii, uint32_t capacity, 
                              (uint32_t*)(pl.img + pl.il.tile_fill), (uint32_t*)(pl.img + pl.il.ranges), counters,
                              capacity, pl.vs.V * ((pl.P + 255) / 256),
                              (uint32_t*)(pl.geom + pl.gl.ssum), slot_capacity, (uint32_t*)(pl.img + pl.il.large),
-                             (uint32_t*)(pl.img + pl.il.seg_off), st));
+                             (uint32_t*)(pl.img + pl.il.seg_off), pl.host_front, st));
   return SR_OK;
 }
 
@@ -444,7 +459,8 @@ int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st) {
   SR_STAGE(8, dbg, st, "accept", launch_accept(aa, items, st));
   SR_STAGE(10, dbg, st, "pair_offsets", launch_pair_offsets(aa, st));
   SR_STAGE(10, dbg, st, "order",
-           launch_order_quads(pl.il.T * quads_per_tile(pl.vs.B), aa.q_cost, (uint32_t*)(pl.img + pl.il.q_order), st));
+           launch_order_quads(pl.il.T * quads_per_tile(pl.vs.B), aa.q_cost, (uint32_t*)(pl.img + pl.il.q_order),
+                              counters, pl.host_counts, st));
   SR_STAGE(10, dbg, st, "pair_write", launch_pair_write(aa, items, st));
   return SR_OK;
 }
@@ -691,25 +707,27 @@ int forward_view(const sr_settings* s, const sr_surfels* g, bool part, int S, co
   pl.il = il;
   uint32_t* host = pinned_counters();
   if (!host) return fail(SR_ERR_HIP, "hipHostMalloc failed");
+  pl.host_front = host;
+  pl.host_counts = next_count_slot(rc);
+  if (!pl.host_counts) return rc;
   if (cap > 0) {
     // Everything enqueued at once on a binning buffer of the caller's
     // capacity; the kernels after the scan do nothing when the instances
-    // exceed it.  The instance count is copied back right after the scan
-    // and waited for only once the rest is enqueued, by when it has long
-    // arrived, so the stream never drains mid-forward.
+    // exceed it.  The scan writes the instance count back and it is waited
+    // for only once the rest is enqueued, by when it has long arrived, so
+    // the stream never drains mid-forward.
     pl.bl = bin_layout(cap, B, il.T, s->pair_store, s->pair_capacity, S, s->slot_capacity);
     pl.bin = (char*)alloc(ctx, pl.bl.total, 1);
     if (!pl.bin) return fail(SR_ERR_ALLOC, "allocation callback failed");
     pl.capacity = cap;
     rc = run_front(pl, g, radii, (uint32_t)cap, (uint32_t)pl.bl.nslot, dbg, st);
     if (rc != SR_OK) return rc;
-    SR_HIP(hipMemcpyAsync(host, pl.counters(), 9 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     hipEvent_t counted = counts_event();
     if (!counted) return fail(SR_ERR_HIP, "hipEventCreate failed");
     SR_HIP(hipEventRecord(counted, st));
     rc = run_binning(pl, radii, dbg, st);
     if (rc == SR_OK) rc = run_blend_fwd(pl, out_color, out_others, dbg, st, semantics, out_semantic);
-    if (rc == SR_OK) rc = post_pair_count(pl, st);
+    if (rc == SR_OK) rc = post_counts(st);
     SR_HIP(hipEventSynchronize(counted));
     if (rc != SR_OK) return rc;
     if (host[1] & kErrPrefiltered)
@@ -723,7 +741,6 @@ int forward_view(const sr_settings* s, const sr_surfels* g, bool part, int S, co
   }
   rc = run_front(pl, g, radii, 0xFFFFFFFFu, 0xFFFFFFFFu, dbg, st);
   if (rc != SR_OK) return rc;
-  SR_HIP(hipMemcpyAsync(host, pl.counters(), 9 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
   SR_HIP(hipStreamSynchronize(st));
   if (host[1] & kErrPrefiltered)
     return fail(SR_ERR_PREFILTERED, "Point is filtered although prefiltered is set. This shouldn't happen!");
@@ -741,7 +758,7 @@ int forward_view(const sr_settings* s, const sr_surfels* g, bool part, int S, co
     if (rc != SR_OK) return rc;
     rc = run_blend_fwd(pl, out_color, out_others, dbg, st, semantics, out_semantic);
     if (rc != SR_OK) return rc;
-    return post_pair_count(pl, st);
+    return post_counts(st);
   }
   rc = clear_lists(pl, dbg, st);
   if (rc != SR_OK) return rc;

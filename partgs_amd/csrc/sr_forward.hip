@@ -615,14 +615,19 @@ SR_DEV void scan1024_excl(uint32_t* s, uint32_t (&x)[N], uint32_t (&total)[N]) {
 // number of each one's first kSegKeys-key segment (seg_off, followed by the
 // total, which also goes to counters[6]);
 // then the same scan for the per-workgroup slot totals of the preprocess (in
-// place), which numbers every record's slots in record order.
+// place), which numbers every record's slots in record order.  host (pinned
+// memory, may be null) receives what the caller waits for, the instances
+// [0], error flags [1] and slots [8]: a copy command after the kernel is a
+// launch of its own in the stream.  Without the two of them a forward and
+// backward of 300k surfels at 800 x 600 takes 679 us instead of 683, and
+// fitting 16 blocks to six views 640 instead of 726.
 constexpr int kScanThreads = 1024;
 __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32_t* count,
                                                               uint32_t* start, uint32_t* fill,
                                                               uint32_t* ranges, uint32_t* counters,
                                                               uint32_t capacity, int nb, uint32_t* ssum,
                                                               uint32_t slot_capacity,
-                                                              uint32_t* large, uint32_t* seg_off) {
+                                                              uint32_t* large, uint32_t* seg_off, uint32_t* host) {
   __shared__ uint32_t s_part[3 * 32];
   const int tid = threadIdx.x;
   const int per = (T + kScanThreads - 1) / kScanThreads;
@@ -677,13 +682,21 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32
     counters[8] = wt[0];
     if (wt[0] > slot_capacity) atomicOr(&counters[1], kErrCapacity | kErrSlots);
   }
+  if (host == nullptr) return;
+  __syncthreads();
+  if (tid == 0) {
+    host[0] = tot3[0];
+    host[1] = __hip_atomic_load(&counters[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    host[8] = wt[0];
+  }
 }
 
 hipError_t launch_scan_tiles(int T, const uint32_t* count, uint32_t* start, uint32_t* fill,
                              uint32_t* ranges, uint32_t* counters, uint32_t capacity, int nb, uint32_t* ssum,
-                             uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off, hipStream_t s) {
+                             uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off, uint32_t* host,
+                             hipStream_t s) {
   hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanThreads), 0, s, T, count, start, fill, ranges,
-                     counters, capacity, nb, ssum, slot_capacity, large, seg_off);
+                     counters, capacity, nb, ssum, slot_capacity, large, seg_off, host);
   return hipGetLastError();
 }
 
@@ -1679,9 +1692,13 @@ __global__ __launch_bounds__(64) void k_pair_offsets(AcceptArgs a) {
 // 1024-lane workgroup), so the blend kernels dispatch the longest per-pixel
 // chains first and the tail of the launch is short work.  The order within a
 // bucket is arbitrary; each quadrant's result does not depend on it.
-__global__ __launch_bounds__(1024) void k_order_quads(int nq, const uint32_t* cost, uint32_t* order) {
+// host (pinned memory, may be null) receives counters[0..8], final from the
+// pair-offset pass on.
+__global__ __launch_bounds__(1024) void k_order_quads(int nq, const uint32_t* cost, uint32_t* order,
+                                                      const uint32_t* counters, uint32_t* host) {
   __shared__ uint32_t s_cnt[64], s_base[64];
   const int tid = threadIdx.x;
+  if (host != nullptr && tid < 9) host[tid] = counters[tid];
   if (tid < 64) s_cnt[tid] = 0;
   __syncthreads();
   auto bucket = [](uint32_t c) {  // 63 for the costliest
@@ -1723,9 +1740,10 @@ __global__ __launch_bounds__(1024) void k_order_quads(int nq, const uint32_t* co
   }
 }
 
-hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, hipStream_t s) {
+hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, const uint32_t* counters,
+                              uint32_t* host, hipStream_t s) {
   if (nq <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_order_quads, dim3(1), dim3(1024), 0, s, nq, cost, order);
+  hipLaunchKernelGGL(k_order_quads, dim3(1), dim3(1024), 0, s, nq, cost, order, counters, host);
   return hipGetLastError();
 }
 

@@ -500,13 +500,15 @@ int set_error(int code, const char* msg);
 hipError_t launch_preprocess(const PreprocessArgs& a, hipStream_t s);
 hipError_t launch_scan_tiles(int T, const uint32_t* count, uint32_t* start, uint32_t* fill,
                              uint32_t* ranges, uint32_t* counters, uint32_t capacity, int nb, uint32_t* ssum,
-                             uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off, hipStream_t s);
+                             uint32_t slot_capacity, uint32_t* large, uint32_t* seg_off, uint32_t* host,
+                             hipStream_t s);
 hipError_t launch_scatter(const ScatterArgs& a, hipStream_t s);
 hipError_t launch_sort_tiles(const SortArgs& a, size_t max_segments, hipStream_t s);
 hipError_t launch_accept(const AcceptArgs& a, size_t max_items, hipStream_t s);
 hipError_t launch_pair_offsets(const AcceptArgs& a, hipStream_t s);
 hipError_t launch_pair_write(const AcceptArgs& a, size_t max_items, hipStream_t s);
-hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, hipStream_t s);
+hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, const uint32_t* counters,
+                              uint32_t* host, hipStream_t s);
 hipError_t launch_iota_u32(uint32_t* p, size_t n, hipStream_t s);
 hipError_t launch_blend_fwd(const BlendArgs& a, hipStream_t s);
 hipError_t launch_blend_semantics(const BlendArgs& a, hipStream_t s);
