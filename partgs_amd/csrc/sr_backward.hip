@@ -17,6 +17,8 @@
 // gradient is accumulated with global atomics, and the result does not
 // depend on scheduling order.
 #include "sr_device.h"
+#include <type_traits>
+
 #include "sr_internal.h"
 #include "sr_pair.h"
 
@@ -25,15 +27,10 @@ namespace sr {
 // Partial-gradient slots: 0..8 dL_dtransMat, 9..10 dL_dmean2D.xy,
 // 11..13 dL_dnormal, 14 dL_dopacity, 15..17 dL_dcolors.
 constexpr int kNumG = 18;
-constexpr int kPre = 8;       // pairs a lane fetches ahead in the per-pair pass
-#ifndef SR_CHAIN_PREFETCH
-#define SR_CHAIN_PREFETCH 4
-#endif
-constexpr int kChainPre = SR_CHAIN_PREFETCH;  // stored pairs a lane fetches ahead in the chain pass
-// waves per quadrant in the chain pass (64 / kSplitBwd = 8 pixels each,
-// 8 lanes per pixel)
-constexpr int kSplitBwd = 8;
-constexpr int kChainSegMin = 16;  // shortest chain segment a lane replays
+constexpr int kChainPre = 4;  // pairs of a batch in the chain pass: three 64-byte pieces
+using V4 = float __attribute__((ext_vector_type(4)));  // a float4 the compiler keeps in registers as a whole
+constexpr int kOwnerQuads = 3 * 64 + 1;  // LDS quads of one quad lane's batches, the odd one against bank conflicts
+constexpr unsigned kChainBlocks = 16384;  // workgroups of the chain pass at most
 #ifndef SR_GRAD_GROUP
 #define SR_GRAD_GROUP 4
 #endif
@@ -216,21 +213,22 @@ struct SegMap {
     s.accum_alpha_rec = A * s.accum_alpha_rec + b[7];
     s.last_dL_dT = A2 * s.last_dL_dT + b2;
   }
+  // in LDS, a lane's words 64 apart
   SR_DEV void save(float* d) const {
     d[0] = A;
-    d[1] = A2;
-    d[2] = b2;
-    d[3] = D;
+    d[64] = A2;
+    d[128] = b2;
+    d[192] = D;
 #pragma unroll
-    for (int x = 0; x < 8; ++x) d[4 + x] = b[x];
+    for (int x = 0; x < 8; ++x) d[64 * (4 + x)] = b[x];
   }
   SR_DEV void load(const float* d) {
     A = d[0];
-    A2 = d[1];
-    b2 = d[2];
-    D = d[3];
+    A2 = d[64];
+    b2 = d[128];
+    D = d[192];
 #pragma unroll
-    for (int x = 0; x < 8; ++x) b[x] = d[4 + x];
+    for (int x = 0; x < 8; ++x) b[x] = d[64 * (4 + x)];
   }
 };
 constexpr int kSegMapFloats = 12;
@@ -291,157 +289,197 @@ SR_DEV void pair_grads(float dLp0, float dLp1, float dLp2, float dLn0, float dLn
   add(14, G * dL_dalpha);
 }
 
-// Backward blend, pass 1 of 2.  One wave64 per 8 x 8 quadrant; each lane
-// walks, back to front, the pairs its pixel blended (the accepted pairs in
-// front of its last contributor, exactly the reference's), running only the
-// per-pixel recurrences and writing each pair's (w, dL/dalpha, dL/ddepth)
-// to the pair store.  The pairs come from the store as contiguous per-lane
-// streams; nothing is staged and there are no barriers, so the serial
-// per-pixel chain carries only the recurrences.  A quadrant some of whose
-// pairs missed the store (q_flag) instead runs the whole backward here over
-// staged records, recomputing those pairs.
+// Backward blend, pass 1 of 2: per pixel, back to front, the pairs it blended
+// (the accepted pairs in front of its last contributor, exactly the
+// reference's), running only the per-pixel recurrences and writing each pair's
+// (w, dL/dalpha, dL/ddepth) to the pair store.  The pairs come from the store
+// as one contiguous run per pixel in entry order (the forward cut it at the
+// last contributor); nothing is staged, so the serial chain carries only the
+// recurrences.
+//
+// A long run is cut into up to 16 segments, one lane each.  Each segment's lane
+// first runs its pairs through SegMap (the state recurrences as an affine map,
+// about a third of a step); the maps of the segments behind a segment, folded
+// onto the chain's initial state, give the state where it starts; then every
+// lane replays its segment with full steps from that state, so the serial
+// chain of a run of n pairs is two passes over n / 16 pairs instead of one over
+// n.  A wave gives its pixels as many lanes each as the quadrant's longest run
+// can have segments (1 to 16, by its cost's class), and a quadrant takes as
+// many waves.  300k surfels at 800 x 600: 98 us and at 400 x 300 49; with 8
+// lanes a pixel in every quadrant and each lane loading its own records 130
+// and 72; with the lanes by class but their own records still 130 and 66.  It
+// moves 316 MB (2.9 TB/s) and issues on 45 % of the cycles.
 template <bool kPart>
-__global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
-  __shared__ float4 s_q0[64], s_q1[64], s_q2[64], s_q3[64], s_q4[64];
-  __shared__ uint2 s_e[64];
-  __shared__ float s_acc[kNumG][64];
-  __shared__ float s_tmp[kNumG][65];
-  __shared__ uint32_t s_took[kPart ? 64 : 1];   // _part: the entry has a pixel with a semantic gradient
-  __shared__ float s_map[8][8][kSegMapFloats];  // per pixel of the wave, each segment's SegMap
+SR_DEV void blend_bwd_stored(const BlendBwdArgs& a, int qi, int lg, int part, float4* s_buf) {
+  // s_buf: a batch of every lane's pairs; between the walks the SegMaps
+  float* s_map = reinterpret_cast<float*>(s_buf);
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
-  if (a.counters[1] & kErrCapacity) return;
-  const int qi = (int)a.q_order[blockIdx.x / kSplitBwd], part = blockIdx.x % kSplitBwd;
   const int tile = qi / Q, q = qi % Q;
   const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
   const int lt = tile - (int)vi.tile_base;
   const int tx = lt % vi.gx, ty = lt / vi.gx;
   const int lane = threadIdx.x;
-  const int cnt = (int)a.sub_count[qi];
-  if (cnt == 0) return;  // no surfel reaches the quadrant: no gradient from it
-  const bool staged = a.q_flag[qi] != 0u;
-  if (staged && part != 0) return;  // the staged path uses all 64 lanes of part 0
-  // pixel of this lane: all 64 in the staged path, 64 / kSplitBwd per part otherwise
-  const int pix = staged ? lane : part * (64 / kSplitBwd) + lane;
-  const bool lane_ok = staged || lane < 64 / kSplitBwd;
-  const uint32_t pxi = (uint32_t)(tx * B + (q % QX) * kQuad + (pix & 7));
-  const uint32_t pyi = (uint32_t)(ty * B + (q / QX) * kQuad + (pix >> 3));
-  const bool inside = lane_ok && pxi < (uint32_t)vi.W && pyi < (uint32_t)vi.H;
-  const float pixx = pixel_centre<kPart>((int)pxi), pixy = pixel_centre<kPart>((int)pyi);
-  ChainBwd ch;
-
-  if (!staged) {
-    // Each pixel's blended pairs are one contiguous run in entry order (the
-    // forward cut the run at the pixel's last contributor), walked from the
-    // back with the next kChainPre pairs in flight.  A wave holds 8 pixels
-    // and gives each 8 lanes: a long run is cut into up to 8 segments, one
-    // per lane.  Each segment's lane first runs its pairs through SegMap (the
-    // state recurrences as an affine map, about a third of a step); the maps
-    // of the segments behind a segment, folded onto the chain's initial
-    // state, give the state where it starts; then every lane replays its
-    // segment with full steps from that state.  The serial chain of a run of
-    // n pairs is two passes over n / 8 pairs instead of one over n.
-    const int ps = lane & 7, sg = lane >> 3;
-    const int pxl = part * 8 + ps;
-    const uint32_t qxi = (uint32_t)(tx * B + (q % QX) * kQuad + (pxl & 7));
-    const uint32_t qyi = (uint32_t)(ty * B + (q / QX) * kQuad + (pxl >> 3));
-    const bool pin = qxi < (uint32_t)vi.W && qyi < (uint32_t)vi.H;
-    const uint2 rg = pin ? a.lane_range[(size_t)qi * 64 + pxl] : make_uint2(0u, 0u);
-    const int n = (int)rg.y, f0 = (int)rg.x;
-    const int seg_len = max(kChainSegMin, (n + 7) / 8);
-    const int nseg = (n + seg_len - 1) / seg_len;
-    const PixelBwd px = pixel_bwd<kPart>(a, vi, n > 0, qxi, qyi);
-    // walk pairs f0 + hi down to f0 + lo, calling fn(index, p0, p1, p2)
-    auto walk = [&](int lo, int hi, auto&& fn) {
-      float4 g0[kChainPre], g1[kChainPre], g2[kChainPre];
-      auto fetch = [&](int at) {
+  const int npx = 64 >> lg;  // pixels of the wave
+  const int ps = lane & (npx - 1), sg = lane >> (6 - lg);
+  const int pxl = part * npx + ps;
+  const uint32_t qxi = (uint32_t)(tx * B + (q % QX) * kQuad + (pxl & 7));
+  const uint32_t qyi = (uint32_t)(ty * B + (q / QX) * kQuad + (pxl >> 3));
+  const bool pin = qxi < (uint32_t)vi.W && qyi < (uint32_t)vi.H;
+  const uint2 rg = pin ? a.lane_range[(size_t)qi * 64 + pxl] : make_uint2(0u, 0u);
+  const int n = (int)rg.y;
+  const int seg_len = chain_segment(n);
+  const int nseg = (n + seg_len - 1) / seg_len;
+  const PixelBwd px = pixel_bwd<kPart>(a, vi, n > 0, qxi, qyi);
+  const int lo = sg * seg_len, hi = min(n, lo + seg_len) - 1;
+  // alpha and values of the pair behind the segment (none behind the last)
+  float la = 0.0f, l[7] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  if (sg < nseg - 1) {
+    const float4* pr = a.ps.rec + kPairQuads * (size_t)(rg.x + (uint32_t)(hi + 1));
+    const float4 e0 = pr[0], e1 = pr[1], e2 = pr[2];
+    la = e0.w;
+    l[0] = e1.w;
+    l[1] = e2.x;
+    l[2] = e2.y;
+    l[3] = e0.x;
+    l[4] = e1.x;
+    l[5] = e1.y;
+    l[6] = e1.z;
+  }
+  // Walks lane segments [lo, hi] (hi < lo: none) from the back, calling
+  // fn(p0, p1, p2) for each pair; the whole wave calls it.  A lane streaming
+  // its own records would touch a cache line of its own per load, and it is
+  // the line rate that bounds the pass: so the four lanes of a quad load the
+  // four lanes' batches together, 64 contiguous bytes at a time, and the
+  // batches change hands in LDS, the next one in flight.  Batches are whole:
+  // up to kChainPre - 1 records in front of lo are read (nothing uses them;
+  // the store is padded).  With kOut, fn's results go to fW the same way.
+  const int ql = lane & 3, qd = lane >> 2;  // place in the quad, quad
+  auto walk = [&](auto out, int lo, int hi, auto&& fn) {
+    constexpr bool kOut = decltype(out)::value;
+    int left[4];     // pairs left of each of the quad's lanes
+    uint32_t at[4];  // and its next batch's first record
 #pragma unroll
-        for (int k = 0; k < kChainPre; ++k) {
-          if (at - k >= lo) {
-            const float4* pr = a.ps.rec + kPairQuads * (size_t)(f0 + at - k);
-            g0[k] = pr[0];
-            g1[k] = pr[1];
-            g2[k] = pr[2];
-          }
-        }
-      };
-      int f = hi;
-      if (f >= lo) fetch(f);
-      while (f >= lo) {
-        float4 c0[kChainPre], c1[kChainPre], c2[kChainPre];
+    for (int o = 0; o < 4; ++o) {
+      left[o] = __shfl(hi - lo + 1, qd * 4 + o);
+      at[o] = (uint32_t)__shfl((int)(rg.x + (uint32_t)hi), qd * 4 + o) - (kChainPre - 1);
+    }
+    int mine = hi - lo + 1;
+    V4 g[4][3] = {};
+    auto fetch = [&]() {
 #pragma unroll
-        for (int k = 0; k < kChainPre; ++k) {
-          c0[k] = g0[k];
-          c1[k] = g1[k];
-          c2[k] = g2[k];
-        }
-        const int at = f;
-        f -= kChainPre;
-        if (f >= lo) fetch(f);  // next batch in flight
+      for (int o = 0; o < 4; ++o) {
+        if (left[o] <= 0) continue;
+        const V4* pr = reinterpret_cast<const V4*>(a.ps.rec + (ptrdiff_t)kPairQuads * (int32_t)at[o] + ql);
 #pragma unroll
-        for (int k = 0; k < kChainPre; ++k)
-          if (at - k >= lo) fn(at - k, c0[k], c1[k], c2[k]);
+        for (int c = 0; c < 3; ++c) g[o][c] = pr[4 * c];
       }
     };
-    const int lo = sg * seg_len, hi = min(n, lo + seg_len) - 1;
-    // alpha and values of the pair behind the segment (none behind the last)
-    float la = 0.0f, l[7] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    if (sg < nseg - 1) {
-      const float4* pr = a.ps.rec + kPairQuads * (size_t)(f0 + hi + 1);
-      const float4 e0 = pr[0], e1 = pr[1], e2 = pr[2];
-      la = e0.w;
-      l[0] = e1.w;
-      l[1] = e2.x;
-      l[2] = e2.y;
-      l[3] = e0.x;
-      l[4] = e1.x;
-      l[5] = e1.y;
-      l[6] = e1.z;
-    }
-    float* maps = &s_map[ps][0][0];
-    if (sg >= 1 && sg < nseg) {  // segment 0's map is never needed
-      SegMap m;
-      float pa = la, pl[7];
+    fetch();
+    while (__ballot(mine > 0) != 0ull) {
 #pragma unroll
-      for (int x = 0; x < 7; ++x) pl[x] = l[x];
-      walk(lo, hi, [&](int, const float4& c0, const float4& c1, const float4& c2) {
-        m.add<kPart>(px, pa, pl, c0.w, c0.y, kPart ? c0.y * c0.y : c0.z, __float_as_uint(c2.z));
-        pa = c0.w;
-        pl[0] = c1.w;
-        pl[1] = c2.x;
-        pl[2] = c2.y;
-        pl[3] = c0.x;
-        pl[4] = c1.x;
-        pl[5] = c1.y;
-        pl[6] = c1.z;
-      });
-      m.save(maps + sg * kSegMapFloats);
-    }
-    __syncthreads();
-    if (sg < nseg) {
-      ch.T = px.T_final;
-      for (int t = nseg - 1; t > sg; --t) {
-        SegMap m;
-        m.load(maps + t * kSegMapFloats);
-        m.apply(ch);
+      for (int o = 0; o < 4; ++o)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) reinterpret_cast<V4*>(s_buf)[o * kOwnerQuads + c * 64 + lane] = g[o][c];
+      uint32_t was[4];
+      int had[4];
+#pragma unroll
+      for (int o = 0; o < 4; ++o) {
+        was[o] = at[o];
+        had[o] = left[o];
+        at[o] -= kChainPre;
+        left[o] -= kChainPre;
       }
-      ch.last_alpha = la;
-      ch.last_c0 = l[0];
-      ch.last_c1 = l[1];
-      ch.last_c2 = l[2];
-      ch.last_depth = l[3];
-      ch.last_n0 = l[4];
-      ch.last_n1 = l[5];
-      ch.last_n2 = l[6];
-      walk(lo, hi, [&](int k, const float4& c0, const float4& c1, const float4& c2) {
-        a.ps.fW[f0 + k] = ch.step<kPart>(px, c0.w, c0.x, c0.y, kPart ? c0.y * c0.y : c0.z, c2.w,
-                                         __float_as_uint(c2.z), c1, c2.x, c2.y);
-      });
+      fetch();  // in flight while this batch is used
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const float4* b = s_buf + ql * kOwnerQuads + qd * 4;
+      auto quad = [&](int w) { return b[(w >> 2) * 64 + (w & 3)]; };
+      float4 r[kChainPre];
+#pragma unroll
+      for (int k = kChainPre - 1; k >= 0; --k) {
+        r[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (kChainPre - 1 - k < mine) r[k] = fn(quad(3 * k), quad(3 * k + 1), quad(3 * k + 2));
+      }
+      mine -= kChainPre;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (kOut) {
+        // rotated so that neither side's accesses share banks
+        auto place = [&](int o, int k) { return (qd * 4 + ((o + qd) & 3)) * 4 + ((k ^ qd) & 3); };
+#pragma unroll
+        for (int k = 0; k < kChainPre; ++k) s_buf[place(ql, k)] = r[k];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int o = 0; o < 4; ++o)
+          if (kChainPre - 1 - ql < had[o]) a.ps.fW[was[o] + (uint32_t)ql] = s_buf[place(o, ql)];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
     }
-    return;
+  };
+  const bool mapped = sg >= 1 && sg < nseg;  // segment 0's map is never needed
+  SegMap m;
+  if (lg > 0) {  // uniform
+    float pa = la, pl[7];
+#pragma unroll
+    for (int x = 0; x < 7; ++x) pl[x] = l[x];
+    walk(std::false_type{}, lo, mapped ? hi : lo - 1, [&](const float4& c0, const float4& c1, const float4& c2) {
+      m.add<kPart>(px, pa, pl, c0.w, c0.y, kPart ? c0.y * c0.y : c0.z, __float_as_uint(c2.z));
+      pa = c0.w;
+      pl[0] = c1.w;
+      pl[1] = c2.x;
+      pl[2] = c2.y;
+      pl[3] = c0.x;
+      pl[4] = c1.x;
+      pl[5] = c1.y;
+      pl[6] = c1.z;
+      return c0;
+    });
+    __syncthreads();
+    if (mapped) m.save(s_map + lane);
+    __syncthreads();
   }
+  ChainBwd ch;
+  ch.T = px.T_final;
+  for (int t = nseg - 1; t > sg; --t) {
+    SegMap behind;
+    behind.load(s_map + t * npx + ps);
+    behind.apply(ch);
+  }
+  __syncthreads();
+  ch.last_alpha = la;
+  ch.last_c0 = l[0];
+  ch.last_c1 = l[1];
+  ch.last_c2 = l[2];
+  ch.last_depth = l[3];
+  ch.last_n0 = l[4];
+  ch.last_n1 = l[5];
+  ch.last_n2 = l[6];
+  walk(std::true_type{}, lo, hi, [&](const float4& c0, const float4& c1, const float4& c2) {
+    return ch.step<kPart>(px, c0.w, c0.x, c0.y, kPart ? c0.y * c0.y : c0.z, c2.w, __float_as_uint(c2.z), c1, c2.x,
+                          c2.y);
+  });
+}
 
-  // Staged path: per chunk, stage the records, run the recurrences and the
-  // gradients together, sum per entry in LDS and store the sums.
+// The whole backward blend of a quadrant whose pairs missed the store: per
+// chunk, the records staged, the pairs recomputed, the recurrences and the
+// gradients together, each entry's sums stored as it is done.  s_buf: LDS that
+// the other path sizes.
+template <bool kPart>
+SR_DEV void blend_bwd_missed(const BlendBwdArgs& a, int qi, float4* s_buf) {
+  float4 *s_q0 = s_buf, *s_q1 = s_buf + 64, *s_q2 = s_buf + 128, *s_q3 = s_buf + 192, *s_q4 = s_buf + 256;
+  uint2* s_e = reinterpret_cast<uint2*>(s_buf + 320);
+  float(*s_tmp)[65] = reinterpret_cast<float(*)[65]>(s_buf + 352);
+  static_assert(4 * kOwnerQuads * 16 >= 352 * 16 + kNumG * 65 * 4 && kNumG >= kMaxSem, "fits the other path's LDS");
+  const int cnt = (int)a.sub_count[qi];
+  const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
+  const int tile = qi / Q, q = qi % Q;
+  const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
+  const int lt = tile - (int)vi.tile_base;
+  const int tx = lt % vi.gx, ty = lt / vi.gx;
+  const int lane = threadIdx.x, pix = lane;
+  const uint32_t pxi = (uint32_t)(tx * B + (q % QX) * kQuad + (pix & 7));
+  const uint32_t pyi = (uint32_t)(ty * B + (q / QX) * kQuad + (pix >> 3));
+  const bool inside = pxi < (uint32_t)vi.W && pyi < (uint32_t)vi.H;
+  const float pixx = pixel_centre<kPart>((int)pxi), pixy = pixel_centre<kPart>((int)pyi);
+  ChainBwd ch;
   const uint32_t rbeg = a.ranges[2 * tile], ntile = a.ranges[2 * tile + 1] - rbeg;
   const uint2* list = a.sub + (size_t)Q * rbeg + (size_t)q * ntile;
   const uint64_t* masks = a.masks + mask_base(Q, rbeg, ntile, tile, q);
@@ -457,25 +495,12 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
   ChainBwd fold = ch;  // the state the current segment started from
   SegMap seg_map;
   const int n_run = inside ? (int)a.lane_range[(size_t)qi * 64 + pix].y : 0;
-  const int seg_len = max(kChainSegMin, (n_run + 7) / 8);
+  const int seg_len = chain_segment(n_run);
   int seg = (n_run + seg_len - 1) / seg_len - 1, seg_start = seg * seg_len, idx = n_run;
   const int nch = (cnt + 63) / 64;
   const bool active = inside && px.last_contributor > 0;
-  // the pixel's semantic gradients (_part)
-  float dLs[kPart ? kMaxSem : 1];
-#pragma unroll
-  for (int x = 0; x < (kPart ? kMaxSem : 1); ++x) {
-    const size_t HW = (size_t)vi.H * vi.W;
-    dLs[x] = kPart && inside && x < a.S
-                 ? a.dL_dsem[(size_t)a.S * vi.pix_base + x * HW + (size_t)vi.W * pyi + pxi] : 0.0f;
-  }
-  ChunkRegs nx{};
-  uint2 v2 = make_uint2(0u, 0u);
-  if (nch > 0) {
-    nx = chunk_load(masks, frag_off, a.rec, lane, nch - 1, chunk_entry(list, cnt, lane, nch - 1, nch));
-    v2 = chunk_entry(list, cnt, lane, nch - 2, nch);
-  }
   for (int c = nch - 1; c >= 0; --c) {
+    const ChunkRegs nx = chunk_load(masks, frag_off, a.rec, lane, c, chunk_entry(list, cnt, lane, c, nch));
     uint64_t mask = active ? nx.mask : 0ull;
     const int m = min(64, cnt - c * 64);
     __syncthreads();
@@ -487,15 +512,10 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
       s_q3[lane] = nx.q3;
       s_q4[lane] = nx.q4;
     }
-#pragma unroll
-    for (int k = 0; k < kNumG; ++k) s_acc[k][lane] = 0.0f;
-    if (kPart) s_took[lane] = 0u;
     __syncthreads();
-    if (c > 0) {  // in flight while this chunk runs
-      const uint2 ve = v2;
-      v2 = chunk_entry(list, cnt, lane, c - 2, nch);
-      nx = chunk_load(masks, frag_off, a.rec, lane, c - 1, ve);
-    }
+    // this lane's entry's slot, and the entries whose sums are stored
+    const uint32_t slot = lane < m ? (uint32_t)slot_of(a.pos_slot, a.pos_quads, rbeg + s_e[lane].y, q) : 0u;
+    uint64_t stored = 0ull;
     if (__ballot(mask != 0ull) != 0ull) {
       // entries from last to first, the wave in step (each lane still walks
       // its own pixel's entries back to front); an entry's 18 partial
@@ -569,22 +589,55 @@ __global__ __launch_bounds__(64) void k_blend_bwd(BlendBwdArgs a) {
 #pragma unroll
         for (int k = 0; k < kNumG; ++k) s_tmp[k][lane] = gk[k];
         __syncthreads();
-        if (lane < kNumG) s_acc[lane][j] = grouped();
+        const float sum = lane < kNumG ? grouped() : 0.0f;
         __syncthreads();
-        if (kPart && a.S > 0 && tookm != 0ull) {  // semantics get their own gradient only
+        // the entry's slot, as store_part writes it
+        const uint32_t at = (uint32_t)__shfl((int)slot, j);
+        const bool sem = kPart && a.S > 0 && tookm != 0ull;
+        if (__ballot(sum != 0.0f) != 0ull || sem) {
+          if (lane < kPartStride) a.part[(size_t)at * kPartStride + lane] = sum;
+          if (lane == 0) a.part_nz[at] = 1;
+          stored |= 1ull << j;
+        }
+        if (sem) {  // semantics get their own gradient only
 #pragma unroll
-          for (int x = 0; x < kMaxSem; ++x) s_tmp[x][lane] = took_w * dLs[x];
+          for (int x = 0; x < kMaxSem; ++x)
+            s_tmp[x][lane] = took && x < a.S ? took_w * a.dL_dsem[(size_t)a.S * vi.pix_base +
+                                                                  x * ((size_t)vi.H * vi.W) + (size_t)vi.W * pyi + pxi]
+                                             : 0.0f;
           __syncthreads();
-          if (lane < a.S)
-            a.sem_part[slot_of(a.pos_slot, a.pos_quads, rbeg + s_e[j].y, q) * (size_t)a.S + lane] = grouped();
-          if (lane == 0) s_took[j] = 1u;
+          if (lane < a.S) a.sem_part[(size_t)at * a.S + lane] = grouped();
           __syncthreads();
         }
       }
     }
+    if (lane < m && ((stored >> lane) & 1ull) == 0ull) a.part_nz[slot] = 0;
     __syncthreads();
-    if (lane < m)
-      store_part(a, rbeg + s_e[lane].y, q, [&](int k) { return s_acc[k][lane]; }, kPart && s_took[lane] != 0u);
+  }
+}
+
+// The quadrants come in cost order, so those of a class are contiguous: work
+// item w is a wave of the first class with w left.
+template <bool kPart>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_blend_bwd(BlendBwdArgs a) {
+  __shared__ float4 s_buf[4 * kOwnerQuads];
+  static_assert(sizeof(s_buf) >= kSegMapFloats * 64 * sizeof(float), "one map a lane");
+  if (a.counters[1] & kErrCapacity) return;
+  const uint32_t* end = a.counters + kCostClass;  // of the classes, in quadrants
+  uint32_t items = 0;
+  for (int c = 0; c <= kSegLog; ++c) items += (end[c] - (c > 0 ? end[c - 1] : 0u)) << (kSegLog - c);
+  for (uint32_t w = blockIdx.x; w < items; w += gridDim.x) {
+    uint32_t first = 0, at = w;
+    int c = 0;
+    for (; c < kSegLog && at >= (end[c] - first) << (kSegLog - c); ++c) {
+      at -= (end[c] - first) << (kSegLog - c);
+      first = end[c];
+    }
+    const int lg = kSegLog - c;
+    const int qi = (int)a.q_order[first + (at >> lg)], part = (int)(at & ((1u << lg) - 1u));
+    if (a.q_flag[qi] == 0u) blend_bwd_stored<kPart>(a, qi, lg, part, s_buf);
+    else if (part == 0) blend_bwd_missed<kPart>(a, qi, s_buf);
+    __syncthreads();
   }
 }
 
@@ -592,8 +645,9 @@ hipError_t launch_blend_bwd(const BlendBwdArgs& a, hipStream_t s) {
   if (a.vs.T == 0) return hipSuccess;
   if (a.vs.B != 8 && a.vs.B != 16 && a.vs.B != 32) return hipErrorInvalidValue;
   const unsigned nblk = (unsigned)(a.vs.T * quads_per_tile(a.vs.B));
-  if (a.is_part) hipLaunchKernelGGL(k_blend_bwd<true>, dim3(nblk * kSplitBwd), dim3(64), 0, s, a);
-  else hipLaunchKernelGGL(k_blend_bwd<false>, dim3(nblk * kSplitBwd), dim3(64), 0, s, a);
+  const unsigned grid = nblk << kSegLog < kChainBlocks ? nblk << kSegLog : kChainBlocks;
+  if (a.is_part) hipLaunchKernelGGL(k_blend_bwd<true>, dim3(grid), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL(k_blend_bwd<false>, dim3(grid), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 

@@ -1692,10 +1692,12 @@ __global__ __launch_bounds__(64) void k_pair_offsets(AcceptArgs a) {
 // 1024-lane workgroup), so the blend kernels dispatch the longest per-pixel
 // chains first and the tail of the launch is short work.  The order within a
 // bucket is arbitrary; each quadrant's result does not depend on it.
-// host (pinned memory, may be null) receives counters[0..8], final from the
-// pair-offset pass on.
+// counters[kCostClass + i] receives the number of quadrants whose cost is at
+// least 256, 64, 32, 16 and 1 (i = 0..kSegLog), which come first in the order
+// in that order.  host (pinned memory, may be null) receives counters[0..8], final from
+// the pair-offset pass on.
 __global__ __launch_bounds__(1024) void k_order_quads(int nq, const uint32_t* cost, uint32_t* order,
-                                                      const uint32_t* counters, uint32_t* host) {
+                                                      uint32_t* counters, uint32_t* host) {
   __shared__ uint32_t s_cnt[64], s_base[64];
   const int tid = threadIdx.x;
   if (host != nullptr && tid < 9) host[tid] = counters[tid];
@@ -1721,6 +1723,9 @@ __global__ __launch_bounds__(1024) void k_order_quads(int nq, const uint32_t* co
   if (tid == 0) {
     uint32_t run = 0;
     for (int b = 0; b < 64; ++b) {
+      // two buckets an octave: costs of 2^k and more are in 0..61 - 2 k
+      const int c = b == 46 ? 0 : b == 50 ? 1 : b == 52 ? 2 : b == 54 ? 3 : b == 63 ? 4 : -1;
+      if (c >= 0) counters[kCostClass + c] = run;
       s_base[b] = run;
       run += s_cnt[b];
     }
@@ -1740,7 +1745,7 @@ __global__ __launch_bounds__(1024) void k_order_quads(int nq, const uint32_t* co
   }
 }
 
-hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, const uint32_t* counters,
+hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, uint32_t* counters,
                               uint32_t* host, hipStream_t s) {
   if (nq <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_order_quads, dim3(1), dim3(1024), 0, s, nq, cost, order, counters, host);
@@ -1865,163 +1870,29 @@ hipError_t launch_pair_write(const AcceptArgs& a, size_t max_items, hipStream_t 
 // full tile list) come out bit-identical.
 // ---------------------------------------------------------------------------
 #ifndef SR_FWD_PREFETCH
-#define SR_FWD_PREFETCH 20
+#define SR_FWD_PREFETCH 8
 #endif
-constexpr int kPre = SR_FWD_PREFETCH;  // stored pairs a lane fetches ahead in the blend kernels
+constexpr int kPre = SR_FWD_PREFETCH;  // stored pairs of a pixel per batch
+constexpr int kPreGroup = 4;           // loaded or not together
+static_assert(kPre % kPreGroup == 0 && kPre <= kPairPad, "whole groups, reads past the last pair within the padding");
 
-// Stored path of the forward blend: every pair of the quadrant is in the
-// store and each pixel's pairs form one contiguous run in entry order.  A
-// wave takes 16 pixels with 4 lanes each; the 4 lanes of a pixel walk the
-// same run in step (each runs the transmittance update, so all agree on
-// where the pixel stops) and split the accumulators: role 0 depth, M1, M2
-// and distortion, role 1 the normal and red, role 2 green and blue, role 3
-// the median and contributor counts.  Every lane executes the same
-// instructions (role values are picked by select), so the serial chain of a
-// long pixel costs a quarter of the full update per pair; each accumulator
-// sees exactly the reference's operations in order.
-// The _part variant sums (x alpha) T where the plain one sums x (alpha T),
-// tracks the median pair's weight, and leaves each blended pair's T in the
-// fW region for the semantic channels' pass.
+// Forward blend of a quadrant whose pairs missed the store: the records staged
+// chunk by chunk, the pairs recomputed, lane = pixel.
 template <bool kPart>
-SR_DEV void blend_fwd_stored(const BlendArgs& a, const ViewInfo& vi, int qi, int tx, int ty, int q, int part) {
-  static_assert(kSplit == 4, "4 waves of 16 pixels x 4 roles per quadrant");
-  const int B = a.vs.B, QX = B / kQuad;
-  const int lane = threadIdx.x, role = lane & 3;
-  const int pix = part * 16 + (lane >> 2);
-  const uint32_t pxi = (uint32_t)(tx * B + (q % QX) * kQuad + (pix & 7));
-  const uint32_t pyi = (uint32_t)(ty * B + (q / QX) * kQuad + (pix >> 3));
-  const bool inside = pxi < (uint32_t)vi.W && pyi < (uint32_t)vi.H;
-  const int cnt = (int)a.sub_count[qi];
-  // lane_range is written by the pair-offset pass, which runs only when the
-  // view has instances: read it for non-empty quadrants only
-  const uint2 rg = (inside && cnt > 0) ? a.lane_range[(size_t)qi * 64 + pix] : make_uint2(0u, 0u);
-  // Each lane loads one record quad per pair: role 0 quad 0 (depth, mm,
-  // mm^2, alpha), role 1 quad 1 (normal, red), roles 2 and 3 quad 2 (green,
-  // blue, tile position); alpha and depth reach the other lanes of the pixel
-  // from role 0 by a quad broadcast.  A lane accumulates x, y and z of its
-  // quad in a0..a2 and w in a3, except that role 0's a3 is the distortion.
-  const int qsel = role < 2 ? role : 2;
-  float T = 1.0f;
-  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f, median_depth = 0.0f, median_weight = 0.0f;
-  float median_contributor = -1.0f;
-  float* pair_T = kPart && a.S > 0 ? reinterpret_cast<float*>(a.ps.fW) : nullptr;
-  uint32_t last_contributor = 0;
-  int blended = 0;
-  bool done = !inside;
-  uint32_t f = rg.x;
-  int left = (int)rg.y;
-  // slots past the run's end keep defined (stale) values; nothing uses them
-  float4 fq[kPre];
-#pragma unroll
-  for (int k = 0; k < kPre; ++k) fq[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  auto fetch = [&](uint32_t at, int n) {
-#pragma unroll
-    for (int k = 0; k < kPre; ++k)
-      if (k < n) fq[k] = a.ps.rec[kPairQuads * (size_t)(at + k) + qsel];
-  };
-  fetch(f, left);
-  while (left > 0 && !done) {  // the four lanes of a pixel share left and done
-    float4 cq[kPre];
-#pragma unroll
-    for (int k = 0; k < kPre; ++k) cq[k] = fq[k];
-    const int n = left;
-    const uint32_t f0 = f;
-    f += kPre;
-    left -= kPre;
-    if (left > 0) fetch(f, left);  // next batch in flight
-    // Straight-line over the batch: every update is computed and kept only
-    // where the pair is live (in the run, the pixel not done) and does not
-    // saturate the pixel, so the body has no per-pair branch.
-#pragma unroll
-    for (int k = 0; k < kPre; ++k) {
-      // forward.cu:383-415; role 0's quad: (depth, mm, mm^2, alpha), mm = mcoef (1 - near / depth)
-      const float4 v = cq[k];
-      const float alpha = quad_bcast0(v.w), depth = quad_bcast0(v.x);
-      const float test_T = T * (1.0f - alpha);
-      const bool live = k < n && !done;
-      const bool sat = test_T < 0.0001f;
-      done = done || (live && sat);
-      const bool ok = live && !sat;
-      const uint32_t contributor = __float_as_uint(v.z) + 1u;  // quad 2's z: position in the tile list
-      const float w = alpha * T;
-      const float A = 1.0f - T;
-      // role 0: the distortion term (mm^2 A + M2 - 2 mm M1), a1 = M1, a2 = M2
-      const float vz = kPart && role == 0 ? v.y * v.y : v.z;
-      const float x3 = role == 0 ? (vz * A + a2) - (2.0f * v.y) * a1 : v.w;
-      auto weighed = [&](float x) { return kPart ? (x * alpha) * T : x * w; };
-      const float n0 = a0 + weighed(v.x), n1 = a1 + weighed(v.y), n2 = a2 + weighed(vz), n3 = a3 + weighed(x3);
-      a0 = ok ? n0 : a0;
-      a1 = ok ? n1 : a1;
-      a2 = ok ? n2 : a2;
-      a3 = ok ? n3 : a3;
-      const bool med = ok && T > 0.5f;
-      median_depth = med ? depth : median_depth;
-      median_contributor = med ? (float)contributor : median_contributor;
-      if (kPart) {
-        median_weight = med ? w : median_weight;
-        if (pair_T != nullptr && ok && role == 0) pair_T[f0 + k] = T;
-      }
-      T = ok ? test_T : T;
-      last_contributor = ok ? contributor : last_contributor;
-      blended += ok ? 1 : 0;
-    }
-  }
-  if (!inside) return;
-  const size_t HW = (size_t)vi.H * vi.W, pid = (size_t)vi.W * pyi + pxi, pb = vi.pix_base;
-  float* final_T = a.final_T + 3 * pb;
-  float* out_color = a.out_color + 3 * pb;
-  float* out_others = a.out_others + (kPart ? 8 : 7) * pb;
-  if (role == 0) {
-    out_others[pid] = a0;
-    final_T[pid + HW] = a1;
-    final_T[pid + 2 * HW] = a2;
-    out_others[pid + 6 * HW] = a3;  // the distortion
-  } else if (role == 1) {
-    out_others[pid + 2 * HW] = a0;
-    out_others[pid + 3 * HW] = a1;
-    out_others[pid + 4 * HW] = a2;
-    out_color[pid] = a3 + T * a.bg[0];
-  } else if (role == 2) {
-    out_color[HW + pid] = a0 + T * a.bg[1];
-    out_color[2 * HW + pid] = a1 + T * a.bg[2];
-  } else {
-    uint32_t* n_contrib = a.n_contrib + 2 * pb;
-    final_T[pid] = T;
-    n_contrib[pid] = last_contributor;
-    n_contrib[pid + HW] = f2u(median_contributor);
-    out_others[pid + HW] = 1.0f - T;
-    out_others[pid + 5 * HW] = median_depth;
-    if (kPart) out_others[pid + 7 * HW] = median_weight;
-    // the backward passes walk only the blended prefix of the run
-    if (cnt > 0) a.lane_range[(size_t)qi * 64 + pix].y = (uint32_t)blended;
-  }
-}
-
-template <bool kPart>
-__global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
+SR_DEV void blend_fwd_missed(const BlendArgs& a, int qi) {
   __shared__ float4 s_q0[64], s_q1[64], s_q2[64], s_q3[64], s_q4[64];
   __shared__ uint32_t s_pos[64];
   __shared__ uint32_t s_rid[kPart ? 64 : 1];
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
-  if (a.counters[1] & kErrCapacity) return;
-  const int qi = (int)a.q_order[blockIdx.x / kSplit], part = blockIdx.x % kSplit;
   const int tile = qi / Q, q = qi % Q;
   const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
   const int lt = tile - (int)vi.tile_base;
   const int tx = lt % vi.gx, ty = lt / vi.gx;
   const int lane = threadIdx.x;
-  const bool staged = a.q_flag[qi] != 0u;
-  if (staged && part != 0) return;  // the staged path uses all 64 lanes of part 0
-  if (!staged) {
-    blend_fwd_stored<kPart>(a, vi, qi, tx, ty, q, part);
-    return;
-  }
-  // staged path: lane = pixel of the quadrant
-  const int pix = lane;
-  const bool lane_ok = true;
+  const int pix = lane;  // of the quadrant
   const uint32_t pxi = (uint32_t)(tx * B + (q % QX) * kQuad + (pix & 7));
   const uint32_t pyi = (uint32_t)(ty * B + (q / QX) * kQuad + (pix >> 3));
-  const bool inside = lane_ok && pxi < (uint32_t)vi.W && pyi < (uint32_t)vi.H;
+  const bool inside = pxi < (uint32_t)vi.W && pyi < (uint32_t)vi.H;
   bool done = !inside;
   const uint32_t rbeg = a.ranges[2 * tile], ntile = a.ranges[2 * tile + 1] - rbeg;
   const int cnt = (int)a.sub_count[qi];
@@ -2160,6 +2031,173 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
     out_others[pid + 6 * HW] = distortion;
     // the backward cuts the pixel's run into the same segments as a stored run
     a.lane_range[(size_t)qi * 64 + pix].y = (uint32_t)blended;
+  }
+}
+
+// Forward blend of the quadrants whose pairs are all in the store, each
+// pixel's pairs one contiguous run in entry order.  A wave takes 16 pixels
+// with 4 lanes each; the 4 lanes of a pixel walk the same run in step (each
+// runs the transmittance update, so all agree on where the pixel stops) and
+// split the accumulators: role 0 depth, M1, M2 and distortion, role 1 the
+// normal and red, roles 2 and 3 green and blue.  Every lane executes the same
+// instructions (role values are picked by select), so the serial chain of a
+// long pixel costs a quarter of the full update per pair; each accumulator
+// sees exactly the reference's operations in order.
+// What bounds it is that chain: a run of hundreds of pairs is blended at the
+// rate one wave issues.  So a batch first runs the transmittances alone (two
+// operations a pair; they only fall, so the last one tells whether the pixel
+// saturates in the batch), and where every pixel of the wave has a whole
+// batch left and none saturates, the updates go in without per-pair
+// conditions.  The last contributor and the median are pairs of the run, looked
+// up once at its end from their counts.  300k surfels: 70 us at 800 x 600 and
+// 79 at 400 x 300, where conditions on every pair and 20 pairs a batch, copied
+// from the prefetch registers (185 a lane, two waves a SIMD), took 94 and 122.
+// Batches of 4, 12 and 16 pairs: 83, 74, 88 and 96, 75, 73 us.
+// The _part variant sums its outputs as (value * alpha) * T (its kernel's
+// expression; the plain one adds value * (alpha * T)), keeps the median pair's
+// weight and leaves each pair's T in fW, which the backward overwrites only
+// later, for the semantic pass.
+template <bool kPart>
+__global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
+  static_assert(kSplit == 4, "4 waves of 16 pixels x 4 roles per quadrant");
+  if (a.counters[1] & kErrCapacity) return;
+  const int qi = (int)a.q_order[blockIdx.x / kSplit], part = blockIdx.x % kSplit;
+  if (a.q_flag[qi] != 0u) {
+    if (part == 0) blend_fwd_missed<kPart>(a, qi);
+    return;
+  }
+  const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
+  const int tile = qi / Q, q = qi % Q;
+  const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
+  const int lt = tile - (int)vi.tile_base;
+  const int tx = lt % vi.gx, ty = lt / vi.gx;
+  const int lane = threadIdx.x, role = lane & 3;
+  const int pix = part * 16 + (lane >> 2);
+  const uint32_t pxi = (uint32_t)(tx * B + (q % QX) * kQuad + (pix & 7));
+  const uint32_t pyi = (uint32_t)(ty * B + (q / QX) * kQuad + (pix >> 3));
+  const bool inside = pxi < (uint32_t)vi.W && pyi < (uint32_t)vi.H;
+  const int cnt = (int)a.sub_count[qi];
+  // lane_range is written by the pair-offset pass, which runs only when the
+  // view has instances: read it for non-empty quadrants only
+  const uint2 rg = (inside && cnt > 0) ? a.lane_range[(size_t)qi * 64 + pix] : make_uint2(0u, 0u);
+  // Each lane loads one record quad per pair: role 0 quad 0 (depth, mm,
+  // mm^2, alpha), role 1 quad 1 (normal, red), roles 2 and 3 quad 2 (green,
+  // blue, tile position); alpha reaches the other lanes of the pixel from
+  // role 0 by a quad broadcast.  A lane accumulates x, y and z of its quad in
+  // a0..a2 and w in a3, except that role 0's a3 is the distortion.
+  const float4* run = a.ps.rec + kPairQuads * (size_t)rg.x + (role < 2 ? role : 2);
+  float T = 1.0f;
+  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f, median_weight = 0.0f;
+  float* pair_T = kPart && a.S > 0 ? reinterpret_cast<float*>(a.ps.fW) + rg.x : nullptr;
+  int blended = 0, in_front = 0;  // pairs blended; those with T above 1/2
+  bool done = false;
+  int left = (int)rg.y;
+  // whole groups, so up to kPreGroup - 1 pairs past the run (nothing uses
+  // them; the store is padded)
+  auto fetch = [&](float4 (&b)[kPre], const float4* at, int n) {
+#pragma unroll
+    for (int g = 0; g < kPre; g += kPreGroup)
+      if (g < n) {
+#pragma unroll
+        for (int k = g; k < g + kPreGroup; ++k) b[k] = at[kPairQuads * k];
+      }
+  };
+  // forward.cu:383-415 for one pair (role 0's quad: depth, mm, mm^2, alpha)
+  auto update = [&](const float4& v, float alpha, float Tk) {
+    const float w = alpha * Tk;
+    const float A = 1.0f - Tk;
+    // role 0: the distortion term (mm^2 A + M2 - 2 mm M1), a1 = M1, a2 = M2
+    const float vz = kPart && role == 0 ? v.y * v.y : v.z;
+    const float x3 = role == 0 ? (vz * A + a2) - (2.0f * v.y) * a1 : v.w;
+    auto weighed = [&](float x) { return kPart ? (x * alpha) * Tk : x * w; };
+    a0 += weighed(v.x);
+    a1 += weighed(v.y);
+    a2 += weighed(vz);
+    a3 += weighed(x3);
+    if (kPart && Tk > 0.5f) median_weight = w;
+  };
+  auto blend = [&](const float4 (&b)[kPre]) {
+    const int n = min(left, kPre);
+    float Tk[kPre + 1];
+    Tk[0] = T;
+#pragma unroll
+    for (int k = 0; k < kPre; ++k) Tk[k + 1] = Tk[k] * (1.0f - quad_bcast0(b[k].w));
+    if (__ballot(n < kPre || !(Tk[kPre] >= 0.0001f)) == 0ull) {  // of the lanes with pairs left
+#pragma unroll
+      for (int k = 0; k < kPre; ++k) {
+        if (kPart && pair_T != nullptr && role == 0) pair_T[blended + k] = Tk[k];
+        update(b[k], quad_bcast0(b[k].w), Tk[k]);
+      }
+      if (__ballot(T > 0.5f) != 0ull) {
+#pragma unroll
+        for (int k = 0; k < kPre; ++k) in_front += Tk[k] > 0.5f ? 1 : 0;
+      }
+      blended += kPre;
+      T = Tk[kPre];
+    } else {
+      const int base = blended;
+#pragma unroll
+      for (int k = 0; k < kPre; ++k) {
+        if (k < n && !done) {
+          if (Tk[k + 1] < 0.0001f) {
+            done = true;
+          } else {
+            if (kPart && pair_T != nullptr && role == 0) pair_T[base + k] = Tk[k];
+            update(b[k], quad_bcast0(b[k].w), Tk[k]);
+            in_front += Tk[k] > 0.5f ? 1 : 0;
+            T = Tk[k + 1];
+            ++blended;
+          }
+        }
+      }
+    }
+    left -= kPre;
+  };
+  float4 b0[kPre], b1[kPre];
+#pragma unroll
+  for (int k = 0; k < kPre; ++k) b0[k] = b1[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  fetch(b0, run, left);
+  while (left > 0 && !done) {  // the four lanes of a pixel share left and done
+    run += kPairQuads * kPre;
+    fetch(b1, run, left - kPre);  // in flight while b0 blends
+    blend(b0);
+    if (left > 0 && !done) {
+      run += kPairQuads * kPre;
+      fetch(b0, run, left - kPre);
+      blend(b1);
+    }
+  }
+  if (!inside) return;
+  const size_t HW = (size_t)vi.H * vi.W, pid = (size_t)vi.W * pyi + pxi, pb = vi.pix_base;
+  float* final_T = a.final_T + 3 * pb;
+  float* out_color = a.out_color + 3 * pb;
+  float* out_others = a.out_others + (kPart ? 8 : 7) * pb;
+  if (role == 0) {
+    out_others[pid] = a0;
+    final_T[pid + HW] = a1;
+    final_T[pid + 2 * HW] = a2;
+    out_others[pid + 6 * HW] = a3;  // the distortion
+    if (kPart) out_others[pid + 7 * HW] = median_weight;
+  } else if (role == 1) {
+    out_others[pid + 2 * HW] = a0;
+    out_others[pid + 3 * HW] = a1;
+    out_others[pid + 4 * HW] = a2;
+    out_color[pid] = a3 + T * a.bg[0];
+  } else if (role == 2) {
+    out_color[HW + pid] = a0 + T * a.bg[1];
+    out_color[2 * HW + pid] = a1 + T * a.bg[2];
+  } else {
+    // quad 0's x: depth, quad 2's z: position in the tile list
+    const float4* first = a.ps.rec + kPairQuads * (size_t)rg.x;
+    auto contributor = [&](int n) { return __float_as_uint(first[kPairQuads * (n - 1) + 2].z) + 1u; };
+    uint32_t* n_contrib = a.n_contrib + 2 * pb;
+    final_T[pid] = T;
+    n_contrib[pid] = blended > 0 ? contributor(blended) : 0u;
+    n_contrib[pid + HW] = f2u(in_front > 0 ? (float)contributor(in_front) : -1.0f);
+    out_others[pid + HW] = 1.0f - T;
+    out_others[pid + 5 * HW] = in_front > 0 ? first[kPairQuads * (in_front - 1)].x : 0.0f;
+    // the backward passes walk only the blended prefix of the run
+    if (cnt > 0) a.lane_range[(size_t)qi * 64 + pix].y = (uint32_t)blended;
   }
 }
 

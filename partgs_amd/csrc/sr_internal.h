@@ -194,6 +194,7 @@ constexpr int kPartStride = 20;  // 18 partial gradients, padded to five float4
 // recomputes its pairs.
 constexpr size_t kFragPerInstance = 24;
 constexpr int kPairQuads = 3;  // float4 per stored pair
+constexpr int kPairPad = 32;   // pairs a blend may read in front of the store's first or past its last
 constexpr uint32_t kNoFrag = 0xFFFFFFFFu;
 // Per-pixel acceptance masks: quadrant (t, q) owns mask slots
 // [mask_base, mask_base + 64 * chunks), chunk c of its sub-list at
@@ -247,7 +248,7 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
   b.frag_cap = pair_capacity > 0 ? (size_t)pair_capacity
                                   : n * (pair_store > 0 ? (size_t)pair_store : kFragPerInstance);
   if (b.frag_cap > 0x7fffffffu) b.frag_cap = 0x7fffffffu;
-  b.prec = off; off += align_up(b.frag_cap * kPairQuads * 16);
+  b.prec = off + kPairPad * kPairQuads * 16; off += align_up((b.frag_cap + 2 * kPairPad) * kPairQuads * 16);
   b.fW = off; off += align_up(b.frag_cap * 16);
   b.sem_part = off; off += align_up(n * Q * (size_t)sem * 4);  // _part: semantic partials per slot
   b.part = off; off += align_up(b.nslot * kPartStride * 4);         // last: see part
@@ -260,6 +261,18 @@ struct PairStore {
   float4* rec;  // kPairQuads per pair
   float4* fW;   // 1 per pair
 };
+// The backward's chain pass cuts a pixel's run of n pairs into segments of
+// chain_segment(n): up to 8 of at least 16 pairs, and 16 from 257 pairs on,
+// where the length of the longest chain bounds the pass and not the extra
+// work (16 from 129 pairs on: 295 instead of 281 us at 1M surfels, 1237 x 823).
+// So a quadrant whose runs are below 16, 32, 64, 256 pairs and any number has
+// at most 1 << k, k = 0..kSegLog, segments a pixel.
+constexpr int kSegLog = 4;
+constexpr int kCostClass = 9;  // counters[9..13]: quadrants by cost, see k_order_quads
+__host__ __device__ inline int chain_segment(int n) {
+  const int len = n > 256 ? (n + 15) >> 4 : (n + 7) >> 3;
+  return len > 16 ? len : 16;
+}
 
 constexpr uint32_t kErrPrefiltered = 1u;
 constexpr uint32_t kErrCapacity = 2u;  // more tile instances (or slots) than the binning capacity
@@ -507,7 +520,7 @@ hipError_t launch_sort_tiles(const SortArgs& a, size_t max_segments, hipStream_t
 hipError_t launch_accept(const AcceptArgs& a, size_t max_items, hipStream_t s);
 hipError_t launch_pair_offsets(const AcceptArgs& a, hipStream_t s);
 hipError_t launch_pair_write(const AcceptArgs& a, size_t max_items, hipStream_t s);
-hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, const uint32_t* counters,
+hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, uint32_t* counters,
                               uint32_t* host, hipStream_t s);
 hipError_t launch_iota_u32(uint32_t* p, size_t n, hipStream_t s);
 hipError_t launch_blend_fwd(const BlendArgs& a, hipStream_t s);
