@@ -257,7 +257,7 @@ int post_counts(hipStream_t st) {
 }
 
 // Per-record gradient outputs of the backward preprocess (record r = v P + i):
-// dL_dtransMat 9, dL_dmean2D 3, dL_dopacity 1, dL_dcolors 3 floats each.
+// dL_dtransMat 9 (or null), dL_dmean2D 3, dL_dopacity 1, dL_dcolors 3 floats each.
 struct RecordGrads {
   float* transMat;
   float* mean2D;
@@ -268,7 +268,7 @@ struct RecordGrads {
 // Workspace of the batched entry points: geometry, image and binning state
 // plus the per-record gradient scratch, each section 256-byte aligned.
 struct BatchLayout {
-  size_t geom, img, bin, g_transMat, g_opacity, g_colors, total;
+  size_t geom, img, bin, g_colors, total;
   GeomLayout gl;
   ImageLayout il;
   BinLayout bl;
@@ -284,8 +284,6 @@ BatchLayout batch_layout(const ViewSet& vs, int P, int capacity, int pair_store,
   b.geom = off; off += align_up(b.gl.total);
   b.img = off; off += align_up(b.il.total);
   b.bin = off; off += align_up(b.bl.total);
-  b.g_transMat = off; off += align_up(R * 9 * 4);
-  b.g_opacity = off; off += align_up(R * 4);
   b.g_colors = off; off += align_up(R * 3 * 4);
   b.total = off;
   return b;
@@ -906,9 +904,10 @@ int sr_backward_batched(const sr_views* v, const sr_surfels* g, void* ws, size_t
   if (ws_bytes < bl.total)
     return fail(SR_ERR_INVALID, "workspace holds %zu bytes, needs %zu", ws_bytes, bl.total);
   Pipeline pl = batch_pipeline(v, g, vs, bl, (char*)ws, capacity);
-  char* w = (char*)ws;
-  RecordGrads rg{(float*)(w + bl.g_transMat), gr->dL_dmeans2D, (float*)(w + bl.g_opacity),
-                 (float*)(w + bl.g_colors)};
+  // a single view's records are its outputs; several views' colour gradients
+  // go to scratch, for the SH pass
+  RecordGrads rg{nullptr, gr->dL_dmeans2D, gr->dL_dopacity,
+                 vs.V == 1 ? gr->dL_dcolors : (float*)((char*)ws + bl.g_colors)};
   return run_backward(pl, g, radii, dL_dcolor, dL_dothers, rg, gr, true, false, st);
 }
 

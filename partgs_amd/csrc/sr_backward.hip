@@ -959,15 +959,14 @@ SR_DEV F3 sh_backward_core(int deg, F3 dir_orig, F3 dL_dRGB, Get S, Put put) {
   return r;
 }
 
-// SH backward against memory: the first view stores c dL_dRGB (and zeros for
-// the inactive coefficients), later views add.  With 16 coefficients and
-// 16-byte aligned rows the surfel's 48 coefficients are read and its 48
+// SH backward of one view against memory: stores c dL_dRGB (and zeros for the
+// inactive coefficients).  With 16 coefficients and 16-byte aligned rows the surfel's 48 coefficients are read and its 48
 // gradients written as twelve float4 each (same values, same order of
 // operations as the scalar form).
-// srow (when not null): the surfel's row staged in LDS by its wave, read
-// instead of sh; with to_row the gradients are written back into it (the
-// caller stores the wave's rows) instead of to dsh.
-template <bool kAdd, bool kRow, bool kToRow>
+// With kRow srow is the surfel's row staged in LDS by its wave, read instead of
+// sh and overwritten with the gradients (the caller stores the wave's rows)
+// instead of dsh.
+template <bool kRow>
 SR_DEV F3 sh_backward(int deg, int M, const float* sh, F3 dir_orig, F3 dL_dRGB, float* dsh, float4* srow) {
   const int nact = (deg + 1) * (deg + 1);
   if (M == 16 && ((reinterpret_cast<uintptr_t>(sh) | reinterpret_cast<uintptr_t>(dsh)) & 15u) == 0u) {
@@ -994,51 +993,38 @@ SR_DEV F3 sh_backward(int deg, int M, const float* sh, F3 dir_orig, F3 dL_dRGB, 
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int j = 4 * i + t, k = j / 3;
-        v[t] = k < nact ? cv[k] * comp(dL_dRGB, j % 3) : (kAdd ? -0.0f : 0.0f);
+        v[t] = k < nact ? cv[k] * comp(dL_dRGB, j % 3) : 0.0f;
       }
-      if (kAdd) {
-        const float4 o = d4[i];
-        d4[i] = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
-      } else if (kToRow) {
-        srow[i] = make_float4(v[0], v[1], v[2], v[3]);
-      } else {
-        d4[i] = make_float4(v[0], v[1], v[2], v[3]);
-      }
+      (kRow ? srow : d4)[i] = make_float4(v[0], v[1], v[2], v[3]);
     }
     return r;
   }
-  if (!kAdd)
-    for (int k = nact; k < M; ++k) dsh[3 * k] = dsh[3 * k + 1] = dsh[3 * k + 2] = 0.0f;
+  for (int k = nact; k < M; ++k) dsh[3 * k] = dsh[3 * k + 1] = dsh[3 * k + 2] = 0.0f;
   return sh_backward_core(
       deg, dir_orig, dL_dRGB, [&](int k) { return f3(sh[3 * k], sh[3 * k + 1], sh[3 * k + 2]); },
       [&](int k, float c) {
-        if (kAdd) {
-          dsh[3 * k] += c * dL_dRGB.x;
-          dsh[3 * k + 1] += c * dL_dRGB.y;
-          dsh[3 * k + 2] += c * dL_dRGB.z;
-        } else {
-          dsh[3 * k] = c * dL_dRGB.x;
-          dsh[3 * k + 1] = c * dL_dRGB.y;
-          dsh[3 * k + 2] = c * dL_dRGB.z;
-        }
+        dsh[3 * k] = c * dL_dRGB.x;
+        dsh[3 * k + 1] = c * dL_dRGB.y;
+        dsh[3 * k + 2] = c * dL_dRGB.z;
       });
 }
 
-// SH backward of one record: stores (first view) or adds c * dL_dRGB to the
-// surfel's dL_dsh and returns the gradient of the mean through the view
-// direction.
-template <bool kRow, bool kToRow>
-SR_DEV F3 sh_grad(const PreprocessBwdArgs& a, bool first, int idx, size_t r, const float* campos, float m0,
-                  float m1, float m2, F3 dRGB, float4* srow) {
+// A record's colour gradient: none through a clamped channel.
+SR_DEV F3 unclamped(const PreprocessBwdArgs& a, size_t r, F3 dRGB) {
   const uchar4 cl = reinterpret_cast<const uchar4*>(a.clamped)[r];
   if (cl.x) dRGB.x = 0.0f;
   if (cl.y) dRGB.y = 0.0f;
   if (cl.z) dRGB.z = 0.0f;
-  const F3 dir_orig = f3(m0 - campos[0], m1 - campos[1], m2 - campos[2]);
-  float* dsh = a.dL_dsh + (size_t)idx * a.M * 3;
-  const float* sh = a.shs + (size_t)idx * a.M * 3;
-  return first ? sh_backward<false, kRow, kToRow>(a.D, a.M, sh, dir_orig, dRGB, dsh, srow)
-               : sh_backward<true, kRow, false>(a.D, a.M, sh, dir_orig, dRGB, dsh, srow);
+  return dRGB;
+}
+
+// SH backward of a surfel's only view: stores its dL_dsh row and returns the
+// gradient of the mean through the view direction.
+template <bool kRow>
+SR_DEV F3 sh_grad(const PreprocessBwdArgs& a, int idx, size_t r, const float* campos, float m0, float m1, float m2,
+                  F3 dRGB, float4* srow) {
+  return sh_backward<kRow>(a.D, a.M, a.shs + (size_t)idx * a.M * 3, f3(m0 - campos[0], m1 - campos[1], m2 - campos[2]),
+                           unclamped(a, r, dRGB), a.dL_dsh + (size_t)idx * a.M * 3, srow);
 }
 
 // Gradients of one surfel summed over the views that see it.
@@ -1048,40 +1034,48 @@ struct SurfelGrad {
 
 // Record r's 18 partial gradients summed over its slots (one per instance
 // and quadrant holding it, a contiguous run in instance order, quadrants in
-// order): a fixed order, so the sums are the same on every run.
+// order): a fixed order, so the sums are the same on every run.  Four flags
+// are in flight at a time, then the sums of kU slots they announce.
+template <int kU>
 SR_DEV void reduce_record(const PreprocessBwdArgs& a, size_t r, float (&gs)[18]) {
 #pragma unroll
   for (int k = 0; k < 18; ++k) gs[k] = 0.0f;
   if (a.tiles[r] == 0 || a.part == nullptr || (a.counters[1] & kErrCapacity)) return;
   const uint2 rs = a.rslot[r];  // the record's slots: its instances in order, each one's quadrants in order
   const uint32_t s0 = rs.x, s1 = rs.x + rs.y;
-  // four flags in flight at a time
   for (uint32_t s = s0; s < s1; s += 4) {
     uint8_t fl[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) fl[t] = a.part_nz[min(s + (uint32_t)t, s1 - 1u)];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      if (s + (uint32_t)t >= s1 || fl[t] == 0) continue;
-      const float4* p = reinterpret_cast<const float4*>(a.part + (size_t)(s + (uint32_t)t) * kPartStride);
-      const float4 p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3], p4 = p[4];
-      gs[0] += p0.x; gs[1] += p0.y; gs[2] += p0.z; gs[3] += p0.w;
-      gs[4] += p1.x; gs[5] += p1.y; gs[6] += p1.z; gs[7] += p1.w;
-      gs[8] += p2.x; gs[9] += p2.y; gs[10] += p2.z; gs[11] += p2.w;
-      gs[12] += p3.x; gs[13] += p3.y; gs[14] += p3.z; gs[15] += p3.w;
-      gs[16] += p4.x; gs[17] += p4.y;
+    for (int t = 0; t < 4; ++t) fl[t] = s + (uint32_t)t < s1 ? fl[t] : 0;
+#pragma unroll
+    for (int u = 0; u < 4; u += kU) {
+      V4 p[kU][5];
+#pragma unroll
+      for (int t = 0; t < kU; ++t) {
+        if (fl[u + t] == 0) continue;
+        const V4* src = reinterpret_cast<const V4*>(a.part + (size_t)(s + (uint32_t)(u + t)) * kPartStride);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) p[t][k] = src[k];
+      }
+#pragma unroll
+      for (int t = 0; t < kU; ++t)
+#pragma unroll
+        for (int k = 0; k < 18; ++k) gs[k] = fl[u + t] ? gs[k] + p[t][k / 4][k % 4] : gs[k];
     }
   }
 }
 
 // Backward preprocess of surfel idx in view v (record r),
 // dsr/cuda_rasterizer/backward.cu:443-630, from the record's reduced blend
-// gradients gs.  Adds the view's contributions to g (and to dL_dsh, owned by
-// this thread) and writes the record's outputs: dL_dtransMat (with the
-// AABB-centre term for a precomputed T), dL_dmean2D (the densification
-// statistic), dL_dopacity and dL_dcolors.
-template <bool kRow, bool kToRow>
-SR_DEV void preprocess_bwd_view(const PreprocessBwdArgs& a, int v, int idx, size_t r, bool first, SurfelGrad& g,
+// gradients gs.  Adds the view's contributions to g and writes the record's
+// outputs: dL_dtransMat (with the AABB-centre term for a precomputed T; may be
+// null), dL_dmean2D (the densification statistic) and, for a single view,
+// dL_dopacity, dL_dcolors and the dL_dsh row.  With several views (kMany) the
+// colour gradients go to dL_dcolors for the SH pass when there are SHs.
+template <bool kMany, bool kRow>
+SR_DEV void preprocess_bwd_view(const PreprocessBwdArgs& a, int v, int idx, size_t r, SurfelGrad& g,
                                 const float (&gs)[18], float4* srow) {
   const ViewInfo& vi = a.vs.v[v];
   const float tanx = vi.tanx, tany = vi.tany;
@@ -1092,7 +1086,6 @@ SR_DEV void preprocess_bwd_view(const PreprocessBwdArgs& a, int v, int idx, size
   const float* pm = a.pm + 16 * v;
   const float* vm = a.vm + 16 * v;
   const float* campos = a.campos + 3 * v;
-  float* gT = a.dL_dtransMat + 9 * r;
   const float m0 = a.means3D[3 * idx], m1 = a.means3D[3 * idx + 1], m2 = a.means3D[3 * idx + 2];
   const bool precomp = a.tprec != nullptr;
   F3 T0, T1, T2, Rc0, Rc1;
@@ -1158,18 +1151,19 @@ SR_DEV void preprocess_bwd_view(const PreprocessBwdArgs& a, int v, int idx, size
   }
   // dL_dtransMat: the blend's sums, with the AABB-centre term only for a
   // precomputed T
-  if (updated) {
-    gT[0] = dT0.x; gT[1] = dT0.y; gT[2] = dT0.z;
-    gT[3] = dT1.x; gT[4] = dT1.y; gT[5] = dT1.z;
-    gT[6] = dT2.x; gT[7] = dT2.y; gT[8] = dT2.z;
-  } else {
+  const float gT2 = updated ? dT0.z : gs[2], gT5 = updated ? dT1.z : gs[5];
+  if (a.dL_dtransMat != nullptr) {
+    float* gT = a.dL_dtransMat + 9 * r;
+    const float full[9] = {dT0.x, dT0.y, dT0.z, dT1.x, dT1.y, dT1.z, dT2.x, dT2.y, dT2.z};
 #pragma unroll
-    for (int k = 0; k < 9; ++k) gT[k] = gs[k];
+    for (int k = 0; k < 9; ++k) gT[k] = updated ? full[k] : gs[k];
   }
-  a.dL_dopacity[r] = gs[14];
-  a.dL_dcolors[3 * r] = gs[15];
-  a.dL_dcolors[3 * r + 1] = gs[16];
-  a.dL_dcolors[3 * r + 2] = gs[17];
+  if (!kMany) a.dL_dopacity[r] = gs[14];
+  if (!kMany || a.shs != nullptr) {
+    a.dL_dcolors[3 * r] = gs[15];
+    a.dL_dcolors[3 * r + 1] = gs[16];
+    a.dL_dcolors[3 * r + 2] = gs[17];
+  }
   if (!precomp) {
     float dM[3][3];
 #pragma unroll
@@ -1203,104 +1197,55 @@ SR_DEV void preprocess_bwd_view(const PreprocessBwdArgs& a, int v, int idx, size
     g.sc[0] += (dRS0.x * Rc0.x + dRS0.y * Rc0.y) + dRS0.z * Rc0.z;
     g.sc[1] += (dRS1.x * Rc1.x + dRS1.y * Rc1.y) + dRS1.z * Rc1.z;
     F3 dm3 = f3(dM[2][0], dM[2][1], dM[2][2]);
-    if (a.shs != nullptr)
-      dm3 = dm3 + sh_grad<kRow, kToRow>(a, first, idx, r, campos, m0, m1, m2, f3(gs[15], gs[16], gs[17]), srow);
+    if (!kMany && a.shs != nullptr)
+      dm3 = dm3 + sh_grad<kRow>(a, idx, r, campos, m0, m1, m2, f3(gs[15], gs[16], gs[17]), srow);
     g.m[0] += dm3.x;
     g.m[1] += dm3.y;
     g.m[2] += dm3.z;
-  } else if (a.shs != nullptr) {
-    const F3 dm3 = sh_grad<kRow, kToRow>(a, first, idx, r, campos, m0, m1, m2, f3(gs[15], gs[16], gs[17]), srow);
+  } else if (!kMany && a.shs != nullptr) {
+    const F3 dm3 = sh_grad<kRow>(a, idx, r, campos, m0, m1, m2, f3(gs[15], gs[16], gs[17]), srow);
     g.m[0] += dm3.x;
     g.m[1] += dm3.y;
     g.m[2] += dm3.z;
   }
   const float depth = a.rec[(size_t)kRecQuads * r + 2].x;  // Tw.z = transMat[8]
-  gm2[0] = (float)(((double)(gT[2] * depth) * 0.5) * (double)(float)W);
-  gm2[1] = (float)(((double)(gT[5] * depth) * 0.5) * (double)(float)H);
+  gm2[0] = (float)(((double)(gT2 * depth) * 0.5) * (double)(float)W);
+  gm2[1] = (float)(((double)(gT5 * depth) * 0.5) * (double)(float)H);
   gm2[2] = 0.0f;
 }
 
-// One thread per surfel, looping over the views; with one view every sum is
-// 0 + x, so the results equal the single-view formulas bit for bit.  Every
-// per-surfel and per-record output is written exactly once (zeros for a
-// record no view sees), so none of them needs clearing beforehand.
-// Degree-3 SH in 16-byte aligned rows move through LDS: each wave loads its
-// 64 surfels' rows (12 KB, contiguous) with coalesced loads and, for one
-// view, stores the gradient rows the same way, instead of each lane moving
-// its 192-byte row in 16-byte pieces 192 bytes apart.
-constexpr int kShRow = 12;  // float4 per degree-3 SH row
-template <bool kRow, bool kToRow>
-SR_DEV void preprocess_bwd_surfel(const PreprocessBwdArgs& a, int idx, float4* srow);
-// Three waves per SIMD (a few registers spill to scratch): with the 48 KB of
-// staged rows, two per SIMD was slower (0.086 against 0.071 ms at 300k surfels).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_preprocess_bwd(
-    PreprocessBwdArgs a) {
-  __shared__ float4 s_sh[256 * kShRow];
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool staged = a.shs != nullptr && a.M == 16 &&
-                      ((reinterpret_cast<uintptr_t>(a.shs) | reinterpret_cast<uintptr_t>(a.dL_dsh)) & 15u) == 0u;
-  const bool to_row = staged && a.vs.V == 1;  // uniform
-  const int w0 = blockIdx.x * blockDim.x + wave * 64;  // the wave's first surfel
-  const int nrow = min(64, a.P - w0) * kShRow;         // float4 of the wave's rows (<= 0: none)
-  float4* wrows = s_sh + wave * 64 * kShRow;
-  if (staged) {
-    const float4* src = reinterpret_cast<const float4*>(a.shs) + (size_t)w0 * kShRow;
-#pragma unroll
-    for (int t = 0; t < kShRow; ++t)
-      if (t * 64 + lane < nrow) wrows[t * 64 + lane] = src[t * 64 + lane];
-  }
-  __syncthreads();
-  if (idx < a.P) {
-    if (to_row) preprocess_bwd_surfel<true, true>(a, idx, wrows + lane * kShRow);
-    else if (staged) preprocess_bwd_surfel<true, false>(a, idx, wrows + lane * kShRow);
-    else preprocess_bwd_surfel<false, false>(a, idx, wrows);
-  }
-  if (to_row) {
-    __syncthreads();
-    float4* dst = reinterpret_cast<float4*>(a.dL_dsh) + (size_t)w0 * kShRow;
-#pragma unroll
-    for (int t = 0; t < kShRow; ++t)
-      if (t * 64 + lane < nrow) dst[t * 64 + lane] = wrows[t * 64 + lane];
-  }
-}
-
-// Gradients of surfel idx over all views; kRow: its SH row is staged in LDS
-// at srow, kToRow: its dL_dsh row goes there too.
-template <bool kRow, bool kToRow>
-SR_DEV void preprocess_bwd_surfel(const PreprocessBwdArgs& a, int idx, float4* srow) {
+// A surfel's outputs but dL_dsh: its records, and the sums over its views.
+// Every per-surfel and per-record output is written exactly once (zeros for a
+// record no view sees), so none of them needs clearing beforehand.  Returns
+// whether some view saw the surfel.
+template <bool kMany, bool kRow>
+SR_DEV bool preprocess_bwd_surfel(const PreprocessBwdArgs& a, int idx, float4* srow) {
   SurfelGrad g{};
   bool any = false;
-  const bool sum_rec = a.dL_dopacity_out != a.dL_dopacity;
   float op = 0.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
-  for (int v = 0; v < a.vs.V; ++v) {
+  const int V = kMany ? a.vs.V : 1;
+  for (int v = 0; v < V; ++v) {
     const size_t r = (size_t)v * a.P + idx;
     if (!(a.radii[r] > 0)) {
+      if (a.dL_dtransMat != nullptr) {
 #pragma unroll
-      for (int k = 0; k < 9; ++k) a.dL_dtransMat[9 * r + k] = 0.0f;
+        for (int k = 0; k < 9; ++k) a.dL_dtransMat[9 * r + k] = 0.0f;
+      }
       a.dL_dmean2D[3 * r] = a.dL_dmean2D[3 * r + 1] = a.dL_dmean2D[3 * r + 2] = 0.0f;
-      a.dL_dopacity[r] = 0.0f;
-      a.dL_dcolors[3 * r] = a.dL_dcolors[3 * r + 1] = a.dL_dcolors[3 * r + 2] = 0.0f;
+      if (!kMany) {
+        a.dL_dopacity[r] = 0.0f;
+        a.dL_dcolors[3 * r] = a.dL_dcolors[3 * r + 1] = a.dL_dcolors[3 * r + 2] = 0.0f;
+      }
       continue;
     }
     float gs[18];
-    reduce_record(a, r, gs);
-    preprocess_bwd_view<kRow, kToRow>(a, v, idx, r, !any, g, gs, srow);
+    reduce_record<kMany ? 2 : 4>(a, r, gs);
+    preprocess_bwd_view<kMany, kRow>(a, v, idx, r, g, gs, srow);
     any = true;
-    if (sum_rec) {
-      op += gs[14];
-      c0 += gs[15];
-      c1 += gs[16];
-      c2 += gs[17];
-    }
-  }
-  if (!any && a.shs != nullptr) {
-    if (kToRow) {
-      for (int k = 0; k < kShRow; ++k) srow[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    } else {
-      float* dsh = a.dL_dsh + (size_t)idx * a.M * 3;
-      for (int k = 0; k < 3 * a.M; ++k) dsh[k] = 0.0f;
-    }
+    op += gs[14];
+    c0 += gs[15];
+    c1 += gs[16];
+    c2 += gs[17];
   }
   a.dL_drots[4 * idx] = g.q[0];
   a.dL_drots[4 * idx + 1] = g.q[1];
@@ -1311,17 +1256,164 @@ SR_DEV void preprocess_bwd_surfel(const PreprocessBwdArgs& a, int idx, float4* s
   a.dL_dmean3D[3 * idx] = g.m[0];
   a.dL_dmean3D[3 * idx + 1] = g.m[1];
   a.dL_dmean3D[3 * idx + 2] = g.m[2];
-  if (sum_rec) {
+  if (kMany) {
     a.dL_dopacity_out[idx] = op;
     a.dL_dcolors_out[3 * idx] = c0;
     a.dL_dcolors_out[3 * idx + 1] = c1;
     a.dL_dcolors_out[3 * idx + 2] = c2;
   }
+  return any;
+}
+
+// Degree-3 SH in 16-byte aligned rows move through LDS: each wave loads its
+// 64 surfels' rows (12 KB, contiguous) with coalesced loads and stores the
+// gradient rows the same way, instead of each lane moving its 192-byte row in
+// 16-byte pieces 192 bytes apart.
+constexpr int kShRow = 12;  // float4 per degree-3 SH row
+constexpr int kShPad = 13;  // its LDS stride where each view reads it, odd against bank conflicts
+__host__ __device__ inline bool sh_rows(const PreprocessBwdArgs& a) {
+  return a.shs != nullptr && a.M == 16 &&
+         ((reinterpret_cast<uintptr_t>(a.shs) | reinterpret_cast<uintptr_t>(a.dL_dsh)) & 15u) == 0u;
+}
+// move(i, k) for the wave's rows from surfel w0 on: float4 i of their memory,
+// k of the LDS rows kStride apart
+template <int kStride, class Move>
+SR_DEV void each_row_quad(int P, int w0, Move move) {
+  const int lane = threadIdx.x & 63, n = min(64, P - w0) * kShRow;
+#pragma unroll
+  for (int t = 0; t < kShRow; ++t)
+    if (t * 64 + lane < n) {
+      const int i = t * 64 + lane, row = i / kShRow;
+      move(i, row * kStride + (i - row * kShRow));
+    }
+}
+
+// Runs surfel(idx, srow, rows) for the workgroup's surfels, one a thread: with
+// rows, srow is the surfel's SH row staged in LDS, which it replaces by its
+// dL_dsh row.
+template <class Surfel>
+SR_DEV void with_sh_rows(const PreprocessBwdArgs& a, Surfel surfel) {
+  __shared__ float4 s_sh[256 * kShRow];
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool rows = sh_rows(a);                        // uniform
+  const int w0 = blockIdx.x * blockDim.x + wave * 64;  // the wave's first surfel
+  float4* wrows = s_sh + wave * 64 * kShRow;
+  float4* srow = wrows + lane * kShRow;
+  if (rows) {
+    const float4* src = reinterpret_cast<const float4*>(a.shs) + (size_t)w0 * kShRow;
+    each_row_quad<kShRow>(a.P, w0, [&](int i, int k) { wrows[k] = src[i]; });
+  }
+  __syncthreads();
+  if (idx < a.P) {
+    const bool any = rows ? surfel(std::true_type{}, idx, srow) : surfel(std::false_type{}, idx, srow);
+    if (!any && rows) {
+      for (int k = 0; k < kShRow; ++k) srow[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    } else if (!any && a.shs != nullptr) {
+      float* dsh = a.dL_dsh + (size_t)idx * a.M * 3;
+      for (int k = 0; k < 3 * a.M; ++k) dsh[k] = 0.0f;
+    }
+  }
+  if (rows) {
+    __syncthreads();
+    float4* dst = reinterpret_cast<float4*>(a.dL_dsh) + (size_t)w0 * kShRow;
+    each_row_quad<kShRow>(a.P, w0, [&](int i, int k) { dst[i] = wrows[k]; });
+  }
+}
+
+// Backward preprocess of a single view, one thread per surfel; three waves per
+// SIMD, with the 48 KB of LDS three workgroups a CU.  Bound by the latencies in
+// front of the sums as much as by memory: 300k surfels of degree 3 59 us (180
+// MB, 3 TB/s), 65 with one slot's sums in flight.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_preprocess_bwd(
+    PreprocessBwdArgs a) {
+  with_sh_rows(a, [&](auto row, int idx, float4* srow) {
+    return preprocess_bwd_surfel<false, decltype(row)::value>(a, idx, srow);
+  });
+}
+
+// Backward preprocess of several views but for the SHs: one thread per surfel,
+// looping over the views.  A million surfels, 16 views: 0.91 ms and the SH pass
+// 0.30, where one kernel that read and wrote the dL_dsh rows once a view, and
+// 64 bytes of per-record gradients, took 3.06.
+__global__ __launch_bounds__(256) void k_preprocess_bwd_views(PreprocessBwdArgs a) {
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx < a.P) preprocess_bwd_surfel<true, false>(a, idx, nullptr);
+}
+
+// SH backward of several views, one thread per surfel: the dL_dsh row summed
+// in registers over the views that see the surfel, and the mean's gradient
+// through the view directions added to dL_dmean3D.
+template <bool kRow>
+__global__ __launch_bounds__(64) void k_sh_bwd_views(PreprocessBwdArgs a) {
+  __shared__ float4 s_sh[kRow ? 64 * kShPad : 1];
+  const int w0 = blockIdx.x * 64, lane = threadIdx.x, idx = w0 + lane;
+  if (kRow) {
+    const float4* src = reinterpret_cast<const float4*>(a.shs) + (size_t)w0 * kShRow;
+    each_row_quad<kShPad>(a.P, w0, [&](int i, int k) { s_sh[k] = src[i]; });
+    __syncthreads();
+  }
+  const bool in = idx < a.P;
+  const float* row = kRow ? reinterpret_cast<const float*>(s_sh + lane * kShPad) : a.shs + (size_t)(in ? idx : 0) * a.M * 3;
+  const int nact = (a.D + 1) * (a.D + 1);
+  float acc[48];
+#pragma unroll
+  for (int k = 0; k < 48; ++k) acc[k] = 0.0f;
+  F3 gm = f3(0.0f, 0.0f, 0.0f);
+  const F3 m = in ? f3(a.means3D[3 * idx], a.means3D[3 * idx + 1], a.means3D[3 * idx + 2]) : gm;
+  for (int v = 0; v < a.vs.V; ++v) {
+    const size_t r = (size_t)v * a.P + idx;
+    if (!in || !(a.radii[r] > 0)) continue;
+    const F3 dRGB = unclamped(a, r, f3(a.dL_dcolors[3 * r], a.dL_dcolors[3 * r + 1], a.dL_dcolors[3 * r + 2]));
+    const float* campos = a.campos + 3 * v;
+    gm = gm + sh_backward_core(
+                  a.D, f3(m.x - campos[0], m.y - campos[1], m.z - campos[2]), dRGB,
+                  [&](int k) { return f3(row[3 * k], row[3 * k + 1], row[3 * k + 2]); },
+                  [&](int k, float c) {
+                    acc[3 * k] += c * dRGB.x;
+                    acc[3 * k + 1] += c * dRGB.y;
+                    acc[3 * k + 2] += c * dRGB.z;
+                  });
+  }
+  if (in) {
+    a.dL_dmean3D[3 * idx] += gm.x;
+    a.dL_dmean3D[3 * idx + 1] += gm.y;
+    a.dL_dmean3D[3 * idx + 2] += gm.z;
+  }
+  if (kRow) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kShRow; ++k)
+      s_sh[lane * kShPad + k] = make_float4(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
+    __syncthreads();
+    float4* dst = reinterpret_cast<float4*>(a.dL_dsh) + (size_t)w0 * kShRow;
+    each_row_quad<kShPad>(a.P, w0, [&](int i, int k) { dst[i] = s_sh[k]; });
+  } else if (in) {
+    float* dsh = a.dL_dsh + (size_t)idx * a.M * 3;
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+      if (k < nact) {
+        dsh[3 * k] = acc[3 * k];
+        dsh[3 * k + 1] = acc[3 * k + 1];
+        dsh[3 * k + 2] = acc[3 * k + 2];
+      }
+    for (int k = 3 * nact; k < 3 * a.M; ++k) dsh[k] = 0.0f;
+  }
 }
 
 hipError_t launch_preprocess_bwd(const PreprocessBwdArgs& a, hipStream_t s) {
   if (a.P == 0 || a.vs.V == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_preprocess_bwd, dim3((a.P + 255) / 256), dim3(256), 0, s, a);
+  const dim3 grid((a.P + 255) / 256);
+  if (a.vs.V == 1) {
+    hipLaunchKernelGGL(k_preprocess_bwd, grid, dim3(256), 0, s, a);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(k_preprocess_bwd_views, grid, dim3(256), 0, s, a);
+  if (a.shs != nullptr) {
+    const dim3 waves((a.P + 63) / 64);
+    if (sh_rows(a)) hipLaunchKernelGGL(k_sh_bwd_views<true>, waves, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL(k_sh_bwd_views<false>, waves, dim3(64), 0, s, a);
+  }
   return hipGetLastError();
 }
 
@@ -1332,10 +1424,8 @@ hipError_t launch_preprocess_bwd(const PreprocessBwdArgs& a, hipStream_t s) {
 // densification statistic (computeAABB, dsp/backward.cu:621-671), then the
 // camera-space homography's adjoint (computeTransMat, :473-545) and the SH
 // backward.  Every output is written (zeros for a culled surfel).
-__global__ __launch_bounds__(256) void k_part_preprocess_bwd(PreprocessBwdArgs a) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= a.P) return;
-  const int S = a.S;
+template <bool kRow>
+SR_DEV bool part_preprocess_bwd_surfel(const PreprocessBwdArgs& a, int idx, float4* srow) {
   float* gT = a.dL_dtransMat + 9 * idx;
   float* gm2 = a.dL_dmean2D + 3 * idx;
   if (!(a.radii[idx] > 0)) {
@@ -1344,26 +1434,10 @@ __global__ __launch_bounds__(256) void k_part_preprocess_bwd(PreprocessBwdArgs a
     a.dL_dopacity[idx] = 0.0f;
     a.dL_dscales[2 * idx] = a.dL_dscales[2 * idx + 1] = 0.0f;
     for (int k = 0; k < 4; ++k) a.dL_drots[4 * idx + k] = 0.0f;
-    for (int ch = 0; ch < S; ++ch) a.dL_dsem[(size_t)idx * S + ch] = 0.0f;
-    if (a.shs != nullptr)
-      for (int k = 0; k < 3 * a.M; ++k) a.dL_dsh[(size_t)idx * a.M * 3 + k] = 0.0f;
-    return;
+    return false;
   }
   float gs[18];
-  reduce_record(a, (size_t)idx, gs);
-  // semantic partials, in the same (instance, quadrant) order
-  {
-    float sm[16];
-    for (int ch = 0; ch < 16; ++ch) sm[ch] = 0.0f;
-    if (S > 0 && a.part != nullptr && a.tiles[idx] > 0 && !(a.counters[1] & kErrCapacity)) {
-      const uint2 rs = a.rslot[idx];  // the record's slots, in the order of reduce_record
-      for (uint32_t sl = rs.x; sl < rs.x + rs.y; ++sl) {
-        if (a.part_nz[sl] == 0) continue;
-        for (int ch = 0; ch < S; ++ch) sm[ch] += a.sem_part[(size_t)sl * S + ch];
-      }
-    }
-    for (int ch = 0; ch < S; ++ch) a.dL_dsem[(size_t)idx * S + ch] = sm[ch];
-  }
+  reduce_record<4>(a, (size_t)idx, gs);
   const ViewInfo& vi = a.vs.v[0];
   const float tanx = vi.tanx, tany = vi.tany;
   const float fx = (float)vi.W / (2.0f * tanx), fy = (float)vi.H / (2.0f * tany);
@@ -1453,24 +1527,57 @@ __global__ __launch_bounds__(256) void k_part_preprocess_bwd(PreprocessBwdArgs a
     a.dL_dscales[2 * idx] = a.dL_dscales[2 * idx + 1] = 0.0f;
     for (int k = 0; k < 4; ++k) a.dL_drots[4 * idx + k] = 0.0f;
   }
-  if (a.shs != nullptr) {
-    F3 dRGB = f3(gs[15], gs[16], gs[17]);
-    const uchar4 cl = reinterpret_cast<const uchar4*>(a.clamped)[idx];
-    if (cl.x) dRGB.x = 0.0f;
-    if (cl.y) dRGB.y = 0.0f;
-    if (cl.z) dRGB.z = 0.0f;
-    const F3 dir_orig = f3(m0 - a.campos[0], m1 - a.campos[1], m2 - a.campos[2]);
-    dm3 = dm3 + sh_backward<false, false, false>(a.D, a.M, a.shs + (size_t)idx * a.M * 3, dir_orig, dRGB,
-                                                  a.dL_dsh + (size_t)idx * a.M * 3, nullptr);
-  }
+  if (a.shs != nullptr)
+    dm3 = dm3 + sh_grad<kRow>(a, idx, (size_t)idx, a.campos, m0, m1, m2, f3(gs[15], gs[16], gs[17]), srow);
   a.dL_dmean3D[3 * idx] = dm3.x;
   a.dL_dmean3D[3 * idx + 1] = dm3.y;
   a.dL_dmean3D[3 * idx + 2] = dm3.z;
+  return true;
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_part_preprocess_bwd(
+    PreprocessBwdArgs a) {
+  with_sh_rows(a, [&](auto row, int idx, float4* srow) {
+    return part_preprocess_bwd_surfel<decltype(row)::value>(a, idx, srow);
+  });
+}
+
+// Semantic gradients: per (surfel, channel), the partials summed over the
+// record's slots in the order of reduce_record, zeros for a culled surfel.  The
+// channels of a surfel are neighbouring lanes, so a slot is one coalesced read:
+// with this and the SH rows through LDS 79 us for 300k surfels and 8 channels,
+// 92 in one kernel with a lane a surfel.
+__global__ __launch_bounds__(256) void k_part_semantics_bwd(PreprocessBwdArgs a) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (size_t)a.P * a.S) return;
+  const uint32_t idx = (uint32_t)(i / (uint32_t)a.S), ch = (uint32_t)(i % (uint32_t)a.S);
+  float sum = 0.0f;
+  if (a.radii[idx] > 0 && a.part != nullptr && a.tiles[idx] > 0 && !(a.counters[1] & kErrCapacity)) {
+    const uint2 rs = a.rslot[idx];
+    for (uint32_t s = rs.x, end = rs.x + rs.y; s < end; s += 4) {
+      uint8_t fl[4];
+      float v[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint32_t sl = min(s + (uint32_t)t, end - 1u);
+        fl[t] = a.part_nz[sl];
+        v[t] = a.sem_part[(size_t)sl * a.S + ch];  // unset, and not used, without the flag
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (s + (uint32_t)t < end && fl[t] != 0) sum += v[t];
+    }
+  }
+  a.dL_dsem[i] = sum;
 }
 
 hipError_t launch_part_preprocess_bwd(const PreprocessBwdArgs& a, hipStream_t s) {
   if (a.P == 0) return hipSuccess;
   hipLaunchKernelGGL(k_part_preprocess_bwd, dim3((a.P + 255) / 256), dim3(256), 0, s, a);
+  if (a.S > 0) {
+    const size_t n = (size_t)a.P * a.S;
+    hipLaunchKernelGGL(k_part_semantics_bwd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
+  }
   return hipGetLastError();
 }
 
