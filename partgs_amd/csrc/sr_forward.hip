@@ -136,9 +136,12 @@ SR_DEV F3 color_from_sh(int deg, int M, const float* sh, F3 dir, uint8_t* clampe
 // whose centres lie between the bounds.  A level set reaching the camera
 // plane (d >= 0) projects unbounded: no box then.
 //
-// The conic is formed about the surfel's centre (Tu - mx Tw, Tv - my Tw), so
-// its extents do not cancel against the image coordinates: they are good to
-// about 1e-6 of the coordinates.  The pixels' own FP32 rho is as good while
+// The conic is formed about the surfel's projected centre (ox, oy) = (Tu.z,
+// Tv.z) / Tw.z, which lies inside it, so its extents do not cancel against the
+// image coordinates: they are good to about 1e-6 of the coordinates.  (mean2D
+// would not do: it is the centre of the 3 sigma conic's box, anywhere on or far
+// off the image when that conic nearly reaches the camera plane while the
+// level set of a faint surfel does not.)  The pixels' own FP32 rho is as good while
 // the two planes of a pixel are not nearly parallel (p.z well above the
 // rounding of its two products; checked at the centre) and the depth varies
 // by less than half over the level set.  Such surfels, nearly all, get a
@@ -166,8 +169,9 @@ SR_DEV short4 cull_box(F3 Tu, F3 Tv, F3 Tw, float mx, float my, float opa, int W
   if (!(d < -1e-3f * (Tw.z * Tw.z))) return all;
   const float fx = c2 / d, fz = -1.0f / d;
   float x0, x1, y0, y1;
-  const F3 U = f3(Tu.x - mx * Tw.x, Tu.y - mx * Tw.y, Tu.z - mx * Tw.z);
-  const F3 V = f3(Tv.x - my * Tw.x, Tv.y - my * Tw.y, Tv.z - my * Tw.z);
+  const float ox = Tu.z / Tw.z, oy = Tv.z / Tw.z;
+  const F3 U = f3(Tu.x - ox * Tw.x, Tu.y - ox * Tw.y, Tu.z - ox * Tw.z);
+  const F3 V = f3(Tv.x - oy * Tw.x, Tv.y - oy * Tw.y, Tv.z - oy * Tw.z);
   const float pa = U.x * V.y, pb = U.y * V.x;
   const bool sound = fabsf(pa - pb) > 0.01f * (fabsf(pa) + fabsf(pb)) && c2 * ww < 0.25f * (Tw.z * Tw.z);
   if (sound) {
@@ -175,11 +179,11 @@ SR_DEV short4 cull_box(F3 Tu, F3 Tv, F3 Tw, float mx, float my, float opa, int W
     const float cy = fx * (V.x * Tw.x + V.y * Tw.y) + fz * (V.z * Tw.z);
     const float hx = sqrtf(fmax_(0.0f, cx * cx - (fx * (U.x * U.x + U.y * U.y) + fz * (U.z * U.z))));
     const float hy = sqrtf(fmax_(0.0f, cy * cy - (fx * (V.x * V.x + V.y * V.y) + fz * (V.z * V.z))));
-    const float gx = 0.02f + 2e-6f * fabsf(mx), gy = 0.02f + 2e-6f * fabsf(my);
-    x0 = ceilf((mx - fmax_(r2, 1.002f * hx - cx)) - gx - shift);
-    x1 = floorf((mx + fmax_(r2, 1.002f * hx + cx)) + gx - shift);
-    y0 = ceilf((my - fmax_(r2, 1.002f * hy - cy)) - gy - shift);
-    y1 = floorf((my + fmax_(r2, 1.002f * hy + cy)) + gy - shift);
+    const float gx = 0.02f + 2e-6f * fmax_(fabsf(mx), fabsf(ox)), gy = 0.02f + 2e-6f * fmax_(fabsf(my), fabsf(oy));
+    x0 = ceilf(fmin_(mx - r2, ox - (1.002f * hx - cx)) - gx - shift);
+    x1 = floorf(fmax_(mx + r2, ox + (1.002f * hx + cx)) + gx - shift);
+    y0 = ceilf(fmin_(my - r2, oy - (1.002f * hy - cy)) - gy - shift);
+    y1 = floorf(fmax_(my + r2, oy + (1.002f * hy + cy)) + gy - shift);
   } else {
     const float cx = fx * (Tu.x * Tw.x + Tu.y * Tw.y) + fz * (Tu.z * Tw.z);
     const float cy = fx * (Tv.x * Tw.x + Tv.y * Tw.y) + fz * (Tv.z * Tw.z);

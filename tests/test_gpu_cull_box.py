@@ -52,3 +52,28 @@ def test_no_accepted_pixel_outside(W, H, grazing, close, size):
     res = gpu_forward(scene)
     _check_forward(scene, res, o)
     _check_backward(scene, res, o, seed=1)
+
+
+@pytest.mark.parametrize("P", [1, 300, 2000])
+def test_faint_surfels_whose_three_sigma_conic_nearly_reaches_the_camera(P):
+    """mean2D, the centre of the 3 sigma conic's box, then lies anywhere; the
+    level set of a faint surfel is a small ellipse about its own centre."""
+    O.set_threads(8)
+    W, H = 53, 37
+    rng = np.random.default_rng(P)
+    cam = look_at((0.0, 0.0, 0.0), target=(0.0, 0.0, 1.0), width=W, height=H)
+    z = rng.uniform(0.5, 5.0, P)
+    means = np.concatenate([rng.uniform(-0.3, 0.3, (P, 2)) * z[:, None], z[:, None]], 1)
+    tilt, turn = rng.uniform(0.2, 1.2, P), rng.uniform(0, 2 * np.pi, P)
+    # about an axis of the image plane by tilt: the depths of the tangents are
+    # sin(tilt) times their scales across the axis, so 9 (Tw.x^2 + Tw.y^2) is
+    # near Tw.z^2 for scales of z / (3 sin(tilt))
+    q = np.stack([np.cos(tilt / 2), np.sin(tilt / 2) * np.cos(turn), np.sin(tilt / 2) * np.sin(turn), np.zeros(P)], 1)
+    s = z / (3 * np.sin(tilt)) * np.sqrt(1 + rng.choice([-1.0, 1.0], P) * 10.0 ** rng.uniform(-5, -1, P))
+    opacity = np.exp(rng.uniform(0, 0.5, (P, 1))) / 255
+    f = lambda a: torch.from_numpy(np.ascontiguousarray(a)).float()  # noqa: E731
+    scene = SurfelScene(f(means), f(np.stack([s, s], 1)), f(q), f(opacity), f(rng.normal(size=(P, 1, 3))), 0, cam,
+                        torch.ones(3))
+    o, rc = oracle_run(scene)
+    assert rc == 0
+    _check_forward(scene, gpu_forward(scene), o)
