@@ -1614,53 +1614,99 @@ constexpr float kSaturatedT = 0.5e-4f;
 // transmittances) are cut: their masks are cleared and their pairs never
 // stored, as the blend never reaches them.  A quadrant whose pairs do not
 // fit is flagged and left to the staged path.
-__global__ __launch_bounds__(64) void k_pair_offsets(AcceptArgs a) {
+// Bound by the chain of loads down the longest lists (hundreds of chunks in a
+// dense tile), so lists above kPoChunks chunks are walked by four waves, each
+// kPoChunks of every 4 kPoChunks, which exchange their transmittances and
+// counts per pixel in LDS; lists that one step covers are read once.  26 us for
+// 300k surfels at 800 x 600 and 230 for 16 views of a million, where one wave
+// a quadrant took 37 and 363; eight waves: 25 and 259.  Reserving the runs of
+// 16 quadrants with one atomic made a workgroup wait for its longest list: 30
+// and 530.
+constexpr int kPoWaves = 4, kPoChunks = 8;
+__global__ __launch_bounds__(kPoWaves * 64) void k_pair_offsets(AcceptArgs a) {
+  constexpr int kU = kPoChunks;  // chunks in flight a wave
+  __shared__ float s_T[kPoWaves][64];
+  __shared__ int s_cut[kPoWaves][64];
+  __shared__ uint32_t s_n[kPoWaves][64];
+  __shared__ unsigned long long s_fill;
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (a.counters[1] & kErrCapacity) return;
   const int qi = blockIdx.x;
   const int tile = qi / Q, q = qi % Q;
   const int cnt = (int)a.sub_count[qi];
   const int nch = (cnt + 63) / 64;
+  const int nw = nch > kU ? kPoWaves : 1;  // uniform
+  if (wave >= nw) return;
+  auto sync = [&]() {
+    if (nw > 1) __syncthreads();
+  };
   const uint32_t rbeg = a.ranges[2 * tile], ntile = a.ranges[2 * tile + 1] - rbeg;
   const size_t base = mask_base(Q, rbeg, ntile, tile, q) + lane;
-#ifndef SR_PO_UNROLL
-#define SR_PO_UNROLL 8
-#endif
-  constexpr int kU = SR_PO_UNROLL;  // mask loads in flight
-  uint32_t tot = 0;
-  int cut = nch;  // first chunk the pixel cannot reach
-  float trun = 1.0f;
-  for (int c0 = 0; c0 < nch; c0 += kU) {
-    uint64_t mk[kU];
-    float tk[kU];
-    // unconditional loads (chunk index clamped into range) so all 2 kU are
-    // in flight together; the values past the end are then dropped
+  const int step = nw * kU;
+  uint64_t mk[kU];
+  // unconditional loads (chunk index clamped into the list) so all are in
+  // flight together; the values past the end are then dropped
+  auto load_masks = [&](int c0) {
+#pragma unroll
+    for (int k = 0; k < kU; ++k) mk[k] = a.masks[base + (size_t)min(c0 + k, nch - 1) * 64];
+  };
+  uint32_t tot = 0, n = 0;  // the pixel's pairs; of this wave's chunks of the step
+  int cut = nch;            // first chunk the pixel cannot reach
+  float T0 = 1.0f;          // transmittance in front of the step
+  for (int t0 = 0; t0 < nch; t0 += step) {
+    const int c0 = t0 + wave * kU;
+    load_masks(c0);
+    float tk[kU], T = T0, all = 1.0f;
+#pragma unroll
+    for (int k = 0; k < kU; ++k) tk[k] = a.chunk_T[base + (size_t)min(c0 + k, nch - 1) * 64];
 #pragma unroll
     for (int k = 0; k < kU; ++k) {
-      const size_t cc = (size_t)min(c0 + k, nch - 1) * 64;
-      mk[k] = a.masks[base + cc];
-      tk[k] = a.chunk_T[base + cc];
+      tk[k] = c0 + k < nch ? tk[k] : 1.0f;
+      all *= tk[k];
     }
+    if (nw > 1) {
+      s_T[wave][lane] = all;
+      __syncthreads();
+      all = 1.0f;
 #pragma unroll
-    for (int k = 0; k < kU; ++k) {
-      const bool in = c0 + k < nch;
-      mk[k] = in ? mk[k] : 0ull;
-      tk[k] = in ? tk[k] : 1.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < kU; ++k) {
-      if (c0 + k < cut) {
-        if (trun < kSaturatedT) {
-          cut = c0 + k;
-        } else {
-          tot += (uint32_t)__popcll(mk[k]);
-          trun *= tk[k];
-        }
+      for (int w = 0; w < kPoWaves; ++w) {
+        if (w == wave) T = T0 * all;
+        all *= s_T[w][lane];
       }
     }
+    T0 *= all;
+    int first = cut;
+#pragma unroll
+    for (int k = 0; k < kU; ++k) {
+      if (T < kSaturatedT) first = min(first, c0 + k);
+      T *= tk[k];
+    }
+    cut = first;
+    if (nw > 1) {
+      s_cut[wave][lane] = first;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kPoWaves; ++w) cut = min(cut, s_cut[w][lane]);
+    }
+    n = 0;
+#pragma unroll
+    for (int k = 0; k < kU; ++k) {
+      if (c0 + k >= cut) {
+        mk[k] = 0ull;
+        if (c0 + k < nch) a.masks[base + (size_t)(c0 + k) * 64] = 0ull;
+      }
+      n += (uint32_t)__popcll(mk[k]);
+    }
+    if (nw > 1) {
+      s_n[wave][lane] = n;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kPoWaves; ++w) tot += s_n[w][lane];
+    } else {
+      tot += n;
+    }
   }
-  for (int c = cut; c < nch; ++c) a.masks[base + (size_t)c * 64] = 0ull;
   uint32_t incl = tot;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -1669,34 +1715,60 @@ __global__ __launch_bounds__(64) void k_pair_offsets(AcceptArgs a) {
   }
   const uint32_t total = __shfl(incl, 63, 64);
   unsigned long long qbase = 0;
-  if (lane == 0 && total > 0) qbase = atomicAdd(a.frag_fill, (unsigned long long)total);
+  if (threadIdx.x == 0 && total > 0) qbase = atomicAdd(a.frag_fill, (unsigned long long)total);
   qbase = __shfl(qbase, 0, 64);
+  if (nw > 1) {
+    if (threadIdx.x == 0) s_fill = qbase;
+    __syncthreads();
+    qbase = s_fill;
+  }
   const bool fits = qbase + total <= (unsigned long long)a.frag_cap;
-  // cost of the quadrant for the blend kernels' longest-first order: its
-  // longest pixel chain (the staged path, when it does not fit, its list)
-  uint32_t mx = tot;
+  if (wave == 0) {
+    // cost of the quadrant for the blend kernels' longest-first order: its
+    // longest pixel chain (the staged path, when it does not fit, its list)
+    uint32_t mx = tot;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
-  if (lane == 0) a.q_cost[qi] = fits ? mx : (uint32_t)cnt;
+    for (int off = 32; off > 0; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
+    if (lane == 0) {
+      a.q_cost[qi] = fits ? mx : (uint32_t)cnt;
+      if (!fits) a.q_flag[qi] = 1u;
+    }
+    a.lane_range[(size_t)qi * 64 + lane] = fits ? make_uint2((uint32_t)qbase + (incl - tot), tot) : make_uint2(0u, 0u);
+  }
   if (!fits) {
-    if (lane == 0) a.q_flag[qi] = 1u;
-    a.lane_range[(size_t)qi * 64 + lane] = make_uint2(0u, 0u);
-    for (int c = 0; c < nch; ++c) a.frag_off[base + (size_t)c * 64] = kNoFrag;
+    for (int c = wave; c < nch; c += nw) a.frag_off[base + (size_t)c * 64] = kNoFrag;
     return;
   }
   uint32_t run = (uint32_t)qbase + (incl - tot);
-  a.lane_range[(size_t)qi * 64 + lane] = make_uint2(run, tot);
-  for (int c0 = 0; c0 < nch; c0 += kU) {
-    uint64_t mk[kU];
+  for (int t0 = 0; t0 < nch; t0 += step) {
+    const int c0 = t0 + wave * kU;
+    if (nch > step) {  // more than one step: the masks again
+      load_masks(c0);
+      n = 0;
 #pragma unroll
-    for (int k = 0; k < kU; ++k) mk[k] = a.masks[base + (size_t)min(c0 + k, nch - 1) * 64];
+      for (int k = 0; k < kU; ++k) {
+        mk[k] = c0 + k < cut ? mk[k] : 0ull;
+        n += (uint32_t)__popcll(mk[k]);
+      }
+      sync();  // the last step's counts are read
+      s_n[wave][lane] = n;
+      sync();
+    }
+    uint32_t at = run, step_n = n;
+    if (nw > 1) {
+      step_n = 0;
 #pragma unroll
-    for (int k = 0; k < kU; ++k) mk[k] = (c0 + k < cut) ? mk[k] : 0ull;
+      for (int w = 0; w < kPoWaves; ++w) {
+        if (w == wave) at = run + step_n;
+        step_n += s_n[w][lane];
+      }
+    }
 #pragma unroll
     for (int k = 0; k < kU; ++k) {
-      if (c0 + k < nch) a.frag_off[base + (size_t)(c0 + k) * 64] = run;
-      run += (uint32_t)__popcll(mk[k]);
+      if (c0 + k < nch) a.frag_off[base + (size_t)(c0 + k) * 64] = at;
+      at += (uint32_t)__popcll(mk[k]);
     }
+    run += step_n;
   }
 }
 
@@ -1724,28 +1796,37 @@ __global__ __launch_bounds__(1024) void k_order_quads(int nq, const uint32_t* co
   // places those with one LDS atomic instead of one per lane.
   const int lane = tid & 63;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  for (int i0 = 0; i0 < nq; i0 += 1024) {  // uniform
-    const int i = i0 + tid;
-    const uint32_t c = i < nq ? cost[i] : 1u;
+  constexpr int kU = 8;  // costs in flight a lane
+  auto each = [&](auto&& fn) {  // fn(quadrant or nq and more, its cost), the whole wave at once
+    for (int i0 = 0; i0 < nq; i0 += 1024 * kU) {  // uniform
+      uint32_t c[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) c[u] = cost[min(i0 + u * 1024 + tid, nq - 1)];
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        if (i0 + u * 1024 < nq) fn(i0 + u * 1024 + tid, c[u]);
+    }
+  };
+  each([&](int i, uint32_t c) {
     const uint64_t zero = __ballot(i < nq && c == 0u);
     if (lane == 0 && zero) atomicAdd(&s_cnt[63], (uint32_t)__popcll(zero));
     if (i < nq && c != 0u) atomicAdd(&s_cnt[bucket(c)], 1u);
-  }
+  });
   __syncthreads();
-  if (tid == 0) {
-    uint32_t run = 0;
-    for (int b = 0; b < 64; ++b) {
-      // two buckets an octave: costs of 2^k and more are in 0..61 - 2 k
-      const int c = b == 46 ? 0 : b == 50 ? 1 : b == 52 ? 2 : b == 54 ? 3 : b == 63 ? 4 : -1;
-      if (c >= 0) counters[kCostClass + c] = run;
-      s_base[b] = run;
-      run += s_cnt[b];
+  if (tid < 64) {
+    uint32_t incl = s_cnt[tid];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)incl, off);
+      if (lane >= off) incl += y;
     }
+    s_base[tid] = incl - s_cnt[tid];
+    // two buckets an octave: costs of 2^k and more are in 0..61 - 2 k
+    const int c = tid == 45 ? 0 : tid == 49 ? 1 : tid == 51 ? 2 : tid == 53 ? 3 : tid == 62 ? 4 : -1;
+    if (c >= 0) counters[kCostClass + c] = incl;
   }
   __syncthreads();
-  for (int i0 = 0; i0 < nq; i0 += 1024) {
-    const int i = i0 + tid;
-    const uint32_t c = i < nq ? cost[i] : 1u;
+  each([&](int i, uint32_t c) {
     const uint64_t zero = __ballot(i < nq && c == 0u);
     uint32_t zbase = 0;
     if (lane == 0 && zero) zbase = atomicAdd(&s_base[63], (uint32_t)__popcll(zero));
@@ -1754,7 +1835,7 @@ __global__ __launch_bounds__(1024) void k_order_quads(int nq, const uint32_t* co
       if (c == 0u) order[zbase + (uint32_t)__popcll(zero & lt)] = (uint32_t)i;
       else order[atomicAdd(&s_base[bucket(c)], 1u)] = (uint32_t)i;
     }
-  }
+  });
 }
 
 hipError_t launch_order_quads(int nq, const uint32_t* cost, uint32_t* order, uint32_t* counters,
@@ -1777,7 +1858,7 @@ hipError_t launch_iota_u32(uint32_t* p, size_t n, hipStream_t s) {
 
 hipError_t launch_pair_offsets(const AcceptArgs& a, hipStream_t s) {
   if (a.vs.T == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_pair_offsets, dim3((unsigned)(a.vs.T * quads_per_tile(a.vs.B))), dim3(64), 0, s, a);
+  hipLaunchKernelGGL(k_pair_offsets, dim3((unsigned)(a.vs.T * quads_per_tile(a.vs.B))), dim3(kPoWaves * 64), 0, s, a);
   return hipGetLastError();
 }
 
