@@ -429,7 +429,7 @@ int run_binning(Pipeline& pl, const int* radii, bool dbg, hipStream_t st) {
   sa.pos_quads = (uint16_t*)(bin + bl.pos_quads);
   sa.sub = (uint2*)(bin + bl.sub);
   sa.sub_count = (uint32_t*)(pl.img + pl.il.sub_count);
-  sa.work = (uint2*)(bin + bl.work);
+  sa.work = (uint4*)(bin + bl.work);
   sa.work_count = counters + 2;
   sa.q_flag = (uint32_t*)(pl.img + pl.il.q_flag);
   SR_STAGE(3, dbg, st, "sort", launch_sort_tiles(sa, segment_capacity((size_t)pl.capacity), st));
@@ -519,7 +519,7 @@ int run_backward(Pipeline& pl, const sr_surfels* g, const int* radii, const floa
     ba.q_order = (const uint32_t*)(pl.img + pl.il.q_order);
     ba.ps = pair_store(pl.bin, pl.bl);
     ba.q_flag = (const uint32_t*)(pl.img + pl.il.q_flag);
-    ba.work = (const uint2*)(pl.bin + pl.bl.work);
+    ba.work = (const uint4*)(pl.bin + pl.bl.work);
     ba.work_count = pl.counters() + 2;
     ba.rec = (const float4*)(pl.geom + pl.gl.rec);
     ba.bg = pl.bg;

@@ -40,14 +40,13 @@ constexpr unsigned kChainBlocks = 16384;  // workgroups of the chain pass at mos
 constexpr int kGradGroup = SR_GRAD_GROUP;
 static_assert(kGradGroup >= 1 && 64 % kGradGroup == 0, "groups tile the 64 pixels");
 
-// Stores the 18 partial sums (g(k) for slot k) of the sub-list entry at
-// tile-list position pos of quadrant q as five float4 in its slot.  Every
+// Stores the 18 partial sums (g(k) for sum k) of a sub-list entry as five
+// float4 in its slot.  Every
 // entry of every sub-list sets its flag exactly once per backward and
 // stores its sums when any is non-zero, so neither buffer needs clearing.
 // (also: some pixel has a semantic gradient for the slot, _part variant).
 template <class G>
-SR_DEV void store_part(const BlendBwdArgs& a, uint32_t pos, int q, G g, bool also = false) {
-  const size_t slot = slot_of(a.pos_slot, a.pos_quads, pos, q);
+SR_DEV void store_part(const BlendBwdArgs& a, size_t slot, G g, bool also = false) {
   bool nz = also;
 #pragma unroll
   for (int k = 0; k < 18; ++k) nz |= g(k) != 0.0f;
@@ -695,6 +694,8 @@ SR_DEV uint64_t wave_transpose64(uint64_t x, int lane) {
 // entry's sums go to its (position, quadrant) slot of the partial-gradient
 // buffer.  The recompute path of pass 1 groups its sums the same way, so
 // the partials have the same bits whichever quadrants missed the pair store.
+// 91 us for 300k surfels at 800 x 600, 53 of them issuing (57 % of the lanes at
+// work: the last group of an entry is rarely full).
 // kSem: the _part variant's semantic channels, rounded up (0: none), whose
 // gradients w dL/dsem are summed the same way into sem_part.
 template <bool kPart, int kSem>
@@ -706,47 +707,39 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
   __shared__ float4 s_e0[64], s_e1[64], s_e2[64];  // per entry: record quads 0..2
   __shared__ unsigned long long s_col[64];         // per entry: the pixels that blended it
   __shared__ uint32_t s_tbase[64];                 // per entry: its first group
-  __shared__ uint8_t s_towner[64 * (64 / kGradGroup)];  // entry of every group
+  __shared__ uint32_t s_head[64];
   __shared__ float s_grp[kNumG + kSem][64];        // group sums of the round
   __shared__ float s_dls[kSem > 0 ? kSem : 1][64]; // per pixel: dL/dsem
-  const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   const int lane = threadIdx.x;
   if (a.counters[1] & kErrCapacity) return;
   const uint32_t nwork = *a.work_count;
+  const int lgQ = a.vs.B == 8 ? 0 : a.vs.B == 16 ? 2 : 4;  // quadrants of a tile
   for (uint32_t w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const uint2 item = a.work[nwork - 1u - w];  // from the end: see work_capacity
-    const int qi = (int)item.x, c = (int)item.y;
-    if (a.q_flag[qi] != 0u) continue;  // done by the staged path of pass 1
-    const int tile = qi / Q, q = qi % Q;
-    const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
-    const int lt = tile - (int)vi.tile_base;
-    const int tx = lt % vi.gx, ty = lt / vi.gx;
-    const int bx = tx * B + (q % QX) * kQuad, by = ty * B + (q / QX) * kQuad;
+    const WorkItem it = unpack_work(a.work[nwork - 1u - w]);  // from the end: see work_capacity
+    if (a.q_flag[it.qi] != 0u) continue;  // done by pass 1
+    const ViewInfo& vi = a.vs.v[it.view];
+    const int bx = it.x0, by = it.y0;
     // lane as pixel (lane & 7, lane >> 3) of the quadrant
-    const uint32_t pxi = (uint32_t)(bx + (lane & 7)), pyi = (uint32_t)(by + (lane >> 3));
-    const bool inside = pxi < (uint32_t)vi.W && pyi < (uint32_t)vi.H;
-    const uint32_t rbeg = a.ranges[2 * tile], ntile = a.ranges[2 * tile + 1] - rbeg;
-    const int cnt = (int)a.sub_count[qi];
-    const uint2* list = a.sub + (size_t)Q * rbeg + (size_t)q * ntile;
-    const size_t slot = mask_base(Q, rbeg, ntile, tile, q) + (size_t)c * 64 + lane;
-    const int e0 = c * 64;
-    const int m = min(64, cnt - e0);
-    uint64_t mask = inside ? a.masks[slot] : 0ull;
-    const uint32_t foff = mask ? a.frag_off[slot] : 0u;
+    const int pxi = bx + (lane & 7), pyi = by + (lane >> 3);
+    const bool inside = pxi < vi.W && pyi < vi.H;
+    const uint32_t rbeg = a.ranges[2 * (it.qi >> lgQ)];
+    const size_t mslot = it.first + 64u * (size_t)it.qi + lane;
+    uint64_t mask = inside ? a.masks[mslot] : 0ull;
+    const uint32_t foff = mask ? a.frag_off[mslot] : 0u;
+    const size_t HW = (size_t)vi.H * vi.W, pid = (size_t)vi.W * pyi + pxi, pb = vi.pix_base;
     uint32_t lc = 0u;
     float4 pg = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float2 pn = make_float2(0.0f, 0.0f);
     if (mask) {
-      const size_t HW = (size_t)vi.H * vi.W, pid = (size_t)vi.W * pyi + pxi, pb = vi.pix_base;
       lc = a.n_contrib[2 * pb + pid];
       const float* dL_dpix = a.dL_dpix + 3 * pb;
       const float* dL_dothers = a.dL_dothers + (kPart ? 8 : 7) * pb;
       pg = make_float4(dL_dpix[pid], dL_dpix[HW + pid], dL_dpix[2 * HW + pid], dL_dothers[2 * HW + pid]);
       pn = make_float2(dL_dothers[3 * HW + pid], dL_dothers[4 * HW + pid]);
     }
-    // lane as entry e0 + lane of the chunk
-    const bool has = lane < m;
-    const uint2 v = has ? list[e0 + lane] : make_uint2(0u, 0xFFFFFFFFu);
+    // lane as entry of the chunk
+    const bool has = (uint32_t)lane < it.m;
+    const uint2 v = has ? a.sub[it.first + lane] : make_uint2(0u, 0xFFFFFFFFu);
     float4 q0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), q1 = q0, q2 = q0;
     if (has) {
       const float4* r = a.rec + (size_t)kRecQuads * v.x;
@@ -754,18 +747,15 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
       q1 = r[1];
       q2 = r[2];
     }
-    __syncthreads();  // the previous item's readers are done
+    wave_lds_fence();  // the previous item's readers are done
     s_pos[lane] = v.y;
     s_e0[lane] = q0;
     s_e1[lane] = q1;
     s_e2[lane] = q2;
 #pragma unroll
-    for (int x = 0; x < kSem; ++x) {
-      const size_t HW = (size_t)vi.H * vi.W;
-      s_dls[x][lane] = mask && x < a.S
-                           ? a.dL_dsem[(size_t)a.S * vi.pix_base + x * HW + (size_t)vi.W * pyi + pxi] : 0.0f;
-    }
-    __syncthreads();
+    for (int x = 0; x < kSem; ++x)
+      s_dls[x][lane] = mask && x < a.S ? a.dL_dsem[(size_t)a.S * pb + x * HW + pid] : 0.0f;
+    wave_lds_fence();
     if (mask) {
       // entries in front of the last contributor: positions rise along the
       // chunk, so they are the first J, found by binary search
@@ -789,18 +779,18 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
     const uint32_t tbase = tincl - ng, ntask = (uint32_t)__shfl((int)tincl, 63, 64);
     s_col[lane] = col;
     s_tbase[lane] = tbase;
-    for (uint32_t i = 0; i < ng; ++i) s_towner[tbase + i] = (uint8_t)lane;
-    __syncthreads();
+    wave_lds_fence();
     float acc[kNumG + kSem];
 #pragma unroll
     for (int k = 0; k < kNumG + kSem; ++k) acc[k] = 0.0f;
+    SlotOwner owner;
     for (uint32_t base = 0; base < ntask; base += 64) {  // uniform
       const uint32_t t = base + (uint32_t)lane;
+      const int j = (int)owner.at(s_head, base, tbase, ng);
       float g[kNumG + kSem];
 #pragma unroll
       for (int k = 0; k < kNumG + kSem; ++k) g[k] = 0.0f;
       if (t < ntask) {
-        const int j = s_towner[t];
         const uint32_t gi = t - s_tbase[j];
         const uint64_t cj = s_col[j];
         // the group's pixels: the set bits of cj from the (gi kGradGroup)-th on
@@ -841,19 +831,20 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
       }
 #pragma unroll
       for (int k = 0; k < kNumG + kSem; ++k) s_grp[k][lane] = g[k];
-      __syncthreads();
+      wave_lds_fence();
       // the entry's lane adds its groups of this round, in order
       const uint32_t lo = max(tbase, base), hi = min(tbase + ng, base + 64u);
       for (uint32_t u = lo; u < hi; ++u) {
 #pragma unroll
         for (int k = 0; k < kNumG + kSem; ++k) acc[k] += s_grp[k][u - base];
       }
-      __syncthreads();
+      wave_lds_fence();
     }
     if (has) {
-      store_part(a, rbeg + v.y, q, [&](int k) { return acc[k]; }, kSem > 0 && ng > 0u);
+      const size_t slot = slot_of(a.pos_slot, a.pos_quads, rbeg + v.y, (int)(it.qi & ((1u << lgQ) - 1u)));
+      store_part(a, slot, [&](int k) { return acc[k]; }, kSem > 0 && ng > 0u);
       if (kSem > 0 && ng > 0u) {
-        float* d = a.sem_part + slot_of(a.pos_slot, a.pos_quads, rbeg + v.y, q) * (size_t)a.S;
+        float* d = a.sem_part + slot * (size_t)a.S;
 #pragma unroll
         for (int x = 0; x < kSem; ++x)
           if (x < a.S) d[x] = acc[kNumG + x];
@@ -864,7 +855,7 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
 
 hipError_t launch_blend_bwd_grad(const BlendBwdArgs& a, size_t max_items, hipStream_t s) {
   if (max_items == 0) return hipSuccess;
-  const unsigned grid = (unsigned)(max_items < 65536 ? max_items : 65536);
+  const unsigned grid = (unsigned)(max_items < kChunkBlocks ? max_items : kChunkBlocks);
   if (!a.is_part) hipLaunchKernelGGL((k_blend_bwd_grad<false, 0>), dim3(grid), dim3(64), 0, s, a);
   else if (a.S == 0) hipLaunchKernelGGL((k_blend_bwd_grad<true, 0>), dim3(grid), dim3(64), 0, s, a);
   else if (a.S <= 4) hipLaunchKernelGGL((k_blend_bwd_grad<true, 4>), dim3(grid), dim3(64), 0, s, a);

@@ -924,10 +924,18 @@ SR_DEV void append_work(const SortArgs& a, int tile, int Q, uint32_t cnt) {
   if (lane == 0 && all > 0) w0 = atomicAdd(a.work_count, all);
   w0 = (uint32_t)__shfl((int)w0, 0);
   if (has) {
-    a.sub_count[(size_t)tile * Q + lane] = cnt;
-    a.q_flag[(size_t)tile * Q + lane] = 0u;
+    const uint32_t qi = (uint32_t)(tile * Q + lane);
+    a.sub_count[qi] = cnt;
+    a.q_flag[qi] = 0u;
     const uint32_t first = w0 + incl - nch;
-    for (uint32_t ch = 0; ch < nch; ++ch) a.work[first + ch] = make_uint2((uint32_t)(tile * Q + lane), ch);
+    const int B = a.vs.B, QX = B / kQuad;
+    const uint32_t view = (uint32_t)view_of_tile(a.vs, (uint32_t)tile);
+    const int lt = tile - (int)a.vs.v[view].tile_base, gx = a.vs.v[view].gx;
+    const int x0 = lt % gx * B + lane % QX * kQuad, y0 = lt / gx * B + lane / QX * kQuad;
+    const uint32_t beg = a.ranges[2 * tile], n = a.ranges[2 * tile + 1] - beg;
+    const size_t e0 = (size_t)Q * beg + (size_t)lane * n;
+    for (uint32_t ch = 0; ch < nch; ++ch)
+      a.work[first + ch] = pack_work(qi, e0 + 64u * ch, min(64u, cnt - 64u * ch), view, x0, y0);
   }
 }
 
@@ -1493,50 +1501,43 @@ hipError_t launch_sort_tiles(const SortArgs& a, size_t max_segments, hipStream_t
 // bit j of pixel p's mask is set when entry j of the chunk reaches
 // alpha >= 1/255 at p.  Only pixels inside an entry's cull box can (the box
 // holds every such pixel), so the wave evaluates exactly the (entry, pixel)
-// pairs of the boxes clipped to the quadrant, 64 pairs per step: an LDS
-// table names the entry of every pair slot, and the slot's offset in the
+// pairs of the boxes clipped to the quadrant, 64 pairs per step: SlotOwner
+// names the entry of every pair slot, and the slot's offset in the
 // entry's box gives the pixel.  The bits go to per-pixel masks in LDS; each
-// accepted pair adds log2(1 - alpha) to its pixel's sum, from which the
-// chunk's transmittance follows.  That transmittance is only compared
-// against half the saturation threshold (a margin of a factor 2 against its
-// rounding, whatever the summation order), so the order in which the lanes
-// add is free.  The chunks of all quadrants are independent, so this, the
+// accepted pair adds -log2(1 - alpha) in 2^-20 to its pixel's sum, from which
+// the chunk's transmittance follows.  That transmittance is only compared
+// against half the saturation threshold, a margin of a factor 2 against its
+// rounding.  LDS atomics bound the pass where they are wide or on floats: with
+// a 64-bit or and a float add a pair it took 77 us (299 for 1M surfels at
+// 1237 x 823), with two 32-bit integer ones 60 (212); with a byte per pair slot
+// naming its entry, whose 4 KB left room for half the waves, 80 (338).  The chunks of all quadrants are independent, so this, the
 // bulk of the pair evaluations, runs balanced over the whole GPU; the blend
 // kernels then visit only accepted pairs.
 // ---------------------------------------------------------------------------
+constexpr float kLogUnit = 1048576.0f;  // 64 pairs of alpha <= 0.99 sum to less than 2^29 of it
 template <bool kPart>
 __global__ __launch_bounds__(64) void k_accept(AcceptArgs a) {
   __shared__ float4 s_q0[64], s_q1[64], s_q2[64];
   __shared__ float s_rej[64];
   __shared__ uint32_t s_start[64];  // running box area before entry j
   __shared__ uint32_t s_geo[64];    // entry j's clipped box: x0 | y0 << 4 | w << 8
-  __shared__ unsigned long long s_mask[64];
-  __shared__ float s_logT[64];          // per pixel: sum of log2(1 - alpha) over its accepted pairs
-  __shared__ uint8_t s_owner[64 * 64];  // entry of every pair slot
+  __shared__ uint32_t s_mask[2][64];  // per pixel: entries 0..31 and 32..63
+  __shared__ uint32_t s_logT[64];   // per pixel: sum of -log2(1 - alpha) over its accepted pairs, in 2^-20
+  __shared__ uint32_t s_head[64];
   // r / w for r < 64 and 1 <= w <= 8 as (r * kDiv[w]) >> 9
   constexpr uint32_t kDiv[9] = {0u, 512u, 256u, 171u, 128u, 103u, 86u, 74u, 64u};
-  const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   const int lane = threadIdx.x;
   if (a.counters[1] & kErrCapacity) return;
   const uint32_t nwork = *a.work_count;
   for (uint32_t w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const uint2 item = a.work[nwork - 1u - w];  // from the end: see work_capacity
-    const int qi = (int)item.x, c = (int)item.y;
-    const int tile = qi / Q, q = qi % Q;
-    const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
-    const int lt = tile - (int)vi.tile_base;
-    const int tx = lt % vi.gx, ty = lt / vi.gx;
-    const int qx0 = tx * B + (q % QX) * kQuad, qy0 = ty * B + (q / QX) * kQuad;
+    const WorkItem it = unpack_work(a.work[nwork - 1u - w]);  // from the end: see work_capacity
+    const ViewInfo& vi = a.vs.v[it.view];
+    const int qx0 = it.x0, qy0 = it.y0;
     const int qw = min(kQuad, vi.W - qx0), qh = min(kQuad, vi.H - qy0);  // pixels inside the image
-    const uint32_t rbeg = a.ranges[2 * tile], ntile = a.ranges[2 * tile + 1] - rbeg;
-    const int cnt = (int)a.sub_count[qi];
-    const uint2* list = a.sub + (size_t)Q * rbeg + (size_t)q * ntile;
-    const int e0 = c * 64;
-    const int m = min(64, cnt - e0);
-    __syncthreads();  // the previous item's readers are done
+    wave_lds_fence();  // the previous item's readers are done
     uint32_t area = 0, geo = 0;
-    if (lane < m) {
-      const uint32_t rid = list[e0 + lane].x;
+    if ((uint32_t)lane < it.m) {
+      const uint32_t rid = a.sub[it.first + lane].x;
       const float4* r = a.rec + (size_t)kRecQuads * rid;
       s_q0[lane] = r[0];
       s_q1[lane] = r[1];
@@ -1561,14 +1562,14 @@ __global__ __launch_bounds__(64) void k_accept(AcceptArgs a) {
     const uint32_t first = incl - area;
     s_start[lane] = first;
     s_geo[lane] = geo;
-    for (uint32_t i = 0; i < area; ++i) s_owner[first + i] = (uint8_t)lane;
-    s_mask[lane] = 0ull;
-    s_logT[lane] = 0.0f;
-    __syncthreads();
+    s_mask[0][lane] = s_mask[1][lane] = 0u;
+    s_logT[lane] = 0u;
+    wave_lds_fence();
+    SlotOwner owner;
     for (uint32_t base = 0; base < total; base += 64) {
       const uint32_t t = base + (uint32_t)lane;
+      const int j = (int)owner.at(s_head, base, first, area);
       if (t < total) {
-        const int j = s_owner[t];
         const uint32_t g = s_geo[j];
         const uint32_t r = t - s_start[j], bw = (g >> 8) & 15u;
         const uint32_t dy = (r * kDiv[bw]) >> 9, dx = r - dy * bw;
@@ -1577,21 +1578,21 @@ __global__ __launch_bounds__(64) void k_accept(AcceptArgs a) {
         if (eval_pair<true>(pixel_centre<kPart>(qx0 + lx), pixel_centre<kPart>(qy0 + ly), s_q0[j], s_q1[j], s_q2[j],
                             s_rej[j], e)) {
           const int p = ly * kQuad + lx;
-          atomicOr(&s_mask[p], 1ull << j);
-          atomicAdd(&s_logT[p], __log2f(1.0f - e.alpha));
+          atomicOr(&s_mask[j >> 5][p], 1u << (j & 31));
+          atomicAdd(&s_logT[p], (uint32_t)(__log2f(1.0f - e.alpha) * -kLogUnit));
         }
       }
     }
-    __syncthreads();
-    const size_t slot = mask_base(Q, rbeg, ntile, tile, q) + (size_t)e0 + lane;
-    a.masks[slot] = s_mask[lane];
-    a.chunk_T[slot] = exp2f(s_logT[lane]);
+    wave_lds_fence();
+    const size_t slot = it.first + 64u * (size_t)it.qi + lane;
+    a.masks[slot] = (uint64_t)s_mask[1][lane] << 32 | s_mask[0][lane];
+    a.chunk_T[slot] = exp2f((float)s_logT[lane] * (-1.0f / kLogUnit));
   }
 }
 
 hipError_t launch_accept(const AcceptArgs& a, size_t max_items, hipStream_t s) {
   if (max_items == 0) return hipSuccess;
-  const unsigned grid = (unsigned)(max_items < 65536 ? max_items : 65536);
+  const unsigned grid = (unsigned)(max_items < kChunkBlocks ? max_items : kChunkBlocks);
   if (a.part) hipLaunchKernelGGL(k_accept<true>, dim3(grid), dim3(64), 0, s, a);
   else hipLaunchKernelGGL(k_accept<false>, dim3(grid), dim3(64), 0, s, a);
   return hipGetLastError();
@@ -1864,39 +1865,29 @@ hipError_t launch_pair_offsets(const AcceptArgs& a, hipStream_t s) {
 
 // Pair-store fill: balanced like the acceptance pass, one wave per
 // (quadrant, chunk).  The chunk's accepted pairs are dealt out 64 per step
-// in pixel order (an LDS table names the pixel of every pair slot; the
+// in pixel order (SlotOwner names the pixel of every pair slot; the
 // slot's rank among the pixel's pairs picks the entry from the pixel's mask
 // bits), so consecutive lanes write consecutive records of a pixel's run.
 // Each lane recomputes its pair and stores the entry data the blend chains
-// need.
+// need.  Bound by its 48 bytes a pair: 232 MB written and 71 read in 79 us for
+// 300k surfels at 800 x 600 (3.8 TB/s; a large copy reaches 4.8).
 template <bool kPart>
 __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
   __shared__ float4 s_q0[64], s_q1[64], s_q2[64], s_q3[64], s_q4[64];
   __shared__ uint32_t s_pos[64];
   __shared__ unsigned long long s_mask[64];
   __shared__ uint32_t s_start[64], s_foff[64];
-  __shared__ uint8_t s_owner[64 * 64];  // pixel of every pair slot
+  __shared__ uint32_t s_head[64];
   __shared__ uint32_t s_rid[kPart ? 64 : 1];
-  const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   const int lane = threadIdx.x;
   if (a.counters[1] & kErrCapacity) return;
   const uint32_t nwork = *a.work_count;
   for (uint32_t w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const uint2 item = a.work[nwork - 1u - w];  // from the end: see work_capacity
-    const int qi = (int)item.x, c = (int)item.y;
-    if (a.q_flag[qi] != 0u) continue;
-    const int tile = qi / Q, q = qi % Q;
-    const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
-    const int lt = tile - (int)vi.tile_base;
-    const int tx = lt % vi.gx, ty = lt / vi.gx;
-    const int qx0 = tx * B + (q % QX) * kQuad, qy0 = ty * B + (q / QX) * kQuad;
-    const uint32_t rbeg = a.ranges[2 * tile], ntile = a.ranges[2 * tile + 1] - rbeg;
-    const int cnt = (int)a.sub_count[qi];
-    const uint2* list = a.sub + (size_t)Q * rbeg + (size_t)q * ntile;
-    const int e0 = c * 64;
-    const int m = min(64, cnt - e0);
+    const WorkItem it = unpack_work(a.work[nwork - 1u - w]);  // from the end: see work_capacity
+    if (a.q_flag[it.qi] != 0u) continue;
+    const int qx0 = it.x0, qy0 = it.y0;
     // lane as pixel: its accepted pairs of the chunk and where they go
-    const size_t slot = mask_base(Q, rbeg, ntile, tile, q) + (size_t)e0 + lane;
+    const size_t slot = it.first + 64u * (size_t)it.qi + lane;
     const uint64_t mm = a.masks[slot];
     const uint32_t foff = mm ? a.frag_off[slot] : 0u;
     const uint32_t n = (uint32_t)__popcll(mm);
@@ -1908,14 +1899,13 @@ __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
     }
     const uint32_t total = (uint32_t)__shfl((int)incl, 63, 64);
     if (total == 0u) continue;  // uniform across the wave
-    __syncthreads();  // the previous item's readers are done
+    wave_lds_fence();  // the previous item's readers are done
     const uint32_t first = incl - n;
     s_mask[lane] = mm;
     s_start[lane] = first;
     s_foff[lane] = foff;
-    for (uint32_t i = 0; i < n; ++i) s_owner[first + i] = (uint8_t)lane;
-    if (lane < m) {
-      const uint2 v = list[e0 + lane];
+    if ((uint32_t)lane < it.m) {
+      const uint2 v = a.sub[it.first + lane];
       const float4* rc = a.rec + (size_t)kRecQuads * v.x;
       s_q0[lane] = rc[0];
       s_q1[lane] = rc[1];
@@ -1925,11 +1915,12 @@ __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
       s_pos[lane] = v.y;
       if (kPart) s_rid[lane] = v.x;
     }
-    __syncthreads();
+    wave_lds_fence();
+    SlotOwner owner;
     for (uint32_t base = 0; base < total; base += 64) {
       const uint32_t t = base + (uint32_t)lane;
+      const int p = (int)owner.at(s_head, base, first, n);
       if (t >= total) continue;
-      const int p = s_owner[t];
       const uint32_t k = t - s_start[p];
       const int j = select_bit(s_mask[p], k);
       Pair e;
@@ -1948,7 +1939,7 @@ __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
 
 hipError_t launch_pair_write(const AcceptArgs& a, size_t max_items, hipStream_t s) {
   if (max_items == 0) return hipSuccess;
-  const unsigned grid = (unsigned)(max_items < 65536 ? max_items : 65536);
+  const unsigned grid = (unsigned)(max_items < kChunkBlocks ? max_items : kChunkBlocks);
   if (a.part) hipLaunchKernelGGL(k_pair_write<true>, dim3(grid), dim3(64), 0, s, a);
   else hipLaunchKernelGGL(k_pair_write<false>, dim3(grid), dim3(64), 0, s, a);
   return hipGetLastError();

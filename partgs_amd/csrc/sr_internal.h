@@ -2,6 +2,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -208,6 +210,70 @@ __host__ __device__ inline size_t mask_base(int Q, uint32_t beg, uint32_t n, int
 // large tiles (appended last, by the sorts of the large tiles)
 // start first (measured: 4 us less per 300k-surfel 800x600 step, in the
 // passes that follow).
+// An item holds what its kernels would otherwise derive with divisions and
+// dependent loads: the quadrant, the chunk's first entry in the sub-list space
+// (40 bits), its entries (1 to 64), the view, and the quadrant's first pixel.
+struct WorkItem {
+  uint32_t qi, m, view;
+  int x0, y0;
+  size_t first;  // the chunk's masks start at first + 64 qi
+};
+__device__ inline uint4 pack_work(uint32_t qi, size_t first, uint32_t m, uint32_t view, int x0, int y0) {
+  return make_uint4(qi, (uint32_t)first, (uint32_t)x0 | (uint32_t)y0 << 16,
+                    view | (m - 1u) << 5 | (uint32_t)(first >> 32) << 11);
+}
+static_assert(kMaxViews <= 32 && kQuad * kQuad == 64, "work item fields");
+// The item, the same value in every lane.
+__device__ inline WorkItem unpack_work(uint4 p) {
+  const uint32_t x = __builtin_amdgcn_readfirstlane(p.x), y = __builtin_amdgcn_readfirstlane(p.y);
+  const uint32_t z = __builtin_amdgcn_readfirstlane(p.z), v = __builtin_amdgcn_readfirstlane(p.w);
+  WorkItem i;
+  i.qi = x;
+  i.m = (v >> 5 & 63u) + 1u;
+  i.view = v & 31u;
+  i.x0 = (int)(z & 0xFFFFu);
+  i.y0 = (int)(z >> 16);
+  i.first = (size_t)(v >> 11) << 32 | y;
+  return i;
+}
+// Owners of slots dealt out 64 a step: owner k has `n` consecutive slots from
+// `start` on, k rising with start, each lane holding one owner.  Step `base`
+// names the owner of slot base + lane (if there is one): the owners whose first
+// slot lies in the step mark it in head (64 words of LDS), and a running maximum
+// over the lanes, from the last step's owner, fills the gaps.
+struct SlotOwner {
+  uint32_t carry = 0u;  // 1 + the owner of the last slot of the step before
+  __device__ inline uint32_t at(uint32_t* head, uint32_t base, uint32_t start, uint32_t n);
+};
+// Orders a single-wave workgroup's LDS accesses.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+constexpr unsigned kChunkBlocks = 65536;  // workgroups that share the work items
+__device__ inline uint32_t SlotOwner::at(uint32_t* head, uint32_t base, uint32_t start, uint32_t n) {
+  const uint32_t lane = threadIdx.x & 63u;
+  head[lane] = 0u;
+  wave_lds_fence();
+  if (n > 0u && start >= base && start < base + 64u) head[start - base] = lane + 1u;
+  wave_lds_fence();
+  uint32_t x = head[lane];
+  wave_lds_fence();
+  auto up = [&](auto ctrl, auto rows) {  // maximum with the lane `ctrl` brings
+    const int y = __builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    x = x > (uint32_t)y ? x : (uint32_t)y;
+  };
+  using std::integral_constant;
+  up(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // within rows of 16 lanes: from 1,
+  up(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});  // 2,
+  up(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});  // 4 and
+  up(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});  // 8 lanes below
+  up(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row 0's last lane to row 1, 2's to 3
+  up(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // lane 31 to rows 2 and 3
+  x = x > carry ? x : carry;
+  carry = (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+  return x - 1u;
+}
 inline size_t work_capacity(int L, int B, int T) {
   const size_t Q = (size_t)quads_per_tile(B);
   return Q * ((size_t)T + ((size_t)(L > 0 ? L : 1) + 63) / 64);
@@ -237,7 +303,7 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
   b.masks = off; off += align_up((n * Q + (size_t)kQuad * kQuad * Q * (size_t)T) * 8);
   const size_t nslots = n * Q + (size_t)kQuad * kQuad * Q * (size_t)T;
   b.chunk_T = off; off += align_up(nslots * 4);  // per mask slot: product of (1 - alpha) over its pairs
-  b.work = off; off += align_up(work_capacity(L, B, T) * 8);
+  b.work = off; off += align_up(work_capacity(L, B, T) * 16);
   b.frag_off = off; off += align_up(nslots * 4);
   b.pay = off; off += align_up(n * 8);
   b.pay2 = off; off += align_up(n * 8);
@@ -336,7 +402,7 @@ struct SortArgs {
   uint16_t* pos_quads;
   uint2* sub;
   uint32_t* sub_count;
-  uint2* work;          // (quadrant index, chunk) items for the acceptance pass
+  uint4* work;          // (quadrant index, chunk) items for the acceptance pass
   uint32_t* work_count;
   uint32_t* q_flag;
 };
@@ -349,7 +415,7 @@ struct AcceptArgs {
   const uint32_t* sub_count;
   const float4* rec;
   const short4* cullbox;  // per record: inclusive pixel box holding every pixel with alpha >= 1/255
-  const uint2* work;
+  const uint4* work;
   const uint32_t* work_count;
   uint64_t* masks;
   float* chunk_T;
@@ -404,7 +470,7 @@ struct BlendBwdArgs {
   const uint32_t* q_order;
   PairStore ps;
   const uint32_t* q_flag;
-  const uint2* work;  // (quadrant, chunk) items of the acceptance pass
+  const uint4* work;  // (quadrant, chunk) items of the acceptance pass
   const uint32_t* work_count;
   const float4* rec;
   const float* bg;
