@@ -200,7 +200,7 @@ struct Pipeline {
 
 PairStore pair_store(char* bin, const BinLayout& bl) {
   PairStore p{};
-  p.rec = (float4*)(bin + bl.prec);
+  p.rec = bin + bl.prec;
   p.fW = (float4*)(bin + bl.fW);
   return p;
 }
@@ -714,7 +714,7 @@ int forward_view(const sr_settings* s, const sr_surfels* g, bool part, int S, co
     // exceed it.  The scan writes the instance count back and it is waited
     // for only once the rest is enqueued, by when it has long arrived, so
     // the stream never drains mid-forward.
-    pl.bl = bin_layout(cap, B, il.T, s->pair_store, s->pair_capacity, S, s->slot_capacity);
+    pl.bl = bin_layout(cap, B, il.T, s->pair_store, s->pair_capacity, S, s->slot_capacity, part);
     pl.bin = (char*)alloc(ctx, pl.bl.total, 1);
     if (!pl.bin) return fail(SR_ERR_ALLOC, "allocation callback failed");
     pl.capacity = cap;
@@ -747,7 +747,7 @@ int forward_view(const sr_settings* s, const sr_surfels* g, bool part, int S, co
   // the slots the forward needs, exactly (the slot region is the layout's
   // last, so the backward locates everything without this count)
   const int slots = (int)(host[8] > 0u ? host[8] : 1u);
-  pl.bl = bin_layout(L, B, il.T, s->pair_store, s->pair_capacity, S, slots);
+  pl.bl = bin_layout(L, B, il.T, s->pair_store, s->pair_capacity, S, slots, part);
   pl.bin = (char*)alloc(ctx, pl.bl.total, 1);
   if (!pl.bin) return fail(SR_ERR_ALLOC, "allocation callback failed");
   pl.capacity = L;
@@ -803,7 +803,7 @@ int backward_view(const sr_settings* s, const sr_surfels* g, bool part, int S, i
   // the binning arrays are laid out for the forward's capacity (R when 0)
   const int cap = s->capacity > 0 ? s->capacity : R;
   if (cap < R) return fail(SR_ERR_INVALID, "capacity %d below num_rendered %d", s->capacity, R);
-  pl.bl = bin_layout(cap, B, pl.il.T, s->pair_store, s->pair_capacity, S);
+  pl.bl = bin_layout(cap, B, pl.il.T, s->pair_store, s->pair_capacity, S, 0, part);
   pl.geom = (char*)geom_buf;
   pl.img = (char*)img_buf;
   pl.bin = (char*)bin_buf;

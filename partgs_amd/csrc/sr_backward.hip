@@ -27,9 +27,17 @@ namespace sr {
 // Partial-gradient slots: 0..8 dL_dtransMat, 9..10 dL_dmean2D.xy,
 // 11..13 dL_dnormal, 14 dL_dopacity, 15..17 dL_dcolors.
 constexpr int kNumG = 18;
-constexpr int kChainPre = 4;  // pairs of a batch in the chain pass: three 64-byte pieces
+constexpr int kChainPre = 4;  // pairs of a batch in the chain pass
 using V4 = float __attribute__((ext_vector_type(4)));  // a float4 the compiler keeps in registers as a whole
-constexpr int kOwnerQuads = 3 * 64 + 1;  // LDS quads of one quad lane's batches, the odd one against bank conflicts
+using V2 = float __attribute__((ext_vector_type(2)));
+template <class T> SR_DEV T load8(const char* p) {  // from an 8-byte aligned place
+  T v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(p, 8), sizeof(T));
+  return v;
+}
+// LDS bytes from one lane's batch to the next: 16 more than its pairs, so that
+// neither the quads' pieces nor the lanes' own reads share banks
+template <bool kPart> constexpr int kOwnerBytes = kChainPre * PairLayout<kPart>::kBytes + 16;
 constexpr unsigned kChainBlocks = 16384;  // workgroups of the chain pass at most
 #ifndef SR_GRAD_GROUP
 #define SR_GRAD_GROUP 4
@@ -304,14 +312,15 @@ SR_DEV void pair_grads(float dLp0, float dLp1, float dLp2, float dLn0, float dLn
 // chain of a run of n pairs is two passes over n / 16 pairs instead of one over
 // n.  A wave gives its pixels as many lanes each as the quadrant's longest run
 // can have segments (1 to 16, by its cost's class), and a quadrant takes as
-// many waves.  300k surfels at 800 x 600: 98 us and at 400 x 300 49; with 8
-// lanes a pixel in every quadrant and each lane loading its own records 130
-// and 72; with the lanes by class but their own records still 130 and 66.  It
-// moves 316 MB (2.9 TB/s) and issues on 45 % of the cycles.
+// many waves.  300k surfels at 800 x 600: 89 us and at 400 x 300 48 (98 and 49
+// with 48-byte records); with 8 lanes a pixel in every quadrant and each lane
+// loading its own records 130 and 72; with the lanes by class but their own
+// records still 130 and 66.
 template <bool kPart>
 SR_DEV void blend_bwd_stored(const BlendBwdArgs& a, int qi, int lg, int part, float4* s_buf) {
   // s_buf: a batch of every lane's pairs; between the walks the SegMaps
   float* s_map = reinterpret_cast<float*>(s_buf);
+  constexpr int kBytes = PairLayout<kPart>::kBytes;
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   const int tile = qi / Q, q = qi % Q;
   const ViewInfo& vi = a.vs.v[view_of_tile(a.vs, (uint32_t)tile)];
@@ -333,19 +342,18 @@ SR_DEV void blend_bwd_stored(const BlendBwdArgs& a, int qi, int lg, int part, fl
   // alpha and values of the pair behind the segment (none behind the last)
   float la = 0.0f, l[7] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   if (sg < nseg - 1) {
-    const float4* pr = a.ps.rec + kPairQuads * (size_t)(rg.x + (uint32_t)(hi + 1));
-    const float4 e0 = pr[0], e1 = pr[1], e2 = pr[2];
-    la = e0.w;
-    l[0] = e1.w;
-    l[1] = e2.x;
-    l[2] = e2.y;
-    l[3] = e0.x;
-    l[4] = e1.x;
-    l[5] = e1.y;
-    l[6] = e1.z;
+    const float* pr = reinterpret_cast<const float*>(a.ps.rec + (size_t)kBytes * (rg.x + (uint32_t)(hi + 1)));
+    la = pr[2];
+    l[0] = pr[4];
+    l[1] = pr[5];
+    l[2] = pr[6];
+    l[3] = pr[3];
+    l[4] = pr[7];
+    l[5] = pr[8];
+    l[6] = pr[9];
   }
   // Walks lane segments [lo, hi] (hi < lo: none) from the back, calling
-  // fn(p0, p1, p2) for each pair; the whole wave calls it.  A lane streaming
+  // fn(depth, m, alpha, position, (normal, red), green, blue) for each pair; the whole wave calls it.  A lane streaming
   // its own records would touch a cache line of its own per load, and it is
   // the line rate that bounds the pass: so the four lanes of a quad load the
   // four lanes' batches together, 64 contiguous bytes at a time, and the
@@ -353,6 +361,7 @@ SR_DEV void blend_bwd_stored(const BlendBwdArgs& a, int qi, int lg, int part, fl
   // up to kChainPre - 1 records in front of lo are read (nothing uses them;
   // the store is padded).  With kOut, fn's results go to fW the same way.
   const int ql = lane & 3, qd = lane >> 2;  // place in the quad, quad
+  char* mine_at = reinterpret_cast<char*>(s_buf) + lane * kOwnerBytes<kPart>;
   auto walk = [&](auto out, int lo, int hi, auto&& fn) {
     constexpr bool kOut = decltype(out)::value;
     int left[4];     // pairs left of each of the quad's lanes
@@ -363,22 +372,30 @@ SR_DEV void blend_bwd_stored(const BlendBwdArgs& a, int qi, int lg, int part, fl
       at[o] = (uint32_t)__shfl((int)(rg.x + (uint32_t)hi), qd * 4 + o) - (kChainPre - 1);
     }
     int mine = hi - lo + 1;
-    V4 g[4][3] = {};
+    // of each lane's batch: 16 bytes at 16 ql and 64 more, then the rest of
+    // the four records, 8 or 16 bytes a lane
+    using Rest = std::conditional_t<kPart, V4, V2>;
+    V4 g[4][2] = {};
+    Rest g2[4] = {};
     auto fetch = [&]() {
 #pragma unroll
       for (int o = 0; o < 4; ++o) {
         if (left[o] <= 0) continue;
-        const V4* pr = reinterpret_cast<const V4*>(a.ps.rec + (ptrdiff_t)kPairQuads * (int32_t)at[o] + ql);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) g[o][c] = pr[4 * c];
+        const char* pr = a.ps.rec + (ptrdiff_t)kBytes * (int32_t)at[o];
+        g[o][0] = load8<V4>(pr + 16 * ql);
+        g[o][1] = load8<V4>(pr + 64 + 16 * ql);
+        g2[o] = load8<Rest>(pr + 128 + (int)sizeof(Rest) * ql);
       }
     };
     fetch();
     while (__ballot(mine > 0) != 0ull) {
 #pragma unroll
-      for (int o = 0; o < 4; ++o)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) reinterpret_cast<V4*>(s_buf)[o * kOwnerQuads + c * 64 + lane] = g[o][c];
+      for (int o = 0; o < 4; ++o) {
+        char* d = reinterpret_cast<char*>(s_buf) + (qd * 4 + o) * kOwnerBytes<kPart>;
+        *reinterpret_cast<V4*>(d + 16 * ql) = g[o][0];
+        *reinterpret_cast<V4*>(d + 64 + 16 * ql) = g[o][1];
+        *reinterpret_cast<Rest*>(d + 128 + (int)sizeof(Rest) * ql) = g2[o];
+      }
       uint32_t was[4];
       int had[4];
 #pragma unroll
@@ -390,13 +407,17 @@ SR_DEV void blend_bwd_stored(const BlendBwdArgs& a, int qi, int lg, int part, fl
       }
       fetch();  // in flight while this batch is used
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      const float4* b = s_buf + ql * kOwnerQuads + qd * 4;
-      auto quad = [&](int w) { return b[(w >> 2) * 64 + (w & 3)]; };
       float4 r[kChainPre];
 #pragma unroll
       for (int k = kChainPre - 1; k >= 0; --k) {
         r[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (kChainPre - 1 - k < mine) r[k] = fn(quad(3 * k), quad(3 * k + 1), quad(3 * k + 2));
+        if (kChainPre - 1 - k < mine) {
+          const char* p = mine_at + kBytes * k;
+          const V4 p0 = load8<V4>(p), p1 = load8<V4>(p + 16);
+          const V2 p2 = load8<V2>(p + 32);
+          const uint32_t pos = kPart ? *reinterpret_cast<const uint32_t*>(p + 40) : __float_as_uint(p0.y);
+          r[k] = fn(p0.w, p0.x, p0.z, pos, make_float4(p1.w, p2.x, p2.y, p1.x), p1.y, p1.z);
+        }
       }
       mine -= kChainPre;
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -419,17 +440,18 @@ SR_DEV void blend_bwd_stored(const BlendBwdArgs& a, int qi, int lg, int part, fl
     float pa = la, pl[7];
 #pragma unroll
     for (int x = 0; x < 7; ++x) pl[x] = l[x];
-    walk(std::false_type{}, lo, mapped ? hi : lo - 1, [&](const float4& c0, const float4& c1, const float4& c2) {
-      m.add<kPart>(px, pa, pl, c0.w, c0.y, kPart ? c0.y * c0.y : c0.z, __float_as_uint(c2.z));
-      pa = c0.w;
-      pl[0] = c1.w;
-      pl[1] = c2.x;
-      pl[2] = c2.y;
-      pl[3] = c0.x;
-      pl[4] = c1.x;
-      pl[5] = c1.y;
-      pl[6] = c1.z;
-      return c0;
+    walk(std::false_type{}, lo, mapped ? hi : lo - 1,
+         [&](float depth, float m_d, float alpha, uint32_t pos, const float4& nr, float g, float b) {
+      m.add<kPart>(px, pa, pl, alpha, m_d, m_d * m_d, pos);
+      pa = alpha;
+      pl[0] = nr.w;
+      pl[1] = g;
+      pl[2] = b;
+      pl[3] = depth;
+      pl[4] = nr.x;
+      pl[5] = nr.y;
+      pl[6] = nr.z;
+      return nr;
     });
     __syncthreads();
     if (mapped) m.save(s_map + lane);
@@ -451,9 +473,9 @@ SR_DEV void blend_bwd_stored(const BlendBwdArgs& a, int qi, int lg, int part, fl
   ch.last_n0 = l[4];
   ch.last_n1 = l[5];
   ch.last_n2 = l[6];
-  walk(std::true_type{}, lo, hi, [&](const float4& c0, const float4& c1, const float4& c2) {
-    return ch.step<kPart>(px, c0.w, c0.x, c0.y, kPart ? c0.y * c0.y : c0.z, c2.w, __float_as_uint(c2.z), c1, c2.x,
-                          c2.y);
+  walk(std::true_type{}, lo, hi, [&](float depth, float m_d, float alpha, uint32_t pos, const float4& nr, float g,
+                                     float b) {
+    return ch.step<kPart>(px, alpha, depth, m_d, m_d * m_d, dist_weight_grad<kPart>(depth), pos, nr, g, b);
   });
 }
 
@@ -466,7 +488,8 @@ SR_DEV void blend_bwd_missed(const BlendBwdArgs& a, int qi, float4* s_buf) {
   float4 *s_q0 = s_buf, *s_q1 = s_buf + 64, *s_q2 = s_buf + 128, *s_q3 = s_buf + 192, *s_q4 = s_buf + 256;
   uint2* s_e = reinterpret_cast<uint2*>(s_buf + 320);
   float(*s_tmp)[65] = reinterpret_cast<float(*)[65]>(s_buf + 352);
-  static_assert(4 * kOwnerQuads * 16 >= 352 * 16 + kNumG * 65 * 4 && kNumG >= kMaxSem, "fits the other path's LDS");
+  static_assert(64 * kOwnerBytes<kPart> >= 352 * 16 + kNumG * 65 * 4 && kNumG >= kMaxSem,
+                "fits the other path's LDS");
   const int cnt = (int)a.sub_count[qi];
   const int B = a.vs.B, QX = B / kQuad, Q = QX * QX;
   const int tile = qi / Q, q = qi % Q;
@@ -619,8 +642,9 @@ SR_DEV void blend_bwd_missed(const BlendBwdArgs& a, int qi, float4* s_buf) {
 // item w is a wave of the first class with w left.
 template <bool kPart>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_blend_bwd(BlendBwdArgs a) {
-  __shared__ float4 s_buf[4 * kOwnerQuads];
-  static_assert(sizeof(s_buf) >= kSegMapFloats * 64 * sizeof(float), "one map a lane");
+  __shared__ float4 s_buf[64 * kOwnerBytes<kPart> / 16];
+  static_assert(sizeof(s_buf) >= kSegMapFloats * 64 * sizeof(float) && sizeof(s_buf) >= 64 * kChainPre * 16,
+                "one map, or one batch of results, a lane");
   if (a.counters[1] & kErrCapacity) return;
   const uint32_t* end = a.counters + kCostClass;  // of the classes, in quadrants
   uint32_t items = 0;

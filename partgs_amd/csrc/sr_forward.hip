@@ -1869,8 +1869,9 @@ hipError_t launch_pair_offsets(const AcceptArgs& a, hipStream_t s) {
 // slot's rank among the pixel's pairs picks the entry from the pixel's mask
 // bits), so consecutive lanes write consecutive records of a pixel's run.
 // Each lane recomputes its pair and stores the entry data the blend chains
-// need.  Bound by its 48 bytes a pair: 232 MB written and 71 read in 79 us for
-// 300k surfels at 800 x 600 (3.8 TB/s; a large copy reaches 4.8).
+// need.  Bound by its 40 bytes a pair: 71 us for 300k surfels at 800 x 600 and
+// 257 for 1M at 1237 x 823, with 48 bytes 79 and 290 (232 MB written and 71 read
+// at 800 x 600, 3.8 TB/s; a large copy reaches 4.8).
 template <bool kPart>
 __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
   __shared__ float4 s_q0[64], s_q1[64], s_q2[64], s_q3[64], s_q4[64];
@@ -1927,12 +1928,14 @@ __global__ __launch_bounds__(64) void k_pair_write(AcceptArgs a) {
       eval_pair<false>(pixel_centre<kPart>(qx0 + (p & 7)), pixel_centre<kPart>(qy0 + (p >> 3)), s_q0[j], s_q1[j],
                        s_q2[j], 0.0f, e);
       const float4 q3 = s_q3[j], q4 = s_q4[j];
-      // the distortion weight m(depth) and its derivative, as the blends form them
-      const float m_d = dist_weight<kPart>(e.depth), dmd_dd = dist_weight_grad<kPart>(e.depth);
-      float4* pr = a.ps.rec + kPairQuads * (size_t)(s_foff[p] + k);
-      pr[0] = make_float4(e.depth, m_d, kPart ? __uint_as_float(s_rid[j]) : m_d * m_d, e.alpha);
-      pr[1] = q3;
-      pr[2] = make_float4(q4.x, q4.y, __uint_as_float(s_pos[j]), dmd_dd);
+      // the distortion weight m(depth), as the blends form it
+      const float m_d = dist_weight<kPart>(e.depth);
+      char* pr = a.ps.rec + (size_t)PairLayout<kPart>::kBytes * (size_t)(s_foff[p] + k);
+      float4* q = reinterpret_cast<float4*>(pr);
+      q[0] = make_float4(m_d, __uint_as_float(kPart ? s_rid[j] : s_pos[j]), e.alpha, e.depth);
+      q[1] = make_float4(q3.w, q4.x, q4.y, q3.x);
+      if (kPart) q[2] = make_float4(q3.y, q3.z, __uint_as_float(s_pos[j]), 0.0f);
+      else *reinterpret_cast<float2*>(pr + 32) = make_float2(q3.y, q3.z);
     }
   }
 }
@@ -1959,6 +1962,12 @@ hipError_t launch_pair_write(const AcceptArgs& a, size_t max_items, hipStream_t 
 constexpr int kPre = SR_FWD_PREFETCH;  // stored pairs of a pixel per batch
 constexpr int kPreGroup = 4;           // loaded or not together
 static_assert(kPre % kPreGroup == 0 && kPre <= kPairPad, "whole groups, reads past the last pair within the padding");
+using V3 = float __attribute__((ext_vector_type(3)));
+template <class T> SR_DEV T load4(const char* p) {  // from a 4-byte aligned place
+  T v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(p, 4), sizeof(float) * (sizeof(T) == 16 ? 3 : sizeof(T) / 4));
+  return v;
+}
 
 // Forward blend of a quadrant whose pairs missed the store: the records staged
 // chunk by chunk, the pairs recomputed, lane = pixel.
@@ -2043,7 +2052,6 @@ SR_DEV void blend_fwd_missed(const BlendArgs& a, int qi) {
     for (int c = 0; c < nch; ++c) {
       const int m = min(64, cnt - c * 64);
       uint64_t mask = done ? 0ull : nx.mask;
-      const uint32_t foff = mask ? nx.foff : kNoFrag;
       __syncthreads();
       if (lane < m) {
         s_pos[lane] = nx.v.y;
@@ -2061,21 +2069,14 @@ SR_DEV void blend_fwd_missed(const BlendArgs& a, int qi) {
         nx = chunk_load(masks, frag_off, a.rec, lane, c + 1, ve);
       }
       if (__ballot(mask != 0ull) == 0ull) continue;
-      uint32_t f = foff;
       while (mask != 0ull) {
         const int j = __builtin_ctzll(mask);
         mask &= mask - 1ull;
         float alpha, depth;
-        if (foff != kNoFrag) {
-          const float4 p0 = a.ps.rec[kPairQuads * (size_t)(f++)];
-          alpha = p0.w;
-          depth = p0.x;
-        } else {
-          Pair e;
-          if (!eval_pair<false>(pixx, pixy, s_q0[j], s_q1[j], s_q2[j], 0.0f, e)) continue;
-          alpha = e.alpha;
-          depth = e.depth;
-        }
+        Pair e;  // none of the quadrant's pairs is stored
+        if (!eval_pair<false>(pixx, pixy, s_q0[j], s_q1[j], s_q2[j], 0.0f, e)) continue;
+        alpha = e.alpha;
+        depth = e.depth;
         const float4 q3 = s_q3[j], q4 = s_q4[j];
         if (!step(alpha, depth, dist_weight<kPart>(depth), s_pos[j], q3, q4.x, q4.y, kPart ? s_rid[j] : 0u)) {
           done = true;
@@ -2122,8 +2123,8 @@ SR_DEV void blend_fwd_missed(const BlendArgs& a, int qi) {
 // pixel's pairs one contiguous run in entry order.  A wave takes 16 pixels
 // with 4 lanes each; the 4 lanes of a pixel walk the same run in step (each
 // runs the transmittance update, so all agree on where the pixel stops) and
-// split the accumulators: role 0 depth, M1, M2 and distortion, role 1 the
-// normal and red, roles 2 and 3 green and blue.  Every lane executes the same
+// split the accumulators: role 0 M1, M2 and distortion, role 1 the normal, role
+// 2 the colour, role 3 the depth.  Every lane executes the same
 // instructions (role values are picked by select), so the serial chain of a
 // long pixel costs a quarter of the full update per pair; each accumulator
 // sees exactly the reference's operations in order.
@@ -2133,10 +2134,10 @@ SR_DEV void blend_fwd_missed(const BlendArgs& a, int qi) {
 // saturates in the batch), and where every pixel of the wave has a whole
 // batch left and none saturates, the updates go in without per-pair
 // conditions.  The last contributor and the median are pairs of the run, looked
-// up once at its end from their counts.  300k surfels: 70 us at 800 x 600 and
-// 79 at 400 x 300, where conditions on every pair and 20 pairs a batch, copied
+// up once at its end from their counts.  300k surfels: 61 us at 800 x 600 and
+// 78 at 400 x 300, where conditions on every pair and 20 pairs a batch, copied
 // from the prefetch registers (185 a lane, two waves a SIMD), took 94 and 122.
-// Batches of 4, 12 and 16 pairs: 83, 74, 88 and 96, 75, 73 us.
+// Batches of 12 and 16 pairs: 63, 69 and 84, 81 us.
 // The _part variant sums its outputs as (value * alpha) * T (its kernel's
 // expression; the plain one adds value * (alpha * T)), keeps the median pair's
 // weight and leaves each pair's T in fW, which the backward overwrites only
@@ -2164,53 +2165,62 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
   // lane_range is written by the pair-offset pass, which runs only when the
   // view has instances: read it for non-empty quadrants only
   const uint2 rg = (inside && cnt > 0) ? a.lane_range[(size_t)qi * 64 + pix] : make_uint2(0u, 0u);
-  // Each lane loads one record quad per pair: role 0 quad 0 (depth, mm,
-  // mm^2, alpha), role 1 quad 1 (normal, red), roles 2 and 3 quad 2 (green,
-  // blue, tile position); alpha reaches the other lanes of the pixel from
-  // role 0 by a quad broadcast.  A lane accumulates x, y and z of its quad in
-  // a0..a2 and w in a3, except that role 0's a3 is the distortion.
-  const float4* run = a.ps.rec + kPairQuads * (size_t)rg.x + (role < 2 ? role : 2);
+  // Each lane loads three words of a record: role 0 (m, .., alpha), role 1 the
+  // normal, role 2 the colour and role 3 (depth, .., ..); alpha reaches the
+  // other lanes of the pixel from role 0 by a quad broadcast.  A lane sums its
+  // words in a0..a2, except that role 0 has m^2 for the second, and the
+  // distortion in a2.
+  constexpr int kBytes = PairLayout<kPart>::kBytes;
+  const char* run = a.ps.rec + (size_t)kBytes * rg.x + (role == 0 ? 0 : role == 1 ? 28 : role == 2 ? 16 : 12);
   float T = 1.0f;
-  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f, median_weight = 0.0f;
+  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, median_weight = 0.0f;
   float* pair_T = kPart && a.S > 0 ? reinterpret_cast<float*>(a.ps.fW) + rg.x : nullptr;
   int blended = 0, in_front = 0;  // pairs blended; those with T above 1/2
   bool done = false;
   int left = (int)rg.y;
   // whole groups, so up to kPreGroup - 1 pairs past the run (nothing uses
   // them; the store is padded)
-  auto fetch = [&](float4 (&b)[kPre], const float4* at, int n) {
+  auto fetch = [&](V3 (&b)[kPre], const char* at, int n) {
 #pragma unroll
     for (int g = 0; g < kPre; g += kPreGroup)
       if (g < n) {
 #pragma unroll
-        for (int k = g; k < g + kPreGroup; ++k) b[k] = at[kPairQuads * k];
+        for (int k = g; k < g + kPreGroup; ++k) b[k] = load4<V3>(at + kBytes * k);
       }
   };
-  // forward.cu:383-415 for one pair (role 0's quad: depth, mm, mm^2, alpha)
-  auto update = [&](const float4& v, float alpha, float Tk) {
+  // forward.cu:383-415 for one pair
+  auto update = [&](const V3& v, float alpha, float Tk) {
     const float w = alpha * Tk;
     const float A = 1.0f - Tk;
-    // role 0: the distortion term (mm^2 A + M2 - 2 mm M1), a1 = M1, a2 = M2
-    const float vz = kPart && role == 0 ? v.y * v.y : v.z;
-    const float x3 = role == 0 ? (vz * A + a2) - (2.0f * v.y) * a1 : v.w;
+    // role 0: the distortion term (m^2 A + M2 - 2 m M1), a0 = M1, a1 = M2
+    const float x1 = role == 0 ? v.x * v.x : v.y;
+    const float x2 = role == 0 ? (x1 * A + a1) - (2.0f * v.x) * a0 : v.z;
     auto weighed = [&](float x) { return kPart ? (x * alpha) * Tk : x * w; };
     a0 += weighed(v.x);
-    a1 += weighed(v.y);
-    a2 += weighed(vz);
-    a3 += weighed(x3);
+    a1 += weighed(x1);
+    a2 += weighed(x2);
     if (kPart && Tk > 0.5f) median_weight = w;
   };
-  auto blend = [&](const float4 (&b)[kPre]) {
+  auto blend = [&](const V3 (&b)[kPre]) {
     const int n = min(left, kPre);
     float Tk[kPre + 1];
     Tk[0] = T;
 #pragma unroll
-    for (int k = 0; k < kPre; ++k) Tk[k + 1] = Tk[k] * (1.0f - quad_bcast0(b[k].w));
+    for (int k = 0; k < kPre; ++k) Tk[k + 1] = Tk[k] * (1.0f - quad_bcast0(b[k].z));
+    if (kPart && pair_T != nullptr) {
+      // a quarter of the batch a lane; behind a saturating pair nobody reads it
+#pragma unroll
+      for (int u = 0; u < kPre / 4; ++u) {
+        const float x = role < 2 ? (role == 0 ? Tk[u] : Tk[kPre / 4 + u])
+                                 : (role == 2 ? Tk[kPre / 2 + u] : Tk[3 * kPre / 4 + u]);
+        const int k = role * (kPre / 4) + u;
+        if (k < n) pair_T[blended + k] = x;
+      }
+    }
     if (__ballot(n < kPre || !(Tk[kPre] >= 0.0001f)) == 0ull) {  // of the lanes with pairs left
 #pragma unroll
       for (int k = 0; k < kPre; ++k) {
-        if (kPart && pair_T != nullptr && role == 0) pair_T[blended + k] = Tk[k];
-        update(b[k], quad_bcast0(b[k].w), Tk[k]);
+        update(b[k], quad_bcast0(b[k].z), Tk[k]);
       }
       if (__ballot(T > 0.5f) != 0ull) {
 #pragma unroll
@@ -2219,15 +2229,13 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
       blended += kPre;
       T = Tk[kPre];
     } else {
-      const int base = blended;
 #pragma unroll
       for (int k = 0; k < kPre; ++k) {
         if (k < n && !done) {
           if (Tk[k + 1] < 0.0001f) {
             done = true;
           } else {
-            if (kPart && pair_T != nullptr && role == 0) pair_T[base + k] = Tk[k];
-            update(b[k], quad_bcast0(b[k].w), Tk[k]);
+            update(b[k], quad_bcast0(b[k].z), Tk[k]);
             in_front += Tk[k] > 0.5f ? 1 : 0;
             T = Tk[k + 1];
             ++blended;
@@ -2237,16 +2245,14 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
     }
     left -= kPre;
   };
-  float4 b0[kPre], b1[kPre];
-#pragma unroll
-  for (int k = 0; k < kPre; ++k) b0[k] = b1[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  V3 b0[kPre] = {}, b1[kPre] = {};
   fetch(b0, run, left);
   while (left > 0 && !done) {  // the four lanes of a pixel share left and done
-    run += kPairQuads * kPre;
+    run += kBytes * kPre;
     fetch(b1, run, left - kPre);  // in flight while b0 blends
     blend(b0);
     if (left > 0 && !done) {
-      run += kPairQuads * kPre;
+      run += kBytes * kPre;
       fetch(b0, run, left - kPre);
       blend(b1);
     }
@@ -2257,29 +2263,29 @@ __global__ __launch_bounds__(64) void k_blend_fwd(BlendArgs a) {
   float* out_color = a.out_color + 3 * pb;
   float* out_others = a.out_others + (kPart ? 8 : 7) * pb;
   if (role == 0) {
-    out_others[pid] = a0;
-    final_T[pid + HW] = a1;
-    final_T[pid + 2 * HW] = a2;
-    out_others[pid + 6 * HW] = a3;  // the distortion
+    final_T[pid + HW] = a0;
+    final_T[pid + 2 * HW] = a1;
+    out_others[pid + 6 * HW] = a2;  // the distortion
     if (kPart) out_others[pid + 7 * HW] = median_weight;
   } else if (role == 1) {
     out_others[pid + 2 * HW] = a0;
     out_others[pid + 3 * HW] = a1;
     out_others[pid + 4 * HW] = a2;
-    out_color[pid] = a3 + T * a.bg[0];
   } else if (role == 2) {
-    out_color[HW + pid] = a0 + T * a.bg[1];
-    out_color[2 * HW + pid] = a1 + T * a.bg[2];
+    out_color[pid] = a0 + T * a.bg[0];
+    out_color[HW + pid] = a1 + T * a.bg[1];
+    out_color[2 * HW + pid] = a2 + T * a.bg[2];
   } else {
-    // quad 0's x: depth, quad 2's z: position in the tile list
-    const float4* first = a.ps.rec + kPairQuads * (size_t)rg.x;
-    auto contributor = [&](int n) { return __float_as_uint(first[kPairQuads * (n - 1) + 2].z) + 1u; };
+    out_others[pid] = a0;  // the depth
+    const char* first = a.ps.rec + (size_t)kBytes * rg.x;
+    auto word = [&](int n, int byte) { return *reinterpret_cast<const uint32_t*>(first + (size_t)kBytes * (n - 1) + byte); };
+    auto contributor = [&](int n) { return word(n, kPart ? 40 : 4) + 1u; };  // tile position
     uint32_t* n_contrib = a.n_contrib + 2 * pb;
     final_T[pid] = T;
     n_contrib[pid] = blended > 0 ? contributor(blended) : 0u;
     n_contrib[pid + HW] = f2u(in_front > 0 ? (float)contributor(in_front) : -1.0f);
     out_others[pid + HW] = 1.0f - T;
-    out_others[pid + 5 * HW] = in_front > 0 ? first[kPairQuads * (in_front - 1)].x : 0.0f;
+    out_others[pid + 5 * HW] = in_front > 0 ? __uint_as_float(word(in_front, 12)) : 0.0f;
     // the backward passes walk only the blended prefix of the run
     if (cnt > 0) a.lane_range[(size_t)qi * 64 + pix].y = (uint32_t)blended;
   }
@@ -2321,19 +2327,19 @@ __global__ __launch_bounds__(64) void k_blend_semantics(BlendArgs a) {
     const uint2 rg = a.lane_range[(size_t)qi * 64 + pix];
     const float* pair_T = reinterpret_cast<const float*>(a.ps.fW);
     for (uint32_t i = 0; i < rg.y; i += kSemPre) {
-      float4 p0[kSemPre];
+      V3 p0[kSemPre];  // m, surfel, alpha
       float T[kSemPre], sv[kSemPre];
 #pragma unroll
       for (int k = 0; k < kSemPre; ++k) {  // past the run's end: its last pair again, not summed
         const size_t f = rg.x + min(i + (uint32_t)k, rg.y - 1u);
-        p0[k] = a.ps.rec[kPairQuads * f];
+        p0[k] = load4<V3>(a.ps.rec + (size_t)PairLayout<true>::kBytes * f);
         T[k] = pair_T[f];
       }
 #pragma unroll
-      for (int k = 0; k < kSemPre; ++k) sv[k] = a.sem[(size_t)__float_as_uint(p0[k].z) * a.S + ch];
+      for (int k = 0; k < kSemPre; ++k) sv[k] = a.sem[(size_t)__float_as_uint(p0[k].y) * a.S + ch];
 #pragma unroll
       for (int k = 0; k < kSemPre; ++k)
-        if (i + (uint32_t)k < rg.y) sum += (sv[k] * p0[k].w) * T[k];
+        if (i + (uint32_t)k < rg.y) sum += (sv[k] * p0[k].z) * T[k];
     }
   }
   const size_t HW = (size_t)vi.H * vi.W;

@@ -175,18 +175,12 @@ struct BinLayout {
 };
 constexpr int kPartStride = 20;  // 18 partial gradients, padded to five float4
 // Accepted-pair store: per accepted (pixel, entry) pair the pair-write pass
-// keeps one 48-byte record with everything the per-pixel blend chains read,
-// so they stream it without staging records:
-//   p0 = (depth, m, m^2, alpha)   m = distortion weight of the depth
-//   p1 = (normal.xyz, r)
-//   p2 = (g, b, position of the entry in the tile list (bits), dm/ddepth)
-// (p0, p1 and p2 are what the forward blend's lanes of roles 0, 1 and 2
-// accumulate, in their accumulators' order; the _part variant keeps the
-// record number in p0.z instead of m^2, for its semantic channels)
-// A lane's consecutive pairs are consecutive records, so the fill writes
-// whole lines.  (The per-pair gradient pass recomputes s and G.)  fW = (w, dL/dalpha, dL/ddepth, 0) is written by the backward chain
-// pass for the per-pair gradient pass, which recomputes the rest of the pair.  All pairs of one pixel of a quadrant are
-// contiguous and in entry order: lane_range holds (first, count) per pixel,
+// keeps one record (PairLayout) with everything the per-pixel blend chains
+// read, so they stream it without staging records.  A lane's consecutive pairs
+// are consecutive records, so the fill writes whole lines.  fW = (w, dL/dalpha,
+// dL/ddepth, 0) is written by the backward chain pass for the per-pair gradient
+// pass, which recomputes the rest of the pair.  All pairs of one pixel of a
+// quadrant are contiguous and in entry order: lane_range holds (first, count) per pixel,
 // frag_off the first pair of each (chunk, pixel).  The forward blend
 // rewrites each count to the pairs the pixel actually blended (a prefix of
 // its run: the ones in front of its last contributor), so the backward
@@ -195,7 +189,14 @@ constexpr int kPartStride = 20;  // 18 partial gradients, padded to five float4
 // flagged (q_flag, frag_off = kNoFrag) and blended by the staged path that
 // recomputes its pairs.
 constexpr size_t kFragPerInstance = 24;
-constexpr int kPairQuads = 3;  // float4 per stored pair
+// A stored pair, as the blend chains read it: m, tile position, alpha, depth,
+// red, green, blue, normal, with m the distortion weight of the depth.  The
+// _part variant has the surfel in place of the position, which follows the
+// normal.  (m^2 and dm/ddepth are formed by the chains: the passes that write
+// and read the store are bound by its bytes.)
+template <bool kPart> struct PairLayout {
+  static constexpr int kBytes = kPart ? 48 : 40;
+};
 constexpr int kPairPad = 32;   // pairs a blend may read in front of the store's first or past its last
 constexpr uint32_t kNoFrag = 0xFFFFFFFFu;
 // Per-pixel acceptance masks: quadrant (t, q) owns mask slots
@@ -289,8 +290,11 @@ inline size_t segment_capacity(size_t n) { return n / kSegKeys + n / kSmallMax +
 // slot_capacity: slots the part region is sized for; 0 sizes it for every
 // (instance, quadrant), which no batch can exceed.
 inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_capacity = 0, int sem = 0,
-                            int slot_capacity = 0) {
+                            int slot_capacity = 0, bool part = false) {
   BinLayout b{};
+  const size_t pair = part ? PairLayout<true>::kBytes : PairLayout<false>::kBytes, pad = kPairPad * pair;
+  static_assert(kPairPad * PairLayout<false>::kBytes % 256 == 0 && kPairPad * PairLayout<true>::kBytes % 256 == 0,
+                "the store stays aligned");
   size_t off = 0;
   const size_t n = (size_t)(L > 0 ? L : 1);
   const size_t Q = (size_t)quads_per_tile(B);
@@ -314,7 +318,7 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
   b.frag_cap = pair_capacity > 0 ? (size_t)pair_capacity
                                   : n * (pair_store > 0 ? (size_t)pair_store : kFragPerInstance);
   if (b.frag_cap > 0x7fffffffu) b.frag_cap = 0x7fffffffu;
-  b.prec = off + kPairPad * kPairQuads * 16; off += align_up((b.frag_cap + 2 * kPairPad) * kPairQuads * 16);
+  b.prec = off + pad; off += align_up(b.frag_cap * pair + 2 * pad);
   b.fW = off; off += align_up(b.frag_cap * 16);
   b.sem_part = off; off += align_up(n * Q * (size_t)sem * 4);  // _part: semantic partials per slot
   b.part = off; off += align_up(b.nslot * kPartStride * 4);         // last: see part
@@ -324,7 +328,7 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
 
 // Device pointers of the accepted-pair store.
 struct PairStore {
-  float4* rec;  // kPairQuads per pair
+  char* rec;    // PairLayout::kBytes per pair
   float4* fW;   // 1 per pair
 };
 // The backward's chain pass cuts a pixel's run of n pairs into segments of
