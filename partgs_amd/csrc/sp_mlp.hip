@@ -1,9 +1,10 @@
 // Point-set MLP of the learned block proposal on gfx950 matrix cores.
 //
 //   k_gemm       C = act(alpha * A B^T + bias) (+ C), A and B bf16 with any
-//                strides, FP32 accumulation on v_mfma_f32_16x16x16_bf16:
-//                64 x 64 output tile per 256-lane workgroup, 32 x 32 per
-//                wave (2 x 2 MFMA tiles), K in steps of 16.
+//                strides, FP32 accumulation on v_mfma_f32_16x16x16_bf16,
+//                32 x 32 per wave (2 x 2 MFMA tiles), K in steps of 16:
+//                64 x 64 output tile per 256-lane workgroup, or, for long
+//                sums on few tiles, 32 x 32 with the sum cut over 16 waves.
 //   k_point_pool the shared per-point MLP 3 -> 64 -> 128 -> 256 (ReLU) fused
 //                with the max-pool over each scene's points: 64 points per
 //                workgroup, layer 1 on the VALU in FP32, layers 2 and 3 on
@@ -17,6 +18,8 @@
 // are rows 4 (lane / 16) + j of column (lane % 16).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "../../include/set_proposal.h"
 
@@ -52,51 +55,110 @@ struct GemmArgs {
   uint16_t* Cb;  // optional bf16 copy of the result (same ldc)
 };
 
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
+// How a wave reads an operand's fragment, 32 rows by 16 k as two 16 x 16 MFMA
+// tiles, four k of a row a lane: element by element at any strides; in one
+// 8-byte load where k is contiguous; or, where the rows are contiguous, as the
+// pairs of rows 2 r, 2 r + 1 at four k, tile 0 taking the even rows and tile 1
+// the odd ones.
+enum class Read { kAny, kQuads, kPairs };
+__device__ inline int row_of(Read how, int tile, int r) { return how == Read::kPairs ? 2 * r + tile : 16 * tile + r; }
+
+template <Read how>
+__device__ inline void read_fragment(bf16x4 (&f)[2], const uint16_t* X, long ld_row, long ld_k, int row0, int rows,
+                                     int k0, int K) {
+  const int lane = threadIdx.x & 63, r = lane & 15, k = k0 + (lane >> 4) * 4;
+  if (how == Read::kPairs) {
+    const int row = row0 + 2 * r;
+    uint32_t p[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      p[t] = row < rows && k + t < K ? *reinterpret_cast<const uint32_t*>(X + row + (long)(k + t) * ld_k) : 0u;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      f[0][t] = (short)(p[t] & 0xFFFFu);
+      f[1][t] = (short)(p[t] >> 16);
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = row0 + 16 * i + r;
+    if (how == Read::kQuads) {
+      f[i] = row < rows && k < K ? *reinterpret_cast<const bf16x4*>(X + row * ld_row + k) : bf16x4{0, 0, 0, 0};
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        f[i][t] = row < rows && k + t < K ? (short)X[row * ld_row + (k + t) * ld_k] : (short)0;
+    }
+  }
+}
+
+// kSlices == 1: 64 x 64 of C a workgroup, 32 x 32 a wave, each element's
+// products summed over k in steps of 16 in order.  kSlices > 1: 32 x 32 a
+// workgroup, every wave a slice of k of its own, the slices' sums added in
+// order in LDS.  The latter is for few tiles and long sums, where the chain of
+// steps down one wave bounds the product: the weight gradients of 8,192 rows
+// (128 x 64 and 256 x 128 by 8,192) were two and eight
+// workgroups, 237 us each, and take 25 and 29; read element by element, where 4
+// k are now one load, the 8,192 x 128 by 256 input gradient took 21 us, now 10.
+constexpr int kDeepSlices = 16;
+template <int kSlices, Read kA, Read kB>
+__global__ __launch_bounds__(kSlices == 1 ? 256 : kSlices * 64) void k_gemm(GemmArgs g) {
+  __shared__ float s_sum[kSlices == 1 ? 1 : kSlices][kSlices == 1 ? 1 : 16 * 64 + 16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int m0 = blockIdx.y * 64 + (wave >> 1) * 32;
-  const int n0 = blockIdx.x * 64 + (wave & 1) * 32;
+  const int m0 = kSlices == 1 ? blockIdx.y * 64 + (wave >> 1) * 32 : blockIdx.y * 32;
+  const int n0 = kSlices == 1 ? blockIdx.x * 64 + (wave & 1) * 32 : blockIdx.x * 32;
   const int r = lane & 15, kq = (lane >> 4) * 4;
+  const int steps = (g.K + 15) / 16, per = (steps + kSlices - 1) / kSlices;
+  const int first = kSlices == 1 ? 0 : wave * per, last = min(steps, first + per);
   f32x4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < g.K; k0 += 16) {
+#pragma unroll 4
+  for (int s = first; s < last; ++s) {
     bf16x4 a[2], b[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int m = m0 + i * 16 + r;
-      const int n = n0 + i * 16 + r;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int k = k0 + kq + t;
-        a[i][t] = (m < g.M && k < g.K) ? (short)g.A[(long)m * g.lda_m + (long)k * g.lda_k] : (short)0;
-        b[i][t] = (n < g.N && k < g.K) ? (short)g.B[(long)n * g.ldb_n + (long)k * g.ldb_k] : (short)0;
-      }
-    }
+    read_fragment<kA>(a, g.A, g.lda_m, g.lda_k, m0, g.M, 16 * s, g.K);
+    read_fragment<kB>(b, g.B, g.ldb_n, g.ldb_k, n0, g.N, 16 * s, g.K);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = mfma(a[i], b[j], acc[i][j]);
+  }
+  auto store = [&](int i, int j, int t, float sum) {
+    const int m = m0 + row_of(kA, i, kq + t);
+    const int n = n0 + row_of(kB, j, r);
+    if (m >= g.M || n >= g.N) return;
+    float v = g.alpha * sum;
+    if (g.bias) v += g.bias[n];
+    if (g.relu) v = v > 0.0f ? v : 0.0f;
+    float* c = g.C + (long)m * g.ldc + n;
+    if (g.accumulate) v += *c;
+    *c = v;
+    if (g.Cb) g.Cb[(long)m * g.ldc + n] = f2bf(v);
+  };
+  if (kSlices == 1) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) store(i, j, t, acc[i][j][t]);
+    return;
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int m = m0 + i * 16 + kq + t;
-        const int n = n0 + j * 16 + r;
-        if (m >= g.M || n >= g.N) continue;
-        float v = g.alpha * acc[i][j][t];
-        if (g.bias) v += g.bias[n];
-        if (g.relu) v = v > 0.0f ? v : 0.0f;
-        float* c = g.C + (long)m * g.ldc + n;
-        if (g.accumulate) v += *c;
-        *c = v;
-        if (g.Cb) g.Cb[(long)m * g.ldc + n] = f2bf(v);
-      }
+      for (int t = 0; t < 4; ++t) s_sum[wave][(8 * i + 4 * j + t) * 64 + lane] = acc[i][j][t];
+  __syncthreads();
+  // wave w: result w of every lane, (i, j, t) = (w / 8, w / 4 % 2, w % 4)
+  static_assert(kSlices == 1 || kSlices == 16, "a result a wave");
+  float sum = 0.0f;
+  for (int w = 0; w < kSlices; ++w) sum += s_sum[w][wave * 64 + lane];
+  store(wave >> 3, wave >> 2 & 1, wave & 3, sum);
 }
 
 // ---------------------------------------------------------------------------
@@ -278,8 +340,39 @@ int sp_gemm_bf16(int M, int N, int K, const uint16_t* A, long lda_m, long lda_k,
   if (M < 0 || N < 0 || K < 0 || (M > 0 && N > 0 && (!A || !B || !C))) return 1;
   if (M == 0 || N == 0) return 0;
   GemmArgs g{M, N, K, A, lda_m, lda_k, B, ldb_n, ldb_k, bias, alpha, relu, accumulate, C, ldc, C_bf16};
-  dim3 grid((N + 63) / 64, (M + 63) / 64);
-  hipLaunchKernelGGL(k_gemm, grid, dim3(256), 0, (hipStream_t)stream, g);
+  // whole 8-byte quads of k, or whole 4-byte pairs of rows, at their alignment
+  auto how = [K](const uint16_t* X, long ld_row, long ld_k, int rows) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(X);
+    if (ld_k == 1 && K % 4 == 0 && ld_row % 4 == 0 && at % 8 == 0) return Read::kQuads;
+    if (ld_row == 1 && rows % 2 == 0 && ld_k % 2 == 0 && at % 4 == 0) return Read::kPairs;
+    return Read::kAny;
+  };
+  const Read ra = how(A, lda_m, lda_k, M), rb = how(B, ldb_n, ldb_k, N);
+  // Long sums on few enough tiles, us with the sum cut and whole: 128 x 64 by 512
+  // 9 and 16, by 1,024 9 and 30; 512 x 512 by 4,096 17 and 156; 1,024 x 1,024 by
+  // 4,096 51 and 159; but 2,048 x 2,048 by 2,048 98 and 85.
+  const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
+  const bool deep = K >= 512 && tiles <= 256;
+  const hipStream_t st = (hipStream_t)stream;
+  auto launch = [&](auto a, auto b) {
+    constexpr Read kA = decltype(a)::value, kB = decltype(b)::value;
+    if (deep)
+      hipLaunchKernelGGL((k_gemm<kDeepSlices, kA, kB>), dim3((N + 31) / 32, (M + 31) / 32), dim3(kDeepSlices * 64), 0,
+                         st, g);
+    else
+      hipLaunchKernelGGL((k_gemm<1, kA, kB>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, st, g);
+  };
+  using Any = std::integral_constant<Read, Read::kAny>;
+  using Quads = std::integral_constant<Read, Read::kQuads>;
+  using Pairs = std::integral_constant<Read, Read::kPairs>;
+  auto with_b = [&](auto a) {
+    if (rb == Read::kQuads) launch(a, Quads{});
+    else if (rb == Read::kPairs) launch(a, Pairs{});
+    else launch(a, Any{});
+  };
+  if (ra == Read::kQuads) with_b(Quads{});
+  else if (ra == Read::kPairs) with_b(Pairs{});
+  else with_b(Any{});
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
