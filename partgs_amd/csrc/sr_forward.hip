@@ -642,23 +642,32 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32
                                                               uint32_t* large, uint32_t* seg_off, uint32_t* host) {
   __shared__ uint32_t s_part[3 * 32];
   const int tid = threadIdx.x;
+  auto each = [](const uint32_t* x, int b, int e, auto&& fn) {  // eight loads in flight
+    int i = b;
+    for (; i + 8 <= e; i += 8) {
+      uint32_t v[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) v[t] = x[i + t];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) fn(i + t, v[t]);
+    }
+    for (; i < e; ++i) fn(i, x[i]);
+  };
   const int per = (T + kScanThreads - 1) / kScanThreads;
   const int b = tid * per;
   const int e = min(T, b + per);
   // this lane's tiles: instances, large tiles, their segments
   uint32_t v3[3] = {0u, 0u, 0u}, tot3[3];
-  for (int i = b; i < e; ++i) {
-    const uint32_t c = count[i];
+  each(count, b, e, [&](int, uint32_t c) {
     v3[0] += c;
     if (c > (uint32_t)kSmallMax) {
       v3[1] += 1u;
       v3[2] += segments_of(c);
     }
-  }
+  });
   scan1024_excl(s_part, v3, tot3);
   uint32_t run = v3[0], at = v3[1], sat = v3[2];
-  for (int i = b; i < e; ++i) {
-    const uint32_t c = count[i];
+  each(count, b, e, [&](int i, uint32_t c) {
     start[i] = run;
     fill[i] = run;
     ranges[2 * i] = c ? run : 0u;
@@ -669,7 +678,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32
       seg_off[at++] = sat;
       sat += segments_of(c);
     }
-  }
+  });
   if (tid == kScanThreads - 1) {
     start[T] = tot3[0];
     counters[0] = tot3[0];
@@ -682,14 +691,13 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int T, const uint32
   const int pb = (nb + kScanThreads - 1) / kScanThreads;
   const int b2 = tid * pb, e2 = min(nb, b2 + pb);
   uint32_t w1[1] = {0u}, wt[1];
-  for (int i = b2; i < e2; ++i) w1[0] += ssum[i];
+  each(ssum, b2, e2, [&](int, uint32_t d) { w1[0] += d; });
   scan1024_excl(s_part, w1, wt);
   uint32_t run3 = w1[0];
-  for (int i = b2; i < e2; ++i) {
-    const uint32_t d = ssum[i];
+  each(ssum, b2, e2, [&](int i, uint32_t d) {
     ssum[i] = run3;
     run3 += d;
-  }
+  });
   if (tid == 0) {
     counters[8] = wt[0];
     if (wt[0] > slot_capacity) atomicOr(&counters[1], kErrCapacity | kErrSlots);
@@ -1163,8 +1171,10 @@ SR_DEV int co_rank(const uint64_t* A, int na, const uint64_t* Bv, int nb, int k)
 // smallest and largest, and the keys moved bin by bin into key2.  Segment s of
 // the tile starts at the first bin boundary at or after kSegKeys s keys, so
 // segments hold kSegKeys keys give or take a bin, and their sorts, one
-// workgroup each, put the tile in order; the payloads move along (24 us for
-// 300k surfels at 800 x 600, 14 of them the keys').  A segment above kSmallMax keys (more
+// workgroup each, put the tile in order; the payloads move along, loaded with
+// the keys: 20 us for 300k surfels at 800 x 600 and 768 for a million and 16
+// views; 24 and 1,153 with each payload's load behind the stores of the one
+// before.  A segment above kSmallMax keys (more
 // than kSegKeys nearly equal depths in one bin) is sorted here: chunks in LDS,
 // then pairwise merges between the tile's two key buffers.
 constexpr int kSplitThreads = 1024, kSplitBins = 4096, kSplitRun = 4;
@@ -1297,11 +1307,25 @@ __global__ __launch_bounds__(kSplitThreads) void k_split_large(SortArgs a) {
     __syncthreads();
     const uint2* pay = a.pay + beg;
     uint2* pay2 = a.pay2 + beg;
-    each([&](uint64_t k, int i) {
-      const uint32_t at = atomicAdd(&bins[bin_of(k)], 1u);
-      dst[at] = k;
-      pay2[at] = pay[i];
-    });
+    for (int i0 = 0; i0 < n; i0 += kU * NT) {  // keys and payloads in flight together
+      uint64_t k[kU];
+      uint2 p[kU];
+      uint32_t at[kU];
+#pragma unroll
+      for (int t = 0; t < kU; ++t) {
+        const int i = min(i0 + t * NT + tid, n - 1);
+        k[t] = src[i];
+        p[t] = pay[i];
+      }
+#pragma unroll
+      for (int t = 0; t < kU; ++t) at[t] = i0 + t * NT + tid < n ? atomicAdd(&bins[bin_of(k[t])], 1u) : 0u;
+#pragma unroll
+      for (int t = 0; t < kU; ++t)
+        if (i0 + t * NT + tid < n) {
+          dst[at[t]] = k[t];
+          pay2[at[t]] = p[t];
+        }
+    }
     __syncthreads();
     for (int sg = 0; sg < nseg; ++sg) {  // uniform
       const uint32_t s0 = seg[sg], s1 = sg + 1 < nseg ? seg[sg + 1] : beg + (uint32_t)n;
