@@ -201,7 +201,7 @@ struct Pipeline {
 PairStore pair_store(char* bin, const BinLayout& bl) {
   PairStore p{};
   p.rec = bin + bl.prec;
-  p.fW = (float4*)(bin + bl.fW);
+  p.fW = (PairOut*)(bin + bl.fW);
   return p;
 }
 

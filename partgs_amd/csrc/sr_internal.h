@@ -173,12 +173,17 @@ struct BinLayout {
   size_t frag_cap;
   size_t sem_part;
 };
-constexpr int kPartStride = 20;  // 18 partial gradients, padded to five float4
+// 18 partial gradients, unpadded, as are a pair's three chain outputs
+// (PairOut): the passes that write and read them are bound by bytes.  Forward
+// + backward with 72 and 12 bytes against 80 and 16: 300k surfels at 800 x 600
+// 561 -> 554 us, 1M at 1237 x 823 1620 -> 1605, the _part variant at 800 x 600
+// 759 -> 748.
+constexpr int kPartStride = 18;
 // Accepted-pair store: per accepted (pixel, entry) pair the pair-write pass
 // keeps one record (PairLayout) with everything the per-pixel blend chains
 // read, so they stream it without staging records.  A lane's consecutive pairs
 // are consecutive records, so the fill writes whole lines.  fW = (w, dL/dalpha,
-// dL/ddepth, 0) is written by the backward chain pass for the per-pair gradient
+// dL/ddepth) is written by the backward chain pass for the per-pair gradient
 // pass, which recomputes the rest of the pair.  All pairs of one pixel of a
 // quadrant are contiguous and in entry order: lane_range holds (first, count) per pixel,
 // frag_off the first pair of each (chunk, pixel).  The forward blend
@@ -319,17 +324,21 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
                                   : n * (pair_store > 0 ? (size_t)pair_store : kFragPerInstance);
   if (b.frag_cap > 0x7fffffffu) b.frag_cap = 0x7fffffffu;
   b.prec = off + pad; off += align_up(b.frag_cap * pair + 2 * pad);
-  b.fW = off; off += align_up(b.frag_cap * 16);
+  b.fW = off; off += align_up(b.frag_cap * 12);
   b.sem_part = off; off += align_up(n * Q * (size_t)sem * 4);  // _part: semantic partials per slot
   b.part = off; off += align_up(b.nslot * kPartStride * 4);         // last: see part
   b.total = off;
   return b;
 }
 
+// What the chain pass leaves of a pair for the per-pair gradient pass.
+struct PairOut {
+  float w, dalpha, ddepth;
+};
 // Device pointers of the accepted-pair store.
 struct PairStore {
   char* rec;    // PairLayout::kBytes per pair
-  float4* fW;   // 1 per pair
+  PairOut* fW;  // 1 per pair
 };
 // The backward's chain pass cuts a pixel's run of n pairs into segments of
 // chain_segment(n): up to 8 of at least 16 pairs, and 16 from 257 pairs on,
