@@ -187,9 +187,9 @@ size_t sr_binning_bytes(int num_rendered, int W, int H, int tile, int pair_store
 /* Accepted pairs (*pairs) and tile instances (*instances) of the calling
  * thread's latest completed sr_forward on the current device: the pairs are
  * those the forward asked the pair store for (the accepted pairs in front
- * of each pixel's saturation point).  The counts are copied back
- * asynchronously at the end of each forward and never waited for: returns
- * SR_OK once such a copy has landed, SR_ERR_INVALID before.  A caller sizes
+ * of each pixel's saturation point).  The forward's kernels write the counts
+ * to host memory and nothing waits for them: returns SR_OK once they have
+ * landed, SR_ERR_INVALID before.  A caller sizes
  * the next forward's pair_capacity from them.  No counterpart in the
  * reference. */
 int sr_pair_count(unsigned long long* pairs, unsigned int* instances);

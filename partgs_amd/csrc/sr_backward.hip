@@ -312,7 +312,7 @@ SR_DEV void pair_grads(float dLp0, float dLp1, float dLp2, float dLn0, float dLn
 // chain of a run of n pairs is two passes over n / 16 pairs instead of one over
 // n.  A wave gives its pixels as many lanes each as the quadrant's longest run
 // can have segments (1 to 16, by its cost's class), and a quadrant takes as
-// many waves.  300k surfels at 800 x 600: 89 us and at 400 x 300 48 (98 and 49
+// many waves.  300k surfels at 800 x 600: 86 us and at 400 x 300 47 (98 and 49
 // with 48-byte records); with 8 lanes a pixel in every quadrant and each lane
 // loading its own records 130 and 72; with the lanes by class but their own
 // records still 130 and 66.
@@ -721,7 +721,7 @@ SR_DEV uint64_t wave_transpose64(uint64_t x, int lane) {
 // entry's sums go to its (position, quadrant) slot of the partial-gradient
 // buffer.  The recompute path of pass 1 groups its sums the same way, so
 // the partials have the same bits whichever quadrants missed the pair store.
-// 91 us for 300k surfels at 800 x 600, 53 of them issuing (57 % of the lanes at
+// 89 us for 300k surfels at 800 x 600, 53 of them issuing (57 % of the lanes at
 // work: the last group of an entry is rarely full).
 // kSem: the _part variant's semantic channels, rounded up (0: none), whose
 // gradients w dL/dsem are summed the same way into sem_part.

@@ -56,31 +56,6 @@ SR_DEV bool eval_pair(float pixx, float pixy, const float4& q0, const float4& q1
   return !(e.alpha < 1.0f / 255.0f);
 }
 
-// Rebuilds a Pair from its stored (alpha, depth), (G, s.x) and s.y: the
-// cheap planes k, l, p.z and the screen offsets are recomputed exactly as in
-// eval_pair, so every field equals eval_pair's.
-SR_DEV void load_pair(float pixx, float pixy, const float4& q0, const float4& q1, const float4& q2,
-                      const float2& fa, const float2& fb, float fc, Pair& e) {
-  const float Tux = q0.x, Tuy = q0.y, Tuz = q0.z, Tvx = q0.w, Tvy = q1.x, Tvz = q1.y;
-  const float Twx = q1.z, Twy = q1.w, Twz = q2.x;
-  e.dx = q2.y - pixx;
-  e.dy = q2.z - pixy;
-  e.rho2d = 2.0f * (e.dx * e.dx + e.dy * e.dy);
-  e.kx = pixx * Twx - Tux;
-  e.ky = pixx * Twy - Tuy;
-  e.kz = pixx * Twz - Tuz;
-  e.lx = pixy * Twx - Tvx;
-  e.ly = pixy * Twy - Tvy;
-  e.lz = pixy * Twz - Tvz;
-  e.pz = e.kx * e.ly - e.ky * e.lx;
-  e.alpha = fa.x;
-  e.depth = fa.y;
-  e.G = fb.x;
-  e.sx = fb.y;
-  e.sy = fc;
-  e.rho3d = e.sx * e.sx + e.sy * e.sy;
-}
-
 // The _part variant ("dsp/") evaluates the same pair at pixel centres + 0.5:
 // its double constants change nothing in FP32 (FilterInvSquare = 1 / FS^2 is
 // 2 (1 - 2e-16), whose product with a float rounds to twice it; 0.2f is the
@@ -89,7 +64,8 @@ SR_DEV void load_pair(float pixx, float pixy, const float4& q0, const float4& q1
 // forward's sums differ between the two.  So the variant runs on the plain
 // kernels' balanced passes (kPart instances) instead of one wave per quadrant
 // evaluating every (entry, pixel): 300k surfels, 800 x 600, 8 channels,
-// forward + backward 15.5 -> 1.03 ms.
+// forward + backward 15.5 -> 0.75 ms (1.03 before the later changes of these
+// passes).
 template <bool kPart>
 SR_DEV float pixel_centre(int i) {
   return kPart ? (float)i + 0.5f : (float)i;
