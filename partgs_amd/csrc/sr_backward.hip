@@ -35,9 +35,6 @@ template <class T> SR_DEV T load8(const char* p) {  // from an 8-byte aligned pl
   __builtin_memcpy(&v, __builtin_assume_aligned(p, 8), sizeof(T));
   return v;
 }
-template <class T> SR_DEV void store8(float* p, T v) {  // to an 8-byte aligned place
-  __builtin_memcpy((void*)__builtin_assume_aligned(p, 8), &v, sizeof(T));
-}
 // LDS bytes from one lane's batch to the next: 16 more than its pairs, so that
 // neither the quads' pieces nor the lanes' own reads share banks
 template <bool kPart> constexpr int kOwnerBytes = kChainPre * PairLayout<kPart>::kBytes + 16;
@@ -51,8 +48,9 @@ constexpr unsigned kChainBlocks = 16384;  // workgroups of the chain pass at mos
 constexpr int kGradGroup = SR_GRAD_GROUP;
 static_assert(kGradGroup >= 1 && 64 % kGradGroup == 0, "groups tile the 64 pixels");
 
-// Stores the 18 partial sums (g(k) for sum k) of a sub-list entry in its
-// slot.  Every entry of every sub-list sets its flag exactly once per backward and
+// Stores the 18 partial sums (g(k) for sum k) of a sub-list entry as five
+// float4 in its slot.  Every
+// entry of every sub-list sets its flag exactly once per backward and
 // stores its sums when any is non-zero, so neither buffer needs clearing.
 // (also: some pixel has a semantic gradient for the slot, _part variant).
 template <class G>
@@ -62,10 +60,12 @@ SR_DEV void store_part(const BlendBwdArgs& a, size_t slot, G g, bool also = fals
   for (int k = 0; k < 18; ++k) nz |= g(k) != 0.0f;
   a.part_nz[slot] = nz ? 1 : 0;  // most entries blend no pixel of the quadrant: only a flag
   if (!nz) return;
-  float* d = a.part + slot * kPartStride;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) store8(d + 4 * k, V4{g(4 * k), g(4 * k + 1), g(4 * k + 2), g(4 * k + 3)});
-  store8(d + 16, V2{g(16), g(17)});
+  float4* d = reinterpret_cast<float4*>(a.part + slot * kPartStride);
+  d[0] = make_float4(g(0), g(1), g(2), g(3));
+  d[1] = make_float4(g(4), g(5), g(6), g(7));
+  d[2] = make_float4(g(8), g(9), g(10), g(11));
+  d[3] = make_float4(g(12), g(13), g(14), g(15));
+  d[4] = make_float4(g(16), g(17), 0.0f, 0.0f);
 }
 
 // Per-pixel inputs of the backward blend (backward.cu:168-236).
@@ -1069,23 +1069,18 @@ SR_DEV void reduce_record(const PreprocessBwdArgs& a, size_t r, float (&gs)[18])
     for (int t = 0; t < 4; ++t) fl[t] = s + (uint32_t)t < s1 ? fl[t] : 0;
 #pragma unroll
     for (int u = 0; u < 4; u += kU) {
-      V4 p[kU][4];
-      V2 p4[kU];
+      V4 p[kU][5];
 #pragma unroll
       for (int t = 0; t < kU; ++t) {
         if (fl[u + t] == 0) continue;
-        const char* src = reinterpret_cast<const char*>(a.part + (size_t)(s + (uint32_t)(u + t)) * kPartStride);
+        const V4* src = reinterpret_cast<const V4*>(a.part + (size_t)(s + (uint32_t)(u + t)) * kPartStride);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) p[t][k] = load8<V4>(src + 16 * k);
-        p4[t] = load8<V2>(src + 64);
+        for (int k = 0; k < 5; ++k) p[t][k] = src[k];
       }
 #pragma unroll
       for (int t = 0; t < kU; ++t)
 #pragma unroll
-        for (int k = 0; k < 18; ++k) {
-          const float x = k < 16 ? p[t][k / 4 & 3][k % 4] : p4[t][k & 1];
-          gs[k] = fl[u + t] ? gs[k] + x : gs[k];
-        }
+        for (int k = 0; k < 18; ++k) gs[k] = fl[u + t] ? gs[k] + p[t][k / 4][k % 4] : gs[k];
     }
   }
 }

@@ -173,12 +173,7 @@ struct BinLayout {
   size_t frag_cap;
   size_t sem_part;
 };
-// 18 partial gradients, unpadded, as are a pair's three chain outputs
-// (PairOut): the passes that write and read them are bound by bytes.  Forward
-// + backward with 72 and 12 bytes against 80 and 16: 300k surfels at 800 x 600
-// 561 -> 554 us, 1M at 1237 x 823 1620 -> 1605, the _part variant at 800 x 600
-// 759 -> 748.
-constexpr int kPartStride = 18;
+constexpr int kPartStride = 20;  // 18 partial gradients, padded to five float4
 // Accepted-pair store: per accepted (pixel, entry) pair the pair-write pass
 // keeps one record (PairLayout) with everything the per-pixel blend chains
 // read, so they stream it without staging records.  A lane's consecutive pairs
@@ -331,7 +326,10 @@ inline BinLayout bin_layout(int L, int B, int T, int pair_store = 0, int pair_ca
   return b;
 }
 
-// What the chain pass leaves of a pair for the per-pair gradient pass.
+// What the chain pass leaves of a pair for the per-pair gradient pass.  Both
+// are bound by bytes: forward + backward with 12 bytes a pair against 16 took
+// 556 us instead of 562 for 300k surfels at 800 x 600 and 1,605 instead of
+// 1,619 for 1M at 1237 x 823.
 struct PairOut {
   float w, dalpha, ddepth;
 };
