@@ -721,10 +721,17 @@ SR_DEV uint64_t wave_transpose64(uint64_t x, int lane) {
 // entry's sums go to its (position, quadrant) slot of the partial-gradient
 // buffer.  The recompute path of pass 1 groups its sums the same way, so
 // the partials have the same bits whichever quadrants missed the pair store.
-// 89 us for 300k surfels at 800 x 600, 53 of them issuing (57 % of the lanes at
+// 88 us for 300k surfels at 800 x 600, 53 of them issuing (57 % of the lanes at
 // work: the last group of an entry is rarely full).
 // kSem: the _part variant's semantic channels, rounded up (0: none), whose
 // gradients w dL/dsem are summed the same way into sem_part.
+// The group sums change hands in rows of kGrpRow floats, 12 at a time: four a
+// read instead of one, and with rows of 12 and not all 18 (20) ten KB of LDS, so
+// that LDS does not hold fewer waves than registers do.  300k surfels at 800 x
+// 600: 88 us with rows of 12, 90 with 8, 16, 20 or one float at a time; 1M at
+// 1237 x 823 274, 280 one at a time; the _part variant with 8 channels, whose
+// dL/dsem are read by four too, 126, was 144.
+constexpr int kGrpRow = 12;
 template <bool kPart, int kSem>
 __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
   __shared__ uint4 s_pm[64];    // per pixel: trimmed mask (lo, hi), first stored pair of the chunk
@@ -735,8 +742,8 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
   __shared__ unsigned long long s_col[64];         // per entry: the pixels that blended it
   __shared__ uint32_t s_tbase[64];                 // per entry: its first group
   __shared__ uint32_t s_head[64];
-  __shared__ float s_grp[kNumG + kSem][64];        // group sums of the round
-  __shared__ float s_dls[kSem > 0 ? kSem : 1][64]; // per pixel: dL/dsem
+  __shared__ V4 s_grp[64][kGrpRow / 4];            // per lane: kGrpRow of its group's sums
+  __shared__ V4 s_dls[kSem > 0 ? 64 : 1][kSem > 0 ? kSem / 4 : 1];  // per pixel: dL/dsem
   const int lane = threadIdx.x;
   if (a.counters[1] & kErrCapacity) return;
   const uint32_t nwork = *a.work_count;
@@ -779,9 +786,11 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
     s_e0[lane] = q0;
     s_e1[lane] = q1;
     s_e2[lane] = q2;
+    if constexpr (kSem > 0) {
+      auto dls = [&](int x) { return mask && x < a.S ? a.dL_dsem[(size_t)a.S * pb + x * HW + pid] : 0.0f; };
 #pragma unroll
-    for (int x = 0; x < kSem; ++x)
-      s_dls[x][lane] = mask && x < a.S ? a.dL_dsem[(size_t)a.S * pb + x * HW + pid] : 0.0f;
+      for (int x = 0; x < kSem; x += 4) s_dls[lane][x / 4] = V4{dls(x), dls(x + 1), dls(x + 2), dls(x + 3)};
+    }
     wave_lds_fence();
     if (mask) {
       // entries in front of the last contributor: positions rise along the
@@ -853,19 +862,35 @@ __global__ __launch_bounds__(64) void k_blend_bwd_grad(BlendBwdArgs a) {
           pair_grads(g4.x, g4.y, g4.z, g4.w, n2.x, n2.y, e, r1, r2.w, fw[k].w, fw[k].dalpha, fw[k].ddepth, pixx, pixy,
                      [&](int s, float val) { g[s] += val; });
 #pragma unroll
-          for (int x = 0; x < kSem; ++x) g[kNumG + x] += fw[k].w * s_dls[x][p];
+          for (int x = 0; x < kSem; x += 4) {
+            const V4 d = s_dls[p][x / 4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) g[kNumG + x + c] += fw[k].w * d[c];
+          }
         }
       }
-#pragma unroll
-      for (int k = 0; k < kNumG + kSem; ++k) s_grp[k][lane] = g[k];
-      wave_lds_fence();
       // the entry's lane adds its groups of this round, in order
       const uint32_t lo = max(tbase, base), hi = min(tbase + ng, base + 64u);
-      for (uint32_t u = lo; u < hi; ++u) {
 #pragma unroll
-        for (int k = 0; k < kNumG + kSem; ++k) acc[k] += s_grp[k][u - base];
+      for (int k0 = 0; k0 < kNumG + kSem; k0 += kGrpRow) {
+        auto sums = [&](auto&& fn) {  // the row's quads, fn(place, first sum)
+#pragma unroll
+          for (int q = 0; q < kGrpRow / 4; ++q)
+            if (k0 + 4 * q < kNumG + kSem) fn(q, k0 + 4 * q);
+        };
+        auto at = [&](int k) { return k < kNumG + kSem ? g[k < kNumG + kSem ? k : 0] : 0.0f; };
+        sums([&](int q, int k) { s_grp[lane][q] = V4{at(k), at(k + 1), at(k + 2), at(k + 3)}; });
+        wave_lds_fence();
+        for (uint32_t u = lo; u < hi; ++u) {
+          sums([&](int q, int k) {
+            const V4 x = s_grp[u - base][q];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              if (k + c < kNumG + kSem) acc[k + c] += x[c];
+          });
+        }
+        wave_lds_fence();
       }
-      wave_lds_fence();
     }
     if (has) {
       const size_t slot = slot_of(a.pos_slot, a.pos_quads, rbeg + v.y, (int)(it.qi & ((1u << lgQ) - 1u)));
